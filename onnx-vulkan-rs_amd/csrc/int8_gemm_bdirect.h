@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
             }
         }
     }
-    if (EPI == EPI_SCALE_BIAS) gemm_emit_range(p, lane, fmn, fmx);
+    if (EPI == EPI_SCALE_BIAS) gemm_emit_range(p, lane, wave, W, fmn, fmx);
 }
 
 }  // namespace hipc
