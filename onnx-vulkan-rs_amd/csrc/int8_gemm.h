@@ -53,6 +53,7 @@ struct GemmArgs {
     int host_zp;                   // zero points given by value instead of by pointer
     int dyn_zp_value, const_zp_value;
     int I, J, K, K_pad;
+    int lda;        // MODE_MM: bytes between rows of A, K or more; a multiple of 16 where p_aligned is set (the bytes from K on are zeros, shifted)
     int p_aligned;  // MODE_MM: rows of A can be read with 128-bit loads
     int xcd_rows, xcd_cols;  // the 8 XCDs as a grid over the tiles (set by gemm_grid)
 
@@ -225,9 +226,17 @@ struct GemmRegs {
     uint4 p[N], q[N];
 };
 
-// ALIGNED (MODE_MM only): rows of A start on 16 bytes and K % 128 == 0, so A is read with
+// The last 128-k stage of an A whose rows are not whole stages long (lda % 128 != 0): a chunk that would begin past the
+// row's end is read from the row's last 16 bytes instead -- `tail_back` bytes back, the same for every chunk of a thread,
+// whose chunks all have the k column `kc`. What is read there meets zeros of the prepacked B, so only the sums over A's
+// row have to leave it out.
+__device__ __forceinline__ int gemm_tail_back(const GemmArgs &p, int kc) {
+    return max(0, (p.K_pad - kBK + kc * 16) - (p.lda - 16));
+}
+
+// ALIGNED (MODE_MM only): rows of A start on 16 bytes, so A is read with
 // unconditional 128-bit loads at base + 32-bit offset (no branch, which keeps the load counters
-// exact and two stages in flight; no per-stage address arithmetic).
+// exact and two stages in flight; the last stage of a ragged row: gemm_tail_back).
 // T is the tile edge: 128, or 64 when 128x128 tiles would leave most CUs idle or alone with one
 // workgroup (several small workgroups per CU then overlap each other's memory and LDS latency).
 template <int MODE, int EPI, bool ALIGNED, int T>
@@ -307,22 +316,23 @@ __global__ void __launch_bounds__(256) int8_gemm_kernel(const GemmArgs p) {
     for (int u = 0; u < kChunks; u++) {
         const int gi = i0 + prow_[u], gj = j0 + qrow_[u];
         p_off[u] = MODE == MODE_CONV ? qfrag_offset(gi, pkc_[u] * 16, p.K_pad)  // a stage of 128 k is 4 KB further on
-                                     : (uint32_t)min(gi, p.I - 1) * (uint32_t)p.K + kc_[u] * 16;
+                                     : (uint32_t)min(gi, p.I - 1) * (uint32_t)p.lda + kc_[u] * 16;
         q_off[u] = MODE == MODE_MM ? qfrag_offset(gj, qkc_[u] * 16, p.K_pad) : 0u;  // a stage of 128 k is 4 KB further on
     }
+    const int last_k0 = p.K_pad - kBK;
+    const uint32_t tail_back = MODE == MODE_MM && ALIGNED ? (uint32_t)gemm_tail_back(p, kc_[0]) : 0u;
     auto load_p = [&](int u, int k0) -> uint4 {
         if (MODE == MODE_CONV) {
             return *reinterpret_cast<const uint4 *>(p.P + (size_t)k0 * 32 + p_off[u]);
         } else if (ALIGNED) {
-            // K % 128 == 0: every chunk is inside the row. Rows past I are clamped, not zeroed:
-            // the rows of a product are independent and those outputs are never stored.
-            // (the sign flip of a u8 operand is applied when the chunk is stored to LDS, so the
-            // load has no consumer until then)
-            return *reinterpret_cast<const uint4 *>(p.P + k0 + p_off[u]);
+            // Rows past I are clamped, not zeroed: the rows of a product are independent and
+            // those outputs are never stored. (The sign flip of a u8 operand is applied when the
+            // chunk is stored to LDS, so the load has no consumer until then.)
+            return *reinterpret_cast<const uint4 *>(p.P + k0 + (p_off[u] - (k0 == last_k0 ? tail_back : 0u)));
         } else {
             const int gi = i0 + row_[u], gk = k0 + kc_[u] * 16;
             if (gi >= p.I || gk >= p.K) return make_uint4(0, 0, 0, 0);
-            const uint8_t *src = p.P + (size_t)gi * p.K + gk;
+            const uint8_t *src = p.P + (size_t)gi * p.lda + gk;
             uint32_t w[4] = {0, 0, 0, 0};
             for (int b = 0; b < 16; b++)
                 if (gk + b < p.K) w[b >> 2] |= (uint32_t)(src[b] ^ (flip & 0xff)) << (8 * (b & 3));
@@ -355,15 +365,16 @@ __global__ void __launch_bounds__(256) int8_gemm_kernel(const GemmArgs p) {
         for (int u = 0; u < kChunks; u++) r.q[u] = load_q(u, k0);
     };
     // `live` false (a stage past the end, only met when the stage count is odd) stores zeros,
-    // which add nothing to the product or to the operand sums.
-    auto store_regs = [&](const GemmRegs<kChunks> &r, int buf, bool live) {
+    // which add nothing to the product or to the operand sums; so does a chunk past A's row in the `last` stage.
+    auto store_regs = [&](const GemmRegs<kChunks> &r, int buf, bool live, bool last) {
         const uint32_t keep = live ? 0xffffffffu : 0u;
+        const uint32_t keep_p = live && !(last && tail_back) ? 0xffffffffu : 0u;
         const uint32_t late_flip = (MODE == MODE_MM && ALIGNED) ? flip : 0u;
 #pragma unroll
         for (int u = 0; u < kChunks; u++) {
             *reinterpret_cast<uint4 *>(lds_p + buf * T * kPitch + prow_[u] * kPitch + pkc_[u] * 16) =
-                make_uint4((r.p[u].x ^ late_flip) & keep, (r.p[u].y ^ late_flip) & keep, (r.p[u].z ^ late_flip) & keep,
-                           (r.p[u].w ^ late_flip) & keep);
+                make_uint4((r.p[u].x ^ late_flip) & keep_p, (r.p[u].y ^ late_flip) & keep_p, (r.p[u].z ^ late_flip) & keep_p,
+                           (r.p[u].w ^ late_flip) & keep_p);
             *reinterpret_cast<uint4 *>(lds_q + buf * T * kPitch + qrow_[u] * kPitch + qkc_[u] * 16) =
                 make_uint4(r.q[u].x & keep, r.q[u].y & keep, r.q[u].z & keep, r.q[u].w & keep);
         }
@@ -407,18 +418,18 @@ __global__ void __launch_bounds__(256) int8_gemm_kernel(const GemmArgs p) {
     GemmRegs<kChunks> r0, r1;
     load_regs(r0, 0);
     load_regs(r1, min(1, nk - 1));
-    store_regs(r0, 0, true);
+    store_regs(r0, 0, true, nk == 1);
     __syncthreads();
     // Two stages per trip and no exit in between, so the memory counters stay exact. With an
     // odd stage count the second half of the last trip multiplies a stage of zeros.
     for (int ks = 0; ks < nk; ks += 2) {
         load_regs(r0, min(ks + 2, nk - 1));
         compute(0);
-        store_regs(r1, 1, ks + 1 < nk);
+        store_regs(r1, 1, ks + 1 < nk, ks + 2 == nk);
         __syncthreads();
         load_regs(r1, min(ks + 3, nk - 1));
         compute(1);
-        store_regs(r0, 0, true);
+        store_regs(r0, 0, true, ks + 3 >= nk);
         __syncthreads();
     }
 
@@ -499,7 +510,7 @@ int gemm_launch(hipc_ctx *ctx, const GemmArgs &g, unsigned batch) {
                                      : gemm_launch_tile<MODE, EPI, ALIGNED, 128>(ctx, g, batch);
 }
 
-// ---- the small-problem variant (MODE_MM, aligned A) ---------------------------------------
+// ---- the small-problem variant (MODE_MM, 16-byte aligned rows of A) ---------------------------------------
 // A product of a few hundred 64x64 tiles. The LDS-staged kernel above is bound by LDS bandwidth
 // there: per 128-k stage a 64x64 tile stores 16 KB and its four 32x32 wavefronts read 32 KB, 384
 // clocks of LDS for 128 clocks of products. Here
@@ -537,7 +548,7 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
     const int ty = (xcd / p.xcd_cols) * rows_per + idx / cols_per, tx = (xcd % p.xcd_cols) * cols_per + idx % cols_per;
     if (idx >= rows_per * cols_per || ty >= tiles_y || tx >= tiles_x) return;
     const int i0 = ty * T, j0 = tx * T;
-    const int nk = p.K / kBK;
+    const int nk = p.K_pad / kBK;
 
     const int zd = (p.host_zp ? p.dyn_zp_value : zp_byte(p.dyn_zp, p.dyn_signed)) - p.dyn_shift;
     const int zc = (p.host_zp ? p.const_zp_value : zp_byte(p.const_zp, p.const_signed)) - p.const_shift;
@@ -548,9 +559,10 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
 #pragma unroll
     for (int u = 0; u < kCh; u++) {
         const int c = tid + 256 * u, row = c >> 3, kc = c & 7;
-        p_off[u] = (uint32_t)min(i0 + row, p.I - 1) * (uint32_t)p.K + kc * 16;  // rows past I: clamped, never stored
+        p_off[u] = (uint32_t)min(i0 + row, p.I - 1) * (uint32_t)p.lda + kc * 16;  // rows past I: clamped, never stored
         l_off[u] = row * kPitch + kc * 16;
     }
+    const uint32_t tail_back = (uint32_t)gemm_tail_back(p, tid & 7);
     // B: fragments j0 / 32 and j0 / 32 + 1 of this wavefront's product step; a step is 1 KB on, a stage 4 KB.
     // Wavefront w will finish fragment (rows w >> 1, columns w & 1) and numbers its operands and
     // accumulators from that one: acc[di][dj] is fragment ((w >> 1) ^ di, (w & 1) ^ dj), so its own
@@ -561,14 +573,15 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
     for (int f = 0; f < 2; f++)
         q_off[f] = qfrag_offset(min(j0 + (f ^ (wave & 1)) * 32, j_last - 31), wave * 32, p.K_pad) + lane * 16;
     const __amdgpu_buffer_rsrc_t rsrc_p = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(p.P), 0, (int)((uint32_t)p.I * (uint32_t)p.K), 0x00020000);
+        const_cast<uint8_t *>(p.P), 0, (int)((uint32_t)p.I * (uint32_t)p.lda), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(p.Q), 0, (int)((uint32_t)(j_last + 1) * (uint32_t)p.K_pad), 0x00020000);
 
     u32x4 ra[kSmallSets][kCh], rb[kSmallSets][kSteps][2];
     auto load_a = [&](int set, int stage) {
 #pragma unroll
-        for (int u = 0; u < kCh; u++) ra[set][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, p_off[u], min(stage, nk - 1) * kBK, 0);
+        for (int u = 0; u < kCh; u++)
+            ra[set][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, p_off[u] - (stage >= nk - 1 ? tail_back : 0u), min(stage, nk - 1) * kBK, 0);
     };
     auto load_b = [&](int set, int stage) {
 #pragma unroll
@@ -577,9 +590,10 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
             for (int f = 0; f < 2; f++)
                 rb[set][step][f] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_q, q_off[f] + step * 1024, min(stage, nk - 1) * kBK * 32, 0);
     };
-    // a stage past the end is stored as zeros: its products add nothing whatever B holds
-    auto store_a = [&](int set, int buf, bool live) {
-        const uint32_t keep = live ? 0xffffffffu : 0u;
+    // a stage past the end is stored as zeros: its products add nothing whatever B holds (and so is, where the sums over
+    // A's rows count, what the last stage read from the row's end: see gemm_tail_back)
+    auto store_a = [&](int set, int buf, int stage) {
+        const uint32_t keep = stage < nk && !(DYN && stage == nk - 1 && tail_back) ? 0xffffffffu : 0u;
 #pragma unroll
         for (int u = 0; u < kCh; u++)
             *reinterpret_cast<u32x4 *>(lds_a + buf * T * kPitch + l_off[u]) = (ra[set][u] ^ flip) & keep;
@@ -624,7 +638,7 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
 
 #pragma unroll
     for (int d = 0; d < kSmallSets; d++) load_a(d, d), load_b(d, d);
-    store_a(0, 0, true);
+    store_a(0, 0, 0);
     load_a(0, kSmallSets);
     __syncthreads();
     // Stage s: multiply it out of LDS buffer s & 1 with B set s % 4, refill that B set with stage
@@ -636,7 +650,7 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
         for (int d = 0; d < kSmallSets; d++) {
             compute(d & 1, d);
             load_b(d, s + d + kSmallSets);
-            store_a((d + 1) % kSmallSets, (d + 1) & 1, s + d + 1 < nk);
+            store_a((d + 1) % kSmallSets, (d + 1) & 1, s + d + 1);
             load_a((d + 1) % kSmallSets, s + d + 1 + kSmallSets);
             __syncthreads();
         }

@@ -1,5 +1,5 @@
 // The int8 matrix product for shapes with hundreds of tiles (MatMulInteger / QLinearMatMul, A with
-// whole 128-byte k stages and 16-byte aligned rows): the constant operand never touches LDS.
+// 16-byte aligned rows): the constant operand never touches LDS.
 //
 // The prepacked B is fragment-major (qfrag_offset): the 16 bytes a lane feeds the matrix core for a
 // 32-column x 32-k fragment lie at fragment base + 16 lane, so a wavefront reads a B fragment with ONE
@@ -68,16 +68,17 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
 #pragma unroll
     for (int u = 0; u < kCh; u++) {
         const int c = tid + 64 * W * u, row = c >> 3, kc = c & 7;
-        p_off[u] = (uint32_t)min(i0 + row, p.I - 1) * (uint32_t)p.K + kc * 16;   // rows past I: clamped, never stored
+        p_off[u] = (uint32_t)min(i0 + row, p.I - 1) * (uint32_t)p.lda + kc * 16;   // rows past I: clamped, never stored
         l_off[u] = row * kPitch + kc * 16;
     }
+    const uint32_t tail_back = (uint32_t)gemm_tail_back(p, tid & 7);
     // B: fragment j of this wavefront's 128 columns at k step g lies g KB behind the fragment column's start
     const int j_last = (p.J + kBN - 1) / kBN * kBN - 1;   // B is packed in whole 128-column tiles
     uint32_t q_off[FJ];
 #pragma unroll
     for (int j = 0; j < FJ; j++) q_off[j] = qfrag_offset(min(j0 + wn * FJ * 32 + j * 32, j_last - 31), 0, p.K_pad) + lane * 16;
     const __amdgpu_buffer_rsrc_t rsrc_p = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(p.P), 0, (int)((uint32_t)p.I * (uint32_t)p.K), 0x00020000);
+        const_cast<uint8_t *>(p.P), 0, (int)((uint32_t)p.I * (uint32_t)p.lda), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(p.Q), 0, (int)((uint32_t)(j_last + 1) * (uint32_t)p.K_pad), 0x00020000);
     const int nk = p.K_pad / kBK, nsteps = nk * 4;
@@ -86,11 +87,13 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
     u32x4 rb[4][FJ];        // B fragments of four consecutive k steps: a ring
     auto load_a = [&](int stage) {
 #pragma unroll
-        for (int u = 0; u < kCh; u++) ra[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, p_off[u], stage * kBK, 0);
+        for (int u = 0; u < kCh; u++)
+            ra[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, p_off[u] - (stage == nk - 1 ? tail_back : 0u), stage * kBK, 0);
     };
-    auto store_a = [&](int buf) {
+    auto store_a = [&](int buf, int stage) {   // (a chunk from the row's end is left out of the sums over the row: gemm_tail_back)
+        const uint32_t keep = DYN && stage >= nk - 1 && tail_back ? 0u : 0xffffffffu;
 #pragma unroll
-        for (int u = 0; u < kCh; u++) *reinterpret_cast<u32x4 *>(lds_p + buf * T * kPitch + l_off[u]) = ra[u] ^ flip;
+        for (int u = 0; u < kCh; u++) *reinterpret_cast<u32x4 *>(lds_p + buf * T * kPitch + l_off[u]) = DYN ? (ra[u] ^ flip) & keep : ra[u] ^ flip;
     };
     auto load_b = [&](int slot, int g) {   // a step past the end reloads the last one (cached, never multiplied)
         const int gc = min(g, nsteps - 1);
@@ -159,7 +162,7 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
         csum[j] = p.const_sum[gj];
         ecol[j] = gemm_emit_column<EPI>(p, gj);
     }
-    store_a(0);
+    store_a(0, 0);
     load_a(min(1, nk - 1));
     __syncthreads();
     read_a(0, 0, 0);
@@ -174,7 +177,7 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
         multiply(1, 1, FI, FJ, 0);
         read_a(1, cur, 3);           // the last read of this buffer
         load_b(1, g0 + 5);
-        store_a(cur ^ 1);            // stage ks + 1 (past the end: a copy of the last stage that nobody multiplies)
+        store_a(cur ^ 1, ks + 1);    // stage ks + 1 (past the end: a copy of the last stage that nobody multiplies)
         multiply(0, 2, FI, FJ, kCh);
         __syncthreads();
         read_a(0, cur ^ 1, 0);

@@ -81,6 +81,33 @@ __global__ void __launch_bounds__(256) int8_mfma_probe_kernel(int iterations, ui
     if (s == 0x7fffffff) sink[0] = s;  // keeps the loop alive; practically never true
 }
 
+// A [M, K] at any address and any K -> rows of `lda` bytes (K rounded up to 16), what is past K being `pad` (zero in the
+// shifted domain). One thread per output word: two aligned 32-bit reads and a byte shift (bytes one by one where the
+// second read would leave A). One pass over A is 1-3 us against the 10 to 350 us that reading such rows byte by byte
+// inside the product cost (1691 x 1728 x 6912 with K % 128 != 0: 378 us -> 47 us on the kernels for aligned rows).
+__global__ void __launch_bounds__(256)
+pad_rows_kernel(const uint8_t *__restrict__ A, uint32_t *__restrict__ out, long rows, int K, int lda, uint32_t pad) {
+    const long words = rows * (lda / 4), total = rows * K;
+    const int off = (int)(reinterpret_cast<uintptr_t>(A) & 3);
+    const uint32_t *base = reinterpret_cast<const uint32_t *>(A - off);
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < words; i += (long)gridDim.x * 256) {
+        const long row = i / (lda / 4);
+        const int k = (int)(i - row * (lda / 4)) * 4;
+        const long at = row * K + k, src = at + off;       // byte offset from A, from `base`
+        uint32_t v = 0;
+        if (at >= off && ((src >> 2) + 2) * 4 - off <= total) {   // both words inside A
+            const uint32_t lo = base[src >> 2], hi = base[(src >> 2) + 1];
+            v = (uint32_t)((((uint64_t)hi << 32) | lo) >> (8 * (int)(src & 3)));
+        } else {
+            for (int b = 0; b < 4; b++)
+                if (at + b < total) v |= (uint32_t)A[at + b] << (8 * b);
+        }
+        const int live = K - k;   // bytes of this word inside the row
+        const uint32_t mask = live >= 4 ? 0xffffffffu : live <= 0 ? 0u : (1u << (8 * live)) - 1u;
+        out[i] = (v & mask) | (pad & ~mask);
+    }
+}
+
 __global__ void __launch_bounds__(256)
 requantize_kernel(const int32_t *__restrict__ acc, const int32_t *__restrict__ bias, const float *__restrict__ ratio,
                   long n, long inner, long axis_len, int y_zp, int out_signed, uint8_t *__restrict__ out) {
@@ -155,8 +182,29 @@ int fill_common(hipc_ctx *ctx, const MmOperands &o, GemmArgs &g) {
     g.dyn_signed = o.a_dtype == HIPC_I8;
     g.const_signed = o.b_dtype == HIPC_I8;
     g.I = (int)o.M, g.J = (int)o.N, g.K = (int)o.K, g.K_pad = o.K_pad;
-    // the fast loader: whole 128-byte k stages, 16-byte aligned rows, 32-bit offsets
-    g.p_aligned = (o.K % kBK == 0) && aligned(o.A, 16) && o.M * o.K < (int64_t(1) << 32);
+    g.lda = g.K;
+    return HIPC_OK;
+}
+
+// The fast kernels read A in 16-byte chunks at 32-bit offsets. Rows that do not start on 16 bytes (an odd K, a view into
+// something larger) are first copied to scratch memory with a pitch that does; an A of 4 GiB or more, or one met for the
+// first time inside a capture (scratch memory cannot grow there), is read byte by byte as it is.
+int align_rows(hipc_ctx *ctx, GemmArgs &g) {
+    const int lda = (int)(ceil_div(g.K, 16) * 16);
+    g.p_aligned = (int64_t)g.I * lda < (int64_t(1) << 32);
+    if (!g.p_aligned || (g.lda % 16 == 0 && aligned(g.P, 16))) return HIPC_OK;
+    const size_t bytes = (size_t)g.I * lda;
+    if (ctx->capturing && ctx->scratch[2].bytes < bytes) {
+        g.p_aligned = 0;
+        return HIPC_OK;
+    }
+    void *rows = nullptr;
+    if (int rc = scratch_get(ctx, 2, bytes, &rows)) return rc;
+    const int64_t blocks = std::min<int64_t>(ceil_div((int64_t)(bytes / 4), 256), 16 * (int64_t)ctx->cu_count);
+    hipLaunchKernelGGL((pad_rows_kernel), dim3((unsigned)blocks), 256, 0, ctx->stream, g.P, static_cast<uint32_t *>(rows), (long)g.I, g.K, lda,
+                       g.dyn_shift ? 0x80808080u : 0u);
+    HIPC_LAUNCHED(ctx);
+    g.P = static_cast<const uint8_t *>(rows), g.lda = lda;
     return HIPC_OK;
 }
 
@@ -217,8 +265,9 @@ int launch_mm_small(hipc_ctx *ctx, const GemmArgs &g) {
     return zero_known ? launch_mm_small_dyn<EPI, false>(ctx, g) : launch_mm_small_dyn<EPI, true>(ctx, g);
 }
 template <int EPI>
-int launch_mm(hipc_ctx *ctx, const GemmArgs &g) {
+int launch_mm(hipc_ctx *ctx, GemmArgs g) {
     if (g.I == 0 || g.J == 0) return HIPC_OK;
+    if (int rc = align_rows(ctx, g)) return rc;
     if (const int big = big_tile_choice(ctx, g)) return launch_mm_big<EPI>(ctx, g, big);
     if (wants_small_tiles(ctx, g)) return launch_mm_small<EPI>(ctx, g);
     return g.p_aligned ? gemm_launch<MODE_MM, EPI, true>(ctx, g, 1) : gemm_launch<MODE_MM, EPI, false>(ctx, g, 1);

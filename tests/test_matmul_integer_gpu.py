@@ -275,3 +275,36 @@ def test_every_route_of_the_integer_product_can_be_forced(ctx, pkg, oracle, opti
     with ctx.options(**options):
         _mm_three_epilogues(ctx, pkg, oracle, m, k, n, np.uint8, np.int8, seed=71)
         _mm_three_epilogues(ctx, pkg, oracle, m, k, n, np.int8, np.uint8, seed=73)
+
+
+@pytest.mark.parametrize("route", [dict(HIPC_GEMM_BIG=1), dict(HIPC_GEMM_BIG=2), dict(HIPC_GEMM_BIG=0, HIPC_GEMM_SMALL=1),
+                                   dict(HIPC_GEMM_BIG=0, HIPC_GEMM_SMALL=0, HIPC_GEMM_TILE=64),
+                                   dict(HIPC_GEMM_BIG=0, HIPC_GEMM_SMALL=0, HIPC_GEMM_TILE=128)],
+                         ids=["tile256", "tile128", "k_split", "staged64", "staged128"])
+@pytest.mark.parametrize("shape", [(133, 16, 70), (70, 112, 140), (257, 400, 131), (129, 1424, 260), (66, 1001, 130), (131, 127, 64)],
+                         ids=lambda s: "M%d_K%d_N%d" % s)
+def test_rows_that_are_not_whole_stages(ctx, pkg, oracle, shape, route):
+    """K a multiple of 16 but not of a stage's 128 (the last stage reads the row's end), and K that is not (the rows are
+    copied to a pitch that is); zero points on both sides, so that the sums over A's rows count, and none."""
+    m, k, n = shape
+    a = rc.pseudo_plus1(m * k, 61).reshape(m, k)
+    for b, za, zb in ((rc.pseudo_plus1(k * n, 62).reshape(k, n), 200, 3), (rc.pseudo_plus1(k * n, 63).view(np.int8).reshape(k, n), 131, None)):
+        want = oracle.matmul_integer(a, b, za, zb or 0)
+        with ctx.options(**route):
+            assert np.array_equal(pkg.ops.matmul_integer(ctx, a, b, za, zb), want)
+
+
+@pytest.mark.parametrize("offset,k", [(4, 256), (3, 128), (1, 45), (2, 16)])
+def test_rows_at_any_address(ctx, pkg, oracle, offset, k):
+    """A inside a larger buffer, at an address that is not a multiple of 16 (or of 4)."""
+    m, n = 37, 75
+    a = rc.pseudo_plus1(m * k, 64).reshape(m, k)
+    b = rc.pseudo_plus1(k * n, 65).view(np.int8).reshape(k, n)
+    weight = pkg.ops.Int8Weight(ctx, b)
+    buf, y, z = ctx.alloc(m * k + offset), ctx.alloc(m * n * 4), ctx.upload(np.array([9, 5], np.uint8))
+    ctx.upload(a, buf, offset)
+    pkg.ops.matmul_integer_device(ctx, buf.at(offset), pkg.U8, weight, z.ptr, z.at(1), y, m)
+    assert np.array_equal(ctx.download(y, np.int32, (m, n)), oracle.matmul_integer(a, b, 9, 5))
+    weight.destroy()
+    for x in (buf, y, z):
+        x.free()
