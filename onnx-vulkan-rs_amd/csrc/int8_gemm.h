@@ -170,6 +170,12 @@ __device__ __forceinline__ EmitColumn gemm_emit_column(const GemmArgs &p, int gj
     }
     return e;
 }
+// One requantized output, still as a number
+__device__ __forceinline__ int gemm_requant(const GemmArgs &p, const EmitColumn &e, int v) {
+    const int q = (int)rintf(__fmul_rn((float)(v + e.qb), e.s)) + p.y_zp;
+    return p.out_signed ? min(max(q, -128), 127) : min(max(q, 0), 255);
+}
+
 template <int EPI>
 __device__ __forceinline__ void gemm_emit_mm(const GemmArgs &p, const EmitColumn &e, int gi, int gj, int v, float &fmn, float &fmx) {
     const size_t at = (size_t)gi * p.J + gj;
@@ -184,16 +190,35 @@ __device__ __forceinline__ void gemm_emit_mm(const GemmArgs &p, const EmitColumn
         fmn = fminf(fmn, o);
         fmx = fmaxf(fmx, o);
     } else {
-        const float t = __fmul_rn((float)(v + e.qb), e.s);
-        int q = (int)rintf(t) + p.y_zp;
-        if (p.out_signed) {
-            q = min(max(q, -128), 127);
-            static_cast<int8_t *>(p.Y)[at] = (int8_t)q;
-        } else {
-            q = min(max(q, 0), 255);
-            static_cast<uint8_t *>(p.Y)[at] = (uint8_t)q;
-        }
+        static_cast<uint8_t *>(p.Y)[at] = (uint8_t)gemm_requant(p, e, v);
     }
+}
+
+// Four requantized outputs of a lane, rows R .. R + 3 of its column, as the bytes of a word. `v`: the sums with
+// everything added (zero points, bias). q = rte(v * ratio) + y_zp is formed in float -- exact wherever it is inside the
+// output's range, and clamped outside it -- so that the conversion saturates and packs at once: six instructions per
+// output. A signed output is clamped 128 higher, as an unsigned one, and has its top bits turned afterwards.
+struct RequantBytes {
+    float ratio, zp;
+    uint32_t flip;
+};
+__device__ __forceinline__ uint32_t gemm_requant4(const RequantBytes &e, const int (&v)[4]) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) w = __builtin_amdgcn_cvt_pk_u8_f32(rintf(__fmul_rn((float)v[i], e.ratio)) + e.zp, i, w);
+    return w ^ e.flip;
+}
+// The same exchanged with the three other lanes of the quad (columns C .. C + 3, C a multiple of 4): the word that comes
+// back holds row R + (lane & 3), columns C .. C + 3. Two steps of a 4 x 4 byte transposition, each one cross-lane move
+// and one byte permutation.
+__device__ __forceinline__ uint32_t gemm_quad_row(uint32_t w) {
+    const int lane = threadIdx.x & 63;
+    // with the neighbouring column: even lanes keep rows 0, 2 of both, odd lanes rows 1, 3
+    const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xb1, 0xf, 0xf, true);   // quad_perm [1, 0, 3, 2]
+    w = (lane & 1) ? __builtin_amdgcn_perm(w, n1, 0x07030501u) : __builtin_amdgcn_perm(n1, w, 0x06020400u);
+    // with the column pair beside it: lanes 0, 1 keep the lower half, lanes 2, 3 the upper
+    const uint32_t n2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x4e, 0xf, 0xf, true);   // quad_perm [2, 3, 0, 1]
+    return (lane & 2) ? __builtin_amdgcn_perm(w, n2, 0x07060302u) : __builtin_amdgcn_perm(n2, w, 0x05040100u);
 }
 
 // Folds the min/max of the floats a workgroup of `waves` wavefronts emitted into the range slot; every thread of the
@@ -697,16 +722,25 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
             }
         }
     };
+    const bool words = EPI == EPI_REQUANT && ((p.J | (int)(reinterpret_cast<uintptr_t>(p.Y) & 3)) & 3) == 0;   // bytes leave four columns at a time
+    const RequantBytes bytes{my_emit.s, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
     read_group(0, 0);
 #pragma unroll
     for (int g = 0; g < 4; g++) {
         if (g + 1 < 4) read_group(g + 1, (g + 1) & 1);
+        int q[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int gi = i0 + ifr * 32 + g * 8 + kg * 4 + e;
             int v = acc[0][0][4 * g + e] + part[g & 1][e] + fixed;
             if (DYN) v -= zc * rs[g & 1][e];
-            if (gi < p.I && gj < p.J) gemm_emit_mm<EPI>(p, my_emit, gi, gj, v, fmn, fmx);
+            if (EPI == EPI_REQUANT && words) q[e] = v + my_emit.qb;
+            else if (gi < p.I && gj < p.J) gemm_emit_mm<EPI>(p, my_emit, gi, gj, v, fmn, fmx);
+        }
+        if (EPI == EPI_REQUANT && words) {
+            const uint32_t w = gemm_quad_row(gemm_requant4(bytes, q));
+            const int gi = i0 + ifr * 32 + g * 8 + kg * 4 + (lane & 3);
+            if (gi < p.I && gj < p.J) *reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(p.Y) + (size_t)gi * p.J + (gj & ~3)) = w;
         }
     }
     if (EPI == EPI_SCALE_BIAS) gemm_emit_range(p, lane, wave, 4, fmn, fmx);
@@ -784,37 +818,35 @@ __device__ __forceinline__ void conv_small_finish(const GemmArgs &p, i32x16 (&ac
     }
     const int ch = i0 + ifr * 32 + r32;
     const int fixed = p.K * zd * zc - zd * chan.csum + (EPI == EPI_REQUANT ? chan.qb : 0);
-    const int lo = p.out_signed ? -128 : 0, hi = p.out_signed ? 127 : 255;
     int out[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-        int v = acc[0][0][r] + part[0][r] + part[1][r] + part[2][r] + fixed;
-        if (DYN) v -= zc * qs[r];
-        if (EPI == EPI_REQUANT) v = min(max((int)rintf(__fmul_rn((float)v, chan.ratio)) + p.y_zp, lo), hi) & 0xff;
-        out[r] = v;
+        out[r] = acc[0][0][r] + part[0][r] + part[1][r] + part[2][r] + fixed;
+        if (DYN) out[r] -= zc * qs[r];
     }
     if (ch >= p.I) return;
     const size_t row = ((size_t)img * p.I + ch) * p.J;
     const bool wide = (p.J & 3) == 0 && (reinterpret_cast<uintptr_t>(p.Y) & (EPI == EPI_REQUANT ? 3 : 15)) == 0;
+    const RequantBytes bytes{chan.ratio, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
 #pragma unroll
     for (int g = 0; g < 4; g++) {
         const int pos = j0 + jf * 32 + g * 8 + kg * 4;   // four consecutive positions: out[4 g ..]
+        const int v[4] = {out[4 * g], out[4 * g + 1], out[4 * g + 2], out[4 * g + 3]};
+        const uint32_t word = EPI == EPI_REQUANT ? gemm_requant4(bytes, v) : 0u;
         if (wide && pos + 3 < p.J) {
             if (EPI == EPI_REQUANT) {
-                const uint32_t word = (uint32_t)out[4 * g] | (uint32_t)out[4 * g + 1] << 8 | (uint32_t)out[4 * g + 2] << 16 |
-                                      (uint32_t)out[4 * g + 3] << 24;
                 *reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(p.Y) + row + pos) = word;
             } else {
                 // written once and several times the operands: kept from displacing them in the caches
-                i32x4 quad = {out[4 * g], out[4 * g + 1], out[4 * g + 2], out[4 * g + 3]};
+                i32x4 quad = {v[0], v[1], v[2], v[3]};
                 __builtin_nontemporal_store(quad, reinterpret_cast<i32x4 *>(static_cast<int32_t *>(p.Y) + row + pos));
             }
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if (pos + e >= p.J) continue;
-                if (EPI == EPI_REQUANT) static_cast<uint8_t *>(p.Y)[row + pos + e] = (uint8_t)out[4 * g + e];
-                else static_cast<int32_t *>(p.Y)[row + pos + e] = out[4 * g + e];
+                if (EPI == EPI_REQUANT) static_cast<uint8_t *>(p.Y)[row + pos + e] = (uint8_t)(word >> (8 * e));
+                else static_cast<int32_t *>(p.Y)[row + pos + e] = v[e];
             }
         }
     }

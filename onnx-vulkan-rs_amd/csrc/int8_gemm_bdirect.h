@@ -197,6 +197,49 @@ __global__ void __launch_bounds__(64 * W) int8_gemm_bdirect_kernel(const GemmArg
 
     const int kzz = p.K * zd * zc;
     float fmn = 0.f, fmx = 0.f;
+    if (EPI == EPI_REQUANT && ((p.J | (int)(reinterpret_cast<uintptr_t>(p.Y) & 3)) & 3) == 0) {
+        // Bytes: a lane's outputs are one column, so four rows of four columns trade places between four lanes, the tile
+        // goes to LDS as words and leaves as whole rows, 16 (or 4) bytes per lane. (The A buffers are free: the last
+        // stage's reads ended before the barrier above. The pitch T + 32 puts the eight rows of a store instruction on
+        // different banks.) What counts is the arithmetic: all workgroups are in their epilogues at the same time.
+        constexpr int kOut = T + 32;
+        static_assert((size_t)T * kOut <= 2 * (size_t)T * kPitch, "the tile of bytes fits the A buffers");
+        const float zp = (float)p.y_zp + (p.out_signed ? 128.f : 0.f);
+        const uint32_t flip_out = p.out_signed ? 0x80808080u : 0u;
+#pragma unroll
+        for (int j = 0; j < FJ; j++) {
+            const int fixed = kzz - zd * csum[j] + ecol[j].qb;
+            const RequantBytes rq{ecol[j].s, zp, flip_out};
+#pragma unroll
+            for (int i = 0; i < FI; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int row = wm * FI * 32 + i * 32 + g * 8 + kg * 4;
+                    int v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = acc[i][j][4 * g + e] + fixed;
+                        if (DYN) v[e] -= zc * lds_sum[row + e];
+                    }
+                    *reinterpret_cast<uint32_t *>(lds_p + (row + (lane & 3)) * kOut + wn * FJ * 32 + j * 32 + (r32 & ~3)) = gemm_quad_row(gemm_requant4(rq, v));
+                }
+        }
+        __syncthreads();
+        uint8_t *Y = static_cast<uint8_t *>(p.Y) + (size_t)i0 * p.J + j0;
+        const int rows = min(T, p.I - i0), cols = min(T, p.J - j0);
+        if (((p.J | (int)(reinterpret_cast<uintptr_t>(p.Y) & 15)) & 15) == 0) {   // (cols is then a multiple of 16 too)
+            for (int c = tid; c < rows * (T / 16); c += 64 * W) {
+                const int row = c / (T / 16), col = c % (T / 16) * 16;
+                if (col < cols) *reinterpret_cast<uint4 *>(Y + (size_t)row * p.J + col) = *reinterpret_cast<const uint4 *>(lds_p + row * kOut + col);
+            }
+        } else {
+            for (int c = tid; c < rows * (T / 4); c += 64 * W) {
+                const int row = c / (T / 4), col = c % (T / 4) * 4;
+                if (col < cols) *reinterpret_cast<uint32_t *>(Y + (size_t)row * p.J + col) = *reinterpret_cast<const uint32_t *>(lds_p + row * kOut + col);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < FI; i++) {
 #pragma unroll

@@ -308,3 +308,19 @@ def test_rows_at_any_address(ctx, pkg, oracle, offset, k):
     weight.destroy()
     for x in (buf, y, z):
         x.free()
+
+
+@pytest.mark.parametrize("route", [dict(HIPC_GEMM_BIG=1), dict(HIPC_GEMM_BIG=2), dict(HIPC_GEMM_BIG=0, HIPC_GEMM_SMALL=1), {}],
+                         ids=["tile256", "tile128", "k_split", "chosen"])
+@pytest.mark.parametrize("n", [272, 260, 131, 7])
+@pytest.mark.parametrize("signed", [False, True])
+def test_requantized_bytes_leave_as_rows(ctx, pkg, oracle, n, signed, route):
+    """Output rows that are whole 16-byte pieces, whole words, neither; both output types; ratios that saturate."""
+    m, k = 145, 144
+    a = rc.pseudo_plus1(m * k, 71).reshape(m, k)
+    b = rc.pseudo_plus1(k * n, 72).view(np.int8).reshape(k, n)
+    b_scale = pkg.synth.uniform_f32(n, 73, 1e-4, 2e-2)
+    zp = -5 if signed else 130
+    want = oracle.qlinear_matmul(a, 0.02, 128, b, b_scale, 0, 0.05, zp, y_signed=signed)
+    with ctx.options(**route):
+        assert np.array_equal(pkg.ops.qlinear_matmul(ctx, a, 0.02, 128, b, b_scale, 0, 0.05, zp, y_signed=signed), want)
