@@ -103,6 +103,7 @@ const OptionName kOptions[] = {
     {"HIPC_GEMM_TILE", &Tuning::gemm_tile},
     {"HIPC_GEMM_BIG", &Tuning::gemm_big},
     {"HIPC_GEMM_SMALL", &Tuning::gemm_small},
+    {"HIPC_GEMM_SKINNY", &Tuning::gemm_skinny},
     {"HIPC_CONV_ROW", &Tuning::conv_row},
     {"HIPC_PREFILL_TILE", &Tuning::prefill_tile},
     {"HIPC_PREFILL_SPLIT", &Tuning::prefill_split},

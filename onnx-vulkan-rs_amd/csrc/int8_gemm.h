@@ -226,7 +226,9 @@ __device__ __forceinline__ uint32_t gemm_quad_row(uint32_t w) {
 // time, about 12 ns each: two per wavefront were 6 us of a 12.8 us product with 64 workgroups, 145 us of one with 756.
 // So the wavefronts meet in LDS first, and the slot is only asked to change when the workgroup has something larger than
 // a plain read of it shows (what is read may be old: the words only grow, so an old value costs an atomic, never an
-// update). Behind a ReLU the minimum is 0 and asks for nothing.
+// update). Read here and not when the workgroup begins: the workgroups of a launch that fits the chip end together, and
+// what the first ones left keeps the others from asking (23 x 1024 x 4096: 6.8 us against 7.6). Behind a ReLU the minimum
+// is 0 and asks for nothing.
 __device__ __forceinline__ void gemm_emit_range(const GemmArgs &p, int lane, int wave, int waves, float fmn, float fmx) {
     if (!p.range) return;
     __shared__ float part[2][16];

@@ -8,6 +8,7 @@
 
 #include "int8_gemm.h"
 #include "int8_gemm_bdirect.h"
+#include "int8_gemm_skinny.h"
 
 namespace hipc {
 
@@ -264,10 +265,50 @@ int launch_mm_small(hipc_ctx *ctx, const GemmArgs &g) {
     const bool zero_known = g.const_shift == 0 && (g.host_zp ? g.const_zp_value == 0 : g.const_zp == nullptr);
     return zero_known ? launch_mm_small_dyn<EPI, false>(ctx, g) : launch_mm_small_dyn<EPI, true>(ctx, g);
 }
+template <int EPI, bool DYN, int RB>
+int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {
+    const int steps = g.K_pad / 64;
+    const int64_t cols16 = ceil_div(g.J, 16);
+    // a workgroup per CU twice over before the columns are taken 32 at a time; four steps of k per wavefront, all in flight
+    // (23 x 1024 x 4096, kernel alone: 3.7 us with 4 wavefronts, 4.5 with 8, 6.3 with 16)
+    const int cb = cols16 > 2 * (int64_t)ctx->cu_count ? 2 : 1;
+    int waves = 4;
+    while (waves < 16 && waves * kSkinnyAhead < steps) waves *= 2;
+    static bool lds_allowed[2][kMaxDevices] = {};
+    const size_t lds = skinny_lds(waves, RB, cb);
+    const dim3 grid((unsigned)ceil_div(cols16, cb));
+    if (cb == 2) {
+        if (int rc = allow_dynamic_lds(ctx, int8_gemm_skinny_kernel<EPI, DYN, RB, 2>, skinny_lds(16, RB, 2), lds_allowed[1])) return rc;
+        hipLaunchKernelGGL((int8_gemm_skinny_kernel<EPI, DYN, RB, 2>), grid, 64 * waves, lds, ctx->stream, g);
+    } else {
+        if (int rc = allow_dynamic_lds(ctx, int8_gemm_skinny_kernel<EPI, DYN, RB, 1>, skinny_lds(16, RB, 1), lds_allowed[0])) return rc;
+        hipLaunchKernelGGL((int8_gemm_skinny_kernel<EPI, DYN, RB, 1>), grid, 64 * waves, lds, ctx->stream, g);
+    }
+    HIPC_LAUNCHED(ctx);
+    gemm_note_scalars(ctx, g, DYN);
+    return HIPC_OK;
+}
+// Up to 64 rows. Kernel alone, against the k-split 64x64 tiles (which are ahead of the LDS-staged ones there): 1 x 1024 x
+// 1024 6.4 -> 2.9 us, 1 x 4096 x 4096 11.4 -> 5.1, 23 x 1024 x 4096 6.6 -> 3.7, 23 x 4096 x 1024 11.1 -> 6.1, 60 x 1024 x
+// 4096 6.8 -> 4.9, 60 x 4096 x 1024 11.3 -> 10.2; against the LDS-staged tiles 64 x 256 x 4096 8.2 -> 4.9.
+template <int EPI>
+int launch_mm_skinny(hipc_ctx *ctx, const GemmArgs &g) {
+    const bool zero_known = g.const_shift == 0 && (g.host_zp ? g.const_zp_value == 0 : g.const_zp == nullptr);
+    if (g.I <= 16) return zero_known ? launch_mm_skinny_rb<EPI, false, 1>(ctx, g) : launch_mm_skinny_rb<EPI, true, 1>(ctx, g);
+    if (g.I <= 32) return zero_known ? launch_mm_skinny_rb<EPI, false, 2>(ctx, g) : launch_mm_skinny_rb<EPI, true, 2>(ctx, g);
+    return zero_known ? launch_mm_skinny_rb<EPI, false, 4>(ctx, g) : launch_mm_skinny_rb<EPI, true, 4>(ctx, g);
+}
+bool wants_skinny(hipc_ctx *ctx, const GemmArgs &g) {
+    if (!g.p_aligned || g.I > kSkinnyRows) return false;
+    if (ctx->tune.gemm_skinny >= 0) return ctx->tune.gemm_skinny != 0;
+    return ctx->tune.gemm_tile < 0 && ctx->tune.gemm_big < 0 && ctx->tune.gemm_small < 0;   // (an override of another kernel is one against this)
+}
+
 template <int EPI>
 int launch_mm(hipc_ctx *ctx, GemmArgs g) {
     if (g.I == 0 || g.J == 0) return HIPC_OK;
     if (int rc = align_rows(ctx, g)) return rc;
+    if (wants_skinny(ctx, g)) return launch_mm_skinny<EPI>(ctx, g);
     if (const int big = big_tile_choice(ctx, g)) return launch_mm_big<EPI>(ctx, g, big);
     if (wants_small_tiles(ctx, g)) return launch_mm_small<EPI>(ctx, g);
     return g.p_aligned ? gemm_launch<MODE_MM, EPI, true>(ctx, g, 1) : gemm_launch<MODE_MM, EPI, false>(ctx, g, 1);

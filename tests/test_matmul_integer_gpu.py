@@ -324,3 +324,27 @@ def test_requantized_bytes_leave_as_rows(ctx, pkg, oracle, n, signed, route):
     want = oracle.qlinear_matmul(a, 0.02, 128, b, b_scale, 0, 0.05, zp, y_signed=signed)
     with ctx.options(**route):
         assert np.array_equal(pkg.ops.qlinear_matmul(ctx, a, 0.02, 128, b, b_scale, 0, 0.05, zp, y_signed=signed), want)
+
+
+@pytest.mark.parametrize("b_dt", [np.int8, np.uint8])
+@pytest.mark.parametrize("shape", [(1, 16, 1), (16, 128, 16), (17, 1008, 100), (32, 2064, 33), (33, 320, 8200), (64, 4096, 132), (5, 8208, 48)],
+                         ids=lambda s: "M%d_K%d_N%d" % s)
+def test_few_rows(ctx, pkg, oracle, shape, b_dt):
+    """Up to 64 rows: 1, 2 and 4 blocks of 16 rows, one and two blocks of columns, 4 to 16 wavefronts along k with fewer
+    steps than they have in flight and more than one round of them; int32, the folded range, bytes."""
+    m, k, n = shape
+    a = rc.pseudo_plus1(m * k, 81).reshape(m, k)
+    b = rc.pseudo_plus1(k * n, 82).view(b_dt).reshape(k, n)
+    want = oracle.matmul_integer(a, b, 131, 17)
+    with ctx.options(HIPC_GEMM_SKINNY=1):
+        weight = pkg.ops.Int8Weight(ctx, b)
+        assert np.array_equal(pkg.ops.matmul_integer(ctx, a, b, 131, 17, weight=weight), want)
+        bias = pkg.synth.uniform_f32(n, 83, -0.5, 0.5)
+        got, folded = pkg.ops.matmul_integer_scale_bias(ctx, a, b, 131, 17, np.float32(0.002), bias, fold_range=True, weight=weight)
+        ref = oracle.rescale(want, np.float32(0.002), bias)
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+        assert folded[0] == np.float32(-min(ref.min(), 0)).view(np.uint32) & 0x7FFFFFFF and folded[1] == np.float32(max(ref.max(), 0)).view(np.uint32)
+        for signed in (False, True):
+            assert np.array_equal(pkg.ops.qlinear_matmul(ctx, a, 0.02, 131, b, 0.01, 17, 0.5, 3, y_signed=signed, weight=weight),
+                                  oracle.qlinear_matmul(a, 0.02, 131, b, 0.01, 17, 0.5, 3, y_signed=signed))
+        weight.destroy()
