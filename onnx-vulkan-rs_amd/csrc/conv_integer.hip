@@ -424,15 +424,9 @@ int hipc_qlinear_conv(hipc_ctx *ctx, const void *X, int x_dtype, float x_scale, 
         HIPC_REFUSE(ctx, n_w_scale > 1 && w_zp != 0, "QLinearConv: w per-channel zero point is not zero (asymmetric weights)");
         HIPC_REQUIRE(ctx, y_scale != 0.f, "QLinear: y_scale is zero");
         HIPC_REQUIRE(ctx, W, "QLinearConv: null weight");
-        // ratio[c] = x_scale * w_scale[c] / y_scale (interp.rs:4693); a per-tensor scale is
-        // broadcast to c_out so the bias stays per channel (interp.rs:4815-4823)
-        std::vector<float> ratio((size_t)g->c_out);
-        for (int64_t c = 0; c < g->c_out; c++) {
-            volatile float t = x_scale * w_scale[n_w_scale == 1 ? 0 : c];
-            ratio[(size_t)c] = t / y_scale;
-        }
+        // a per-tensor scale is broadcast to c_out so the bias stays per channel (interp.rs:4815-4823)
         const float *dratio = nullptr;
-        int rc = ratio_resident(ctx, W->ratios, ratio, &dratio);
+        int rc = ratio_resident(ctx, W->ratios, x_scale, w_scale, n_w_scale, y_scale, g->c_out, &dratio);
         if (rc != HIPC_OK) return rc;
         ConvEpilogue ep;
         ep.requant = 1;

@@ -493,14 +493,8 @@ int hipc_qlinear_matmul(hipc_ctx *ctx, const void *A, int a_dtype, float a_scale
         if (rc != HIPC_OK) return rc;
         if (M == 0) return HIPC_OK;
         HIPC_REQUIRE(ctx, A && Y, "QLinearMatMul: null operand");
-        // ratio[c] = a_scale * b_scale[c] / y_scale, f32, left to right (interp.rs:4693)
-        std::vector<float> ratio((size_t)n_b_scale);
-        for (int64_t c = 0; c < n_b_scale; c++) {
-            volatile float t = a_scale * b_scale[c];
-            ratio[(size_t)c] = t / y_scale;
-        }
         const float *dratio = nullptr;
-        rc = ratio_resident(ctx, B->ratios, ratio, &dratio);
+        rc = ratio_resident(ctx, B->ratios, a_scale, b_scale, n_b_scale, y_scale, n_b_scale, &dratio);
         if (rc != HIPC_OK) return rc;
         ga.host_zp = 1, ga.dyn_zp_value = a_zp, ga.const_zp_value = b_zp;
         ga.Y = Y;

@@ -268,11 +268,18 @@ def requantize(ctx: Context, acc, bias, ratio, inner, y_zp, out_signed=False):
     return out
 
 
+def _f32_vector(v):
+    """`v` as a contiguous float32 vector: itself where it is one."""
+    if type(v) is np.ndarray and v.dtype == np.float32 and v.ndim == 1 and v.flags.c_contiguous:
+        return v
+    return np.ascontiguousarray(np.atleast_1d(v), np.float32)
+
+
 def qlinear_matmul_device(ctx, A, a_dtype, a_scale, a_zp, weight: Int8Weight, b_scale, b_zp, y_scale, y_zp, y_dtype, Y, M):
-    bs = np.ascontiguousarray(np.atleast_1d(b_scale), np.float32)
+    bs = _f32_vector(b_scale)
     ctx._check(ctx.lib.hipc_qlinear_matmul(
-        ctx.handle, _ptr(A), a_dtype, float(a_scale), int(a_zp), weight.handle, bs.ctypes.data_as(C.POINTER(C.c_float)),
-        bs.size, int(b_zp), float(y_scale), int(y_zp), y_dtype, _ptr(Y), M))
+        ctx.handle, _ptr(A), a_dtype, float(a_scale), int(a_zp), weight.handle, bs, bs.size, int(b_zp), float(y_scale),
+        int(y_zp), y_dtype, _ptr(Y), M))
 
 
 def qlinear_matmul(ctx: Context, A, a_scale, a_zp, B, b_scale, b_zp, y_scale, y_zp, y_signed=False,
@@ -352,11 +359,10 @@ def conv_integer(ctx: Context, X, W, x_zp, w_zp, geom: ConvGeom, weight: ConvWei
 
 def qlinear_conv_device(ctx, X, x_dtype, x_scale, x_zp, weight: ConvWeight, w_scale: np.ndarray, w_zp, y_scale, y_zp,
                         y_dtype, bias, geom: ConvGeom, Y):
-    ws = np.ascontiguousarray(np.atleast_1d(w_scale), np.float32)
+    ws = _f32_vector(w_scale)
     ctx._check(ctx.lib.hipc_qlinear_conv(
-        ctx.handle, _ptr(X), x_dtype, float(x_scale), int(x_zp), weight.handle,
-        ws.ctypes.data_as(C.POINTER(C.c_float)), ws.size, int(w_zp), float(y_scale), int(y_zp), y_dtype, _ptr(bias),
-        C.byref(geom), _ptr(Y)))
+        ctx.handle, _ptr(X), x_dtype, float(x_scale), int(x_zp), weight.handle, ws, ws.size, int(w_zp), float(y_scale),
+        int(y_zp), y_dtype, _ptr(bias), geom, _ptr(Y)))
 
 
 def qlinear_conv(ctx: Context, X, x_scale, x_zp, W, w_scale, w_zp, y_scale, y_zp, bias, geom: ConvGeom,

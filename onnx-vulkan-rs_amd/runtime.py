@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes as C
+import importlib.util
 import os
 
 import numpy as np
@@ -134,14 +135,14 @@ SIGNATURES = {
 
 def source_build_id():
     """The build id of the sources in this tree, as csrc/Makefile computes it: sha256 over the sorted
-    ``*.hip`` and ``*.h`` of csrc/, the public header and the Makefile (first 16 hex digits).
+    ``*.hip`` and ``*.h`` of csrc/, fastcall.cpp, the public header and the Makefile (first 16 hex digits).
     None when the sources are not there (a library deployed on its own)."""
     import glob
     import hashlib
     csrc = os.path.join(_HERE, "csrc")
     names = sorted(os.path.basename(f) for f in glob.glob(os.path.join(csrc, "*.hip")) + glob.glob(os.path.join(csrc, "*.h")))
-    files = [os.path.join(csrc, n) for n in names] + [os.path.join(_HERE, "..", "include", "hipcompute.h"),
-                                                      os.path.join(csrc, "Makefile")]
+    files = [os.path.join(csrc, n) for n in names] + [os.path.join(csrc, "fastcall.cpp"),
+                                                      os.path.join(_HERE, "..", "include", "hipcompute.h"), os.path.join(csrc, "Makefile")]
     if not names or not all(os.path.exists(f) for f in files):
         return None
     h = hashlib.sha256()
@@ -169,8 +170,27 @@ def load_library():
         if want is not None and built != want:
             raise HipComputeError(3, f"{path} is stale: built from sources with id {built}, the tree has {want}; "
                                      f"rebuild it (make -C onnx-vulkan-rs_amd/csrc)")
+        _bind_fast(lib, built)
         _lib = lib
     return _lib
+
+
+def _bind_fast(lib, build_id: str):
+    """Puts the native entry points (csrc/fastcall.cpp) in the place of the ctypes functions that only enqueue. The
+    module belongs to this build of the library, like the library to the sources."""
+    path = os.path.join(_HERE, "_fastcall.so")
+    if not os.path.exists(path):
+        raise HipComputeError(3, f"{path} is missing: build it with __graft_entry__.build() (make -C onnx-vulkan-rs_amd/csrc)")
+    spec = importlib.util.spec_from_file_location("onnx_vulkan_rs_amd._fastcall", path)
+    fast = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(fast)
+    if fast.build_id != build_id:
+        raise HipComputeError(3, f"{path} is stale: built with id {fast.build_id}, the library has {build_id}; rebuild both")
+    for name in SIGNATURES:
+        fn = getattr(lib, name)
+        call = fast.bind(name, C.cast(fn, _vp).value, fn)
+        if call is not None:
+            setattr(lib, name, call)
 
 
 def hipc_dtype(dt) -> int:

@@ -29,11 +29,9 @@ int scratch_get(hipc_ctx *ctx, int slot, size_t bytes, void **out) {
     *out = s.ptr;
     return HIPC_OK;
 }
-int ratio_resident(hipc_ctx *, RatioCache &cache, const std::vector<float> &ratio, const float **out) {
+int ratio_resident(hipc_ctx *, RatioCache &cache, float, const float *, int64_t, float, int64_t count, const float **out) {
     if (cache.dev) gpu_model::release(cache.dev);
-    cache.dev = static_cast<float *>(gpu_model::alloc(ratio.size() * sizeof(float)));
-    std::memcpy(cache.dev, ratio.data(), ratio.size() * sizeof(float));
-    cache.host = ratio;
+    cache.dev = static_cast<float *>(gpu_model::alloc((size_t)count * sizeof(float)));
     *out = cache.dev;
     return HIPC_OK;
 }
