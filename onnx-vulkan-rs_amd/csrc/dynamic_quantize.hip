@@ -10,9 +10,19 @@
 // workgroups arrive in. The reference replaces `/` by a double-single reciprocal
 // because Vulkan's OpFDiv may be 2.5 ULP off; here `__fdiv_rn` is the IEEE
 // division, so the operator's definition is evaluated as written.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "internal.h"
 
 namespace hipc {
+
+// up to how many values dql_small_kernel takes: where its repeated reads (of a GELU: evaluations) cost what a second launch
+// does (feed-forward block of 32 tokens of 1024: 26.0 -> 23.4 us, of 60: 28.7 -> 29.5; of 4 tokens through a GELU of 4 x
+// 4096: 25.0 -> 19.1, of 8: 25.0 -> 24.4)
+constexpr int64_t kSmallPlain = 40960, kSmallGelu = 16384;
+
 
 // Range partials of hipc_dynamic_quantize_linear_static: {bits(-min), bits(max)} per workgroup of
 // the first pass, kParamPartsMax pairs = 16 KiB, part of the library's device image. In host code
@@ -28,80 +38,117 @@ int dql_static_init(hipc_ctx *ctx) {
     return HIPC_OK;
 }
 
+// Division by a value that is the same for every element (a quantizer's scale, GELU's divisor), correctly rounded, in five
+// instructions instead of the ten of a general IEEE division: q = v * rc with rc = 1 / d rounded to nearest is within 1.5 ulp,
+// and each correction adds the exactly formed remainder times rc. After the first one q is within just over half an ulp; the
+// second one then rounds what the true quotient rounds to: its error is below b 2^-26 ulp for a divisor mantissa b < 2,
+// while a quotient is never closer than 2^-24 / b ulp to a midpoint (Markstein's theorem). No remainder may be lost below
+// the smallest number and no product may overflow: the callers see to that.
+__device__ __forceinline__ float div_by(float v, float d, float rc) {
+    float q = v * rc;
+    q = fmaf(fmaf(-q, d, v), rc, q);
+    return fmaf(fmaf(-q, d, v), rc, q);
+}
+
 // What the quantizer reads: x itself, or DecomposedGelu(x), the exact GELU written out as
-// Div -> Erf -> Add -> Mul -> Mul and fused by the reference (rewrite.rs:683-735). Every step rounds
-// on its own, as the five kernels it replaces do (shaders/elementwise.rs:71-118): this file is
+// Div -> Erf -> Add -> Mul -> Mul and fused by the reference (rewrite.rs:683-735). Every one of the five rounds
+// on its own, as the kernels it replaces do (shaders/elementwise.rs:71-118): this file is
 // compiled with floating-point contraction off, so the fused quantizer and the plain GELU kernel
 // below evaluate bit for bit the same function.
+enum { GELU_OFF = 0, GELU_SQRT2 = 1, GELU_ANY = 2 };   // GELU_SQRT2: the divisor is sqrt(2) as a float, which exported graphs have
 struct GeluParams {
-    int on;             // 0: the identity
+    int on;             // one of the above (the kernels are instantiated on it)
     float divisor, offset, factor;
     int factor_first;   // x * ((erf + offset) * factor) instead of (x * (erf + offset)) * factor
 };
 
-__device__ __forceinline__ float erf_approx(float x) {  // shaders/elementwise.rs:71-80 (Abramowitz-Stegun 7.1.26)
-    const float s = x > 0.f ? 1.f : (x < 0.f ? -1.f : 0.f);
+// shaders/elementwise.rs:71-80 (Abramowitz-Stegun 7.1.26); |x| <= 32. The passes over a GELU are bound by these
+// instructions (16 M values: 21 us a pass at 40 of them, for 65 MB), so:
+//   * 1 / (1 + p a), an argument in [1, 12]: the hardware's estimate and one correction, which for every one of the 2^23
+//     mantissas gives the correctly rounded reciprocal;
+//   * exp(-a^2) as 2^h times (1 + r ln 2), h + r being -a^2 log2(e) to 48 bits: no range reduction, since the hardware's
+//     exponential takes the whole range and nothing here overflows.
+__device__ __forceinline__ float erf_approx(float x) {
     const float a = fabsf(x);
-    const float t = 1.f / (1.f + 0.3275911f * a);
-    const float poly = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-    return s * (1.f - poly * expf(-a * a));
+    const float y = fmaf(0.3275911f, a, 1.f);
+    const float r0 = __builtin_amdgcn_rcpf(y);
+    const float t = fmaf(fmaf(-y, r0, 1.f), r0, r0);
+    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
+    constexpr float log2e = 1.44269502f, ln2 = 0.693147181f;
+    const float s = -(a * a), h = s * log2e, r = fmaf(s, log2e, -h);
+    const float e2 = __builtin_amdgcn_exp2f(h), e = fmaf(e2, r * ln2, e2);
+    return copysignf(fmaf(-poly, e, 1.f), x);   // (for x = 0 the caller multiplies by 0)
 }
 
+// Past 32 the error function has long been 1 (from 10.2 on): clamping there keeps infinities out of the quotient and the square.
+template <int GELU>
 __device__ __forceinline__ float gelu_load(float v, const GeluParams &g) {
-    if (!g.on) return v;
-    const float e = erf_approx(v / g.divisor) + g.offset;
+    if (GELU == GELU_OFF) return v;
+    float x;
+    if (GELU == GELU_SQRT2) {
+        // div_by with a single correction: for this divisor it gives the IEEE quotient for every one of the 2^23 mantissas
+        constexpr float d = 1.41421356f, rc = 1.f / d;
+        const float c = __builtin_amdgcn_fmed3f(v, -64.f, 64.f), q = c * rc;
+        x = fmaf(fmaf(-q, d, c), rc, q);
+    } else {
+        x = fminf(fmaxf(v / g.divisor, -32.f), 32.f);
+    }
+    const float e = erf_approx(x) + g.offset;
     return g.factor_first ? v * (e * g.factor) : (v * e) * g.factor;
 }
+template <int GELU>
+__device__ __forceinline__ float4 gelu_load4(float4 v, const GeluParams &g) {
+    return make_float4(gelu_load<GELU>(v.x, g), gelu_load<GELU>(v.y, g), gelu_load<GELU>(v.z, g), gelu_load<GELU>(v.w, g));
+}
 
+template <int GELU>
 __global__ void __launch_bounds__(256)
 decomposed_gelu_kernel(const float *__restrict__ x, long n, GeluParams g, float *__restrict__ y) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) y[i] = gelu_load(x[i], g);
+    if (i < n) y[i] = gelu_load<GELU>(x[i], g);
 }
 
 __global__ void dql_clear_range_kernel(uint32_t *range) {
     if (threadIdx.x < 2) range[threadIdx.x] = 0u;
 }
 
-__global__ void __launch_bounds__(256)
-dql_range_kernel(const float *__restrict__ x, long n, uint32_t *__restrict__ range, int vec_ok, int per_block, GeluParams g) {
-    float mn = 0.f, mx = 0.f;
-    auto L = [&](float4 v) { return g.on ? make_float4(gelu_load(v.x, g), gelu_load(v.y, g), gelu_load(v.z, g), gelu_load(v.w, g)) : v; };
-    const long tid = (long)blockIdx.x * 256 + threadIdx.x;
-    const long nthreads = (long)gridDim.x * 256;
+// min and max of zero and `n` values at x, taken by `nthreads` threads of which this one is `tid`
+template <int GELU>
+__device__ __forceinline__ void dql_scan(const float *__restrict__ x, long n, long tid, long nthreads, int vec_ok, const GeluParams &g, float &mn, float &mx) {
+    mn = 0.f, mx = 0.f;
+    auto take = [&](float4 v) {
+        v = gelu_load4<GELU>(v, g);
+        mn = fminf(mn, fminf(fminf(v.x, v.y), fminf(v.z, v.w)));
+        mx = fmaxf(mx, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+    };
+    long i = tid;
     if (vec_ok) {
         const long n4 = n >> 2;
         const float4 *x4 = reinterpret_cast<const float4 *>(x);
-        long i = tid;
         for (; i + 3 * nthreads < n4; i += 4 * nthreads) {  // four independent loads in flight
-            const float4 a = L(x4[i]), b = L(x4[i + nthreads]), c = L(x4[i + 2 * nthreads]), d = L(x4[i + 3 * nthreads]);
-            mn = fminf(mn, fminf(fminf(fminf(a.x, a.y), fminf(a.z, a.w)), fminf(fminf(b.x, b.y), fminf(b.z, b.w))));
-            mn = fminf(mn, fminf(fminf(fminf(c.x, c.y), fminf(c.z, c.w)), fminf(fminf(d.x, d.y), fminf(d.z, d.w))));
-            mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(a.x, a.y), fmaxf(a.z, a.w)), fmaxf(fmaxf(b.x, b.y), fmaxf(b.z, b.w))));
-            mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(c.x, c.y), fmaxf(c.z, c.w)), fmaxf(fmaxf(d.x, d.y), fmaxf(d.z, d.w))));
+            const float4 a = x4[i], b = x4[i + nthreads], c = x4[i + 2 * nthreads], d = x4[i + 3 * nthreads];
+            take(a), take(b), take(c), take(d);
         }
-        for (; i < n4; i += nthreads) {
-            const float4 v = L(x4[i]);
-            mn = fminf(mn, fminf(fminf(v.x, v.y), fminf(v.z, v.w)));
-            mx = fmaxf(mx, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
-        }
-        for (long i = (n4 << 2) + tid; i < n; i += nthreads) {
-            const float v = gelu_load(x[i], g);
-            mn = fminf(mn, v);
-            mx = fmaxf(mx, v);
-        }
-    } else {
-        for (long i = tid; i < n; i += nthreads) {
-            const float v = gelu_load(x[i], g);
-            mn = fminf(mn, v);
-            mx = fmaxf(mx, v);
-        }
+        for (; i < n4; i += nthreads) take(x4[i]);
+        i = (n4 << 2) + tid;
+    }
+    for (; i < n; i += nthreads) {
+        const float v = gelu_load<GELU>(x[i], g);
+        mn = fminf(mn, v);
+        mx = fmaxf(mx, v);
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         mn = fminf(mn, __shfl_xor(mn, off, 64));
         mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     }
+}
+
+template <int GELU>
+__global__ void __launch_bounds__(256)
+dql_range_kernel(const float *__restrict__ x, long n, uint32_t *__restrict__ range, int vec_ok, int per_block, GeluParams g) {
+    float mn, mx;
+    dql_scan<GELU>(x, n, (long)blockIdx.x * 256 + threadIdx.x, (long)gridDim.x * 256, vec_ok, g, mn, mx);
     __shared__ float smn[4], smx[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) smn[wave] = mn, smx[wave] = mx;
@@ -129,55 +176,132 @@ __device__ __forceinline__ void dql_params(const uint32_t *range, float &scale, 
     zp = rintf(fminf(fmaxf(__fdiv_rn(neg_min, scale), 0.f), 255.f));
 }
 
-__device__ __forceinline__ uint32_t dql_one(float v, float scale, float zp) {
-    const float q = __fadd_rn(rintf(__fdiv_rn(v, scale)), zp);
-    return (uint32_t)fminf(fmaxf(q, 0.f), 255.f);
+// The codes of four values: sat(rte(v / scale) + zp), packed. `rcp` is 1 / scale where div_by may be used -- a scale within
+// 2^-100 .. 2^100, so that |v| <= 255 scale and the remainders of every quotient that does not round to 0 stay in range --
+// and 0 where it may not.
+template <bool FAST>
+__device__ __forceinline__ uint32_t dql_four_by(float4 v, float scale, float rcp, float zp) {
+    const float in[4] = {v.x, v.y, v.z, v.w};
+    uint32_t w = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float q = FAST ? div_by(in[j], scale, rcp) : __fdiv_rn(in[j], scale);
+        w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(__fadd_rn(rintf(q), zp), 0.f, 255.f), j, w);
+    }
+    return w;
+}
+__device__ __forceinline__ uint32_t dql_four(float4 v, float scale, float rcp, float zp) {
+    return rcp != 0.f ? dql_four_by<true>(v, scale, rcp, zp) : dql_four_by<false>(v, scale, rcp, zp);
+}
+__device__ __forceinline__ float dql_rcp(float scale) { return scale >= 0x1p-100f && scale <= 0x1p100f ? __fdiv_rn(1.f, scale) : 0.f; }
+
+// 256 threads join `nparts` {bits(-min), bits(max)} pairs; the maximum of non-negative floats is the maximum of their
+// bit patterns
+__device__ __forceinline__ void dql_join(const uint32_t *__restrict__ pairs, int nparts, uint32_t (&joined)[2]) {
+    __shared__ uint32_t wave_max[4][2];
+    uint32_t a = 0, b = 0;
+    for (int i = threadIdx.x; i < nparts; i += 256) a = max(a, pairs[2 * i]), b = max(b, pairs[2 * i + 1]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        a = max(a, (uint32_t)__shfl_xor((int)a, off, 64));
+        b = max(b, (uint32_t)__shfl_xor((int)b, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6][0] = a, wave_max[threadIdx.x >> 6][1] = b;
+    __syncthreads();
+    joined[0] = max(max(wave_max[0][0], wave_max[1][0]), max(wave_max[2][0], wave_max[3][0]));
+    joined[1] = max(max(wave_max[0][1], wave_max[1][1]), max(wave_max[2][1], wave_max[3][1]));
 }
 
-// four values per thread, packed into one 32-bit store where the output allows it
+// V runs of four values per thread, 1024 values apart, each packed into one 32-bit store where the output allows it; the
+// values are asked for before the range pairs are joined
+template <int GELU, int V>
 __global__ void __launch_bounds__(256)
 dql_quantize_kernel(const float *__restrict__ x, long n, const uint32_t *__restrict__ range, int nparts,
                     uint8_t *__restrict__ y, float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, int vec_ok,
                     GeluParams g) {
+    const long first = (long)blockIdx.x * (256 * V) + threadIdx.x;   // this thread's first run, counted in runs
+    float4 v[V];
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+        const long run = first + 256 * u, base = run << 2;
+        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (vec_ok && base + 4 <= n) {
+            v[u] = reinterpret_cast<const float4 *>(x)[run];
+        } else {
+            if (base < n) v[u].x = x[base];
+            if (base + 1 < n) v[u].y = x[base + 1];
+            if (base + 2 < n) v[u].z = x[base + 2];
+            if (base + 3 < n) v[u].w = x[base + 3];
+        }
+    }
     float scale, zp;
     if (nparts > 0) {
-        // range holds nparts pairs: every workgroup joins them itself; the maximum of
-        // non-negative floats is the maximum of their bit patterns
-        __shared__ uint32_t joined[2];
-        __shared__ uint32_t wave_max[4][2];
-        uint32_t a = 0, b = 0;
-        for (int i = threadIdx.x; i < nparts; i += 256) a = max(a, range[2 * i]), b = max(b, range[2 * i + 1]);
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            a = max(a, (uint32_t)__shfl_xor((int)a, off, 64));
-            b = max(b, (uint32_t)__shfl_xor((int)b, off, 64));
-        }
-        if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6][0] = a, wave_max[threadIdx.x >> 6][1] = b;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            joined[0] = max(max(wave_max[0][0], wave_max[1][0]), max(wave_max[2][0], wave_max[3][0]));
-            joined[1] = max(max(wave_max[0][1], wave_max[1][1]), max(wave_max[2][1], wave_max[3][1]));
-        }
-        __syncthreads();
+        uint32_t joined[2];
+        dql_join(range, nparts, joined);
         dql_params(joined, scale, zp);
     } else {
         dql_params(range, scale, zp);
     }
-    const long i4 = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i4 == 0) {
+    const float rcp = dql_rcp(scale);
+    if (first == 0) {
         *scale_out = scale;
         *zp_out = (uint8_t)zp;
     }
-    const long base = i4 << 2;
-    if (base >= n) return;
-    if (vec_ok && base + 4 <= n) {
-        float4 v = reinterpret_cast<const float4 *>(x)[i4];
-        if (g.on) v = make_float4(gelu_load(v.x, g), gelu_load(v.y, g), gelu_load(v.z, g), gelu_load(v.w, g));
-        const uint32_t packed = dql_one(v.x, scale, zp) | dql_one(v.y, scale, zp) << 8 |
-                                dql_one(v.z, scale, zp) << 16 | dql_one(v.w, scale, zp) << 24;
-        reinterpret_cast<uint32_t *>(y)[i4] = packed;
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+        const long run = first + 256 * u, base = run << 2;
+        const uint32_t w = dql_four(gelu_load4<GELU>(v[u], g), scale, rcp, zp);
+        if (vec_ok && base + 4 <= n) {
+            reinterpret_cast<uint32_t *>(y)[run] = w;
+        } else {
+            for (int j = 0; j < 4; j++)
+                if (base + j < n) y[base + j] = (uint8_t)(w >> (8 * j));
+        }
+    }
+}
+
+// Few values: one launch instead of two. Every workgroup takes the range of all of them and quantizes its own 4096; what
+// that reads again comes from the caches and costs less than the second launch, whose 1.6 us (2.2 us of the host's time)
+// nothing hides.
+template <int GELU>
+__global__ void __launch_bounds__(1024)
+dql_small_kernel(const float *__restrict__ x, long n, uint8_t *__restrict__ y, float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, GeluParams g) {
+    const long run = (long)blockIdx.x * 1024 + threadIdx.x, base = run << 2;
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (base + 4 <= n) {
+        own = reinterpret_cast<const float4 *>(x)[run];
     } else {
-        for (long i = base; i < n && i < base + 4; i++) y[i] = (uint8_t)dql_one(gelu_load(x[i], g), scale, zp);
+        if (base < n) own.x = x[base];
+        if (base + 1 < n) own.y = x[base + 1];
+        if (base + 2 < n) own.z = x[base + 2];
+    }
+    own = gelu_load4<GELU>(own, g);
+    float mn, mx;
+    if (gridDim.x == 1) {
+        mn = fminf(0.f, fminf(fminf(own.x, own.y), fminf(own.z, own.w))), mx = fmaxf(0.f, fmaxf(fmaxf(own.x, own.y), fmaxf(own.z, own.w)));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            mn = fminf(mn, __shfl_xor(mn, off, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        }
+    } else {
+        dql_scan<GELU>(x, n, threadIdx.x, 1024, 1, g, mn, mx);
+    }
+    __shared__ float smn[16], smx[16];
+    if ((threadIdx.x & 63) == 0) smn[threadIdx.x >> 6] = mn, smx[threadIdx.x >> 6] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; w++) mn = fminf(mn, smn[w]), mx = fmaxf(mx, smx[w]);
+    const uint32_t joined[2] = {__float_as_uint(-mn) & 0x7fffffffu, __float_as_uint(mx) & 0x7fffffffu};   // (-0.0 counts as 0)
+    float scale, zp;
+    dql_params(joined, scale, zp);
+    if (run == 0) *scale_out = scale, *zp_out = (uint8_t)zp;
+    const uint32_t w = dql_four(own, scale, dql_rcp(scale), zp);
+    if (base + 4 <= n) {
+        reinterpret_cast<uint32_t *>(y)[run] = w;
+    } else {
+        for (int j = 0; j < 3; j++)
+            if (base + j < n) y[base + j] = (uint8_t)(w >> (8 * j));
     }
 }
 
@@ -213,34 +337,52 @@ int dql_launch(hipc_ctx *ctx, const void *X, int64_t n, void *Y, void *scale_out
     HIPC_REQUIRE(ctx, !(range_ready && !range), "DynamicQuantizeLinear: range_ready needs a caller-owned range slot");
     const int vec_ok = aligned(X, 16) && aligned(Y, 4);
     const float *x = static_cast<const float *>(X);
-    int nparts = 0;
-    if (!range_ready && !range) {
-        // no slot of the caller's to fill: per-workgroup pairs in the context's block, joined by the
-        // second pass -- no clearing launch and no atomics
-        slot = parts ? parts : reinterpret_cast<uint32_t *>(static_cast<char *>(ctx->params) + kParamParts);
-        nparts = (int)std::min<long>(std::max<long>(ceil_div(n, 256 * 16), 1), kParamPartsMax);
-        hipLaunchKernelGGL((dql_range_kernel), (unsigned)nparts, 256, 0, ctx->stream, x, (long)n, slot, vec_ok, 1, gelu);
+    auto launch = [&](auto gelu_kind) -> int {
+        constexpr int GELU = decltype(gelu_kind)::value;
+        if (!range_ready && !range && vec_ok && n <= (GELU ? kSmallGelu : kSmallPlain)) {
+            hipLaunchKernelGGL((dql_small_kernel<GELU>), (unsigned)ceil_div(n, 4096), 1024, 0, ctx->stream, x, (long)n, static_cast<uint8_t *>(Y),
+                               static_cast<float *>(scale_out), static_cast<uint8_t *>(zp_out), gelu);
+            HIPC_LAUNCHED(ctx);
+            return HIPC_OK;
+        }
+        int nparts = 0;
+        if (!range_ready && !range) {
+            // no slot of the caller's to fill: per-workgroup pairs in the context's block, joined by the
+            // second pass -- no clearing launch and no atomics
+            slot = parts ? parts : reinterpret_cast<uint32_t *>(static_cast<char *>(ctx->params) + kParamParts);
+            nparts = (int)std::min<long>(std::max<long>(ceil_div(n, 256 * 16), 1), kParamPartsMax);
+            hipLaunchKernelGGL((dql_range_kernel<GELU>), (unsigned)nparts, 256, 0, ctx->stream, x, (long)n, slot, vec_ok, 1, gelu);
+            HIPC_LAUNCHED(ctx);
+        } else if (!range_ready) {
+            hipLaunchKernelGGL((dql_clear_range_kernel), 1, 64, 0, ctx->stream, slot);
+            HIPC_LAUNCHED(ctx);
+            // enough workgroups to pull from every HBM channel, few enough that the atomics are noise
+            const long want = ceil_div(n, 256 * 16);
+            const unsigned grid = (unsigned)std::min<long>(std::max<long>(want, 1), 8L * ctx->cu_count);
+            hipLaunchKernelGGL((dql_range_kernel<GELU>), grid, 256, 0, ctx->stream, x, (long)n, slot, vec_ok, 0, gelu);
+            HIPC_LAUNCHED(ctx);
+        }
+        // sixteen values per thread where that leaves every SIMD a wavefront: a workgroup joins all the range pairs, a trip
+        // to memory of its own (4 M values through a GELU: 13.2 -> 11.0 us); else four
+        const long quads = ceil_div(n, 4);
+        HIPC_REQUIRE(ctx, ceil_div(quads, 256) < (int64_t(1) << 31), "DynamicQuantizeLinear: tensor too large");
+        if (quads >= 4 * 256 * (int64_t)ctx->cu_count)
+            hipLaunchKernelGGL((dql_quantize_kernel<GELU, 4>), (unsigned)ceil_div(quads, 4 * 256), 256, 0, ctx->stream, x, (long)n, slot, nparts, static_cast<uint8_t *>(Y),
+                               static_cast<float *>(scale_out), static_cast<uint8_t *>(zp_out), vec_ok, gelu);
+        else
+            hipLaunchKernelGGL((dql_quantize_kernel<GELU, 1>), (unsigned)ceil_div(quads, 256), 256, 0, ctx->stream, x, (long)n, slot, nparts, static_cast<uint8_t *>(Y),
+                               static_cast<float *>(scale_out), static_cast<uint8_t *>(zp_out), vec_ok, gelu);
         HIPC_LAUNCHED(ctx);
-    } else if (!range_ready) {
-        hipLaunchKernelGGL((dql_clear_range_kernel), 1, 64, 0, ctx->stream, slot);
-        HIPC_LAUNCHED(ctx);
-        // enough workgroups to pull from every HBM channel, few enough that the atomics are noise
-        const long want = ceil_div(n, 256 * 16);
-        const unsigned grid = (unsigned)std::min<long>(std::max<long>(want, 1), 8L * ctx->cu_count);
-        hipLaunchKernelGGL((dql_range_kernel), grid, 256, 0, ctx->stream, x, (long)n, slot, vec_ok, 0, gelu);
-        HIPC_LAUNCHED(ctx);
-    }
-    const long quads = ceil_div(n, 4);
-    HIPC_REQUIRE(ctx, ceil_div(quads, 256) < (int64_t(1) << 31), "DynamicQuantizeLinear: tensor too large");
-    hipLaunchKernelGGL((dql_quantize_kernel), (unsigned)ceil_div(quads, 256), 256, 0, ctx->stream, x, (long)n, slot, nparts, static_cast<uint8_t *>(Y), static_cast<float *>(scale_out), static_cast<uint8_t *>(zp_out),
-        vec_ok, gelu);
-    HIPC_LAUNCHED(ctx);
-    return HIPC_OK;
+        return HIPC_OK;
+    };
+    if (gelu.on == GELU_SQRT2) return launch(std::integral_constant<int, GELU_SQRT2>{});
+    if (gelu.on == GELU_ANY) return launch(std::integral_constant<int, GELU_ANY>{});
+    return launch(std::integral_constant<int, GELU_OFF>{});
 }
 
 int gelu_params(hipc_ctx *ctx, float divisor, float offset, float factor, int factor_first, GeluParams *out) {
     HIPC_REQUIRE(ctx, divisor == divisor && offset == offset && factor == factor && divisor != 0.f, "DecomposedGelu: bad constants");
-    *out = GeluParams{1, divisor, offset, factor, factor_first != 0};
+    *out = GeluParams{divisor == 1.41421356f ? GELU_SQRT2 : GELU_ANY, divisor, offset, factor, factor_first != 0};
     return HIPC_OK;
 }
 
@@ -251,7 +393,7 @@ extern "C" {
 int hipc_dynamic_quantize_linear(hipc_ctx *ctx, const void *X, int64_t n, void *Y, void *scale_out, void *zp_out,
                                  void *range, int range_ready) {
     return entry(ctx, [&]() -> int {
-        return dql_launch(ctx, X, n, Y, scale_out, zp_out, range, range_ready, GeluParams{0, 1.f, 0.f, 1.f, 0});
+        return dql_launch(ctx, X, n, Y, scale_out, zp_out, range, range_ready, GeluParams{});
     });
 }
 
@@ -262,7 +404,7 @@ int hipc_dynamic_quantize_linear_static(hipc_ctx *ctx, const void *X, int64_t n,
         HIPC_REQUIRE(ctx, ctx->dql_static, "DynamicQuantizeLinear (static): the static array was not found on this device");
         // every pair the second pass reads is written by the first pass of this same call, so
         // what an earlier (larger) call left in the array is never seen and nothing needs clearing
-        return dql_launch(ctx, X, n, Y, scale_out, zp_out, nullptr, 0, GeluParams{0, 1.f, 0.f, 1.f, 0},
+        return dql_launch(ctx, X, n, Y, scale_out, zp_out, nullptr, 0, GeluParams{},
                           static_cast<uint32_t *>(ctx->dql_static));
     });
 }
@@ -285,8 +427,10 @@ int hipc_decomposed_gelu(hipc_ctx *ctx, const void *X, int64_t n, float divisor,
         if (n == 0) return HIPC_OK;
         HIPC_REQUIRE(ctx, X && Y && aligned(X, 4) && aligned(Y, 4), "DecomposedGelu: null or unaligned tensor");
         HIPC_REQUIRE(ctx, ceil_div(n, 256) < (int64_t(1) << 31), "DecomposedGelu: tensor too large");
-        hipLaunchKernelGGL((decomposed_gelu_kernel), (unsigned)ceil_div(n, 256), 256, 0, ctx->stream, static_cast<const float *>(X), (long)n, gp,
-                                                                                    static_cast<float *>(Y));
+        if (gp.on == GELU_SQRT2)
+            hipLaunchKernelGGL((decomposed_gelu_kernel<GELU_SQRT2>), (unsigned)ceil_div(n, 256), 256, 0, ctx->stream, static_cast<const float *>(X), (long)n, gp, static_cast<float *>(Y));
+        else
+            hipLaunchKernelGGL((decomposed_gelu_kernel<GELU_ANY>), (unsigned)ceil_div(n, 256), 256, 0, ctx->stream, static_cast<const float *>(X), (long)n, gp, static_cast<float *>(Y));
         HIPC_LAUNCHED(ctx);
         return HIPC_OK;
     });

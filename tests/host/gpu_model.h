@@ -144,6 +144,9 @@ inline void gpu_model_nt_store(U v, T *p) { *p = v; }
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8 gpu_model_mfma
 inline float gpu_model_rcp(float v) { return 1.f / v; }
 #define __builtin_amdgcn_rcpf gpu_model_rcp
+#define __builtin_amdgcn_exp2f std::exp2
+inline float gpu_model_fmed3(float v, float lo, float hi) { return std::min(std::max(v, lo), hi); }
+#define __builtin_amdgcn_fmed3f gpu_model_fmed3
 inline int gpu_model_sdot4(int, int, int c, bool) { return c; }
 #define __builtin_amdgcn_sdot4 gpu_model_sdot4
 template <typename P>

@@ -137,3 +137,26 @@ def test_fused_gelu_quantization_of_nothing_and_bad_constants(ctx, pkg):
     assert y.size == 0 and scale == 1.0 and zp == 0
     with pytest.raises(pkg.HipComputeError):
         pkg.ops.decomposed_gelu(ctx, np.ones(4, np.float32), divisor=0.0)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4095, 4097, 16383, 16384, 16386, 40959, 40960, 40961, 262144 * 4 + 5])
+def test_sizes_around_the_launch_forms(ctx, pkg, oracle, n):
+    """One launch up to 40960 values (16384 through a GELU), two behind it, sixteen values per thread from a million on:
+    the last size of each form and the first of the next; divisors the quotient of which is formed either way."""
+    x = pkg.synth.normal_f32(n, 91)
+    y, s, z = pkg.ops.dynamic_quantize_linear(ctx, x)
+    wy, ws, wz = oracle.dynamic_quantize_linear(x)
+    assert np.array_equal(y, wy) and np.float32(s) == np.float32(ws) and z == wz
+    for divisor in (pkg.ops.SQRT2_F32, 1.5):
+        y, s, z = pkg.ops.dynamic_quantize_linear_gelu(ctx, x, divisor)
+        wy, ws, wz = pkg.ops.dynamic_quantize_linear(ctx, pkg.ops.decomposed_gelu(ctx, x, divisor))
+        assert np.array_equal(y, wy) and s == ws and z == wz
+
+
+@pytest.mark.parametrize("scale", [1e-38, 2.0 ** -101, 2.0 ** -99, 1.0, 2.0 ** 99, 2.0 ** 101, 1e38])
+def test_scales_at_the_ends_of_the_float_range(ctx, pkg, oracle, scale):
+    """Where the quotient is formed from the scale's reciprocal, and where it is not."""
+    x = (pkg.synth.uniform_f32(5000, 92, -1.0, 1.0) * np.float32(scale)).astype(np.float32)
+    y, s, z = pkg.ops.dynamic_quantize_linear(ctx, x)
+    wy, ws, wz = oracle.dynamic_quantize_linear(x)
+    assert np.array_equal(y, wy) and np.float32(s) == np.float32(ws) and z == wz
