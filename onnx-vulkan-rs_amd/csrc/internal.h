@@ -477,6 +477,14 @@ int nbits_prefill(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void
 bool nbits_prefill_f32_takes(const void *A, const hipc_nbits_weight *w, int64_t M);
 int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int64_t M, int terms);   // f16 terms per f32 row: 2 (22 bits), 1 (11) or 3 (all 24)
 
+// A few rows (matmul_nbits_rows.hip): up to 64 of f16, or of f32 as f16 terms -- up to 16 split by the kernel itself, more by
+// a launch in front (one term or two; see nbits_prefill_f32).
+constexpr int kFewRows = 64;
+bool nbits_rows_takes(const void *A, const hipc_nbits_weight *w, int64_t M, int terms);
+int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, const hipc_nbits_weight *w, void *Y, int y_f16, int M);
+int nbits_rows_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms);
+int nbits_rows_f32_split(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms);
+
 // offsets inside ctx->params
 constexpr size_t kParamRange = 0;   // 8 B  {bits(-min), bits(max)}
 constexpr size_t kParamParts = 256; // 16 KiB: per-workgroup {bits(-min), bits(max)} pairs of DynamicQuantizeLinear

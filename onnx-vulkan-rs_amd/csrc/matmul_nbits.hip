@@ -1221,6 +1221,12 @@ int packed_run(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weigh
     // accuracy_level 1 pins f32 activations: all 24 bits go through the matrix cores (3 bf16
     // terms). Unset, or 2 / 3 / 4 (f16 / bf16 / int8 are enough): 2 terms. f16 activations are exact in 2.
     const int NT = (accuracy_level == 1 && a_dtype == HIPC_F32) ? 3 : 2;
+    // a few rows (one of f32 is a matter of its own: launch_gemv)
+    const int terms = a_dtype == HIPC_F16 ? 1 : NT == 3 ? 3 : M > 32 && accuracy_level >= 2 ? 1 : 2;
+    if ((a_dtype == HIPC_F16 || M > 1) && nbits_rows_takes(A, w, M, terms)) {
+        if (a_dtype == HIPC_F16) return nbits_rows_f16(ctx, A, 1, nullptr, w, Y, 1, (int)M);
+        return M <= 16 ? nbits_rows_f32(ctx, A, w, Y, (int)M, terms) : nbits_rows_f32_split(ctx, A, w, Y, (int)M, terms);
+    }
     // many rows of f16: the tiled kernel reads the weight once per row tile instead of once per 16 rows
     if (a_dtype == HIPC_F16 && nbits_prefill_takes(A, w, M)) return nbits_prefill(ctx, A, w, Y, M);
     // many rows of f32: two f16 rows each (22 bits) through the same kernel; one (11 bits beside the row's own

@@ -27,11 +27,10 @@
 #include <cstdlib>
 
 #include "internal.h"
+#include "nbits_f16.h"
 
 namespace hipc {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPK = 64;          // k values per stage
@@ -61,11 +60,6 @@ struct PrefillArgs {
     const int *exps;
     int pair_rows;
 };
-
-// two f16 values as one word, the first in the low half
-__device__ __forceinline__ uint32_t two_halves(__half lo, __half hi) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-}
 
 // eight nibbles (order k0 k2 k4 k6 k1 k3 k5 k7) -> eight f16 values q - zp in k order, as four words of pairs
 __device__ __forceinline__ uint4 dequant8(uint32_t w, uint32_t zb) {
@@ -341,40 +335,6 @@ __global__ void __launch_bounds__(256) mmnb_prefill_kernel(const PrefillArgs p) 
 // covers k = 32 j + 16 kg + 8 h + 0..7 -- an order of its own, which only has to be the same for both operands: A
 // is read from LDS at that offset. LDS carries A alone (half the traffic and half the writes of the kernel above,
 // and no conversion ahead of a barrier).
-
-// 1024 + zp and 64 + zp as f16 in both halves of a word (zb carries 128 + zp)
-struct ZeroPair {
-    f16x2 unit, sixteenth;
-};
-__device__ __forceinline__ ZeroPair zero_pair(uint32_t zb) {
-    const uint32_t zp = zb - 128u, a = 0x6400u + zp, b = 0x5400u + (zp << 4);
-    return {__builtin_bit_cast(f16x2, a | (a << 16)), __builtin_bit_cast(f16x2, b | (b << 16))};
-}
-// eight nibbles (k0 k2 k4 k6 in the low half, k1 k3 k5 k7 in the high half) -> the f16 values q - zp in k order.
-// Nibbles 0 and 2 of each half sit where the low mantissa bits are: or-ed with the exponent of 1024 that is
-// 1024 + q. Nibbles 1 and 3 sit four bits higher: 1024 + 16 q, and one fused multiply-add by 1/16 makes q - zp
-// of it ((1024 + 16 q) / 16 = 64 + q is exact). One shift instead of three.
-// (x & mask) | 0x64006400 as one instruction: v_and_or_b32 can take one scalar operand only, so the compiler, which
-// keeps both constants in scalar registers, emits two; the exponent pattern is handed over in a vector register
-__device__ __forceinline__ uint32_t and_or_1024(uint32_t x, uint32_t mask, uint32_t ones) {
-#ifdef HIPC_HOST_MODEL
-    return (x & mask) | ones;
-#else
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(ones));
-    return r;
-#endif
-}
-__device__ __forceinline__ f16x8 dequant_operand(uint32_t w, const ZeroPair &z, uint32_t ones) {
-    const f16x2 sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const uint32_t w8 = w >> 8;
-    const f16x2 p0 = __builtin_bit_cast(f16x2, and_or_1024(w, 0x000f000fu, ones)) - z.unit;
-    const f16x2 p1 = __builtin_bit_cast(f16x2, and_or_1024(w, 0x00f000f0u, ones)) * sixteenth - z.sixteenth;
-    const f16x2 p2 = __builtin_bit_cast(f16x2, and_or_1024(w8, 0x000f000fu, ones)) - z.unit;
-    const f16x2 p3 = __builtin_bit_cast(f16x2, and_or_1024(w8, 0x00f000f0u, ones)) * sixteenth - z.sixteenth;
-    return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-__device__ __forceinline__ uint32_t word_of(const uint4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
 
 // NJ: 32-column blocks per wavefront. 2: a 128x128 tile. 3: a 128x192 tile -- a third less LDS traffic per product,
 // and a matrix of 512 x 11008 becomes 232 workgroups for 256 CUs where 128x128 tiles make 344, two of them on every
@@ -1075,6 +1035,23 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
         hipLaunchKernelGGL((mmnb_prefill_join_rows_kernel<false>), dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, ctx->stream, static_cast<const float *>(sums), exps, (int)M, (int)w->N, static_cast<float *>(Y), terms);
     HIPC_LAUNCHED(ctx);
     return HIPC_OK;
+}
+
+// up to 64 rows of f32, split here and multiplied as f16 rows by the kernel for a few rows (matmul_nbits_rows.hip)
+int nbits_rows_f32_split(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms) {
+    const size_t e_bytes = ((size_t)M * sizeof(int) + 255) & ~(size_t)255;
+    void *split = nullptr;
+    if (int rc = scratch_get(ctx, 2, (size_t)terms * M * w->K * sizeof(__half) + e_bytes, &split)) return rc;
+    __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + e_bytes);
+    int *exps = static_cast<int *>(split);
+    if (terms == 1)
+        hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 1>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), M, (int)w->K, A2, exps);
+    else if (terms == 3)
+        hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 3>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), M, (int)w->K, A2, exps);
+    else
+        hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 2>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), M, (int)w->K, A2, exps);
+    HIPC_LAUNCHED(ctx);
+    return nbits_rows_f16(ctx, A2, terms, exps, w, Y, 0, M);
 }
 
 #endif  // HIPC_PREFILL_WIDE

@@ -171,6 +171,8 @@ inline T __shfl_xor(T v, int, int = 64) { return v; }
 inline float __uint_as_float(uint32_t u) { float f; std::memcpy(&f, &u, 4); return f; }
 inline uint32_t __float_as_uint(float f) { uint32_t u; std::memcpy(&u, &f, 4); return u; }
 inline float __expf(float v) { return std::exp(v); }
+inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xffffffu) * (b & 0xffffffu); }
+inline int __any(int v) { return v; }
 inline float rsqrtf(float v) { return 1.f / std::sqrt(v); }
 inline float __fmul_rn(float a, float b) { return a * b; }
 inline float __fdiv_rn(float a, float b) { return a / b; }

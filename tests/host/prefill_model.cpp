@@ -150,7 +150,11 @@ int main() {
                               {16, 640, 96, 128, 0}, {1, 1152, 1536, 32, 1}, {2, 256, 1024, 256, 1},
                               // the stand-alone launches of a gemma3-1b token (one k tile per wavefront up to sixteen tiles,
                               // four column tiles per workgroup on the widest, four k tiles per wavefront on the longest), a ragged k
-                              {1, 1024, 1152, 32, 1}, {1, 1152, 13824, 32, 1}, {1, 6912, 1152, 32, 1}, {1, 1480, 64, 32, 1}};
+                              {1, 1024, 1152, 32, 1}, {1, 1152, 13824, 32, 1}, {1, 6912, 1152, 32, 1}, {1, 1480, 64, 32, 1},
+                              // the kernel for a few rows: one, two and four row blocks, stages that end in the middle of k,
+                              // k split over workgroups, a last tile of k with 8 values, one to four column tiles per wavefront
+                              {2, 1152, 13824, 32, 1}, {8, 6912, 1152, 32, 1}, {16, 2056, 4100, 64, 1}, {13, 136, 40, 128, 0}, {23, 1288, 1152, 32, 1},
+                              {32, 4104, 272, 128, 0}, {33, 1152, 600, 64, 1}, {64, 2048, 1030, 32, 1}, {50, 520, 13824, 32, 0}};
     for (const auto &s : few)
         for (int dt : {HIPC_F32, HIPC_F16}) rows(s[0], s[1], s[2], s[3], s[4] != 0, dt);
     gpu_model::Registry &g = gpu_model::reg();

@@ -442,3 +442,39 @@ def test_one_row_on_the_streaming_kernel(ctx, pkg, oracle, shape):
     assert close(lean, want, RTOL32), ("lean", worst(lean, want))
     assert close(streaming, want, RTOL32), ("streaming", worst(streaming, want))
     assert close(lean, streaming, RTOL32)
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("bs,with_zp", [(32, True), (64, False), (128, True)])
+@pytest.mark.parametrize("shape", [(2, 136, 40), (4, 1152, 1030), (5, 1000, 200), (8, 2056, 16), (9, 72, 600), (16, 4096, 272), (17, 1288, 90),
+                                   (32, 520, 1040), (33, 2048, 131), (64, 1152, 96), (64, 264, 2064), (7, 8, 33)], ids=lambda s: "M%d_K%d_N%d" % s)
+def test_a_few_rows(ctx, pkg, oracle, shape, bs, with_zp, dtype):
+    """2 to 64 rows: every number of row blocks and result registers, rows that fill their stage of LDS once and several
+    times, k split over workgroups, a last tile of k with eight values, columns that end inside a tile."""
+    m, k, n = shape
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=500 + n, with_zp=with_zp, scale_dtype=dtype)
+    a = pkg.synth.normal_f32(m * k, 501).reshape(m, k).astype(dtype)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    want = oracle.matmul_nbits(a, B, scales, zp, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, weight=w)
+    assert close(got, want, RTOL32 if dtype == np.float32 else RTOL16), worst(got, want)
+    w.destroy()
+
+
+@pytest.mark.parametrize("m", [3, 16, 20])
+@pytest.mark.parametrize("level", [0, 1])
+def test_a_few_rows_of_very_different_size(ctx, pkg, oracle, m, level):
+    """Rows that are not split as they are: values above 2^15, rows whose largest value is small, subnormal, zero."""
+    k, n, bs = 640, 80, 32
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=511)
+    a = pkg.synth.normal_f32(m * k, 512).reshape(m, k)
+    a[0] *= np.float32(1e30)
+    a[1] *= np.float32(1e-20)
+    a[2] = 0
+    a[m - 1, ::3] *= np.float32(1e5)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    want = oracle.matmul_nbits(a.astype(np.float32), B, scales, zp, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a.astype(np.float32), None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    for r in range(m):   # each row against its own size
+        assert np.max(np.abs(got[r] - want[r])) <= 1e-5 * max(np.max(np.abs(want[r])), 1e-37), r
+    w.destroy()
