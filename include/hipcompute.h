@@ -180,7 +180,8 @@ int hipc_matmul_nbits(hipc_ctx *ctx, const void *A, int a_dtype, const void *B, 
 /* Repack a constant weight once (the role `packed_b` plays for MatMulInteger,
  * interp.rs:2712-2768; the reference feeds MatMulNBits the ONNX layout directly).
  * The operands are device pointers in the ONNX layout above and may be released
- * after the next flush. A block_size below 32 or not a power of two has no tiled form:
+ * after the next flush. A block_size that is not a power of two or below 16, and one of 16 with
+ * K * N < 16384 or K no multiple of 8, has no tiled form:
  * its handle holds copies of the tensors as they are and hipc_matmul_nbits_packed runs
  * the kernel of hipc_matmul_nbits on them (the same results, bit for bit). */
 int hipc_prepack_matmul_nbits(hipc_ctx *ctx, const void *B, size_t b_len, const void *scales,
@@ -190,13 +191,13 @@ void hipc_nbits_weight_destroy(hipc_ctx *ctx, hipc_nbits_weight *w);
 /* bytes of device memory the prepacked form occupies */
 size_t hipc_nbits_weight_bytes(const hipc_nbits_weight *w);
 /* MatMulNBits on a prepacked weight. `accuracy_level` as in the operator, a lower bound on what the
- * activations may be reduced to (the reference never reads it and computes in f32). One row of f32, and
- * up to 16 against 32768 columns or more: 0 (unset), 2, 3 and 4 enter the matrix cores as two bf16 terms
+ * activations may be reduced to (the reference never reads it and computes in f32). One row of f32
+ * (blocks of 32 and more), and up to 16 against 32768 columns or more: 0 (unset), 2, 3 and 4 enter the matrix cores as two bf16 terms
  * (16 significant bits, less error than f32 accumulation over K adds), 1 pins f32 and uses three terms (all
  * 24 bits). Otherwise the kernels use f16: an f16 row as it is, an f32 row
  * as f16 terms of the row times a power of two (none up to 16 rows whose largest value lies in [1/8, 2^15),
  * else the one that puts the row's largest value into [2^14, 2^15)):
- * two terms (22 bits) at level 0, one (11 bits of every value) from 33 rows on at levels 2, 3 and 4, which allow
+ * two terms (22 bits) at level 0 (three with blocks of 16), one (11 bits of every value) from 33 rows on at levels 2, 3 and 4, which allow
  * f16, bf16 or int8 activations, three (every bit of the row's values) at level 1.
  * The tiled kernel keeps its accumulators in units of the open quantisation block's scale: there a
  * scale of magnitude below 2^-64 counts as 2^-64 (what such a block adds is below

@@ -38,7 +38,7 @@
 
 namespace hipc {
 
-constexpr int kScratchSlots = 5;
+constexpr int kScratchSlots = 6;
 
 // grow-only device scratch reused by operators that need a temporary (packed
 // B of a raw call, the i32 accumulator of a QLinear op). One in-order stream
@@ -143,7 +143,7 @@ struct hipc_graph {
 // A MatMulNBits weight repacked for the matrix cores: 1 KiB tiles of 16 columns x 128 k. Lane l
 // of tile (nt, cg) = Wq[(nt * n_cg + cg) * 64 + l] holds, in word j, the eight nibbles
 // k = 128 cg + 32 j + 8 (l >> 4) .. + 8 of column 16 nt + (l & 15), in the order k0 k2 k4 k6 k1 k3 k5 k7. Sc / Zb hold SG scales
-// and (128 + zero point) bytes per tile column, SG = 4, 2, 1 for block sizes 32, 64, >= 128.
+// and (128 + zero point) bytes per tile column, SG = 8, 4, 2, 1 for block sizes 16, 32, 64, >= 128.
 struct hipc_nbits_weight {
     int64_t K = 0, N = 0, block_size = 0;
     int n_tiles = 0, n_cg = 0, SG = 0;
@@ -152,8 +152,8 @@ struct hipc_nbits_weight {
     float *Sc = nullptr;
     uint8_t *Zb = nullptr;
     size_t bytes = 0;
-    // A block_size below 32 or not a power of two has no tiled form (a 32-k product step would straddle scale
-    // groups): the handle then keeps device copies of the operator's own tensors (Wq is null) and the product
+    // A block_size below 16 or not a power of two has no tiled form (a product step would straddle scale groups), and a
+    // small weight in blocks of 16 gets none (see has_tiled_form): the handle then keeps device copies of the operator's own tensors (Wq is null) and the product
     // runs on the kernel that reads that layout. Only hipc_matmul_nbits_packed takes such a handle.
     void *raw_B = nullptr, *raw_scales = nullptr, *raw_zp = nullptr;
     int raw_scale_dtype = 0;

@@ -108,7 +108,7 @@ mmnb_direct_kernel(const AT *__restrict__ A, const uint32_t *__restrict__ B, con
 // Lane l's 128-bit element holds, in word j, the 8 nibbles k = 32*c + 8*(l >> 4) .. +8
 // of column n -- exactly the B operand of one 16x16x32 MFMA per word -- in the nibble order
 // k0 k2 k4 k6 k1 k3 k5 k7, so that (word >> 4 i) & 0x000f000f is the pair (k_2i, k_2i+1).
-// SG scale groups per tile (4 when block_size == 32, 2 for 64, 1 for >= 128).
+// SG scale groups per tile (8 when block_size == 16, 4 for 32, 2 for 64, 1 for >= 128).
 template <typename ST>
 __global__ void __launch_bounds__(256)
 mmnb_prepack_kernel(const uint32_t *__restrict__ B, const ST *__restrict__ scales, const uint8_t *__restrict__ zp,
@@ -141,8 +141,7 @@ mmnb_prepack_kernel(const uint32_t *__restrict__ B, const ST *__restrict__ scale
     Wq[idx] = make_uint4(v[0], v[1], v[2], v[3]);
     if (w == 0) {
         for (int g = 0; g < SG; g++) {
-            const int c = cg * 4 + g * (4 / SG);
-            const int b = c >> cpb_shift;
+            const int b = SG == 8 ? cg * 8 + g : (cg * 4 + g * (4 / SG)) >> cpb_shift;
             float s = 0.f;
             int z = 8;
             if (n < N && b < n_blocks) {
@@ -1060,21 +1059,25 @@ int hipc_prepack_matmul_nbits(hipc_ctx *ctx, const void *B, size_t b_len, const 
 
 namespace {
 
-// tile counts and scale grouping of the tiled form of a weight (K, N, block_size set; block_size a power of two >= 32), and
+// Which weights the matrix-core kernels have a form for. Blocks of 16 take it from 16384 values on: one row
+// of a smaller weight is a launch and little else on either kernel, and the handle stays what the caller passed in.
+bool has_tiled_form(int64_t K, int64_t N, int64_t block_size) {
+    return is_pow2(block_size) && (block_size >= 32 || (block_size == 16 && K % 8 == 0 && K * N >= 16384));
+}
+// tile counts and scale grouping of the tiled form of a weight (K, N, block_size set), and
 // the bytes of its three arrays
 void tiled_geometry(hipc_nbits_weight *w, size_t *wq_bytes, size_t *sc_bytes, size_t *zb_bytes) {
     const int n_chunks = (int)ceil_div(w->K, 32);
     w->n_tiles = (int)ceil_div(w->N, 16);
     w->n_cg = (int)ceil_div(n_chunks, 4);
-    const int cpb = (int)(w->block_size / 32);
-    w->SG = cpb >= 4 ? 1 : 4 / cpb;
+    w->SG = w->block_size >= 128 ? 1 : (int)(128 / w->block_size);
     const size_t tiles = (size_t)w->n_tiles * w->n_cg;
     *wq_bytes = tiles * 1024, *sc_bytes = tiles * 16 * w->SG * 4, *zb_bytes = tiles * 16 * w->SG;
 }
 // the launch that writes the tiled form from the operator's tensors (device pointers)
 hipError_t tiled_fill(hipc_ctx *ctx, const hipc_nbits_weight *w, const void *B, const void *scales, int scale_dtype, const void *zp) {
     const int n_blocks = (int)ceil_div(w->K, w->block_size);
-    const int cpb = (int)(w->block_size / 32);
+    const int cpb_shift = w->block_size >= 32 ? log2i((int)(w->block_size / 32)) : 0;
     const size_t tiles = (size_t)w->n_tiles * w->n_cg;
     const int row_words = (int)(n_blocks * w->block_size / 8);
     const int zp_row = (n_blocks + 1) / 2;
@@ -1082,10 +1085,10 @@ hipError_t tiled_fill(hipc_ctx *ctx, const hipc_nbits_weight *w, const void *B, 
     const dim3 grid((unsigned)ceil_div(threads, 256)), block(256);
     if (scale_dtype == HIPC_F16)
         hipLaunchKernelGGL((mmnb_prepack_kernel<__half>), grid, block, 0, ctx->stream, static_cast<const uint32_t *>(B), static_cast<const __half *>(scales), static_cast<const uint8_t *>(zp),
-            w->Wq, w->Sc, w->Zb, (int)w->N, n_blocks, row_words, zp_row, (long)tiles, w->n_cg, log2i(cpb), w->SG, w->interleave_half);
+            w->Wq, w->Sc, w->Zb, (int)w->N, n_blocks, row_words, zp_row, (long)tiles, w->n_cg, cpb_shift, w->SG, w->interleave_half);
     else
         hipLaunchKernelGGL((mmnb_prepack_kernel<float>), grid, block, 0, ctx->stream, static_cast<const uint32_t *>(B), static_cast<const float *>(scales), static_cast<const uint8_t *>(zp),
-            w->Wq, w->Sc, w->Zb, (int)w->N, n_blocks, row_words, zp_row, (long)tiles, w->n_cg, log2i(cpb), w->SG, w->interleave_half);
+            w->Wq, w->Sc, w->Zb, (int)w->N, n_blocks, row_words, zp_row, (long)tiles, w->n_cg, cpb_shift, w->SG, w->interleave_half);
     return hipGetLastError();
 }
 
@@ -1103,7 +1106,7 @@ int hipc::nbits_prepack(hipc_ctx *ctx, const void *B, size_t b_len, const void *
     if (rc != HIPC_OK) return rc;
     HIPC_REQUIRE(ctx, N > 0 && B && scales, "MatMulNBits prepack: empty weight");
     HIPC_REQUIRE(ctx, aligned(B, 4), "MatMulNBits: packed weight must be 4-byte aligned");
-    const bool tiled = block_size >= 32 && is_pow2(block_size);
+    const bool tiled = has_tiled_form(K, N, block_size) && (block_size >= 32 || any_block_size);   // (the decoder's kernels know no blocks of 16)
     HIPC_REFUSE(ctx, !tiled && (!any_block_size || interleave_half != 0),
                 "MatMulNBits prepack: block_size %ld (below 32, or not a power of two) has no tiled form", (long)block_size);
     hipc_nbits_weight *w = new hipc_nbits_weight();
@@ -1201,6 +1204,37 @@ int hipc_matmul_nbits_packed(hipc_ctx *ctx, const void *A, int a_dtype, const hi
 
 namespace {
 
+// Blocks of 16: up to 16 rows, and more where it is the better kernel, on the one for a few rows, the others on the tiled
+// kernel. Nothing here accumulates less than the kernel of the operator's layout, which computes in f32: an f32 row keeps all
+// 24 bits (three f16 terms) unless accuracy_level allows less. That kernel, which unpacks the weight and multiplies it
+// with vector instructions once per four rows, took -> this: f32 1 x 6912 x 1152 28.0 -> 8.6 us, 8 rows 145 -> 7.9, 60 x 1152 x
+// 13824 1641 -> 30; f16 20 x 2048 x 11008 384 -> 9.9, 100 rows 1881 -> 22.7; 200 x 256 x 256 27.8 -> 9.5.
+int packed_run16(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weight *w, void *Y, int64_t M, int accuracy_level) {
+    const bool f16 = a_dtype == HIPC_F16;
+    const size_t esz = f16 ? 2 : 4;
+    if (!aligned(A, 16)) {   // (the kernels read 16-byte pieces: rows that do not start on one are moved first)
+        void *copy = nullptr;
+        if (int rc = scratch_get(ctx, 5, (size_t)M * w->K * esz, &copy)) return rc;
+        HIPC_TRY(ctx, hipMemcpyAsync(copy, A, (size_t)M * w->K * esz, hipMemcpyDeviceToDevice, ctx->stream));
+        A = copy;
+    }
+    // as many rows at a time as the kernels' 32-bit offsets reach
+    const int64_t most = std::max<int64_t>(16, (((int64_t(1) << 31) - 1) / 3 / std::max(w->K, w->N) - 64) / 128 * 128);
+    for (int64_t m0 = 0; m0 < M; m0 += most) {
+        const int rows = (int)std::min(most, M - m0);
+        const char *a = static_cast<const char *>(A) + (size_t)m0 * w->K * esz;
+        char *y = static_cast<char *>(Y) + (size_t)m0 * w->N * esz;
+        const int terms = f16 ? 1 : accuracy_level < 2 ? 3 : rows > 32 ? 1 : 2;
+        int rc;
+        if (nbits_rows_takes(a, w, rows, terms))
+            rc = f16 ? nbits_rows_f16(ctx, a, 1, nullptr, w, y, 1, rows) : rows <= 16 ? nbits_rows_f32(ctx, a, w, y, rows, terms) : nbits_rows_f32_split(ctx, a, w, y, rows, terms);
+        else
+            rc = f16 ? nbits_prefill(ctx, a, w, y, rows) : nbits_prefill_f32(ctx, a, w, y, rows, terms);
+        if (rc != HIPC_OK) return rc;
+    }
+    return HIPC_OK;
+}
+
 int packed_run(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weight *w, void *Y, int64_t M, int accuracy_level) {
     HIPC_REQUIRE(ctx, w, "MatMulNBits: null weight");
     HIPC_REFUSE(ctx, a_dtype != HIPC_F32 && a_dtype != HIPC_F16, "MatMulNBits: A must be f32 or f16, got %d", a_dtype);
@@ -1210,13 +1244,14 @@ int packed_run(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weigh
     HIPC_REQUIRE(ctx, M >= 0 && M < (int64_t(1) << 30), "MatMulNBits: bad M=%ld", (long)M);
     if (M == 0) return HIPC_OK;
     HIPC_REQUIRE(ctx, A && Y, "MatMulNBits: null operand");
-    if (!w->Wq) {   // a handle in the operator's own layout (block_size below 32 or not a power of two)
+    if (!w->Wq) {   // a handle in the operator's own layout (see has_tiled_form)
         const bool af16 = a_dtype == HIPC_F16, sf16 = w->raw_scale_dtype == HIPC_F16;
         if (af16 && sf16) return launch_direct<__half, __half>(ctx, A, w->raw_B, w->raw_scales, w->raw_zp, Y, M, w->K, w->N, w->block_size);
         if (af16) return launch_direct<__half, float>(ctx, A, w->raw_B, w->raw_scales, w->raw_zp, Y, M, w->K, w->N, w->block_size);
         if (sf16) return launch_direct<float, __half>(ctx, A, w->raw_B, w->raw_scales, w->raw_zp, Y, M, w->K, w->N, w->block_size);
         return launch_direct<float, float>(ctx, A, w->raw_B, w->raw_scales, w->raw_zp, Y, M, w->K, w->N, w->block_size);
     }
+    if (w->SG == 8) return packed_run16(ctx, A, a_dtype, w, Y, M, accuracy_level);
     const size_t esz = a_dtype == HIPC_F16 ? 2 : 4;
     // accuracy_level 1 pins f32 activations: all 24 bits go through the matrix cores (3 bf16
     // terms). Unset, or 2 / 3 / 4 (f16 / bf16 / int8 are enough): 2 terms. f16 activations are exact in 2.
@@ -1248,7 +1283,7 @@ int packed_run(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weigh
 int tiled_from_onnx_layout(hipc_ctx *ctx, const void *A, int a_dtype, const void *B, const void *scales, int scale_dtype, const void *zp, void *Y,
                            int64_t M, int64_t K, int64_t N, int64_t block_size, int accuracy_level, bool *taken) {
     *taken = false;
-    if (block_size < 32 || !is_pow2(block_size)) return HIPC_OK;
+    if (!has_tiled_form(K, N, block_size)) return HIPC_OK;
     hipc_nbits_weight w;
     w.K = K, w.N = N, w.block_size = block_size;
     size_t wq_bytes, sc_bytes, zb_bytes;

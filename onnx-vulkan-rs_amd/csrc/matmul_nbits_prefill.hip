@@ -333,7 +333,9 @@ __global__ void __launch_bounds__(256) mmnb_prefill_kernel(const PrefillArgs p) 
 // (r32, kg) takes tile lanes q = 2 kg and 2 kg + 1 of its column: two 16-byte loads per 128 k), turns a word into
 // the operand in registers (nine instructions) and uses it for every 32-row block it owns. A k step (j, h) then
 // covers k = 32 j + 16 kg + 8 h + 0..7 -- an order of its own, which only has to be the same for both operands: A
-// is read from LDS at that offset. LDS carries A alone (half the traffic and half the writes of the kernel above,
+// is read from LDS at that offset. With blocks of 16 (SG 8) the lane takes tile lanes q = kg and 2 + kg instead and the step
+// covers k = 32 j + 16 h + 8 kg + 0..7: one block, whose scale costs as many vector instructions as two steps of the
+// matrix core take (2e10 operations: 24 us with few tiles, 96 with long k; 2341 and 7845 on vector instructions alone). LDS carries A alone (half the traffic and half the writes of the kernel above,
 // and no conversion ahead of a barrier).
 
 // NJ: 32-column blocks per wavefront. 2: a 128x128 tile. 3: a 128x192 tile -- a third less LDS traffic per product,
@@ -408,33 +410,38 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int nt = min(j0 / 16 + wn * (2 * NJ) + j * 2 + (r32 >> 4), p.n_tiles - 1);  // tiles past N: clamped, never stored
-        b_at[j] = (uint32_t)nt * (uint32_t)p.n_cg * 64 + (r32 & 15) + 32 * kg;
+        b_at[j] = (uint32_t)nt * (uint32_t)p.n_cg * 64 + (r32 & 15) + (SG == 8 ? 16 : 32) * kg;
         sc_at[j] = ((uint32_t)nt * (uint32_t)p.n_cg * 16 + (r32 & 15)) * SG;
     }
     struct BRegs {
         uint4 w[NJ][2];
         float s[NJ][SG];
-        uint32_t z[NJ];  // SG bytes of 128 + zp
+        uint32_t z[NJ][SG == 8 ? 2 : 1];  // SG bytes of 128 + zp
     };
     auto load_b = [&](BRegs &b, int cg) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             const uint4 *src = (p.Wq + (size_t)cg * 64) + b_at[j];
             b.w[j][0] = src[0];
-            b.w[j][1] = src[16];
+            b.w[j][1] = src[SG == 8 ? 32 : 16];
             const float *sc = (p.Sc + (size_t)cg * 16 * SG) + sc_at[j];
             const uint8_t *zb = (p.Zb + (size_t)cg * 16 * SG) + sc_at[j];
-            if (SG == 4) {
+            if (SG >= 4) {
                 const float4 v = *reinterpret_cast<const float4 *>(sc);
                 b.s[j][0] = v.x, b.s[j][1 % SG] = v.y, b.s[j][2 % SG] = v.z, b.s[j][3 % SG] = v.w;
-                b.z[j] = *reinterpret_cast<const uint32_t *>(zb);
+                if (SG == 8) {
+                    const float4 u = *reinterpret_cast<const float4 *>(sc + 4);
+                    b.s[j][4 % SG] = u.x, b.s[j][5 % SG] = u.y, b.s[j][6 % SG] = u.z, b.s[j][7 % SG] = u.w;
+                    b.z[j][SG == 8] = *reinterpret_cast<const uint32_t *>(zb + 4);
+                }
+                b.z[j][0] = *reinterpret_cast<const uint32_t *>(zb);
             } else if (SG == 2) {
                 const float2 v = *reinterpret_cast<const float2 *>(sc);
                 b.s[j][0] = v.x, b.s[j][1 % SG] = v.y;
-                b.z[j] = *reinterpret_cast<const uint16_t *>(zb);
+                b.z[j][0] = *reinterpret_cast<const uint16_t *>(zb);
             } else {
                 b.s[j][0] = sc[0];
-                b.z[j] = zb[0];
+                b.z[j][0] = zb[0];
             }
         }
     };
@@ -484,40 +491,43 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
     asm volatile("" : "+v"(ones));
 #endif
     // One stage = 64 k = the k steps (j, h) with j = 2 half + 0 / 1 of the weight tile the stage lies in;
-    // a scale group opens at every second step (SG 4), every stage (SG 2) or every even stage (SG 1).
+    // a scale group opens at every step (SG 8), every second step (SG 4), every stage (SG 2) or every even stage (SG 1).
     // the zero points of a stage as f16 pairs (with one scale group per weight tile: of the whole tile, made once per trip)
     struct ZeroPairs {
-        ZeroPair at[NJ][SG == 4 ? 2 : 1];
+        ZeroPair at[NJ][SG == 8 ? 4 : SG == 4 ? 2 : 1];
     };
     auto zero_pairs = [&](const BRegs &b, int half) {
         ZeroPairs zp;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            if (SG == 4) {
-                zp.at[j][0] = zero_pair((b.z[j] >> (16 * half)) & 0xffu);
-                zp.at[j][SG == 4 ? 1 : 0] = zero_pair((b.z[j] >> (16 * half + 8)) & 0xffu);
+            if constexpr (SG == 8) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) zp.at[j][g] = zero_pair((b.z[j][half] >> (8 * g)) & 0xffu);
+            } else if constexpr (SG == 4) {
+                zp.at[j][0] = zero_pair((b.z[j][0] >> (16 * half)) & 0xffu);
+                zp.at[j][1] = zero_pair((b.z[j][0] >> (16 * half + 8)) & 0xffu);
             } else {
-                zp.at[j][0] = zero_pair(SG == 2 ? (b.z[j] >> (8 * half)) & 0xffu : b.z[j]);
+                zp.at[j][0] = zero_pair(SG == 2 ? (b.z[j][0] >> (8 * half)) & 0xffu : b.z[j][0]);
             }
         }
         return zp;
     };
     auto compute = [&](const BRegs &b, const ZeroPairs &zp, int buf, int half) {   // (b.s holds ratios by now)
-        const uint8_t *ba = lds_a + buf * T * kPPitch + (wm * kWT + r32) * kPPitch + kg * 32;
+        const uint8_t *ba = lds_a + buf * T * kPPitch + (wm * kWT + r32) * kPPitch + kg * (SG == 8 ? 16 : 32);
 #pragma unroll
         for (int step = 0; step < 4; step++) {
             const int word = half * 2 + (step >> 1), h = step & 1;
-            const bool opens = SG == 4 ? h == 0 : SG == 2 ? step == 0 : step == 0 && half == 0;
+            const bool opens = SG == 8 ? true : SG == 4 ? h == 0 : SG == 2 ? step == 0 : step == 0 && half == 0;
             f16x8 af[kF], wf[NJ];
             if (opens) {
-                const int g = SG == 4 ? word : SG == 2 ? half : 0;
+                const int g = SG == 8 ? 2 * word + h : SG == 4 ? word : SG == 2 ? half : 0;
 #pragma unroll
                 for (int j = 0; j < NJ; j++) reopen(j, b.s[j][g % SG]);
             }
 #pragma unroll
-            for (int i = 0; i < kF; i++) af[i] = *reinterpret_cast<const f16x8 *>(ba + i * 32 * kPPitch + (step >> 1) * 64 + h * 16);
+            for (int i = 0; i < kF; i++) af[i] = *reinterpret_cast<const f16x8 *>(ba + i * 32 * kPPitch + (step >> 1) * 64 + h * (SG == 8 ? 32 : 16));
 #pragma unroll
-            for (int j = 0; j < NJ; j++) wf[j] = dequant_operand(word_of(b.w[j][h], word), zp.at[j][SG == 4 ? step >> 1 : 0], ones);
+            for (int j = 0; j < NJ; j++) wf[j] = dequant_operand(word_of(b.w[j][h], word), zp.at[j][SG == 8 ? step : SG == 4 ? step >> 1 : 0], ones);
 #pragma unroll
             for (int i = 0; i < kF; i++)
 #pragma unroll
@@ -830,11 +840,13 @@ int prefill_launch_wide(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) {
             default: return prefill_launch_direct<1, 2, 3>(ctx, a);
         }
     if (tile == 64) switch (SG) {
+            case 8: return prefill_launch_direct<8, 1, 1>(ctx, a);
             case 4: return prefill_launch_direct<4, 1, 1>(ctx, a);
             case 2: return prefill_launch_direct<2, 1, 1>(ctx, a);
             default: return prefill_launch_direct<1, 1, 1>(ctx, a);
         }
-    if (ctx->tune.prefill_direct != 0) switch (SG) {
+    if (ctx->tune.prefill_direct != 0 || SG == 8) switch (SG) {
+            case 8: return prefill_launch_direct<8, 2, 2>(ctx, a);
             case 4: return prefill_launch_direct<4, 2, 2>(ctx, a);
             case 2: return prefill_launch_direct<2, 2, 2>(ctx, a);
             default: return prefill_launch_direct<1, 2, 2>(ctx, a);
@@ -862,10 +874,11 @@ int prefill_launch(hipc_ctx *ctx, const PrefillArgs &a) {
     // 128x192 where that shortens the longest queue of a SIMD: rounds of workgroups over the CUs times the wavefront's
     // 32-column blocks (512 x 11008: 344 tiles of 128x128 are two rounds of 2, 232 of 128x192 one round of 3)
     const int64_t cus = std::max(1, ctx->cu_count);
-    if (tile == 128 && tiles128 >= 256 && ctx->tune.prefill_direct != 0 && ceil_div(tiles192, cus) * 3 < ceil_div(tiles128, cus) * 2) tile = 192;
-    if (forced == 64 || forced == 128 || (forced == 192 && ctx->tune.prefill_direct != 0)) tile = forced;
+    if (SG != 8 && tile == 128 && tiles128 >= 256 && ctx->tune.prefill_direct != 0 && ceil_div(tiles192, cus) * 3 < ceil_div(tiles128, cus) * 2) tile = 192;
+    if (forced == 64 || forced == 128 || (forced == 192 && SG != 8 && ctx->tune.prefill_direct != 0)) tile = forced;
     if (a.pair_rows > 0 && tile == 64) tile = 128;   // paired rows are the two row blocks of a wavefront: 128-row tiles
-    return tile == 64 && ctx->tune.prefill_direct == 0 ? prefill_launch_tile<SG, 64>(ctx, a) : prefill_launch_wide(ctx, a, SG, tile);
+    if constexpr (SG == 8) return prefill_launch_wide(ctx, a, SG, tile);   // (blocks of 16: one kernel; three column blocks leave no registers for the scales)
+    else return tile == 64 && ctx->tune.prefill_direct == 0 ? prefill_launch_tile<SG, 64>(ctx, a) : prefill_launch_wide(ctx, a, SG, tile);
 }
 
 }  // namespace
@@ -880,6 +893,7 @@ int nbits_prefill(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void
     a.A = static_cast<const __half *>(A), a.Wq = w->Wq, a.Sc = w->Sc, a.Zb = w->Zb, a.Y = static_cast<__half *>(Y);
     a.M = (int)M, a.K = (int)w->K, a.N = (int)w->N, a.n_tiles = w->n_tiles, a.n_cg = w->n_cg;
     switch (w->SG) {
+        case 8: return prefill_launch<8>(ctx, a);
         case 4: return prefill_launch<4>(ctx, a);
         case 2: return prefill_launch<2>(ctx, a);
         default: return prefill_launch<1>(ctx, a);
@@ -994,6 +1008,7 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
         a.A = A1, a.Wq = w->Wq, a.Sc = w->Sc, a.Zb = w->Zb, a.Y = nullptr, a.Yf32 = static_cast<float *>(Y), a.exps = exps;
         a.M = (int)M, a.K = (int)w->K, a.N = (int)w->N, a.n_tiles = w->n_tiles, a.n_cg = w->n_cg;
         switch (w->SG) {
+            case 8: return prefill_launch<8>(ctx, a);
             case 4: return prefill_launch<4>(ctx, a);
             case 2: return prefill_launch<2>(ctx, a);
             default: return prefill_launch<1>(ctx, a);
@@ -1001,7 +1016,7 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
     }
     // two terms: the pairs of the kernel that keeps the weight out of LDS; three (f32 pinned: all 24 bits), or the
     // kernel with both operands in LDS: `terms` M rows, and a launch that adds them
-    const bool paired = terms == 2 && ctx->tune.prefill_direct != 0;
+    const bool paired = terms == 2 && (ctx->tune.prefill_direct != 0 || w->SG == 8);
     const int64_t rows2 = paired ? 64 * ceil_div(M, 32) : terms * M;
     const size_t a2_bytes = (size_t)rows2 * w->K * sizeof(__half), e_bytes = ((size_t)M * sizeof(int) + 255) & ~(size_t)255;
     void *split = nullptr, *sums = nullptr;
@@ -1023,6 +1038,7 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
     if (paired) a.exps = exps, a.pair_rows = (int)M;
     int rc;
     switch (w->SG) {
+        case 8: rc = prefill_launch<8>(ctx, a); break;
         case 4: rc = prefill_launch<4>(ctx, a); break;
         case 2: rc = prefill_launch<2>(ctx, a); break;
         default: rc = prefill_launch<1>(ctx, a); break;

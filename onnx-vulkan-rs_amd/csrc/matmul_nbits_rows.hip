@@ -51,7 +51,7 @@ constexpr size_t kRowsHead = 128;
 __host__ __device__ inline int rows_pitch(int M) { return M | 1; }
 __host__ __device__ inline size_t rows_operands(int M, int terms, int stage_tiles) { return (size_t)stage_tiles * 4 * terms * 4 * rows_pitch(M) * 16; }
 
-// SG: scale groups per 128-k tile. NT: f16 terms per row. RB: blocks of 16 rows; NR: result registers per block in use (M <=
+// SG: scale groups per 128-k tile (8, 4, 2, 1 for blocks of 16, 32, 64, 128 and more). NT: f16 terms per row. RB: blocks of 16 rows; NR: result registers per block in use (M <=
 // 4 NR with one block: then register r of lane group g is row g + 4 r, else row 4 g + r). T: 16-column tiles per wavefront.
 // P: pieces of the rows a thread holds at most (kRowsPieces of f32, kRowsPieces16 of f16, or a quarter: a launch starts with
 // its instruction cache empty, and code for pieces that do not exist is 0.3 us a kilobyte).
@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
     struct Stage {
         uint4 wq[T];
         float s[T][SG > 1 ? SG : 1];
-        uint32_t z[T];
+        uint32_t z[T][SG == 8 ? 2 : 1];
     };
     // (buffer loads: what a lane adds is computed once, the tile's place is a scalar -- three instructions a tile instead of
     // a dozen. Every scalar offset is a tile's of the weight, the lane's part stays inside the tile.)
@@ -87,17 +87,24 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
         for (int t = 0; t < T; t++) {
             const uint32_t tl = (uint32_t)min(nt0 + t, p.n_tiles - 1) * (uint32_t)p.n_cg + (uint32_t)tile;
             st.wq[t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r_wq, v_wq, tl * 1024u, 0));
-            if constexpr (SG == 4) {
+            if constexpr (SG == 8) {
+                const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r_sc, v_sc, tl * 512u, 0));
+                const float4 u = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r_sc, v_sc + 16u, tl * 512u, 0));
+                const uint2 z = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r_zb, v_zb, tl * 128u, 0));
+                st.s[t][0] = v.x, st.s[t][1] = v.y, st.s[t][2] = v.z, st.s[t][3] = v.w;
+                st.s[t][4 % SG] = u.x, st.s[t][5 % SG] = u.y, st.s[t][6 % SG] = u.z, st.s[t][7 % SG] = u.w;
+                st.z[t][0] = z.x, st.z[t][SG == 8] = z.y;
+            } else if constexpr (SG == 4) {
                 const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r_sc, v_sc, tl * 256u, 0));
                 st.s[t][0] = v.x, st.s[t][1] = v.y, st.s[t][2] = v.z, st.s[t][3] = v.w;
-                st.z[t] = __builtin_amdgcn_raw_buffer_load_b32(r_zb, v_zb, tl * 64u, 0);
+                st.z[t][0] = __builtin_amdgcn_raw_buffer_load_b32(r_zb, v_zb, tl * 64u, 0);
             } else if constexpr (SG == 2) {
                 const float2 v = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r_sc, v_sc, tl * 128u, 0));
                 st.s[t][0] = v.x, st.s[t][1] = v.y;
-                st.z[t] = __builtin_amdgcn_raw_buffer_load_b16(r_zb, v_zb, tl * 32u, 0);
+                st.z[t][0] = __builtin_amdgcn_raw_buffer_load_b16(r_zb, v_zb, tl * 32u, 0);
             } else {
                 st.s[t][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_sc, v_sc, tl * 64u, 0));
-                st.z[t] = __builtin_amdgcn_raw_buffer_load_b8(r_zb, v_zb, tl * 16u, 0);
+                st.z[t][0] = __builtin_amdgcn_raw_buffer_load_b8(r_zb, v_zb, tl * 16u, 0);
             }
         }
     };
@@ -117,10 +124,17 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
     uint32_t ones = 0x64006400u;   // kept in a vector register (see and_or_1024)
     HIPC_PIN_VGPR(ones);
 
+    // blocks of 16: a product step of 32 k covers two of them, k groups 0 and 1 the first, 2 and 3 the second. Each is a
+    // product of its own with the other half of the weight operand zeroed (the matrix cores have the time)
+    const uint32_t first16 = SG == 8 && g4 < 2 ? ~0u : 0u;
+    const auto masked = [](const f16x8 &w, uint32_t keep) {
+        const uint4 v = __builtin_bit_cast(uint4, w);
+        return __builtin_bit_cast(f16x8, make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep));
+    };
     auto compute = [&](const Stage &st, int first_chunk) {
         f32x4 d[RB][T];
         ZeroPair z[T];
-        constexpr int CPG = 4 / SG;   // chunks per scale group
+        constexpr int CPG = SG == 8 ? 1 : 4 / SG;   // chunks per scale group
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             f16x8 a[RB][NT];
@@ -132,8 +146,27 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
             const int g = j / CPG;
 #pragma unroll
             for (int t = 0; t < T; t++) {
-                if (first) z[t] = zero_pair((st.z[t] >> (8 * g)) & 0xffu);
+                if constexpr (SG == 8) {
+                    z[t] = zero_pair((st.z[t][j >> 1] >> (16 * (j & 1) + (first16 ? 0 : 8))) & 0xffu);   // of the lane's own block
+                } else {
+                    if (first) z[t] = zero_pair((st.z[t][0] >> (8 * g)) & 0xffu);
+                }
                 const f16x8 w = dequant_operand(word_of(st.wq[t], j), z[t], ones);
+                if constexpr (SG == 8) {
+                    const f16x8 w0 = masked(w, first16), w1 = masked(w, ~first16);
+#pragma unroll
+                    for (int b = 0; b < RB; b++) {
+                        f32x4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = v0;
+#pragma unroll
+                        for (int e = NT - 1; e >= 0; e--) {
+                            v0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], w0, v0, 0, 0, 0);
+                            v1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], w1, v1, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int r = 0; r < NR; r++) acc[b][t][r] = fmaf(st.s[t][(2 * j + 1) % SG], v1[r], fmaf(st.s[t][2 * j % SG], v0[r], acc[b][t][r]));
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int b = 0; b < RB; b++) {
                     f32x4 v = first ? f32x4{0.f, 0.f, 0.f, 0.f} : d[b][t];
@@ -336,7 +369,7 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
 
 // Y = sum over the workgroups' partial rows, in order, times 2^exps[row] where given; four results per thread
 template <bool VEC>   // VEC: N is a multiple of four and Y's rows take 16-byte (f16: 8-byte) stores
-__global__ void __launch_bounds__(64)
+static __global__ void __launch_bounds__(64)
 mmnb_rows_join_kernel(const float *__restrict__ part, void *__restrict__ Y, long total, int splits, int N, const int *__restrict__ exps, int y_f16) {
     const long i = ((long)blockIdx.x * 64 + threadIdx.x) * (VEC ? 4 : 1);
     if (i >= total) return;
@@ -394,15 +427,16 @@ struct RowsPlan {
 // column tile: 24 x 2048 x 8320 9.2 us without that term, 7.6 with it), and a split costs a second launch, some 6000 clocks with its own trip through memory.
 bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT, int RB, int NR, RowsPlan *best) {
     const int cus = std::max(1, ctx->cu_count), max_waves = kRowsWaves;
+    const int most_splits = std::min(w->n_cg, std::max(16, (int)ceil_div(w->n_cg, 8)));   // (up to eight tiles of k fit any launch)
     double best_cost = 0;
     bool found = false;
     static const int shapes[][2] = {{4, 1}, {2, 1}, {1, 1}, {2, 2}, {1, 2}};   // column tiles per wavefront, wavefronts side by side
     for (const auto &shape : shapes) {
-        if (RB > 2 && shape[0] == 4) continue;   // (registers)
+        if ((RB > 2 || w->SG == 8) && shape[0] == 4) continue;   // (registers)
         if ((NT * M > 64) != (shape[1] > 1)) continue;   // a stage is at least a round of the wavefronts along k: eight of them only up to 64 rows
         const int cw = shape[0] * shape[1];
         const int64_t groups = ceil_div(w->n_tiles, cw);
-        for (int splits = 1; splits <= 16 && splits <= w->n_cg; splits++) {
+        for (int splits = 1; splits <= most_splits; splits++) {
             const int st = (int)ceil_div(w->n_cg, splits);
             if ((int)ceil_div(w->n_cg, st) != splits) continue;
             RowsPlan pl;
@@ -463,10 +497,14 @@ int rows_launch(hipc_ctx *ctx, const RowsArgs &a, const RowsPlan &pl) {
 template <int SRC, int NT, int RB, int NR, int T>
 int rows_launch_sg(hipc_ctx *ctx, const RowsArgs &a, const RowsPlan &pl, int SG) {
     switch (SG) {
+        case 8:
+            if constexpr (T <= 2) return rows_launch<8, SRC, NT, RB, NR, T>(ctx, a, pl);
+            break;   // (rows_plan: never)
         case 4: return rows_launch<4, SRC, NT, RB, NR, T>(ctx, a, pl);
         case 2: return rows_launch<2, SRC, NT, RB, NR, T>(ctx, a, pl);
-        default: return rows_launch<1, SRC, NT, RB, NR, T>(ctx, a, pl);
+        case 1: return rows_launch<1, SRC, NT, RB, NR, T>(ctx, a, pl);
     }
+    return fail(ctx, HIPC_ERR_INVALID, "MatMulNBits rows: no kernel for %d scale groups and %d column tiles", SG, T);
 }
 template <int SRC, int NT, int RB, int NR>
 int rows_run(hipc_ctx *ctx, RowsArgs a, const hipc_nbits_weight *w) {
@@ -500,19 +538,8 @@ int rows_run(hipc_ctx *ctx, RowsArgs a, const hipc_nbits_weight *w) {
 
 }  // namespace
 
-// Which row counts come here (kernel time of the call, before -> after; the streaming kernel 16 rows at a time, the tiled
-// kernel from 17 rows of f16 and 33 of f32 on): 8 x 1152 x 13824 11.5 -> 7.4 us, 16 rows 23 -> 9.8, 32 rows 46 -> 21; 8 x 6912
-// x 1152 10.4 -> 8.6, 16 rows 19 -> 10.2; f16 2048 -> 11008: 1 row 7.3 -> 6.5, 4 rows 11.2 -> 6.5, 16 rows 24 -> 7.8, 17 rows
-// 11.3 -> 8.6; 24 x 512 -> 1152 5.4 -> 4.5, but -> 16384 5.5 -> 5.9. From 33 rows on only where the tiled kernel has few tiles: f16 48 x 6912 x 1152 27.4 -> 11.6, but 48 x 4096 x
-// 4096 18.1 -> 21.4; f32 (which the tiled kernel takes 64 rows at a time) 48 x 6912 x 1152 41 -> 22.7, 48 x 4096 x 4096 39 ->
-// 25, but 64 x 2048 x 8192 32.6 -> 37. A weight of 2048 column tiles or more and up to 16 rows stay on the streaming kernel,
-// whose wavefronts each walk all of k and meet nobody: 4 x 1152 x 262144 35.7 us there (5.5 TB/s), 50 here.
-bool nbits_rows_takes(const void *A, const hipc_nbits_weight *w, int64_t M, int terms) {
-    if (M > kFewRows || terms * M > 128 || w->K % 8 != 0 || !aligned(A, 16)) return false;
-    if (M <= 16) return w->n_tiles < 2048;
-    if (M <= 32) return terms > 1 || w->n_tiles <= 300 || w->n_cg > 4;
-    return w->n_tiles <= (terms > 1 ? 300 : 128);
-}
+// (this file is compiled twice: HIPC_ROWS_F16 is the half whose rows arrive as f16)
+#ifdef HIPC_ROWS_F16
 
 // rows of f16, `terms` of them per row of the result (term e of row m is row e M + m of A); exps / y_f16 as in RowsArgs
 int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, const hipc_nbits_weight *w, void *Y, int y_f16, int M) {
@@ -525,6 +552,23 @@ int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, con
     if (M <= 16) return rows_run<SRC_F16, 1, 1, 4>(ctx, a, w);
     return M <= 32 ? rows_run<SRC_F16, 1, 2, 4>(ctx, a, w) : rows_run<SRC_F16, 1, 4, 4>(ctx, a, w);
 }
+
+#else
+
+// Which row counts come here (kernel time of the call, before -> after; the streaming kernel 16 rows at a time, the tiled
+// kernel from 17 rows of f16 and 33 of f32 on): 8 x 1152 x 13824 11.5 -> 7.4 us, 16 rows 23 -> 9.8, 32 rows 46 -> 21; 8 x 6912
+// x 1152 10.4 -> 8.6, 16 rows 19 -> 10.2; f16 2048 -> 11008: 1 row 7.3 -> 6.5, 4 rows 11.2 -> 6.5, 16 rows 24 -> 7.8, 17 rows
+// 11.3 -> 8.6; 24 x 512 -> 1152 5.4 -> 4.5, but -> 16384 5.5 -> 5.9. From 33 rows on only where the tiled kernel has few tiles: f16 48 x 6912 x 1152 27.4 -> 11.6, but 48 x 4096 x
+// 4096 18.1 -> 21.4; f32 (which the tiled kernel takes 64 rows at a time) 48 x 6912 x 1152 41 -> 22.7, 48 x 4096 x 4096 39 ->
+// 25, but 64 x 2048 x 8192 32.6 -> 37. A weight of 2048 column tiles or more and up to 16 rows stay on the streaming kernel,
+// whose wavefronts each walk all of k and meet nobody: 4 x 1152 x 262144 35.7 us there (5.5 TB/s), 50 here.
+bool nbits_rows_takes(const void *A, const hipc_nbits_weight *w, int64_t M, int terms) {
+    if (M > kFewRows || terms * M > 128 || w->K % 8 != 0 || !aligned(A, 16)) return false;
+    if (M <= 16) return w->n_tiles < 2048 || w->SG == 8;   // (the streaming kernel has no form for blocks of 16)
+    if (M <= 32) return terms > 1 || w->n_tiles <= 300 || w->n_cg > 4;
+    return w->n_tiles <= (terms > 1 ? 300 : 128);
+}
+
 // up to 16 rows of f32, as two f16 terms or three
 int nbits_rows_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms) {
     RowsArgs a{};
@@ -532,5 +576,7 @@ int nbits_rows_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, voi
     if (terms == 3) return M <= 4 ? rows_run<SRC_F32, 3, 1, 1>(ctx, a, w) : M <= 8 ? rows_run<SRC_F32, 3, 1, 2>(ctx, a, w) : rows_run<SRC_F32, 3, 1, 4>(ctx, a, w);
     return M <= 4 ? rows_run<SRC_F32, 2, 1, 1>(ctx, a, w) : M <= 8 ? rows_run<SRC_F32, 2, 1, 2>(ctx, a, w) : rows_run<SRC_F32, 2, 1, 4>(ctx, a, w);
 }
+
+#endif
 
 }  // namespace hipc

@@ -139,7 +139,7 @@ int main() {
     // (M, K, N, block, zero points): ragged in every direction, a partial last stage, an odd stage count, one tile,
     // more tiles than one XCD rectangle holds, every scale grouping
     const int64_t shapes[][5] = {{17, 72, 16, 32, 1},   {100, 1000, 200, 32, 1}, {130, 384, 131, 64, 1}, {257, 640, 96, 128, 1},
-                                 {64, 256, 1024, 256, 0}, {129, 512, 392, 64, 0},  {300, 1152, 200, 128, 1}};
+                                 {64, 256, 1024, 256, 0}, {129, 512, 392, 64, 0},  {300, 1152, 200, 128, 1}, {131, 520, 392, 16, 1}};
     for (const auto &s : shapes) {
         product(s[0], s[1], s[2], s[3], s[4] != 0, HIPC_F16);
         if (s[0] > 32) product(s[0], s[1], s[2], s[3], s[4] != 0, HIPC_F32);
@@ -154,7 +154,9 @@ int main() {
                               // the kernel for a few rows: one, two and four row blocks, stages that end in the middle of k,
                               // k split over workgroups, a last tile of k with 8 values, one to four column tiles per wavefront
                               {2, 1152, 13824, 32, 1}, {8, 6912, 1152, 32, 1}, {16, 2056, 4100, 64, 1}, {13, 136, 40, 128, 0}, {23, 1288, 1152, 32, 1},
-                              {32, 4104, 272, 128, 0}, {33, 1152, 600, 64, 1}, {64, 2048, 1030, 32, 1}, {50, 520, 13824, 32, 0}};
+                              {32, 4104, 272, 128, 0}, {33, 1152, 600, 64, 1}, {64, 2048, 1030, 32, 1}, {50, 520, 13824, 32, 0},
+                              // blocks of 16
+                              {1, 1160, 1030, 16, 1}, {8, 2048, 600, 16, 0}, {40, 520, 1030, 16, 1}};
     for (const auto &s : few)
         for (int dt : {HIPC_F32, HIPC_F16}) rows(s[0], s[1], s[2], s[3], s[4] != 0, dt);
     gpu_model::Registry &g = gpu_model::reg();

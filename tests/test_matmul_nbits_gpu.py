@@ -478,3 +478,27 @@ def test_a_few_rows_of_very_different_size(ctx, pkg, oracle, m, level):
     for r in range(m):   # each row against its own size
         assert np.max(np.abs(got[r] - want[r])) <= 1e-5 * max(np.max(np.abs(want[r])), 1e-37), r
     w.destroy()
+
+
+@pytest.mark.parametrize("dtype,level", [(np.float16, 0), (np.float32, 0), (np.float32, 4)])
+@pytest.mark.parametrize("shape", [(1, 1160, 1030), (2, 512, 1040), (16, 2056, 200), (20, 136, 600), (43, 1288, 96), (65, 1000, 131), (130, 648, 400), (300, 1152, 1100)],
+                         ids=lambda s: "M%d_K%d_N%d" % s)
+def test_blocks_of_sixteen_on_the_matrix_cores(ctx, pkg, oracle, shape, dtype, level):
+    """Blocks of 16, two to a product step of the kernel for a few rows, one to a step of the tiled kernel (64- and
+    128-row tiles): a last block with eight values, an odd number of blocks, rows that do not start on 16 bytes."""
+    m, k, n = shape
+    B, scales, zp = pkg.synth.nbits_weight(n, k, 16, seed=600 + n, scale_dtype=dtype)
+    a = pkg.synth.normal_f32(m * k, 601).reshape(m, k).astype(dtype)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, 16)
+    want = oracle.matmul_nbits(a, B, scales, zp, k, n, 16)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, 16, accuracy_level=level, weight=w)
+    assert got.dtype == dtype
+    if level:    # one f16 term of a row from 33 rows on: 11 bits of every value
+        assert worst(got, want) <= 1e-3 * np.abs(want).max()
+    else:
+        assert close(got, want, RTOL16 if dtype == np.float16 else RTOL32), worst(got, want)
+    moved = ctx.upload(np.concatenate([np.zeros(2, dtype), a.reshape(-1)]))
+    out = ctx.alloc(m * n * a.itemsize)
+    pkg.ops.matmul_nbits_packed_device(ctx, moved.at(2 * a.itemsize), pkg.ops.hipc_dtype(a.dtype), w, out, m, level)
+    assert np.array_equal(ctx.download(out, dtype, (m, n)), got)
+    moved.free(), out.free(), w.destroy()
