@@ -13,15 +13,14 @@
 // match. Padding taps read the zero point, so they contribute nothing and the
 // zero-point algebra of the plain matmul applies unchanged
 // (shaders/conv_integer.rs:112-119, 350-371).
-// A window along one axis (H = 1, 1 x kw: the vocoder shapes) skips even that
-// copy: each workgroup reads the input positions its 64 outputs see straight
-// from NCHW, transposes them in registers and keeps them in LDS for the whole
-// product (int8_conv_row_kernel).
-// Grouped convolutions and channel counts that are not multiples of 16 take a
-// direct kernel, one output per thread, as the reference does for grouped ones.
+// That is the general route. What most convolutions take skips even that copy: each workgroup reads the input positions its
+// 64 or 128 outputs see straight from NCHW, transposes them in registers and keeps them in LDS for the whole product --
+// int8_conv_slab_kernel (int8_conv_slab.h), and for few tiles along one axis int8_conv_row_kernel.
+// Grouped convolutions, and what fits neither (channel counts off 16 whose slab exceeds LDS), take a direct kernel, one
+// output per thread.
 #include <algorithm>
 
-#include "int8_gemm.h"
+#include "int8_conv_slab.h"
 
 namespace hipc {
 
@@ -109,6 +108,42 @@ pack_conv_w_kernel(const uint8_t *__restrict__ W, uint8_t *__restrict__ Wp, int3
     if (threadIdx.x == 0) rowsum[o] = part[0];
 }
 
+// W [O, C, kh, kw] -> fragment-major bytes in the step order of int8_conv_slab_kernel: a step is 32 k of one tap, or, with a
+// single 16-channel chunk (kw2: pairs of taps per filter row), 16 channels of two taps. Zeros where there is no channel or tap.
+__global__ void __launch_bounds__(256)
+pack_conv_slab_kernel(const uint8_t *__restrict__ W, uint8_t *__restrict__ Ws, int32_t *__restrict__ rowsum, int O, int C,
+                      int kh, int kw, int kw2, int npair, int steps, int is_signed, int shift) {
+    const int o = blockIdx.x;
+    const bool tap_pairs = C <= 16;
+    int local = 0;
+    for (int k = threadIdx.x; k < steps * 32; k += 256) {
+        const int step = k >> 5, half = (k >> 4) & 1;
+        int r, t, c;
+        if (tap_pairs) {
+            r = step / kw2, t = 2 * (step - r * kw2) + half, c = k & 15;
+        } else {
+            const int tap = step / npair;
+            r = tap / kw, t = tap - r * kw, c = (step - tap * npair) * 32 + (k & 31);
+        }
+        uint8_t out = 0;
+        if (o < O && c < C && t < kw) {
+            const uint8_t v = W[((size_t)o * C + c) * kh * kw + r * kw + t];
+            const int sv = (is_signed ? (int)(int8_t)v : (int)v) - shift;
+            local += sv;
+            out = (uint8_t)sv;
+        }
+        Ws[qfrag_offset(o, k, steps * 32)] = out;
+    }
+    __shared__ int part[256];
+    part[threadIdx.x] = local;
+    __syncthreads();
+    for (int n = 128; n > 0; n >>= 1) {
+        if (threadIdx.x < n) part[threadIdx.x] += part[threadIdx.x + n];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) rowsum[o] = part[0];
+}
+
 struct DirectConvArgs {
     const uint8_t *X, *W;
     const uint8_t *x_zp, *w_zp;
@@ -172,6 +207,7 @@ struct hipc_conv_weight {
     int w_dtype = HIPC_I8;
     uint8_t *raw = nullptr;  // ONNX layout copy, for the direct path
     uint8_t *Wp = nullptr;   // [O_pad, K_pad], (kh, kw, c) order; null when the MFMA path does not apply
+    uint8_t *Ws = nullptr;   // the same in the step order of int8_conv_slab_kernel; null where that is Wp's own, or group > 1
     int32_t *rowsum = nullptr;
     int O_pad = 0, K_pad = 0;
     mutable hipc::RatioCache ratios;  // QLinearConv's requantisation ratios as last used
@@ -216,6 +252,102 @@ struct ConvEpilogue {
     int y_zp = 0, out_signed = 0;
 };
 
+// one output per thread, any geometry
+int run_direct(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *W, const void *x_zp, const void *w_zp,
+               int host_zp, int x_zp_value, int w_zp_value, const hipc_conv_geom *g, int64_t ho, int64_t wo, void *Y, const ConvEpilogue &ep) {
+    const int64_t total = g->n * g->c_out * ho * wo;
+    DirectConvArgs d{};
+    d.X = static_cast<const uint8_t *>(X), d.W = W->raw;
+    d.x_zp = static_cast<const uint8_t *>(x_zp), d.w_zp = static_cast<const uint8_t *>(w_zp);
+    d.x_signed = x_dtype == HIPC_I8, d.w_signed = W->w_dtype == HIPC_I8;
+    d.host_zp = host_zp, d.x_zp_value = x_zp_value, d.w_zp_value = w_zp_value;
+    d.n = (int)g->n, d.C = (int)g->c_in, d.H = (int)g->h, d.Wd = (int)g->w, d.O = (int)g->c_out;
+    d.kh = (int)g->kh, d.kw = (int)g->kw, d.sh = (int)g->stride_h, d.sw = (int)g->stride_w, d.dh = (int)g->dil_h,
+    d.dw = (int)g->dil_w, d.pt = (int)g->pad_top, d.pl = (int)g->pad_left, d.group = (int)g->group;
+    d.Ho = (int)ho, d.Wo = (int)wo;
+    d.Y = Y;
+    d.requant = ep.requant, d.ratio = ep.ratio, d.ratio_step = ep.ratio_step, d.qbias = ep.qbias, d.y_zp = ep.y_zp,
+    d.out_signed = ep.out_signed;
+    hipLaunchKernelGGL((conv_direct_kernel), dim3((unsigned)ceil_div(total, 256)), 256, 0, ctx->stream, d);
+    HIPC_LAUNCHED(ctx);
+    if (host_zp) {
+        note_scalar(ctx, HIPC_SCALAR_A_ZERO_POINT, offsetof(DirectConvArgs, x_zp_value));
+        note_scalar(ctx, HIPC_SCALAR_B_ZERO_POINT, offsetof(DirectConvArgs, w_zp_value));
+    }
+    if (ep.requant) note_scalar(ctx, HIPC_SCALAR_Y_ZERO_POINT, offsetof(DirectConvArgs, y_zp));
+    return HIPC_OK;
+}
+
+// product steps of int8_conv_slab_kernel: chunks, pairs of them per tap, taps or pairs of taps per filter row
+void slab_steps(const hipc_conv_geom &g, ConvSlabArgs *a) {
+    a->nch = (int)ceil_div(g.c_in, 16);
+    const bool tap_pairs = a->nch == 1;
+    a->npair = tap_pairs ? 1 : (a->nch + 1) / 2;
+    a->kw2 = (int)(tap_pairs ? ceil_div(g.kw, 2) : g.kw);
+    a->pairs = tap_pairs;
+    a->steps = (int)g.kh * a->kw2 * a->npair;
+}
+
+template <int EPI, bool DYN, int WK, int WP, bool RAGGED>
+int slab_launch(hipc_ctx *ctx, const ConvSlabArgs &a, size_t lds) {
+    static bool lds_allowed[kMaxDevices] = {};
+    if (int rc = allow_dynamic_lds(ctx, int8_conv_slab_kernel<EPI, DYN, WK, WP, RAGGED>, kSlabLds, lds_allowed)) return rc;
+    hipLaunchKernelGGL((int8_conv_slab_kernel<EPI, DYN, WK, WP, RAGGED>), dim3(8u * (unsigned)a.per_xcd), 256, lds, ctx->stream, a);
+    HIPC_LAUNCHED(ctx);
+    gemm_note_scalars(ctx, a.g, DYN);
+    return HIPC_OK;
+}
+template <int EPI, bool DYN, int WK, int WP>
+int slab_launch_ragged(hipc_ctx *ctx, const ConvSlabArgs &a, size_t lds) {
+    return a.g.C % 16 ? slab_launch<EPI, DYN, WK, WP, true>(ctx, a, lds) : slab_launch<EPI, DYN, WK, WP, false>(ctx, a, lds);
+}
+template <int WK, int WP>
+int slab_launch_as(hipc_ctx *ctx, ConvSlabArgs a, size_t lds, bool requant, bool sums) {
+    a.adv_tap = WK / a.npair, a.adv_q = WK % a.npair;
+    if (requant) return sums ? slab_launch_ragged<EPI_REQUANT, true, WK, WP>(ctx, a, lds) : slab_launch_ragged<EPI_REQUANT, false, WK, WP>(ctx, a, lds);
+    return sums ? slab_launch_ragged<EPI_I32, true, WK, WP>(ctx, a, lds) : slab_launch_ragged<EPI_I32, false, WK, WP>(ctx, a, lds);
+}
+
+// positions a slab of int8_conv_slab_kernel needs for `tile` consecutive outputs, whichever they are: rounded up to fours
+// from a multiple of four on, and the padding position
+int64_t slab_positions(const hipc_conv_geom &g, int64_t ho, int64_t wo, int64_t tile) {
+    tile = std::min(tile, ho * wo);
+    const int64_t rows = wo % tile == 0 ? 1 : tile % wo == 0 ? tile / wo : std::min(ho, (tile + wo - 2) / wo + 1);
+    const int64_t span = (g.kh - 1) * g.dil_h + 1;
+    const int64_t within = (std::min(g.h, span) - 1) * g.w + std::min(g.w, (std::min(tile, wo) - 1) * g.stride_w + (g.kw - 1) * g.dil_w + 1);
+    const int64_t across = rows > 1 ? std::min(g.h, (rows - 1) * g.stride_h + span) * g.w : 0;
+    return (std::max(within, across) + 3 + 3) / 4 * 4 + 2;
+}
+
+// The slab kernel, where what 64 outputs see of the input fits LDS (*taken).
+int run_slab(hipc_ctx *ctx, const GemmArgs &ga, const hipc_conv_weight *W, const hipc_conv_geom *g, int64_t ho, int64_t wo, bool requant, bool sums, bool *taken) {
+    *taken = false;
+    if (g->h * g->w < 4) return HIPC_OK;
+    ConvSlabArgs a{};
+    a.g = ga;
+    slab_steps(*g, &a);
+    a.frag_steps = W->Ws ? a.steps : W->K_pad / 32;
+    if (W->Ws) a.g.P = W->Ws;
+    const auto slab_of = [&](int64_t tile) { return (size_t)a.nch * slab_positions(*g, ho, wo, tile) * 16; };
+    const auto lds_of = [&](int64_t tile) { return slab_of(tile) + (size_t)(g->kh * a.kw2 * (a.pairs ? 2 : 1) * tile * 2); };
+    const int64_t J = ho * wo, cus = std::max(1, ctx->cu_count), o64 = ceil_div(g->c_out, 64);
+    // Few tiles of 64 x 64 and enough steps to share: the four wavefronts of a workgroup split k. Else a wavefront keeps its k
+    // to itself and takes 32 channels: 128 channels x 64 positions, or, where the channels would leave wavefronts of the
+    // last tile idle, 64 x 128.
+    const bool by_k = o64 * ceil_div(J, 64) * g->n <= 2 * cus && a.steps >= 8;
+    const bool wide = !by_k && o64 % 2 == 1 && o64 <= 3 && J > 64 && lds_of(128) <= kSlabLds;
+    const int tile = wide ? 128 : 64;
+    size_t lds = lds_of(tile);
+    if (lds > kSlabLds) return HIPC_OK;
+    *taken = true;
+    if (by_k) lds = std::max(lds, kSmallLds);
+    a.SP = (int)slab_positions(*g, ho, wo, tile), a.tab_at = (int)slab_of(tile);
+    a.o_tiles = (int)(by_k || wide ? o64 : ceil_div(g->c_out, 128)), a.p_tiles = (int)ceil_div(J, tile);
+    a.items = (int)((int64_t)a.o_tiles * a.p_tiles * g->n), a.per_xcd = (int)ceil_div(a.items, 8);
+    a.by_o_tiles = magic_of((uint32_t)a.o_tiles), a.by_p_tiles = magic_of((uint32_t)a.p_tiles), a.by_wo = magic_of((uint32_t)wo);
+    return by_k ? slab_launch_as<4, 1>(ctx, a, lds, requant, sums) : wide ? slab_launch_as<1, 2>(ctx, a, lds, requant, sums) : slab_launch_as<1, 1>(ctx, a, lds, requant, sums);
+}
+
 int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *W, const void *x_zp, const void *w_zp,
              int host_zp, int x_zp_value, int w_zp_value, const hipc_conv_geom *g, void *Y, const ConvEpilogue &ep) {
     int64_t ho = 0, wo = 0;
@@ -228,7 +360,7 @@ int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *
     if (total == 0) return HIPC_OK;
     HIPC_REQUIRE(ctx, X && Y, "Conv: null tensor");
 
-    if (W->Wp) {
+    if (W->rowsum) {
         GemmArgs ga{};
         ga.P = W->Wp;
         ga.const_sum = W->rowsum;
@@ -243,23 +375,22 @@ int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *
         ga.Y = Y;
         ga.ratio = ep.ratio, ga.ratio_step = ep.ratio_step, ga.qbias = ep.qbias, ga.y_zp = ep.y_zp,
         ga.out_signed = ep.out_signed;
-        HIPC_REQUIRE(ctx, g->n <= 65535, "Conv: batch %ld too large", (long)g->n);
+        // the row sums of the activations only matter when the weight's zero point, in the signed domain, is not zero
+        const bool zero_known = ga.const_shift == 0 && (host_zp ? w_zp_value == 0 : w_zp == nullptr);
         // few 64x64 tiles and a long k: the wavefronts of a workgroup split k and the weight stays out of LDS
         // (the gemm_small option, 0 / 1, overrides: tuning, tests)
         const int forced = ctx->tune.gemm_small;
         const int64_t tiles64 = ceil_div(ga.I, 64) * ceil_div(ga.J, 64) * g->n;
         const bool small = forced >= 0 ? forced != 0 : (tiles64 <= 2 * (int64_t)ctx->cu_count && ga.K_pad >= 4 * kBK);
-        // the row sums of the activations only matter when the weight's zero point, in the signed domain, is not zero
-        const bool zero_known = ga.const_shift == 0 && (host_zp ? w_zp_value == 0 : w_zp == nullptr);
 
-        // A convolution along W alone whose per-tile input slab fits LDS reads the NCHW activation
-        // directly: no transposed copy at all, whatever the number of tiles (on 8 x 512 x 4096 inputs,
-        // k = 7, it still finishes before the tiled route: 120 against 147 us).
+        // A convolution along W alone with few tiles, whose input slab fits LDS: the kernel made for it, one instruction
+        // cheaper wherever int8_conv_slab_kernel allows for rows, padding and odd addresses (192 x 4096, k = 7: 6.5 against
+        // 7.0 us; with more tiles than two per CU that kernel does not split k and is the faster one).
         // The conv_row option set to 0 takes the general route (tuning, tests).
         const bool row_off = ctx->tune.conv_row == 0;
         const int64_t slab_pos = (3 + 63 * g->stride_w + (g->kw - 1) * g->dil_w + 1 + 3) / 4 * 4;
         const size_t slab_bytes = (size_t)(slab_pos * g->c_in);
-        if (!row_off && g->h == 1 && g->kh == 1 && ho == 1 && g->pad_top == 0 && g->w % 4 == 0 && aligned(X, 4) &&
+        if (W->Wp && !row_off && tiles64 <= 2 * (int64_t)ctx->cu_count && g->h == 1 && g->kh == 1 && ho == 1 && g->pad_top == 0 && g->w % 4 == 0 && aligned(X, 4) &&
             slab_bytes <= 64 * 1024) {
             ga.Q = static_cast<const uint8_t *>(X);
             ga.slab_pos = (int)slab_pos;
@@ -277,6 +408,15 @@ int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *
             return HIPC_OK;
         }
 
+        // any other whose slab fits
+        ga.Q = static_cast<const uint8_t *>(X);
+        bool taken = false;
+        if (!row_off) {
+            rc = run_slab(ctx, ga, W, g, ho, wo, ep.requant != 0, !zero_known, &taken);
+            if (taken) return rc;
+        }
+        if (!W->Wp) return run_direct(ctx, X, x_dtype, W, x_zp, w_zp, host_zp, x_zp_value, w_zp_value, g, ho, wo, Y, ep);
+        HIPC_REQUIRE(ctx, g->n <= 65535, "Conv: batch %ld too large", (long)g->n);
         // NHWC copy of the activation, shifted to the signed domain
         void *xt = nullptr;
         const size_t x_bytes = (size_t)(g->n * g->c_in * g->h * g->w);
@@ -308,26 +448,7 @@ int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *
                           : gemm_launch<MODE_CONV, EPI_I32, true>(ctx, ga, (unsigned)g->n);
     }
 
-    DirectConvArgs d{};
-    d.X = static_cast<const uint8_t *>(X), d.W = W->raw;
-    d.x_zp = static_cast<const uint8_t *>(x_zp), d.w_zp = static_cast<const uint8_t *>(w_zp);
-    d.x_signed = x_dtype == HIPC_I8, d.w_signed = W->w_dtype == HIPC_I8;
-    d.host_zp = host_zp, d.x_zp_value = x_zp_value, d.w_zp_value = w_zp_value;
-    d.n = (int)g->n, d.C = (int)g->c_in, d.H = (int)g->h, d.Wd = (int)g->w, d.O = (int)g->c_out;
-    d.kh = (int)g->kh, d.kw = (int)g->kw, d.sh = (int)g->stride_h, d.sw = (int)g->stride_w, d.dh = (int)g->dil_h,
-    d.dw = (int)g->dil_w, d.pt = (int)g->pad_top, d.pl = (int)g->pad_left, d.group = (int)g->group;
-    d.Ho = (int)ho, d.Wo = (int)wo;
-    d.Y = Y;
-    d.requant = ep.requant, d.ratio = ep.ratio, d.ratio_step = ep.ratio_step, d.qbias = ep.qbias, d.y_zp = ep.y_zp,
-    d.out_signed = ep.out_signed;
-    hipLaunchKernelGGL((conv_direct_kernel), dim3((unsigned)ceil_div(total, 256)), 256, 0, ctx->stream, d);
-    HIPC_LAUNCHED(ctx);
-    if (host_zp) {
-        note_scalar(ctx, HIPC_SCALAR_A_ZERO_POINT, offsetof(DirectConvArgs, x_zp_value));
-        note_scalar(ctx, HIPC_SCALAR_B_ZERO_POINT, offsetof(DirectConvArgs, w_zp_value));
-    }
-    if (ep.requant) note_scalar(ctx, HIPC_SCALAR_Y_ZERO_POINT, offsetof(DirectConvArgs, y_zp));
-    return HIPC_OK;
+    return run_direct(ctx, X, x_dtype, W, x_zp, w_zp, host_zp, x_zp_value, w_zp_value, g, ho, wo, Y, ep);
 }
 
 }  // namespace
@@ -371,11 +492,23 @@ int hipc_prepack_conv_w(hipc_ctx *ctx, const void *W, int w_dtype, const hipc_co
         if (e == hipSuccess)
             e = hipMemcpyAsync(w->raw, W, raw_bytes, hipMemcpyDeviceToDevice, ctx->stream);
         const bool mfma = g->group == 1 && g->c_in % 16 == 0;
-        if (e == hipSuccess && mfma) {
+        if (e == hipSuccess && g->group == 1) {
             w->O_pad = (int)(ceil_div(g->c_out, kBM) * kBM);
+            e = hipMalloc(reinterpret_cast<void **>(&w->rowsum), (size_t)w->O_pad * 4);
+        }
+        if (e == hipSuccess && g->group == 1 && g->c_in % 32 != 0) {
+            ConvSlabArgs a{};
+            slab_steps(*g, &a);
+            e = hipMalloc(reinterpret_cast<void **>(&w->Ws), (size_t)w->O_pad * a.steps * 32);
+            if (e == hipSuccess) {
+                hipLaunchKernelGGL((pack_conv_slab_kernel), dim3((unsigned)w->O_pad), 256, 0, ctx->stream, static_cast<const uint8_t *>(W), w->Ws, w->rowsum, (int)g->c_out, (int)g->c_in, (int)g->kh, (int)g->kw,
+                    a.kw2, a.npair, a.steps, w_dtype == HIPC_I8, w_dtype == HIPC_U8 ? 128 : 0);
+                e = hipGetLastError();
+            }
+        }
+        if (e == hipSuccess && mfma) {
             w->K_pad = (int)(ceil_div(g->c_in * g->kh * g->kw, kBK) * kBK);
             e = hipMalloc(reinterpret_cast<void **>(&w->Wp), (size_t)w->O_pad * w->K_pad);
-            if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&w->rowsum), (size_t)w->O_pad * 4);
             if (e == hipSuccess) {
                 hipLaunchKernelGGL((pack_conv_w_kernel), dim3((unsigned)w->O_pad), 256, 0, ctx->stream, static_cast<const uint8_t *>(W), w->Wp, w->rowsum, (int)g->c_out, (int)g->c_in, (int)g->kh, (int)g->kw,
                     w->O_pad, w->K_pad, w_dtype == HIPC_I8, w_dtype == HIPC_U8 ? 128 : 0);
@@ -385,6 +518,7 @@ int hipc_prepack_conv_w(hipc_ctx *ctx, const void *W, int w_dtype, const hipc_co
         if (e != hipSuccess) {
             if (w->raw) (void)hipFree(w->raw);
             if (w->Wp) (void)hipFree(w->Wp);
+            if (w->Ws) (void)hipFree(w->Ws);
             if (w->rowsum) (void)hipFree(w->rowsum);
             delete w;
             return fail(ctx, HIPC_ERR_BACKEND, "Conv prepack: %s", hipGetErrorString(e));
@@ -399,6 +533,7 @@ void hipc_conv_weight_destroy(hipc_ctx *ctx, hipc_conv_weight *w) {
     entry_void(ctx, [&] {
         if (w->raw) ctx->deferred.push_back(w->raw);
         if (w->Wp) ctx->deferred.push_back(w->Wp);
+        if (w->Ws) ctx->deferred.push_back(w->Ws);
         if (w->rowsum) ctx->deferred.push_back(w->rowsum);
         ratio_release(ctx, w->ratios);
         delete w;

@@ -764,9 +764,7 @@ struct ConvChannel {
     float ratio = 0.f;
 };
 template <int EPI>
-__device__ __forceinline__ ConvChannel conv_small_channel(const GemmArgs &p, int i0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ch = i0 + (wave >> 1) * 32 + (lane & 31);
+__device__ __forceinline__ ConvChannel conv_channel(const GemmArgs &p, int ch) {
     ConvChannel c;
     c.csum = p.const_sum[ch];  // I_pad rows exist
     const int cc = min(ch, p.I - 1);
@@ -775,6 +773,41 @@ __device__ __forceinline__ ConvChannel conv_small_channel(const GemmArgs &p, int
         if (p.qbias) c.qb = p.qbias[cc];
     }
     return c;
+}
+template <int EPI>
+__device__ __forceinline__ ConvChannel conv_small_channel(const GemmArgs &p, int i0) {
+    return conv_channel<EPI>(p, i0 + (int)(threadIdx.x >> 7) * 32 + (int)(threadIdx.x & 31));
+}
+// A lane's 16 finished outputs of channel `ch` and of the 32 positions from `j0` on, as four runs of four. Four bytes leave as
+// one store wherever they begin (the hardware takes any address), four int32 where the row allows 16-byte stores.
+template <int EPI>
+__device__ __forceinline__ void conv_store(const GemmArgs &p, const ConvChannel &chan, const int (&out)[16], int img, int ch, int j0) {
+    const int kg = (threadIdx.x >> 5) & 1;
+    const size_t row = ((size_t)img * p.I + ch) * p.J;
+    const bool wide = EPI == EPI_REQUANT || ((p.J & 3) == 0 && (reinterpret_cast<uintptr_t>(p.Y) & 15) == 0);
+    const RequantBytes bytes{chan.ratio, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const int pos = j0 + g * 8 + kg * 4;   // four consecutive positions: out[4 g ..]
+        const int v[4] = {out[4 * g], out[4 * g + 1], out[4 * g + 2], out[4 * g + 3]};
+        const uint32_t word = EPI == EPI_REQUANT ? gemm_requant4(bytes, v) : 0u;
+        if (wide && pos + 3 < p.J) {
+            if (EPI == EPI_REQUANT) {
+                __builtin_memcpy(static_cast<uint8_t *>(p.Y) + row + pos, &word, 4);
+            } else {
+                // written once and several times the operands: kept from displacing them in the caches
+                i32x4 quad = {v[0], v[1], v[2], v[3]};
+                __builtin_nontemporal_store(quad, reinterpret_cast<i32x4 *>(static_cast<int32_t *>(p.Y) + row + pos));
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (pos + e >= p.J) continue;
+                if (EPI == EPI_REQUANT) static_cast<uint8_t *>(p.Y)[row + pos + e] = (uint8_t)(word >> (8 * e));
+                else static_cast<int32_t *>(p.Y)[row + pos + e] = v[e];
+            }
+        }
+    }
 }
 
 template <int EPI, bool DYN>
@@ -826,32 +859,7 @@ __device__ __forceinline__ void conv_small_finish(const GemmArgs &p, i32x16 (&ac
         out[r] = acc[0][0][r] + part[0][r] + part[1][r] + part[2][r] + fixed;
         if (DYN) out[r] -= zc * qs[r];
     }
-    if (ch >= p.I) return;
-    const size_t row = ((size_t)img * p.I + ch) * p.J;
-    const bool wide = (p.J & 3) == 0 && (reinterpret_cast<uintptr_t>(p.Y) & (EPI == EPI_REQUANT ? 3 : 15)) == 0;
-    const RequantBytes bytes{chan.ratio, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const int pos = j0 + jf * 32 + g * 8 + kg * 4;   // four consecutive positions: out[4 g ..]
-        const int v[4] = {out[4 * g], out[4 * g + 1], out[4 * g + 2], out[4 * g + 3]};
-        const uint32_t word = EPI == EPI_REQUANT ? gemm_requant4(bytes, v) : 0u;
-        if (wide && pos + 3 < p.J) {
-            if (EPI == EPI_REQUANT) {
-                *reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(p.Y) + row + pos) = word;
-            } else {
-                // written once and several times the operands: kept from displacing them in the caches
-                i32x4 quad = {v[0], v[1], v[2], v[3]};
-                __builtin_nontemporal_store(quad, reinterpret_cast<i32x4 *>(static_cast<int32_t *>(p.Y) + row + pos));
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (pos + e >= p.J) continue;
-                if (EPI == EPI_REQUANT) static_cast<uint8_t *>(p.Y)[row + pos + e] = (uint8_t)(word >> (8 * e));
-                else static_cast<int32_t *>(p.Y)[row + pos + e] = v[e];
-            }
-        }
-    }
+    if (ch < p.I) conv_store<EPI>(p, chan, out, img, ch, j0 + jf * 32);
 }
 
 // The same arrangement for a convolution with few 64x64 tiles (MODE_CONV): the gathered activation

@@ -168,6 +168,8 @@ inline T atomicMax(T *p, T v) { const T old = *p; if (v > old) *p = v; return ol
 inline void __syncthreads() {}
 template <typename T>
 inline T __shfl_xor(T v, int, int = 64) { return v; }
+template <typename T>
+inline T __shfl(T v, int, int = 64) { return v; }
 inline float __uint_as_float(uint32_t u) { float f; std::memcpy(&f, &u, 4); return f; }
 inline uint32_t __float_as_uint(float f) { uint32_t u; std::memcpy(&u, &f, 4); return u; }
 inline float __expf(float v) { return std::exp(v); }

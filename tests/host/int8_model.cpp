@@ -189,6 +189,15 @@ int main(int argc, char **argv) {
     conv(1, 32, 1, 200, 64, 1, 5, 1, 2, 1, 2, 0, 4, 0, 4, 4, HIPC_I8, "grouped, 1 x 5, stride 2, dilation 2");
     conv(1, 20, 9, 11, 33, 2, 4, 1, 1, 2, 1, 1, 0, 0, 3, 1, HIPC_U8, "ragged channels, 2 x 4");
     if (!quick) conv(1, 512, 1, 1024, 512, 1, 7, 1, 1, 1, 1, 0, 3, 0, 3, 1, HIPC_U8, "512 channels, 1 x 7");
+    // straight from NCHW in two dimensions: k split over wavefronts or not, 64 and 128 positions per workgroup, odd numbers of
+    // channel chunks, fewer than 16 channels (pairs of taps), planes of no whole number of words, images smaller than a tile
+    conv(2, 48, 13, 11, 40, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, HIPC_U8, "48 channels, 3 x 3");
+    conv(3, 64, 7, 7, 70, 3, 3, 2, 2, 1, 1, 1, 1, 1, 1, 1, HIPC_I8, "7 x 7 images, stride 2");
+    conv(quick ? 2 : 14, 3, 61, 57, 40, 7, 7, 2, 2, 1, 1, 3, 3, 3, 3, 1, HIPC_U8, "3 channels, 7 x 7, stride 2");
+    conv(quick ? 40 : 130, 16, 18, 18, 130, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, HIPC_U8, "pointwise");
+    conv(quick ? 40 : 130, 5, 18, 18, 24, 3, 2, 1, 1, 2, 3, 4, 1, 2, 5, 1, HIPC_U8, "5 channels, wide padding");
+    conv(3, 80, 1, 443, 80, 1, 5, 1, 1, 1, 5, 0, 10, 0, 10, 1, HIPC_U8, "one axis, 443 positions");
+    conv(1, 20, 3, 2, 8, 1, 1, 1, 1, 1, 1, 2, 3, 2, 3, 1, HIPC_U8, "six positions");
     report("convolutions");
     for (hipc::Scratch &s : ctx.scratch)
         if (s.ptr) gpu_model::release(s.ptr);

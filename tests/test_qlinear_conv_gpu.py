@@ -270,3 +270,29 @@ def test_a_recorded_graph_survives_scratch_growth_and_new_scales(ctx, pkg, oracl
         for b in [dX, dY, dB] + filler:
             b.free()
         ctx.flush()
+
+
+SLABS = [  # convolutions straight from NCHW: geometry, pads (top, left, bottom, right)
+    (dict(c_in=48, c_out=40, t=11, kw=3, dil=1, n=2, h=13, kh=3), (1, 1, 1, 1)),        # k split over wavefronts, an odd number of chunks
+    (dict(c_in=64, c_out=70, t=7, kw=3, dil=1, n=3, h=7, kh=3, stride=2), (1, 1, 1, 1)),  # images smaller than a tile, 49 bytes a plane
+    (dict(c_in=3, c_out=40, t=57, kw=7, dil=1, n=14, h=61, kh=7, stride=2), (3, 3, 3, 3)),  # pairs of taps, 64 channels x 128 positions
+    (dict(c_in=16, c_out=130, t=18, kw=1, dil=1, n=130, h=18), (0, 0, 0, 0)),           # one step, 128 channels x 64 positions
+    (dict(c_in=20, c_out=24, t=18, kw=2, dil=3, n=60, h=18, kh=3), (4, 1, 2, 5)),       # padding wider than the window, ragged channels
+    (dict(c_in=80, c_out=80, t=443, kw=5, dil=5, n=3), (0, 10, 0, 10)),                 # one axis, 443 positions
+    (dict(c_in=20, c_out=8, t=2, kw=1, dil=1, h=3), (2, 3, 2, 3)),                      # six positions, most outputs padding only
+]
+
+
+@pytest.mark.parametrize("signs", [(np.uint8, np.int8), (np.int8, np.uint8)], ids=["u8xi8", "i8xu8"])
+@pytest.mark.parametrize("cfg,pads", SLABS, ids=lambda v: str(v).replace(" ", ""))
+def test_convolutions_straight_from_nchw(ctx, pkg, oracle, cfg, pads, signs):
+    X, W, w_scale, bias, kw = _qconv_case(pkg, seed=160, **cfg)
+    kw["pads"] = pads
+    X, W = X.view(signs[0]), W.view(signs[1])
+    geom, og = pkg.ConvGeom.make(X.shape, W.shape, **kw), oracle.conv_geom(X.shape, W.shape, **kw)
+    x_zp = 100 if signs[0] == np.uint8 else -20
+    w_zp = 0 if signs[1] == np.int8 else 131
+    acc = pkg.ops.conv_integer(ctx, X, W, x_zp, w_zp, geom)
+    assert np.array_equal(acc, oracle.conv_integer(X, W, x_zp, w_zp, og))
+    got = pkg.ops.qlinear_conv(ctx, X, 0.03, x_zp, W, np.float32(0.004), w_zp, 0.7, -5, bias, geom, y_signed=True)
+    assert np.array_equal(got, oracle.qlinear_conv(X, 0.03, x_zp, W, np.float32(0.004), w_zp, 0.7, -5, bias, og, True))
