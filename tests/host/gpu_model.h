@@ -153,6 +153,7 @@ template <typename P>
 inline float gpu_model_fdot2(P, P, float c, bool) { return c; }
 #define __builtin_amdgcn_fdot2_f32_bf16 gpu_model_fdot2
 inline uint32_t gpu_model_perm(uint32_t a, uint32_t, uint32_t) { return a; }
+inline unsigned __builtin_amdgcn_alignbyte(unsigned hi, unsigned lo, unsigned by) { return (unsigned)((((unsigned long long)hi << 32) | lo) >> (8 * (by & 3))); }
 #define __builtin_amdgcn_perm gpu_model_perm
 #define __builtin_amdgcn_cvt_pk_u8_f32 gpu_model_cvt_pk_u8
 inline uint32_t gpu_model_cvt_pk_u8(float, uint32_t, uint32_t w) { return w; }

@@ -198,6 +198,8 @@ int main(int argc, char **argv) {
     conv(quick ? 40 : 130, 5, 18, 18, 24, 3, 2, 1, 1, 2, 3, 4, 1, 2, 5, 1, HIPC_U8, "5 channels, wide padding");
     conv(3, 80, 1, 443, 80, 1, 5, 1, 1, 1, 5, 0, 10, 0, 10, 1, HIPC_U8, "one axis, 443 positions");
     conv(1, 20, 3, 2, 8, 1, 1, 1, 1, 1, 1, 2, 3, 2, 3, 1, HIPC_U8, "six positions");
+    conv(2, 24, 13, 11, 24, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 24, HIPC_U8, "depthwise, 3 x 3");
+    conv(1, 10, 9, 14, 20, 5, 7, 2, 2, 2, 1, 5, 4, 5, 6, 10, HIPC_I8, "depthwise, two outputs per channel, 5 x 7, stride 2, wide padding");
     report("convolutions");
     for (hipc::Scratch &s : ctx.scratch)
         if (s.ptr) gpu_model::release(s.ptr);

@@ -296,3 +296,24 @@ def test_convolutions_straight_from_nchw(ctx, pkg, oracle, cfg, pads, signs):
     assert np.array_equal(acc, oracle.conv_integer(X, W, x_zp, w_zp, og))
     got = pkg.ops.qlinear_conv(ctx, X, 0.03, x_zp, W, np.float32(0.004), w_zp, 0.7, -5, bias, geom, y_signed=True)
     assert np.array_equal(got, oracle.qlinear_conv(X, 0.03, x_zp, W, np.float32(0.004), w_zp, 0.7, -5, bias, og, True))
+
+
+DEPTH = [  # depthwise: geometry, pads (top, left, bottom, right)
+    (dict(c_in=24, c_out=24, t=11, kw=3, dil=1, n=2, h=13, kh=3, group=24), (1, 1, 1, 1)),
+    (dict(c_in=10, c_out=20, t=14, kw=7, dil=1, h=9, kh=5, stride=2, group=10), (5, 4, 5, 6)),   # two outputs per channel, a column of padding only
+    (dict(c_in=5, c_out=5, t=4, kw=4, dil=1, n=3, h=4, kh=1, group=5), (0, 3, 0, 7)),            # the narrowest row
+    (dict(c_in=7, c_out=7, t=203, kw=8, dil=1, stride=2, group=7), (0, 0, 0, 3)),
+    (dict(c_in=6, c_out=6, t=3, kw=3, dil=1, h=20, kh=3, group=6), (1, 1, 1, 1)),                # too narrow: one output per thread
+]
+
+
+@pytest.mark.parametrize("x_type", [np.uint8, np.int8], ids=["u8", "i8"])
+@pytest.mark.parametrize("cfg,pads", DEPTH, ids=lambda v: str(v).replace(" ", ""))
+def test_depthwise_convolutions(ctx, pkg, oracle, cfg, pads, x_type):
+    X, W, w_scale, bias, kw = _qconv_case(pkg, seed=170, **cfg)
+    kw["pads"] = pads
+    X, x_zp = X.view(x_type), 100 if x_type == np.uint8 else -20
+    geom, og = pkg.ConvGeom.make(X.shape, W.shape, **kw), oracle.conv_geom(X.shape, W.shape, **kw)
+    assert np.array_equal(pkg.ops.conv_integer(ctx, X, W, x_zp, None, geom), oracle.conv_integer(X, W, x_zp, 0, og))
+    got = pkg.ops.qlinear_conv(ctx, X, 0.03, x_zp, W, w_scale, 0, 0.1, -5, bias, geom, y_signed=True)
+    assert np.array_equal(got, oracle.qlinear_conv(X, 0.03, x_zp, W, w_scale, 0, 0.1, -5, bias, og, True))
