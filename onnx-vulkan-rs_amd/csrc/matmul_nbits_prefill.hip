@@ -51,9 +51,9 @@ struct PrefillArgs {
     int ksplit, split_stages;
     float *Ypart;
     float *Yf32;   // when set, the result is written here as f32 and Y is not used (rows of f32 activations, see nbits_prefill_f32)
-    // Paired rows (set together; only the kernel that keeps the weight out of LDS, 128-row tiles): A holds the two
+    // Paired rows (set together; only the kernel that keeps the weight out of LDS): A holds the two
     // f16 terms of `pair_rows` f32 rows, 32 rows of high terms followed by the 32 rows of their low terms, so that a
-    // wavefront's two row blocks are the two terms of the same 32 rows; it adds them and stores row r of the result
+    // wavefront's two row blocks (64-row tiles: two wavefronts') are the two terms of the same 32 rows; it adds them and stores row r of the result
     // times 2^exps[r] -- into Yf32, or unscaled into the k split's partials [split][pair_rows][N].
     // exps without pair_rows: A holds one f16 term per f32 row and row r of the f32 result is stored times 2^exps[r]
     // (any of the kernels; the k split's partials stay unscaled).
@@ -637,6 +637,33 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
                     const float4 o = slot[((g - 1) * NJ * 4 + j * 4 + q) * 256 + tid];
                     acc[0][j][4 * q] += o.x, acc[0][j][4 * q + 1] += o.y, acc[0][j][4 * q + 2] += o.z, acc[0][j][4 * q + 3] += o.w;
                 }
+    }
+    if constexpr (MI == 1) {
+        if (p.pair_rows > 0) {
+            // paired rows: the tile's two row blocks, of two wavefronts. The one with the low terms hands its sums over
+            // (behind what the groups exchanged; 8 KB, once per tile), the other adds them and stores. Few rows are
+            // bound by the serial chain of each tile: 128-row tiles left most CUs idle (130 x 2048 x 2560: 60 tiles,
+            // 30.8 us; 200 of these, 17.6 us).
+            float4 *slot = reinterpret_cast<float4 *>(lds_raw) + (KG - 1) * NJ * 4 * 256;
+            if (wm == 1) {
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        slot[(j * 4 + q) * 128 + wn * 64 + lane] = make_float4(acc[0][j][4 * q], acc[0][j][4 * q + 1], acc[0][j][4 * q + 2], acc[0][j][4 * q + 3]);
+            }
+            __syncthreads();   // (the second group of wavefronts has left)
+            if (wm == 1) return;
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const float4 o = slot[(j * 4 + q) * 128 + wn * 64 + lane];
+                    acc[0][j][4 * q] += o.x, acc[0][j][4 * q + 1] += o.y, acc[0][j][4 * q + 2] += o.z, acc[0][j][4 * q + 3] += o.w;
+                }
+            prefill_store_pairs<NJ>(p, acc, i0 >> 1, j0 + wn * kWN, r32, kg);
+            return;
+        }
         prefill_store<kF, NJ>(p, acc, i0 + wm * kWT, j0 + wn * kWN, r32, kg);
     } else if constexpr (KG == 2) {
         // group g keeps row block g and hands the other one over: [group][16-byte piece][thread] in LDS (the A
@@ -777,7 +804,7 @@ template <int SG, int MI, int NJ, int KG>
 int prefill_launch_direct_groups(hipc_ctx *ctx, const PrefillArgs &a, dim3 grid) {
     const bool full = a.K % (2 * kPK) == 0;
     // one group: at most 36 KB, inside the limit that needs no permission; two: their A buffers, then the hand-over
-    constexpr size_t lds = KG == 1 ? prefill_lds(64 * MI) / 2 : std::max(KG * prefill_lds(64 * MI) / 2, (size_t)(MI == 2 ? 2 : KG - 1) * NJ * 4 * 256 * 16);
+    constexpr size_t lds = KG == 1 ? prefill_lds(64 * MI) / 2 : std::max(KG * prefill_lds(64 * MI) / 2, (size_t)(MI == 2 ? 4 : 2 * (KG - 1) + 1) * NJ * 4 * 128 * 16);
     if (KG > 1 && lds > 64 * 1024) {
         static bool lds_allowed[2][kMaxDevices] = {};
         if (int rc = full ? allow_dynamic_lds(ctx, mmnb_prefill_direct_kernel<SG, MI, NJ, KG, true>, lds, lds_allowed[1])
@@ -794,7 +821,9 @@ int prefill_launch_direct_groups(hipc_ctx *ctx, const PrefillArgs &a, dim3 grid)
 template <int SG, int MI, int NJ>
 int prefill_launch_direct(hipc_ctx *ctx, PrefillArgs a) {
     dim3 grid;
-    if (int rc = prefill_plan(ctx, a, 64 * MI, 64 * NJ, MI == 2, &grid)) return rc;
+    // (64-row tiles split a long k as the larger ones do when even they are too few: f16 100 x 8192 x 1024, 32 tiles,
+    // 32.0 us as they are, 13.7 us four ways)
+    if (int rc = prefill_plan(ctx, a, 64 * MI, 64 * NJ, true, &grid)) return rc;
     if constexpr (MI == 2) {
         // Two k groups per workgroup when the launch leaves the second wavefront slot of the SIMDs empty (no more
         // workgroups than CUs) and every group gets two trips or more; prefill_groups 1 / 2 forces the choice.
@@ -876,7 +905,6 @@ int prefill_launch(hipc_ctx *ctx, const PrefillArgs &a) {
     const int64_t cus = std::max(1, ctx->cu_count);
     if (SG != 8 && tile == 128 && tiles128 >= 256 && ctx->tune.prefill_direct != 0 && ceil_div(tiles192, cus) * 3 < ceil_div(tiles128, cus) * 2) tile = 192;
     if (forced == 64 || forced == 128 || (forced == 192 && SG != 8 && ctx->tune.prefill_direct != 0)) tile = forced;
-    if (a.pair_rows > 0 && tile == 64) tile = 128;   // paired rows are the two row blocks of a wavefront: 128-row tiles
     if constexpr (SG == 8) return prefill_launch_wide(ctx, a, SG, tile);   // (blocks of 16: one kernel; three column blocks leave no registers for the scales)
     else return tile == 64 && ctx->tune.prefill_direct == 0 ? prefill_launch_tile<SG, 64>(ctx, a) : prefill_launch_wide(ctx, a, SG, tile);
 }

@@ -502,3 +502,20 @@ def test_blocks_of_sixteen_on_the_matrix_cores(ctx, pkg, oracle, shape, dtype, l
     pkg.ops.matmul_nbits_packed_device(ctx, moved.at(2 * a.itemsize), pkg.ops.hipc_dtype(a.dtype), w, out, m, level)
     assert np.array_equal(ctx.download(out, dtype, (m, n)), got)
     moved.free(), out.free(), w.destroy()
+
+
+@pytest.mark.parametrize("bs,level", [(16, 0), (32, 0), (64, 0), (128, 0), (32, 4)])
+@pytest.mark.parametrize("shape", [(65, 1024, 130), (95, 520, 64), (97, 1160, 1100), (128, 648, 96), (70, 4224, 200), (66, 8200, 100)], ids=lambda s: "M%d_K%d_N%d" % s)
+def test_f32_rows_on_small_tiles(ctx, pkg, oracle, shape, bs, level):
+    """Rows of f32 on 64-row tiles: the last tile with one row, one missing and full; one group of wavefronts and two;
+    k split over workgroups (k of 4224 and more), the last split shorter than the others."""
+    m, k, n = shape
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=700 + n)
+    a = pkg.synth.normal_f32(m * k, 701).reshape(m, k)
+    a[0] *= np.float32(1e20)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    want = oracle.matmul_nbits(a, B, scales, zp, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    for rows in (slice(0, 1), slice(1, m)):   # the large row against its own size
+        assert np.max(np.abs(got[rows] - want[rows])) <= (1e-3 if level else 1e-5) * np.max(np.abs(want[rows])), rows
+    w.destroy()
