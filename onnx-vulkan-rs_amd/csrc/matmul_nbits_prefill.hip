@@ -965,11 +965,9 @@ mmnb_prefill_split_rows_kernel(const float *__restrict__ A, int M, int K, __half
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    // bits of mx: exponent field - 127 = floor(log2 mx) for a normal number; zero, subnormal or infinite rows are not scaled
-    const int ef = (int)((__float_as_uint(mx) >> 23) & 0xffu);
-    const int e = (ef == 0 || ef == 255) ? 0 : ef - 127 - 14;
+    const int e = row_exponent(__float_as_uint(mx));
     if (tid == 0) exps[m] = e;
-    const float down = __uint_as_float((uint32_t)(127 - e) << 23);   // 2^-e: e is in [-140, 113], 2^-e a normal number
+    const float down = two_to_minus(e);
     uint2 *hi_row = reinterpret_cast<uint2 *>(A2 + hi_at * K), *lo_row = reinterpret_cast<uint2 *>(A2 + lo_at * K);
     auto split4 = [&](const float4 &v, int c) {
         const float a[4] = {v.x * down, v.y * down, v.z * down, v.w * down};

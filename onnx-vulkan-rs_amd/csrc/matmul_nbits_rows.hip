@@ -296,13 +296,11 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
                 if (i16 == 0) atomicMax(&head[at_m[u]], (int)__float_as_uint(mx));
             }
             __syncthreads();
-            // zero, subnormal and infinite rows are not scaled
-            auto exponent = [](int bits) { const int ef = (bits >> 23) & 0xff; return ef == 0 || ef == 255 ? 0 : ef - 127 - 14; };
 #pragma unroll
             for (int u = 0; u < P; u++)
-                if (tid + u * nthreads < items) split(u, __uint_as_float((uint32_t)(127 - exponent(head[at_m[u]])) << 23));
+                if (tid + u * nthreads < items) split(u, two_to_minus(row_exponent((uint32_t)head[at_m[u]])));
             __syncthreads();
-            if (tid < 16) head[tid] = exponent(head[tid]);
+            if (tid < 16) head[tid] = row_exponent((uint32_t)head[tid]);
             __syncthreads();
         } else {
             __syncthreads();

@@ -16,6 +16,13 @@ __device__ __forceinline__ uint32_t two_halves(__half lo, __half hi) {
     return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
 }
 
+// An f32 row enters as f16 terms of the row times 2^-e, with the e that brings its largest magnitude (given as bits) into
+// [2^14, 2^15). 2^-e has to be a normal number: rows whose largest value is below 2^-113, subnormal and zero ones among them,
+// are all scaled by 2^127, which their terms hold as well (a subnormal's last bit becomes 2^-22); a row with an infinity is
+// scaled like one of the largest finite value.
+__device__ __forceinline__ int row_exponent(uint32_t largest) { return min(max((int)(largest >> 23), 14), 254) - 127 - 14; }
+__device__ __forceinline__ float two_to_minus(int e) { return __uint_as_float((uint32_t)(127 - e) << 23); }
+
 // 1024 + zp and 64 + zp as f16 in both halves of a word (zb carries 128 + zp)
 struct ZeroPair {
     f16x2 unit, sixteenth;

@@ -519,3 +519,42 @@ def test_f32_rows_on_small_tiles(ctx, pkg, oracle, shape, bs, level):
     for rows in (slice(0, 1), slice(1, m)):   # the large row against its own size
         assert np.max(np.abs(got[rows] - want[rows])) <= (1e-3 if level else 1e-5) * np.max(np.abs(want[rows])), rows
     w.destroy()
+
+
+def unpacked(B, scales, zp, k, n, bs):
+    """The weight's (q - zp) and scales, [N, K] in 64 bits."""
+    nb = -(-k // bs)
+    codes = np.stack([B & 15, B >> 4], axis=-1).reshape(n, -1)[:, :k].astype(np.float64)
+    if zp is None:
+        z = np.full((n, nb), 8.0)
+    else:
+        z = np.stack([zp & 15, zp >> 4], axis=-1).reshape(n, -1)[:, :nb].astype(np.float64)
+    s = np.asarray(scales).reshape(n, nb).astype(np.float64)
+    return codes - np.repeat(z, bs, axis=1)[:, :k], np.repeat(s, bs, axis=1)[:, :k]
+
+
+@pytest.mark.parametrize("bs", [16, 32, 128])
+@pytest.mark.parametrize("level", [0, 1])
+@pytest.mark.parametrize("m", [1, 3, 16, 20, 40, 70])
+def test_rows_of_tiny_values(ctx, pkg, oracle, m, level, bs):
+    """Rows whose largest value lies anywhere down to the smallest normal number, subnormal rows, and an ordinary row
+    with a run of tiny values (a whole slice of k, where k is split over workgroups): the power of two a row is scaled by
+    stays a number. Scales near 2^10 keep the results in the normal range, so the bound is the rows' own."""
+    k, n = 2176, 80
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=521)
+    scales = (scales * np.float32(2.0**15)).astype(np.float32)
+    a = pkg.synth.normal_f32(m * k, 522).reshape(m, k)
+    a /= np.abs(a).max(axis=1, keepdims=True)           # the largest of a row is 1
+    for r in range(m):
+        a[r] *= np.float32(2.0) ** -(110 + (7 * r + 3) % 18)      # 2^-110 .. 2^-127
+    a[m // 2] = pkg.synth.normal_f32(k, 523)
+    a[m // 2, 128:1280] *= np.float32(2.0**-113)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    w.destroy()
+    d, s = unpacked(B, scales, zp, k, n, bs)
+    want = a.astype(np.float64) @ (d * s).T
+    assert np.all(np.isfinite(got))
+    for r in range(m):
+        # 16 bits of a value or better (2^-16, over sqrt(K) of them), an f32 sum, and subnormal inputs' own last bits
+        assert np.max(np.abs(got[r] - want[r])) <= 2e-5 * np.max(np.abs(want[r])) + 2.0**-149 * np.sum(np.abs(d * s), axis=1).max(), r
