@@ -195,10 +195,11 @@ size_t hipc_nbits_weight_bytes(const hipc_nbits_weight *w);
  * (blocks of 32 and more), and up to 16 against 32768 columns or more: 0 (unset), 2, 3 and 4 enter the matrix cores as two bf16 terms
  * (16 significant bits, less error than f32 accumulation over K adds), 1 pins f32 and uses three terms (all
  * 24 bits). Otherwise the kernels use f16: an f16 row as it is, an f32 row
- * as f16 terms of the row times a power of two (none up to 16 rows whose largest value lies in [1/8, 2^15),
- * else the one that puts the row's largest value into [2^14, 2^15)):
- * two terms (22 bits) at level 0 (three with blocks of 16), one (11 bits of every value) from 33 rows on at levels 2, 3 and 4, which allow
- * f16, bf16 or int8 activations, three (every bit of the row's values) at level 1.
+ * as f16 terms of the row times the power of two that puts its largest value into [2^14, 2^15)
+ * (up to 16 rows with largest values in [1/4, 64) share one, which puts them between 2^7 and 2^15):
+ * two terms (22 bits of a value, but no less than 2^-39 -- of shared ones, 2^-32 -- of the row's largest) at level 0 (three with blocks of 16), one (11 bits of every value) from 33 rows on at levels 2, 3 and 4, which allow
+ * f16, bf16 or int8 activations, three (all 24 bits of a value down to 2^-30 of the row's largest, and 2^-54 of that one
+ * below) at level 1.
  * The tiled kernel keeps its accumulators in units of the open quantisation block's scale: there a
  * scale of magnitude below 2^-64 counts as 2^-64 (what such a block adds is below
  * 2^-64 x 15 x sum |a|), and a column whose scales are all below it is stored as 0. */

@@ -934,7 +934,7 @@ int nbits_prefill(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void
 // are stored as A2[m] = hi, A2[M + m] = lo; one workgroup per row. PAIRED: 32 rows of high terms are followed by the
 // 32 rows of their low terms (row m: hi at 64 (m / 32) + m % 32, lo 32 rows on), the grid covers a multiple of 32
 // rows and the rows past M are zeros.
-template <bool PAIRED, int TERMS = 2>   // TERMS 1: the high terms alone, M rows; 3: a third term (all 24 bits of the row's values), rows 2 M + m
+template <bool PAIRED, int TERMS = 2>   // TERMS 1: the high terms alone, M rows; 3: a third, rows 2 M + m (see split_terms)
 static __global__ void __launch_bounds__(256)
 mmnb_prefill_split_rows_kernel(const float *__restrict__ A, int M, int K, __half *__restrict__ A2, int *__restrict__ exps) {
     __shared__ float red[4];
@@ -971,24 +971,23 @@ mmnb_prefill_split_rows_kernel(const float *__restrict__ A, int M, int K, __half
     uint2 *hi_row = reinterpret_cast<uint2 *>(A2 + hi_at * K), *lo_row = reinterpret_cast<uint2 *>(A2 + lo_at * K);
     auto split4 = [&](const float4 &v, int c) {
         const float a[4] = {v.x * down, v.y * down, v.z * down, v.w * down};
-        __half hi[4], lo[4], lo2[4];
+        _Float16 t[4][TERMS];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            hi[t] = __float2half(a[t]);
-            const float r = a[t] - __half2float(hi[t]);   // (exact, like the next one)
-            lo[t] = __float2half(r);
-            lo2[t] = __float2half(r - __half2float(lo[t]));
-        }
-        hi_row[c] = make_uint2(two_halves(hi[0], hi[1]), two_halves(hi[2], hi[3]));
-        if (TERMS >= 2) lo_row[c] = make_uint2(two_halves(lo[0], lo[1]), two_halves(lo[2], lo[3]));
-        if (TERMS == 3) lo_row[c + (size_t)M * (K / 4)] = make_uint2(two_halves(lo2[0], lo2[1]), two_halves(lo2[2], lo2[3]));
+        for (int i = 0; i < 4; i++) split_terms<TERMS>(a[i], t[i]);
+        const auto piece = [&](int e) {
+            return make_uint2(two_halves(__builtin_bit_cast(__half, t[0][e]), __builtin_bit_cast(__half, t[1][e])),
+                              two_halves(__builtin_bit_cast(__half, t[2][e]), __builtin_bit_cast(__half, t[3][e])));
+        };
+        hi_row[c] = piece(0);
+        if constexpr (TERMS >= 2) lo_row[c] = piece(1);
+        if constexpr (TERMS == 3) lo_row[c + (size_t)M * (K / 4)] = piece(2);
     };
 #pragma unroll
     for (int u = 0; u < kHeld; u++)
         if (tid + 256 * u < nv) split4(held[u], tid + 256 * u);
     for (int c = tid + 256 * kHeld; c < nv; c += 256) split4(row[c], c);
 }
-// Y[m] = (P[m] + P[M + m]) 2^e[m], or with three terms (P[m] + (P[M + m] + P[2 M + m])) 2^e[m]: the small ones first
+// Y[m] = (P[m] + P[M + m]) 2^e[m], or with three terms join_terms(P[m], P[M + m], P[2 M + m]) 2^e[m]
 template <bool VEC>   // VEC: N is a multiple of four and Y is aligned for 16-byte stores
 static __global__ void __launch_bounds__(256)
 mmnb_prefill_join_rows_kernel(const float *__restrict__ P, const int *__restrict__ exps, int M, int N, float *__restrict__ Y, int terms) {
@@ -996,16 +995,15 @@ mmnb_prefill_join_rows_kernel(const float *__restrict__ P, const int *__restrict
     if (i >= plane) return;
     const int e = exps[(int)(i / N)];
     if (VEC) {
-        const float4 a = *reinterpret_cast<const float4 *>(P + i);
-        float4 b = *reinterpret_cast<const float4 *>(P + i + plane);
+        const float4 a = *reinterpret_cast<const float4 *>(P + i), b = *reinterpret_cast<const float4 *>(P + i + plane);
+        float4 v = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
         if (terms == 3) {
             const float4 c = *reinterpret_cast<const float4 *>(P + i + 2 * plane);
-            b = make_float4(b.x + c.x, b.y + c.y, b.z + c.z, b.w + c.w);
+            v = make_float4(join_terms(a.x, b.x, c.x), join_terms(a.y, b.y, c.y), join_terms(a.z, b.z, c.z), join_terms(a.w, b.w, c.w));
         }
-        *reinterpret_cast<float4 *>(Y + i) = make_float4(ldexpf(a.x + b.x, e), ldexpf(a.y + b.y, e), ldexpf(a.z + b.z, e), ldexpf(a.w + b.w, e));
+        *reinterpret_cast<float4 *>(Y + i) = make_float4(ldexpf(v.x, e), ldexpf(v.y, e), ldexpf(v.z, e), ldexpf(v.w, e));
     } else {
-        const float b = terms == 3 ? P[i + plane] + P[i + 2 * plane] : P[i + plane];
-        Y[i] = ldexpf(P[i] + b, e);
+        Y[i] = ldexpf(terms == 3 ? join_terms(P[i], P[i + plane], P[i + 2 * plane]) : P[i] + P[i + plane], e);
     }
 }
 

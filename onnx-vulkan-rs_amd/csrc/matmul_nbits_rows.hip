@@ -11,8 +11,10 @@
 //   * products run on v_mfma_f32_16x16x32_f16. A nibble becomes the exact integer q - zp (nbits_f16.h), so no sums of the
 //     activations are needed to take a bias out; an f16 row is one operand, exact;
 //   * an f32 row is two f16 terms of the row times a power of two that brings its largest value (in the workgroup's range
-//     of k) into [2^14, 2^15): 22 bits, the terms chained into the same accumulator. Up to 16 rows are split by the
-//     workgroup itself (SRC_F32); more are split once by a launch in front (nbits_prefill's), and travel as f16 rows;
+//     of k) into [2^14, 2^15), or to 2^7 at least, or three terms where every bit counts (split_terms).
+//     No row goes unscaled: beside values near 1, f16's smallest step (2^-24) would cost the small values of a row most of
+//     their bits, in columns where the large ones meet a zero all that counts. Up to 16 rows are split by the workgroup itself (SRC_F32);
+//     more are split once by a launch in front (nbits_prefill's), and travel as f16 rows;
 //   * the wavefronts' partial sums meet in LDS, in a fixed order. With few columns and a long k the range of k is also
 //     split over workgroups, and a second launch adds their partial rows (rows_plan weighs that launch against the bytes).
 #include <algorithm>
@@ -45,9 +47,10 @@ struct RowsArgs {
     int loops;         // workgroups take one column group after another (gridDim.x of them at a time)
 };
 
-// LDS of a workgroup: 32 words of flags and exponents, operands [chunk][term][4 k groups][rows, made odd], partial sums --
+// LDS of a workgroup: 32 words of flags and magnitudes, operands [chunk][term][4 k groups][rows, made odd], partial sums --
 // behind the operands where the workgroup takes several column groups, over them where it takes one
 constexpr size_t kRowsHead = 128;
+constexpr int kUsualExponent = -9;   // see the splitting of SRC_F32 rows
 __host__ __device__ inline int rows_pitch(int M) { return M | 1; }
 __host__ __device__ inline size_t rows_operands(int M, int terms, int stage_tiles) { return (size_t)stage_tiles * 4 * terms * 4 * rows_pitch(M) * 16; }
 
@@ -64,7 +67,10 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
     const int M = p.M, MP = rows_pitch(M);
     const int tile0 = blockIdx.y * p.split_tiles, tile1 = min(p.n_cg, tile0 + p.split_tiles);
     const int group_tiles = p.WN * T, groups = (p.n_tiles + group_tiles - 1) / group_tiles;
-    int *head = reinterpret_cast<int *>(smem);   // SRC_F32: [0..15] row m has a value that needs no scaling up, [16] one needs scaling down; then exponents
+    // SRC_F32: [0..15] row m has a value of 1/4 or more, [16] some value is 64 or more; where not every row is a usual one,
+    // the largest magnitude of row m in this workgroup's range of k, as bits
+    int *head = reinterpret_cast<int *>(smem);
+    bool usual = true;
     uint4 *As = smem + kRowsHead / 16;
     float *red = reinterpret_cast<float *>(reinterpret_cast<char *>(As) + (p.loops ? rows_operands(M, NT, p.stage_tiles) : 0));
 
@@ -131,8 +137,30 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
         const uint4 v = __builtin_bit_cast(uint4, w);
         return __builtin_bit_cast(f16x8, make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep));
     };
+    // Where the registers allow it (128 hold twice the wavefronts of 129) the first terms' products have a sum of their own --
+    // an f16 by a four-bit integer 32 times over leaves next to no rounding to do -- that the others' joins once per scale
+    // group. The step between the second and third of three terms, and before it where all share a sum, is in the weight:
+    // times 2^-11 and 2^-22, exact for small integers.
+    constexpr bool APART = RB == 1 && NT > 1 && (T == 1 || (T == 2 && (NT == 3 || SG < 8)));
+    constexpr int ND = APART ? 2 : 1;
+    const auto joined = [](const f32x4 (&v)[ND], int r) {
+        if constexpr (APART) return fmaf(v[1][r], NT == 3 ? 1.f / kTermStep : 1.f, v[0][r]);
+        else return v[0][r];
+    };
+    const auto weight_for = [](const f16x8 &w, int e) {
+        const int steps = NT < 3 ? 0 : APART ? e - 1 : e;
+        return steps <= 0 ? w : w * (_Float16)(steps == 1 ? 1.f / kTermStep : 1.f / (kTermStep * kTermStep));
+    };
     auto compute = [&](const Stage &st, int first_chunk) {
-        f32x4 d[RB][T];
+        f32x4 d[RB][T][ND];
+        // three terms, and registers left: a tile's scale groups are added up among themselves first, one rounding at the size of
+        // the whole sum a tile instead of one a group
+        constexpr bool BY_TILE = APART && NT == 3 && T == 1 && SG < 8;
+        f32x4 tile_sum[RB][T];
+        const auto add = [&](int b, int t, int r, bool opens, float s, float v) {
+            if (!BY_TILE) acc[b][t][r] = fmaf(s, v, acc[b][t][r]);
+            else tile_sum[b][t][r] = opens ? s * v : fmaf(s, v, tile_sum[b][t][r]);
+        };
         ZeroPair z[T];
         constexpr int CPG = SG == 8 ? 1 : 4 / SG;   // chunks per scale group
 #pragma unroll
@@ -156,30 +184,44 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
                     const f16x8 w0 = masked(w, first16), w1 = masked(w, ~first16);
 #pragma unroll
                     for (int b = 0; b < RB; b++) {
-                        f32x4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = v0;
+                        f32x4 v0[ND], v1[ND];
+#pragma unroll
+                        for (int e = 0; e < ND; e++) v0[e] = v1[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                         for (int e = NT - 1; e >= 0; e--) {
-                            v0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], w0, v0, 0, 0, 0);
-                            v1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], w1, v1, 0, 0, 0);
+                            const int c = APART && e > 0;
+                            v0[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], weight_for(w0, e), v0[c], 0, 0, 0);
+                            v1[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], weight_for(w1, e), v1[c], 0, 0, 0);
                         }
 #pragma unroll
-                        for (int r = 0; r < NR; r++) acc[b][t][r] = fmaf(st.s[t][(2 * j + 1) % SG], v1[r], fmaf(st.s[t][2 * j % SG], v0[r], acc[b][t][r]));
+                        for (int r = 0; r < NR; r++) add(b, t, r, j == 0, st.s[t][2 * j % SG], joined(v0, r)), add(b, t, r, false, st.s[t][(2 * j + 1) % SG], joined(v1, r));
                     }
                     continue;
                 }
 #pragma unroll
                 for (int b = 0; b < RB; b++) {
-                    f32x4 v = first ? f32x4{0.f, 0.f, 0.f, 0.f} : d[b][t];
+                    if (first)
 #pragma unroll
-                    for (int e = NT - 1; e >= 0; e--) v = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], w, v, 0, 0, 0);
-                    d[b][t] = v;
+                        for (int e = 0; e < ND; e++) d[b][t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = NT - 1; e >= 0; e--) {
+                        const int c = APART && e > 0;
+                        d[b][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], weight_for(w, e), d[b][t][c], 0, 0, 0);
+                    }
                     if (last) {
 #pragma unroll
-                        for (int r = 0; r < NR; r++) acc[b][t][r] = fmaf(st.s[t][g], v[r], acc[b][t][r]);
+                        for (int r = 0; r < NR; r++) add(b, t, r, g == 0, st.s[t][g], joined(d[b][t], r));
                     }
                 }
             }
         }
+        if constexpr (BY_TILE)
+#pragma unroll
+            for (int b = 0; b < RB; b++)
+#pragma unroll
+                for (int t = 0; t < T; t++)
+#pragma unroll
+                    for (int r = 0; r < NR; r++) acc[b][t][r] += tile_sum[b][t][r];
     };
     // This wavefront's tiles of a stage [t0, t1) in LDS; `cur` is the first of them, and on leaving the first of the next
     // stage (a stage is a whole number of rounds of the wavefronts) or group, the tile after it always on its way.
@@ -218,7 +260,7 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
             const int b = q / (T * NR), t = q / NR % T, r = q % NR;
             const int m = b * 16 + (NR == 4 ? 4 * g4 + r : g4 + 4 * r), n = (group * group_tiles + wn * T + t) * 16 + i16;
             if (m >= M || n >= p.N) continue;
-            if (SRC == SRC_F32) v = ldexpf(v, head[m]);
+            if (SRC == SRC_F32) v = ldexpf(v, usual ? kUsualExponent : row_exponent((uint32_t)head[m]));
             const size_t at = (size_t)m * p.N + n;
             if (p.Ypart) {
                 p.Ypart[(size_t)blockIdx.y * M * p.N + at] = v;
@@ -259,32 +301,32 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
         };
         auto split = [&](int u, float down) {
             const float v[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
-            f16x8 t[3];
+            f16x8 t[NT];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float x = v[i] * down;
-                t[0][i] = (_Float16)x;
-                const float r = x - (float)t[0][i];   // (exact, like the next one)
-                t[1][i] = (_Float16)r;
-                if (NT == 3) t[2][i] = (_Float16)(r - (float)t[1][i]);
+                _Float16 terms[NT];
+                split_terms<NT>(v[i] * down, terms);
+#pragma unroll
+                for (int e = 0; e < NT; e++) t[e][i] = terms[e];
             }
 #pragma unroll
             for (int e = 0; e < NT; e++) As[slot(at_c[u] >> 2, at_c[u] & 3, e, at_m[u])] = __builtin_bit_cast(uint4, t[e]);
         };
         __syncthreads();   // the flags are cleared
-        // Rows as they usually are -- every value below 2^15, the largest 2^kPlain or more, so that what the terms leave (at
-        // most 2^-25) is below the row's 22nd bit (three terms: 24th) -- are split as they are, without waiting for their maxima.
-        constexpr float kPlain = NT == 3 ? 0.5f : 0.125f;
+        // Rows as they usually are, every one's largest value in [1/4, 64), are all scaled by 2^9 as their pieces arrive, without
+        // waiting for the maxima: that puts the largest value between 2^7 and 2^15, and what two terms lose (2^-25) at 2^-32
+        // of it at most. (8 x 1152 x 4096: 4.9 us, 5.3 with a power of two for each row; 16 x 1152 x 13824 9.0 and 10.4)
 #pragma unroll
         for (int u = 0; u < P; u++) {
             if (tid + u * nthreads >= items) continue;
             const float mx = largest(u);
-            if (mx >= kPlain) head[at_m[u]] = 1;
-            if (!(mx < 32768.f)) head[16] = 1;
-            split(u, 1.f);
+            if (mx >= 0.25f) head[at_m[u]] = 1;
+            if (!(mx < 64.f)) head[16] = 1;
+            split(u, two_to_minus(kUsualExponent));
         }
         __syncthreads();
         if (__any(head[16] != 0 || (lane < M && head[lane & 15] == 0))) {   // (the same in every wavefront)
+            usual = false;
             // the largest magnitude of each row, as bits (non-negative floats order like them)
             __syncthreads();
             if (tid < 16) head[tid] = 0;
@@ -300,11 +342,6 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
             for (int u = 0; u < P; u++)
                 if (tid + u * nthreads < items) split(u, two_to_minus(row_exponent((uint32_t)head[at_m[u]])));
             __syncthreads();
-            if (tid < 16) head[tid] = row_exponent((uint32_t)head[tid]);
-            __syncthreads();
-        } else {
-            __syncthreads();
-            if (tid < 16) head[tid] = 0;
         }
         for (int group = blockIdx.x; group < groups; group += gridDim.x) {
             if (group != (int)blockIdx.x) __syncthreads();   // the sums of the group before have been read

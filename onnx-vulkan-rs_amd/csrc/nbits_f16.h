@@ -22,6 +22,22 @@ __device__ __forceinline__ uint32_t two_halves(__half lo, __half hi) {
 // scaled like one of the largest finite value.
 __device__ __forceinline__ int row_exponent(uint32_t largest) { return min(max((int)(largest >> 23), 14), 254) - 127 - 14; }
 __device__ __forceinline__ float two_to_minus(int e) { return __uint_as_float((uint32_t)(127 - e) << 23); }
+// Each term is the nearest f16 of what the ones before leave (exactly formed). Of two terms, which hold 22 bits, the second is
+// as it comes: of a small value up to 2^-25 is lost where that is more, 2^-39 of a largest value of 2^14. Three stand for every
+// bit of the row's values, so the second and third are 2^11 and 2^22 times what they stand for: 2^-47 is lost at most, and 24
+// bits are held of values down to 2^-23 -- of 2^-1 were the terms as they come.
+constexpr float kTermStep = 0x1p11f;
+template <int NT>
+__device__ __forceinline__ void split_terms(float x, _Float16 (&t)[NT]) {
+    constexpr float step = NT == 3 ? kTermStep : 1.f;
+    t[0] = (_Float16)x;
+    if constexpr (NT >= 2) {
+        const float r = (x - (float)t[0]) * step;
+        t[1] = (_Float16)r;
+        if constexpr (NT == 3) t[2] = (_Float16)((r - (float)t[1]) * step);
+    }
+}
+__device__ __forceinline__ float join_terms(float d0, float d1, float d2) { return fmaf(fmaf(d2, 1.f / kTermStep, d1), 1.f / kTermStep, d0); }
 
 // 1024 + zp and 64 + zp as f16 in both halves of a word (zb carries 128 + zp)
 struct ZeroPair {

@@ -558,3 +558,52 @@ def test_rows_of_tiny_values(ctx, pkg, oracle, m, level, bs):
     for r in range(m):
         # 16 bits of a value or better (2^-16, over sqrt(K) of them), an f32 sum, and subnormal inputs' own last bits
         assert np.max(np.abs(got[r] - want[r])) <= 2e-5 * np.max(np.abs(want[r])) + 2.0**-149 * np.sum(np.abs(d * s), axis=1).max(), r
+
+
+@pytest.mark.parametrize("m", [2, 8, 16, 24, 40])
+@pytest.mark.parametrize("bs,level", [(32, 0), (64, 1), (128, 0), (16, 0), (16, 1)])
+def test_small_values_beside_a_large_one(ctx, pkg, bs, level, m):
+    """An activation row as language models have them, one value of ordinary size among small ones, against columns whose
+    weight for that value is zero: the small ones count in full. They are whole multiples of 2^-32 times at most 127, so
+    every sum is exact in f32 and so must the result be: two f16 terms of a scaled row hold any 22 bits that end 2^-31 below
+    a largest value near 1 or earlier."""
+    k, n = 640, 48
+    rng = np.random.default_rng(77)
+    q = np.full((n, k), 8, np.uint8)
+    small = rng.choice(np.arange(1, k), 32, replace=False)
+    q[:, small] = rng.integers(0, 16, (n, 32))
+    B = pkg.synth.pack_nibbles(q, bs)
+    scales = np.ones(n * (-(-k // bs)), np.float32)
+    a = np.zeros((m, k), np.float32)
+    a[:, 0] = 0.6
+    a[:, small] = rng.integers(-127, 128, (m, 32)) * 2.0**-32
+    w = pkg.ops.NBitsWeight(ctx, B, scales, None, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    w.destroy()
+    want = a[:, small].astype(np.float64) @ (q[:, small].astype(np.float64) - 8).T
+    assert np.array_equal(got, want.astype(np.float32))
+
+
+@pytest.mark.parametrize("m", [1, 2, 16, 20, 40, 70])
+@pytest.mark.parametrize("bs,level", [(16, 0), (16, 1), (32, 1)])
+def test_every_bit_of_a_small_value_beside_a_large_one(ctx, pkg, bs, level, m):
+    """Where three terms are promised (accuracy_level 1, and blocks of 16, unless a level allows less): 24 significant
+    bits of a value 2^30 times smaller than the row's largest. One product per result, so the result is that product,
+    correctly rounded but for the bias some kernels carry (the nearest f32, or its neighbours)."""
+    k, n = 512, 32
+    rng = np.random.default_rng(78)
+    q = np.full((n, k), 8, np.uint8)
+    q[:, 7] = rng.integers(9, 16, n)
+    B = pkg.synth.pack_nibbles(q, bs)
+    scales = np.ones(n * (k // bs), np.float32)
+    a = np.zeros((m, k), np.float32)
+    a[:, 300] = 1.5
+    a[:, 7] = (rng.integers(1 << 23, 1 << 24, m) | 1) * 2.0**-53
+    w = pkg.ops.NBitsWeight(ctx, B, scales, None, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    w.destroy()
+    want = np.outer(a[:, 7].astype(np.float64), q[:, 7].astype(np.float64) - 8)
+    # the terms leave up to half a unit of the value's last bit, and f32 rounds the product and the terms' sum once each;
+    # one row of blocks of 32 is multiplied as 128 + q, and 128 + zp taken back: roundings at 143 times the result's size
+    bound = 4 * 2.0**-24 * (143 if m == 1 and bs == 32 else 1)
+    assert np.all(np.abs(got - want) <= bound * np.abs(want))
