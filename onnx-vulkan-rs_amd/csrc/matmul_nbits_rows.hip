@@ -58,8 +58,10 @@ __host__ __device__ inline size_t rows_operands(int M, int terms, int stage_tile
 // 4 NR with one block: then register r of lane group g is row g + 4 r, else row 4 g + r). T: 16-column tiles per wavefront.
 // P: pieces of the rows a thread holds at most (kRowsPieces of f32, kRowsPieces16 of f16, or a quarter: a launch starts with
 // its instruction cache empty, and code for pieces that do not exist is 0.3 us a kilobyte).
+// Two column tiles of blocks of 16 are told to keep within 128 registers (four wavefronts on a SIMD), which rows_plan counts
+// on and they would miss by a few (one row, 1152 -> 13824 in two terms: 8.6 us, so 7.0).
 template <int SG, int SRC, int NT, int RB, int NR, int T, int P>
-__global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsArgs p) {
+__global__ void __launch_bounds__(64 * kRowsWaves, SG == 8 && RB == 1 && T == 2 && P <= 4 ? 4 : 1) mmnb_rows_kernel(const RowsArgs p) {
     extern __shared__ uint4 smem[];
     const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave % p.WK, wn = wave / p.WK;
@@ -131,10 +133,11 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
     HIPC_PIN_VGPR(ones);
 
     // blocks of 16: a product step of 32 k covers two of them, k groups 0 and 1 the first, 2 and 3 the second. Each is a
-    // product of its own with the other half of the weight operand zeroed (the matrix cores have the time)
+    // product of its own with the other half of one operand zeroed (the matrix cores have the time): of a row's first term,
+    // which may hold an infinity that a weight of zero would make NaN of, and of the weight for the others, which are finite
     const uint32_t first16 = SG == 8 && g4 < 2 ? ~0u : 0u;
-    const auto masked = [](const f16x8 &w, uint32_t keep) {
-        const uint4 v = __builtin_bit_cast(uint4, w);
+    const auto masked = [](const f16x8 &o, uint32_t keep) {
+        const uint4 v = __builtin_bit_cast(uint4, o);
         return __builtin_bit_cast(f16x8, make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep));
     };
     // Where the registers allow it (128 hold twice the wavefronts of 129) the first terms' products have a sum of their own --
@@ -190,8 +193,8 @@ __global__ void __launch_bounds__(64 * kRowsWaves) mmnb_rows_kernel(const RowsAr
 #pragma unroll
                         for (int e = NT - 1; e >= 0; e--) {
                             const int c = APART && e > 0;
-                            v0[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], weight_for(w0, e), v0[c], 0, 0, 0);
-                            v1[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][e], weight_for(w1, e), v1[c], 0, 0, 0);
+                            v0[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(e ? a[b][e] : masked(a[b][e], first16), e ? weight_for(w0, e) : w, v0[c], 0, 0, 0);
+                            v1[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(e ? a[b][e] : masked(a[b][e], ~first16), e ? weight_for(w1, e) : w, v1[c], 0, 0, 0);
                         }
 #pragma unroll
                         for (int r = 0; r < NR; r++) add(b, t, r, j == 0, st.s[t][2 * j % SG], joined(v0, r)), add(b, t, r, false, st.s[t][(2 * j + 1) % SG], joined(v1, r));

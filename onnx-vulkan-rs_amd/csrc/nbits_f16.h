@@ -32,7 +32,9 @@ __device__ __forceinline__ void split_terms(float x, _Float16 (&t)[NT]) {
     constexpr float step = NT == 3 ? kTermStep : 1.f;
     t[0] = (_Float16)x;
     if constexpr (NT >= 2) {
-        const float r = (x - (float)t[0]) * step;
+        // (an infinity leaves infinity minus itself: the maximum makes a number of that, which the infinite first term outweighs.
+        // Any other remainder is 8 at most, half a step of f16 below 2^15.)
+        const float r = fmaxf(x - (float)t[0], -8.f) * step;
         t[1] = (_Float16)r;
         if constexpr (NT == 3) t[2] = (_Float16)((r - (float)t[1]) * step);
     }

@@ -607,3 +607,34 @@ def test_every_bit_of_a_small_value_beside_a_large_one(ctx, pkg, bs, level, m):
     # one row of blocks of 32 is multiplied as 128 + q, and 128 + zp taken back: roundings at 143 times the result's size
     bound = 4 * 2.0**-24 * (143 if m == 1 and bs == 32 else 1)
     assert np.all(np.abs(got - want) <= bound * np.abs(want))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("m", [1, 3, 16, 20, 40, 70])
+def test_infinite_activations_with_blocks_of_sixteen(ctx, pkg, m, dtype):
+    """One infinite value in a row: what the operator's own layout gives -- an infinity of the product's sign, NaN where
+    the weight is zero -- and nothing in other rows."""
+    k, n, bs = 512, 64, 16
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=531, scale_dtype=dtype)
+    a = pkg.synth.normal_f32(m * k, 532).reshape(m, k).astype(dtype)
+    a[0, 37] = np.inf
+    if m > 2:
+        a[2, 500] = -np.inf
+        a[1, 3] = 6e4 if dtype == np.float16 else 1e8       # (finite)
+    want = pkg.ops.matmul_nbits(ctx, a[:, :], B, scales, zp, k, n, bs) if m <= 16 else None
+    d, s = unpacked(B, scales, zp, k, n, bs)
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, weight=w)
+    w.destroy()
+    for r, at, sign in ((0, 37, 1), (2, 500, -1)):
+        if r >= m:
+            continue
+        zero = d[:, at] == 0
+        assert np.all(np.isnan(got[r][zero])) and np.array_equal(got[r][~zero], sign * np.sign(d[~zero, at]) * np.inf)
+        assert want is None or np.array_equal(got[r], want[r], equal_nan=True)
+    rest = [r for r in range(m) if r not in (0, 2)]
+    exact = a[rest].astype(np.float64) @ (d * s).T
+    with np.errstate(over="ignore"):
+        assert np.all(np.isfinite(got[rest]) == np.isfinite(exact.astype(dtype)))
+    ok = np.isfinite(got[rest])
+    assert np.all(np.abs(got[rest] - exact)[ok] <= (1e-2 if dtype == np.float16 else 1e-3) + 2e-3 * np.abs(exact)[ok])
