@@ -308,6 +308,9 @@ int allow_dynamic_lds(hipc_ctx *ctx, K kernel, size_t bytes, bool (&done)[kMaxDe
 // Returns ctx->scratch[slot] grown to at least `bytes`. Growth allocates, so it is
 // refused while a capture is open.
 int scratch_get(hipc_ctx *ctx, int slot, size_t bytes, void **out);
+// whether it would: inside a capture only what the slot has grown to before. A call that was never run eagerly takes a route
+// that needs no scratch memory there, where it has one
+inline bool scratch_fits(const hipc_ctx *ctx, int slot, size_t bytes) { return !ctx->capturing || ctx->scratch[slot].bytes >= bytes; }
 // host bytes -> device through the context's pinned staging ring; records only (see StageRing)
 int stage_upload(hipc_ctx *ctx, void *dst, const void *host, size_t bytes);
 // looks up this device's address of the static range-partials array of the DynamicQuantizeLinear
@@ -475,12 +478,14 @@ bool nbits_prefill_takes(const void *A, const hipc_nbits_weight *w, int64_t M);
 int nbits_prefill(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int64_t M);
 // f32 activations, more than 32 rows: the same kernel on two f16 rows per row (see matmul_nbits_prefill.hip)
 bool nbits_prefill_f32_takes(const void *A, const hipc_nbits_weight *w, int64_t M);
+bool nbits_prefill_f32_fits(hipc_ctx *ctx, const hipc_nbits_weight *w, int64_t M, int terms);   // its scratch memory (see scratch_fits)
 int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int64_t M, int terms);   // f16 terms per f32 row: 2 (22 bits), 1 (11) or 3 (all 24)
 
 // A few rows (matmul_nbits_rows.hip): up to 64 of f16, or of f32 as f16 terms -- up to 16 split by the kernel itself, more by
 // a launch in front (one term or two; see nbits_prefill_f32).
 constexpr int kFewRows = 64;
-bool nbits_rows_takes(const void *A, const hipc_nbits_weight *w, int64_t M, int terms);
+bool nbits_rows_takes(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weight *w, int64_t M, int terms);
+size_t nbits_split_bytes(int64_t rows, int64_t M, int64_t K);   // scratch memory (slot 2) of M f32 rows as `rows` f16 rows and their exponents
 int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, const hipc_nbits_weight *w, void *Y, int y_f16, int M);
 int nbits_rows_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms);
 int nbits_rows_f32_split(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms);

@@ -102,6 +102,45 @@ mmnb_direct_kernel(const AT *__restrict__ A, const uint32_t *__restrict__ B, con
     }
 }
 
+// The tiled form in blocks of 16, without matrix cores, scratch memory or a demand on the rows' address: for calls inside a
+// capture that can have no scratch memory. A wavefront takes 16 columns and four rows through all of k, its lanes the
+// eight values of a column that share a word.
+template <typename AT>
+__global__ void __launch_bounds__(64)
+mmnb_plain16_kernel(const AT *__restrict__ A, const uint4 *__restrict__ Wq, const float *__restrict__ Sc, const uint8_t *__restrict__ Zb, AT *__restrict__ Y, int M, int K, int N,
+                    int n_cg) {
+    const int lane = threadIdx.x, i16 = lane & 15, g4 = lane >> 4, m0 = blockIdx.y * 4, n = blockIdx.x * 16 + i16;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int cg = 0; cg < n_cg; cg++) {
+        const size_t tile = (size_t)blockIdx.x * n_cg + cg;
+        const uint4 q = Wq[tile * 64 + lane];
+        const uint32_t words[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k0 = cg * 128 + 32 * j + 8 * g4;
+            if (k0 >= K) continue;   // (K is a multiple of 8)
+            const size_t at = (tile * 16 + i16) * 8 + 2 * j + (g4 >> 1);
+            const float s = Sc[at];
+            const int z = (int)Zb[at] - 128;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {   // (the word holds k0 k2 k4 k6 k1 k3 k5 k7)
+                const int k = k0 + (i < 4 ? 2 * i : 2 * i - 7);
+                const float wv = (float)((int)((words[j] >> (4 * i)) & 15u) - z) * s;
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (m0 + r < M) acc[r] = fmaf(to_f32<AT>(A[(size_t)(m0 + r) * K + k]), wv, acc[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float v = acc[r];
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (g4 == 0 && m0 + r < M && n < N) Y[(size_t)(m0 + r) * N + n] = from_f32<AT>(v);
+    }
+}
+
 // ----------------------------------------------------------------- prepack
 
 // Tile (nt, cg): 16 columns n = 16*nt + (lane & 15), four 32-k chunks c = 4*cg + j.
@@ -1204,6 +1243,17 @@ int hipc_matmul_nbits_packed(hipc_ctx *ctx, const void *A, int a_dtype, const hi
 
 namespace {
 
+template <typename AT>
+int launch_plain16(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int64_t M) {
+    for (int64_t m0 = 0; m0 < M; m0 += 4 * 65535) {   // grid.y is limited to 65535 row groups
+        const int rows = (int)std::min<int64_t>(M - m0, 4 * 65535);
+        hipLaunchKernelGGL((mmnb_plain16_kernel<AT>), dim3((unsigned)w->n_tiles, (unsigned)ceil_div(rows, 4)), 64, 0, ctx->stream, static_cast<const AT *>(A) + m0 * w->K,
+                           static_cast<const uint4 *>(w->Wq), static_cast<const float *>(w->Sc), static_cast<const uint8_t *>(w->Zb), static_cast<AT *>(Y) + m0 * w->N, rows, (int)w->K, (int)w->N, w->n_cg);
+        HIPC_LAUNCHED(ctx);
+    }
+    return HIPC_OK;
+}
+
 // Blocks of 16: up to 16 rows, and more where it is the better kernel, on the one for a few rows, the others on the tiled
 // kernel. Nothing here accumulates less than the kernel of the operator's layout, which computes in f32: an f32 value keeps all
 // 24 bits (three f16 terms; down to 2^-30 of its row's largest, see split_terms) unless accuracy_level allows less. That kernel, which unpacks the weight and multiplies it
@@ -1213,6 +1263,8 @@ int packed_run16(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_wei
     const bool f16 = a_dtype == HIPC_F16;
     const size_t esz = f16 ? 2 : 4;
     if (!aligned(A, 16)) {   // (the kernels read 16-byte pieces: rows that do not start on one are moved first)
+        if (!scratch_fits(ctx, 5, (size_t)M * w->K * esz))
+            return f16 ? launch_plain16<__half>(ctx, A, w, Y, M) : launch_plain16<float>(ctx, A, w, Y, M);
         void *copy = nullptr;
         if (int rc = scratch_get(ctx, 5, (size_t)M * w->K * esz, &copy)) return rc;
         HIPC_TRY(ctx, hipMemcpyAsync(copy, A, (size_t)M * w->K * esz, hipMemcpyDeviceToDevice, ctx->stream));
@@ -1226,8 +1278,10 @@ int packed_run16(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_wei
         char *y = static_cast<char *>(Y) + (size_t)m0 * w->N * esz;
         const int terms = f16 ? 1 : accuracy_level < 2 ? 3 : rows > 32 ? 1 : 2;
         int rc;
-        if (nbits_rows_takes(a, w, rows, terms))
+        if (nbits_rows_takes(ctx, a, a_dtype, w, rows, terms))
             rc = f16 ? nbits_rows_f16(ctx, a, 1, nullptr, w, y, 1, rows) : rows <= 16 ? nbits_rows_f32(ctx, a, w, y, rows, terms) : nbits_rows_f32_split(ctx, a, w, y, rows, terms);
+        else if (!f16 && (rows <= 32 || !nbits_prefill_f32_fits(ctx, w, rows, terms)))   // (rows the tiled kernel does not take come here inside a capture only)
+            rc = launch_plain16<float>(ctx, a, w, y, rows);
         else
             rc = f16 ? nbits_prefill(ctx, a, w, y, rows) : nbits_prefill_f32(ctx, a, w, y, rows, terms);
         if (rc != HIPC_OK) return rc;
@@ -1258,7 +1312,7 @@ int packed_run(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weigh
     const int NT = (accuracy_level == 1 && a_dtype == HIPC_F32) ? 3 : 2;
     // a few rows (one of f32 is a matter of its own: launch_gemv)
     const int terms = a_dtype == HIPC_F16 ? 1 : NT == 3 ? 3 : M > 32 && accuracy_level >= 2 ? 1 : 2;
-    if ((a_dtype == HIPC_F16 || M > 1) && nbits_rows_takes(A, w, M, terms)) {
+    if ((a_dtype == HIPC_F16 || M > 1) && nbits_rows_takes(ctx, A, a_dtype, w, M, terms)) {
         if (a_dtype == HIPC_F16) return nbits_rows_f16(ctx, A, 1, nullptr, w, Y, 1, (int)M);
         return M <= 16 ? nbits_rows_f32(ctx, A, w, Y, (int)M, terms) : nbits_rows_f32_split(ctx, A, w, Y, (int)M, terms);
     }
@@ -1292,8 +1346,9 @@ int tiled_from_onnx_layout(hipc_ctx *ctx, const void *A, int a_dtype, const void
     // only where a tiled kernel will take the rows (otherwise sixteen rows at a time on the decode kernel: no gain)
     const bool many = a_dtype == HIPC_F16 ? nbits_prefill_takes(A, &w, M) : nbits_prefill_f32_takes(A, &w, M);
     if (!many) return HIPC_OK;
-    *taken = true;
     const size_t wq_r = (wq_bytes + 255) & ~(size_t)255, sc_r = (sc_bytes + 255) & ~(size_t)255;
+    if (!scratch_fits(ctx, 4, wq_r + sc_r + zb_bytes)) return HIPC_OK;
+    *taken = true;
     void *block = nullptr;
     if (int rc = scratch_get(ctx, 4, wq_r + sc_r + zb_bytes, &block)) return rc;
     w.Wq = static_cast<uint4 *>(block);

@@ -759,9 +759,11 @@ int prefill_plan(hipc_ctx *ctx, PrefillArgs &a, int TM, int TN, bool may_split, 
     a.split_stages = (int)(ceil_div(ceil_div(nk, ksplit), 2) * 2);
     a.ksplit = (int)ceil_div(nk, a.split_stages);
     a.Ypart = nullptr;
+    const size_t part_bytes = (size_t)a.ksplit * a.M * a.N * sizeof(float);
+    if (a.ksplit > 1 && !scratch_fits(ctx, 0, part_bytes)) a.split_stages = (int)(ceil_div(nk, 2) * 2), a.ksplit = 1;
     if (a.ksplit > 1) {
         void *part = nullptr;
-        if (int rc = scratch_get(ctx, 0, (size_t)a.ksplit * a.M * a.N * sizeof(float), &part)) return rc;
+        if (int rc = scratch_get(ctx, 0, part_bytes, &part)) return rc;
         a.Ypart = static_cast<float *>(part);
     }
     *grid = dim3(gx, (unsigned)a.ksplit);
@@ -1016,15 +1018,29 @@ bool nbits_prefill_f32_takes(const void *A, const hipc_nbits_weight *w, int64_t 
     return M > 32 && w->K % 8 == 0 && aligned(A, 16) && (3 * M + 64) * w->K < (int64_t(1) << 31) && 3 * M * w->N < (int64_t(1) << 31);
 }
 
+namespace {
+// the exponents of M rows, padded, in front of the f16 rows
+size_t split_exps_bytes(int64_t M) { return ((size_t)M * sizeof(int) + 255) & ~(size_t)255; }
+// two terms: the pairs of the kernel that keeps the weight out of LDS; three (f32 pinned: all 24 bits), or the
+// kernel with both operands in LDS: `terms` M rows, and a launch that adds them
+bool split_paired(hipc_ctx *ctx, const hipc_nbits_weight *w, int terms) { return terms == 2 && (ctx->tune.prefill_direct != 0 || w->SG == 8); }
+}  // namespace
+size_t nbits_split_bytes(int64_t rows, int64_t M, int64_t K) { return (size_t)rows * K * sizeof(__half) + split_exps_bytes(M); }
+
+bool nbits_prefill_f32_fits(hipc_ctx *ctx, const hipc_nbits_weight *w, int64_t M, int terms) {
+    const bool paired = split_paired(ctx, w, terms);
+    if (!scratch_fits(ctx, 2, nbits_split_bytes(paired ? 64 * ceil_div(M, 32) : terms * M, M, w->K))) return false;
+    return terms == 1 || paired || scratch_fits(ctx, 3, (size_t)terms * M * w->N * sizeof(float));
+}
+
 int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int64_t M, int terms) {
     HIPC_REFUSE(ctx, !nbits_prefill_f32_takes(A, w, M), "MatMulNBits prefill: shape or alignment not taken by the tiled kernel");
     if (terms == 1) {
         // one f16 term per row (11 bits beside the row's own power of two): M rows through the kernel, which scales
         // the rows of its f32 result back itself (after a k split, the reduce launch does)
-        const size_t e_bytes = ((size_t)M * sizeof(int) + 255) & ~(size_t)255;
         void *split = nullptr;
-        if (int rc = scratch_get(ctx, 2, (size_t)M * w->K * sizeof(__half) + e_bytes, &split)) return rc;
-        __half *A1 = reinterpret_cast<__half *>(static_cast<char *>(split) + e_bytes);
+        if (int rc = scratch_get(ctx, 2, nbits_split_bytes(M, M, w->K), &split)) return rc;
+        __half *A1 = reinterpret_cast<__half *>(static_cast<char *>(split) + split_exps_bytes(M));
         int *exps = static_cast<int *>(split);
         hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 1>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), (int)M, (int)w->K, A1, exps);
         HIPC_LAUNCHED(ctx);
@@ -1038,16 +1054,13 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
             default: return prefill_launch<1>(ctx, a);
         }
     }
-    // two terms: the pairs of the kernel that keeps the weight out of LDS; three (f32 pinned: all 24 bits), or the
-    // kernel with both operands in LDS: `terms` M rows, and a launch that adds them
-    const bool paired = terms == 2 && (ctx->tune.prefill_direct != 0 || w->SG == 8);
+    const bool paired = split_paired(ctx, w, terms);
     const int64_t rows2 = paired ? 64 * ceil_div(M, 32) : terms * M;
-    const size_t a2_bytes = (size_t)rows2 * w->K * sizeof(__half), e_bytes = ((size_t)M * sizeof(int) + 255) & ~(size_t)255;
     void *split = nullptr, *sums = nullptr;
-    if (int rc = scratch_get(ctx, 2, a2_bytes + e_bytes, &split)) return rc;
+    if (int rc = scratch_get(ctx, 2, nbits_split_bytes(rows2, M, w->K), &split)) return rc;
     if (!paired)
         if (int rc = scratch_get(ctx, 3, (size_t)terms * M * w->N * sizeof(float), &sums)) return rc;
-    __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + e_bytes);
+    __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + split_exps_bytes(M));
     int *exps = static_cast<int *>(split);
     if (paired)
         hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<true, 2>), dim3((unsigned)(rows2 / 2)), dim3(256), 0, ctx->stream, static_cast<const float *>(A), (int)M, (int)w->K, A2, exps);
@@ -1079,10 +1092,9 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
 
 // up to 64 rows of f32, split here and multiplied as f16 rows by the kernel for a few rows (matmul_nbits_rows.hip)
 int nbits_rows_f32_split(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void *Y, int M, int terms) {
-    const size_t e_bytes = ((size_t)M * sizeof(int) + 255) & ~(size_t)255;
     void *split = nullptr;
-    if (int rc = scratch_get(ctx, 2, (size_t)terms * M * w->K * sizeof(__half) + e_bytes, &split)) return rc;
-    __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + e_bytes);
+    if (int rc = scratch_get(ctx, 2, nbits_split_bytes(terms * M, M, w->K), &split)) return rc;
+    __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + split_exps_bytes(M));
     int *exps = static_cast<int *>(split);
     if (terms == 1)
         hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 1>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), M, (int)w->K, A2, exps);

@@ -463,9 +463,9 @@ struct RowsPlan {
 // (17.7 TB/s of L2 over 256 CUs), of rows and of weight alike: few columns per workgroup read the rows often, many leave
 // CUs without work, the code of a tile's products is fetched by an empty instruction cache (600 clocks per row block and
 // column tile: 24 x 2048 x 8320 9.2 us without that term, 7.6 with it), and a split costs a second launch, some 6000 clocks with its own trip through memory.
-bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT, int RB, int NR, RowsPlan *best) {
+bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT, int RB, int NR, bool may_split, RowsPlan *best) {
     const int cus = std::max(1, ctx->cu_count), max_waves = kRowsWaves;
-    const int most_splits = std::min(w->n_cg, std::max(16, (int)ceil_div(w->n_cg, 8)));   // (up to eight tiles of k fit any launch)
+    const int most_splits = may_split ? std::min(w->n_cg, std::max(16, (int)ceil_div(w->n_cg, 8))) : 1;   // (up to eight tiles of k fit any launch)
     double best_cost = 0;
     bool found = false;
     static const int shapes[][2] = {{4, 1}, {2, 1}, {1, 1}, {2, 2}, {1, 2}};   // column tiles per wavefront, wavefronts side by side
@@ -513,6 +513,13 @@ bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT
     return found;
 }
 
+// ... for this call: without a split of k where its scratch memory is not to be had
+size_t rows_part_bytes(const hipc_nbits_weight *w, int M, const RowsPlan &pl) { return (size_t)pl.splits * M * w->N * sizeof(float); }
+bool rows_plan_now(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT, int RB, int NR, RowsPlan *pl) {
+    if (!rows_plan(ctx, w, M, src, NT, RB, NR, true, pl)) return false;
+    return pl->splits == 1 || scratch_fits(ctx, 0, rows_part_bytes(w, M, *pl)) || rows_plan(ctx, w, M, src, NT, RB, NR, false, pl);
+}
+
 template <int SG, int SRC, int NT, int RB, int NR, int T, int P>
 int rows_launch_p(hipc_ctx *ctx, const RowsArgs &a, const RowsPlan &pl) {
     static bool lds_allowed[kMaxDevices] = {};
@@ -547,7 +554,7 @@ int rows_launch_sg(hipc_ctx *ctx, const RowsArgs &a, const RowsPlan &pl, int SG)
 template <int SRC, int NT, int RB, int NR>
 int rows_run(hipc_ctx *ctx, RowsArgs a, const hipc_nbits_weight *w) {
     RowsPlan pl;
-    HIPC_REFUSE(ctx, !rows_plan(ctx, w, a.M, SRC, NT, RB, NR, &pl), "MatMulNBits rows: no launch shape for %d rows", a.M);
+    HIPC_REFUSE(ctx, !rows_plan_now(ctx, w, a.M, SRC, NT, RB, NR, &pl), "MatMulNBits rows: no launch shape for %d rows", a.M);
     a.Wq = w->Wq, a.Sc = w->Sc, a.Zb = w->Zb;
     a.K = (int)w->K, a.N = (int)w->N, a.n_tiles = w->n_tiles, a.n_cg = w->n_cg;
     a.WK = pl.WK, a.WN = pl.WN, a.split_tiles = pl.split_tiles, a.stage_tiles = pl.stage_tiles;
@@ -555,7 +562,7 @@ int rows_run(hipc_ctx *ctx, RowsArgs a, const hipc_nbits_weight *w) {
     a.Ypart = nullptr;
     if (pl.splits > 1) {
         void *part = nullptr;
-        if (int rc = scratch_get(ctx, 0, (size_t)pl.splits * a.M * a.N * sizeof(float), &part)) return rc;
+        if (int rc = scratch_get(ctx, 0, rows_part_bytes(w, a.M, pl), &part)) return rc;
         a.Ypart = static_cast<float *>(part);
     }
     int rc;
@@ -600,11 +607,18 @@ int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, con
 // 4096 18.1 -> 21.4; f32 (which the tiled kernel takes 64 rows at a time) 48 x 6912 x 1152 41 -> 22.7, 48 x 4096 x 4096 39 ->
 // 25, but 64 x 2048 x 8192 32.6 -> 37. A weight of 2048 column tiles or more and up to 16 rows stay on the streaming kernel,
 // whose wavefronts each walk all of k and meet nobody: 4 x 1152 x 262144 35.7 us there (5.5 TB/s), 50 here.
-bool nbits_rows_takes(const void *A, const hipc_nbits_weight *w, int64_t M, int terms) {
+// Inside a capture, only where the scratch memory is to be had or not needed.
+bool nbits_rows_takes(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weight *w, int64_t M, int terms) {
     if (M > kFewRows || terms * M > 128 || w->K % 8 != 0 || !aligned(A, 16)) return false;
-    if (M <= 16) return w->n_tiles < 2048 || w->SG == 8;   // (the streaming kernel has no form for blocks of 16)
-    if (M <= 32) return terms > 1 || w->n_tiles <= 300 || w->n_cg > 4;
-    return w->n_tiles <= (terms > 1 ? 300 : 128);
+    const bool shape = M <= 16 ? w->n_tiles < 2048 || w->SG == 8   // (the streaming kernel has no form for blocks of 16)
+                     : M <= 32 ? terms > 1 || w->n_tiles <= 300 || w->n_cg > 4 : w->n_tiles <= (terms > 1 ? 300 : 128);
+    if (!shape || !ctx->capturing) return shape;
+    const bool split_in_front = a_dtype == HIPC_F32 && M > 16;
+    if (split_in_front && !scratch_fits(ctx, 2, nbits_split_bytes(terms * M, M, w->K))) return false;
+    const int src = a_dtype == HIPC_F32 && M <= 16 ? SRC_F32 : SRC_F16;
+    const int RB = M > 32 ? 4 : M > 16 ? 2 : 1, NR = M <= 4 ? 1 : M <= 8 ? 2 : 4;   // (as nbits_rows_f32 and nbits_rows_f16 dispatch)
+    RowsPlan pl;
+    return rows_plan_now(ctx, w, (int)M, src, terms, RB, NR, &pl);
 }
 
 // up to 16 rows of f32, as two f16 terms or three

@@ -42,6 +42,8 @@ bool nbits_prefill_takes(const void *, const hipc_nbits_weight *, int64_t) { ret
 int nbits_rows_f32_split(hipc_ctx *, const void *, const hipc_nbits_weight *, void *, int, int) { return HIPC_ERR_UNSUPPORTED; }
 int nbits_prefill(hipc_ctx *, const void *, const hipc_nbits_weight *, void *, int64_t) { return HIPC_ERR_UNSUPPORTED; }
 bool nbits_prefill_f32_takes(const void *, const hipc_nbits_weight *, int64_t) { return false; }
+bool nbits_prefill_f32_fits(hipc_ctx *, const hipc_nbits_weight *, int64_t, int) { return false; }
+size_t nbits_split_bytes(int64_t, int64_t, int64_t) { return 0; }
 int nbits_prefill_f32(hipc_ctx *, const void *, const hipc_nbits_weight *, void *, int64_t, int) { return HIPC_ERR_UNSUPPORTED; }
 }  // namespace hipc
 extern "C" {

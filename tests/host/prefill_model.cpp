@@ -23,6 +23,7 @@ alignas(16) thread_local uint4 smem[160 * 1024 / 16];
 thread_local float wgt[40960];
 int scratch_get(hipc_ctx *ctx, int slot, size_t bytes, void **out) {
     Scratch &s = ctx->scratch[slot];
+    if (s.bytes < bytes && ctx->capturing) return HIPC_ERR_UNSUPPORTED;
     if (s.bytes < bytes) {
         if (s.ptr) gpu_model::release(s.ptr);
         s.ptr = gpu_model::alloc(bytes);   // exactly what was asked for: stricter than the library's rounding
@@ -120,6 +121,19 @@ void rows(int64_t M, int64_t K, int64_t N, int64_t bs, bool with_zp, int a_dtype
             MUST(hipc_matmul_nbits_packed(&ctx, A, a_dtype, w, Y, M, 0));
         }
         ctx.tune.gemv_lean = -1;
+        // a first call inside a capture: no scratch memory to be had; rows that start off 16 bytes too (blocks of 16 copy those)
+        hipc::Scratch grown[hipc::kScratchSlots];
+        std::swap(ctx.scratch, grown);
+        ctx.capturing = true;
+        void *moved = gpu_model::alloc((size_t)(M * K + 1) * esz);
+        std::memset(moved, 0, (size_t)(M * K + 1) * esz);
+        for (void *from : {A, static_cast<void *>(static_cast<char *>(moved) + esz)}) {
+            const int rc = hipc_matmul_nbits_packed(&ctx, from, a_dtype, w, Y, M, 0);
+            if (rc != HIPC_OK && (rc != HIPC_ERR_UNSUPPORTED || bs == 16)) MUST(rc);   // (a long k on the streaming kernel wants some)
+        }
+        ctx.capturing = false;
+        std::swap(ctx.scratch, grown);
+        gpu_model::release(moved);
         hipc_nbits_weight_destroy(&ctx, w);
     }
     for (void *p : {A, Y, B, S, Z}) gpu_model::release(p);

@@ -638,3 +638,54 @@ def test_infinite_activations_with_blocks_of_sixteen(ctx, pkg, m, dtype):
         assert np.all(np.isfinite(got[rest]) == np.isfinite(exact.astype(dtype)))
     ok = np.isfinite(got[rest])
     assert np.all(np.abs(got[rest] - exact)[ok] <= (1e-2 if dtype == np.float16 else 1e-3) + 2e-3 * np.abs(exact)[ok])
+
+
+FIRST_IN_A_CAPTURE = [  # (M, K, N, block, activations, elements the rows are off 16 bytes): what an unrecorded first call wants scratch memory for
+    (2, 4096, 256, 32, np.float32, 0),       # k split over workgroups
+    (6, 6912, 1152, 128, np.float16, 0),
+    (24, 640, 600, 32, np.float32, 0),       # rows split into terms by a launch in front
+    (100, 8192, 1024, 64, np.float16, 0),    # 64-row tiles with k split
+    (1, 6912, 1152, 16, np.float32, 0), (16, 4096, 272, 16, np.float32, 0), (20, 1288, 600, 16, np.float32, 0), (65, 1000, 131, 16, np.float32, 0),
+    (100, 8192, 1024, 16, np.float16, 0),
+    (1, 1160, 130, 16, np.float32, 1), (5, 1160, 130, 16, np.float16, 1), (43, 520, 96, 16, np.float32, 2),   # rows off 16 bytes
+]
+
+
+@pytest.mark.parametrize("layout", ["handle", "operator"])
+@pytest.mark.parametrize("case", FIRST_IN_A_CAPTURE, ids=lambda c: "M%d_K%d_N%d_bs%d_%s_off%d" % (*c[:4], c[4].__name__, c[5]))
+def test_a_first_call_inside_a_capture(pkg, oracle, case, layout):
+    """A context that has never run the operator records it: scratch memory cannot grow there, and the call takes a route
+    that needs none. The graph is replayed with eager work in between, which may then grow the scratch memory."""
+    m, k, n, bs, dtype, off = case
+    if layout == "operator" and bs != 16 and m > 16:
+        pytest.skip("many rows on the operator's layout write the tiled form to scratch memory")
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=541, scale_dtype=dtype)
+    a = pkg.synth.normal_f32(m * k, 542).reshape(m, k).astype(dtype)
+    want = oracle.matmul_nbits(a, B, scales, zp, k, n, bs)
+    rtol = RTOL32 if dtype == np.float32 else RTOL16
+    with pkg.Context(0) as c:
+        dt = pkg.ops.hipc_dtype(a.dtype)
+        dA = c.upload(np.concatenate([np.zeros(off, dtype), a.reshape(-1)]))
+        dY = c.alloc(m * n * a.itemsize)
+        if layout == "handle":
+            w = pkg.ops.NBitsWeight(c, B, scales, zp, k, n, bs)
+            call = lambda: pkg.ops.matmul_nbits_packed_device(c, dA.at(off * a.itemsize), dt, w, dY, m)  # noqa: E731
+        else:
+            held = [c.upload(v) for v in (B, scales, zp)]
+            call = lambda: pkg.ops.matmul_nbits_device(c, dA.at(off * a.itemsize), dt, held[0], B.size, held[1], dt, scales.size, held[2], zp.size, dY, m, k, n, bs)  # noqa: E731
+        c.flush()
+        c.capture_begin()
+        try:
+            call()
+        finally:
+            graph = c.capture_end()
+        for _ in range(3):
+            c.fill(dY, 0, m * n * a.itemsize // 4 * 4, 0)
+            c.graph_launch(graph)
+            got = c.download(dY, dtype, (m, n))
+            assert close(got, want, rtol), worst(got, want)
+            call()
+            assert close(c.download(dY, dtype, (m, n)), want, rtol)
+        c.graph_destroy(graph)
+        if layout == "handle":
+            w.destroy()
