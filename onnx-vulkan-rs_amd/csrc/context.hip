@@ -194,25 +194,28 @@ int stage_upload(hipc_ctx *ctx, void *dst, const void *host, size_t bytes) {
 
 int ratio_resident(hipc_ctx *ctx, RatioCache &cache, float x_scale, const float *w_scale, int64_t n, float y_scale, int64_t count, const float **out) {
     const bool same_pair = memcmp(&cache.x_scale, &x_scale, sizeof x_scale) == 0 && memcmp(&cache.y_scale, &y_scale, sizeof y_scale) == 0;
-    if (cache.dev && same_pair && cache.count == count && cache.w_scale.size() == (size_t)n &&
+    if (cache.dev && same_pair && cache.ratio.size() == (size_t)count && cache.w_scale.size() == (size_t)n &&
         memcmp(cache.w_scale.data(), w_scale, (size_t)n * sizeof(float)) == 0) {
         *out = cache.dev;
         return HIPC_OK;
     }
-    HIPC_REFUSE(ctx, ctx->capturing, "QLinear: the requantisation ratios changed and would have to be uploaded inside a capture; run the operator once before capturing");
     std::vector<float> ratio((size_t)count);
     for (int64_t c = 0; c < count; c++) {
         volatile float t = x_scale * w_scale[n == 1 ? 0 : c];   // (rounded on its own)
         ratio[(size_t)c] = t / y_scale;
     }
-    // A new block every time the ratios change: earlier launches, and graphs recorded with the old
-    // scales, keep reading the old one (it is retired, not rewritten).
-    retire(ctx, cache.dev);
-    cache.dev = nullptr;
-    cache.w_scale.clear();
-    HIPC_TRY(ctx, hipMalloc(reinterpret_cast<void **>(&cache.dev), std::max<size_t>(ratio.size() * sizeof(float), 16)));
-    if (int rc = stage_upload(ctx, cache.dev, ratio.data(), ratio.size() * sizeof(float))) return rc;
-    cache.x_scale = x_scale, cache.y_scale = y_scale, cache.count = count;
+    if (!cache.dev || cache.ratio.size() != ratio.size() || memcmp(cache.ratio.data(), ratio.data(), ratio.size() * sizeof(float)) != 0) {
+        HIPC_REFUSE(ctx, ctx->capturing, "QLinear: the requantisation ratios changed and would have to be uploaded inside a capture; run the operator once before capturing");
+        // A new block every time the ratios change: earlier launches, and graphs recorded with the old
+        // scales, keep reading the old one (it is retired, not rewritten).
+        retire(ctx, cache.dev);
+        cache.dev = nullptr;
+        cache.ratio.clear();
+        HIPC_TRY(ctx, hipMalloc(reinterpret_cast<void **>(&cache.dev), std::max<size_t>(ratio.size() * sizeof(float), 16)));
+        if (int rc = stage_upload(ctx, cache.dev, ratio.data(), ratio.size() * sizeof(float))) return rc;
+        cache.ratio = std::move(ratio);
+    }
+    cache.x_scale = x_scale, cache.y_scale = y_scale;
     cache.w_scale.assign(w_scale, w_scale + n);
     *out = cache.dev;
     return HIPC_OK;

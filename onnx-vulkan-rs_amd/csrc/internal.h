@@ -278,17 +278,17 @@ inline void retire(hipc_ctx *ctx, void *p) {
 #define HIPC_LAUNCHED(ctx) HIPC_TRY((ctx), hipGetLastError())
 
 // Requantisation ratios of a QLinear operator, kept with the weight handle: ratio[c] = x_scale * w_scale[c] / y_scale in
-// f32, left to right (interp.rs:4693), formed on the host from the operator's scale attributes. As long as those do not
-// change between calls the device copy is reused, so a call neither uploads nor synchronises and can be captured -- nor
-// does it form them again (4096 of them were 3 us of every call).
+// f32, left to right (interp.rs:4693), formed on the host from the operator's scale attributes. As long as the ratios do not
+// change between calls the device copy is reused, so a call neither uploads nor synchronises and can be captured; as long as
+// the attributes do not, they are not even formed again (4096 of them were 3 us of every call).
 struct RatioCache {
     float *dev = nullptr;
-    float x_scale = 0.f, y_scale = 0.f;   // the attributes they were formed from
-    int64_t count = 0;
+    std::vector<float> ratio;             // what `dev` holds
+    float x_scale = 0.f, y_scale = 0.f;   // the attributes the last call formed it from
     std::vector<float> w_scale;
 };
 // *out = device pointer to `count` ratios from `n` weight scales (count, or 1: the same for all), uploading them first when
-// an attribute differs from the last call's; that upload is refused while a capture is open
+// one differs from the last call's; that upload is refused while a capture is open
 int ratio_resident(hipc_ctx *ctx, RatioCache &cache, float x_scale, const float *w_scale, int64_t n, float y_scale, int64_t count, const float **out);
 void ratio_release(hipc_ctx *ctx, RatioCache &cache);
 

@@ -317,3 +317,36 @@ def test_depthwise_convolutions(ctx, pkg, oracle, cfg, pads, x_type):
     assert np.array_equal(pkg.ops.conv_integer(ctx, X, W, x_zp, None, geom), oracle.conv_integer(X, W, x_zp, 0, og))
     got = pkg.ops.qlinear_conv(ctx, X, 0.03, x_zp, W, w_scale, 0, 0.1, -5, bias, geom, y_signed=True)
     assert np.array_equal(got, oracle.qlinear_conv(X, 0.03, x_zp, W, w_scale, 0, 0.1, -5, bias, og, True))
+
+
+def test_scales_with_the_same_quotients_keep_the_resident_ratios(ctx, pkg, oracle):
+    """What must be resident before a capture is the ratios: a recorded call whose scales differ from the last one's but
+    give the same quotients (both activation scales doubled; one weight scale written out per channel) needs no upload."""
+    X, W, w_scale, bias, kw = _qconv_case(pkg, 64, 64, 512, 7, 3, seed=77)
+    geom, og = pkg.ConvGeom.make(X.shape, W.shape, **kw), oracle.conv_geom(X.shape, W.shape, **kw)
+    one = np.float32(0.01)
+    ys = _y_scale(0.02, np.full(64, one, np.float32), 64 * 7)
+    weight = pkg.ops.ConvWeight(ctx, W, geom)
+    dX, dY, dB = ctx.upload(X), ctx.alloc(X.size), ctx.upload(bias.astype(np.int32))
+    run = lambda xs, ws, s: pkg.ops.qlinear_conv_device(ctx, dX, pkg.U8, xs, 128, weight, ws, 0, s, 128, pkg.U8, dB, geom, dY)  # noqa: E731
+    run(0.02, one, ys)
+    ctx.flush()
+    for xs, ws, s in ((0.04, one, 2 * ys), (0.01, np.full(64, one, np.float32), ys / 2), (0.02, one, ys)):
+        ctx.capture_begin()
+        try:
+            run(xs, ws, s)
+        finally:
+            graph = ctx.capture_end()
+        ctx.fill(dY, 0, X.size, 0)
+        ctx.graph_launch(graph)
+        want = oracle.qlinear_conv(X, xs, 128, W, ws, 0, s, 128, bias, og)
+        assert np.array_equal(ctx.download(dY, np.uint8, X.shape), want)
+        ctx.graph_destroy(graph)
+    ctx.capture_begin()
+    with pytest.raises(pkg.HipComputeError) as e:
+        run(0.02, one, 2 * ys)
+    assert e.value.code == 2
+    ctx.graph_destroy(ctx.capture_end())
+    weight.destroy()
+    for b in (dX, dY, dB):
+        b.free()
