@@ -121,7 +121,8 @@ void hipc_graph_destroy(hipc_ctx *ctx, hipc_graph *graph);
  * crates/onnx-vulkan-core/src/plan.rs:52-68: "a push-constant word that moves with the step"). Here a graph
  * keeps, for every call that recorded work while the capture was open (numbered from 0 in call order,
  * `hipc_graph_op_count` of them), the scalars of that call a replay may change without recording again:
- *   QLinearMatMul, QLinearConv        the three zero points given by value
+ *   QLinearMatMul, QLinearConv        the three zero points given by value (of a convolution on the kernels that split k
+ *                                     for a few tiles, the weight's only if it was not recorded as 0 of an int8 weight)
  *   MatMulIntegerScaleBias            the relu attribute (0 / 1)
  * `hipc_graph_set_scalar` changes one (a kernel-node parameter update of the instantiated graph); the next
  * `hipc_graph_launch` uses it. Everything that decides a launch's grid (M, the conv geometry) and everything

@@ -479,15 +479,25 @@ int hipc_graph_set_scalar(hipc_ctx *ctx, hipc_graph *graph, int op, int which, i
         HIPC_REQUIRE(ctx, !ctx->capturing, "hipc_graph_set_scalar while a capture is open");
         HIPC_REQUIRE(ctx, op >= 0 && op < (int)graph->ops.size(), "hipc_graph_set_scalar: the graph recorded %zu operator calls, not %d", graph->ops.size(), op + 1);
         int changed = 0;
+        bool other_kernel = false;
         for (const ScalarPatch &sp : graph->ops[(size_t)op].patches) {
             if (sp.which != which) continue;
             hipKernelNodeParams params{};
             HIPC_TRY(ctx, hipGraphKernelNodeGetParams(sp.node, &params));
             HIPC_REQUIRE(ctx, params.kernelParams && params.kernelParams[0], "hipc_graph_set_scalar: the kernel node carries no arguments");
             memcpy(static_cast<char *>(params.kernelParams[0]) + sp.offset, &value, sizeof value);
+            const bool replace = sp.func && value != 0 && params.func != sp.func;
+            if (replace) params.func = const_cast<void *>(sp.func), other_kernel = true;
             HIPC_TRY(ctx, hipGraphKernelNodeSetParams(sp.node, &params));           // the graph itself, for later instantiations
-            HIPC_TRY(ctx, hipGraphExecKernelNodeSetParams(graph->exec, sp.node, &params));
+            if (!replace) HIPC_TRY(ctx, hipGraphExecKernelNodeSetParams(graph->exec, sp.node, &params));
             changed++;
+        }
+        if (other_kernel) {   // (once per node: the kernel that reads the scalar stays, whatever the next value)
+            hipGraphExec_t exec = nullptr;
+            HIPC_TRY(ctx, hipGraphInstantiate(&exec, graph->graph, nullptr, nullptr, 0));
+            (void)hipStreamSynchronize(ctx->stream);   // replays of the old one may be under way
+            (void)hipGraphExecDestroy(graph->exec);
+            graph->exec = exec;
         }
         HIPC_REFUSE(ctx, changed == 0, "hipc_graph_set_scalar: operator call %d of the graph has no scalar %d that a replay can change", op, which);
         return HIPC_OK;

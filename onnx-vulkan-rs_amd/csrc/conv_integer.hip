@@ -19,6 +19,7 @@
 // Depthwise convolutions have a kernel of their own (conv_depth_kernel). Other grouped ones, and what fits neither (channel counts off 16 whose slab exceeds LDS), take a direct kernel, one
 // output per thread.
 #include <algorithm>
+#include <type_traits>
 
 #include "int8_conv_slab.h"
 
@@ -234,7 +235,9 @@ pack_conv_depth_kernel(const uint8_t *__restrict__ W, uint32_t *__restrict__ F, 
     rowsum[o] = sum;
 }
 
-template <int EPI, int SW, int NW>   // SW: stride along the row; NW: words of a filter row
+// SW: stride along the row; NW: words of a filter row; SUMS: the weight's zero point is not zero, which takes the sums of each
+// window (calls come here with one of zero; a recorded call may be given another)
+template <int EPI, int SW, int NW, bool SUMS>
 __global__ void __launch_bounds__(256) conv_depth_kernel(const DepthConvArgs a) {
     constexpr int NB = (3 * SW + 4 * NW + 3) / 4;   // words of input four outputs span
     const GemmArgs &p = a.g;
@@ -246,6 +249,7 @@ __global__ void __launch_bounds__(256) conv_depth_kernel(const DepthConvArgs a) 
     const int ci = div_by_magic(o, a.by_per_group);
     const int zd = (p.host_zp ? p.dyn_zp_value : zp_byte(p.dyn_zp, p.dyn_signed)) - p.dyn_shift;
     const uint32_t zd4 = (uint32_t)(zd & 0xff) * 0x01010101u, flip4 = p.dyn_shift ? 0x80808080u : 0u;
+    const int zc = SUMS ? p.const_zp_value : 0;
     const ConvChannel chan = conv_channel<EPI>(p, o);
 
     // word j of the span begins at column iw: where it is loaded from, how far that is off, which of its bytes exist
@@ -262,7 +266,7 @@ __global__ void __launch_bounds__(256) conv_depth_kernel(const DepthConvArgs a) 
     }
     const uint8_t *x = p.Q + ((size_t)img * p.C + ci) * p.H * p.W;
     const uint32_t *filter = a.filter + (size_t)o * p.kh * NW;
-    int out[4] = {0, 0, 0, 0};
+    int out[4] = {0, 0, 0, 0}, sum[4] = {0, 0, 0, 0};
     for (int r = 0; r < p.kh; r++) {
         const int ih = oh * p.sh - p.pt + r * p.dh;
         const bool inside = ih >= 0 && ih < p.H;
@@ -282,11 +286,19 @@ __global__ void __launch_bounds__(256) conv_depth_kernel(const DepthConvArgs a) 
                 const int b = i * SW + 4 * k;   // first byte of output i's taps 4 k ..
                 out[i] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_alignbyte(w[b / 4 + 1 < NB ? b / 4 + 1 : NB], w[b / 4], b % 4), f, out[i], false);
             }
+            if (SUMS) {
+                const int ones = p.kw - 4 * k >= 4 ? 0x01010101 : 0x01010101 & ((1 << (8 * (p.kw - 4 * k))) - 1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int b = i * SW + 4 * k;
+                    sum[i] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_alignbyte(w[b / 4 + 1 < NB ? b / 4 + 1 : NB], w[b / 4], b % 4), ones, sum[i], false);
+                }
+            }
         }
     }
-    const int fixed = -zd * chan.csum + (EPI == EPI_REQUANT ? chan.qb : 0);
+    const int fixed = -zd * chan.csum + p.kh * p.kw * zd * zc + (EPI == EPI_REQUANT ? chan.qb : 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) out[i] += fixed;
+    for (int i = 0; i < 4; i++) out[i] += SUMS ? fixed - zc * sum[i] : fixed;
     const size_t at = (size_t)row * p.Wo + ow;
     if (EPI == EPI_REQUANT) {
         const RequantBytes bytes{chan.ratio, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
@@ -401,7 +413,13 @@ int slab_launch(hipc_ctx *ctx, const ConvSlabArgs &a, size_t lds) {
     if (int rc = allow_dynamic_lds(ctx, int8_conv_slab_kernel<EPI, DYN, WK, WP, RAGGED>, kSlabLds, lds_allowed)) return rc;
     hipLaunchKernelGGL((int8_conv_slab_kernel<EPI, DYN, WK, WP, RAGGED>), dim3(8u * (unsigned)a.per_xcd), 256, lds, ctx->stream, a);
     HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, a.g, DYN);
+    const void *with_sums = nullptr;
+    if (!DYN && ctx->capturing) {
+        static bool sums_allowed[kMaxDevices] = {};
+        if (int rc = allow_dynamic_lds(ctx, int8_conv_slab_kernel<EPI, true, WK, WP, RAGGED>, kSlabLds, sums_allowed)) return rc;
+        with_sums = reinterpret_cast<const void *>(int8_conv_slab_kernel<EPI, true, WK, WP, RAGGED>);
+    }
+    gemm_note_scalars(ctx, a.g, DYN, with_sums);
     return HIPC_OK;
 }
 template <int EPI, bool DYN, int WK, int WP>
@@ -459,17 +477,17 @@ int run_slab(hipc_ctx *ctx, const GemmArgs &ga, const hipc_conv_weight *W, const
 int depth_words(const hipc_conv_geom &g) { return g.group == g.c_in && g.kw <= 8 ? (int)ceil_div(g.kw, 4) : 0; }
 template <int EPI>
 int depth_launch(hipc_ctx *ctx, const DepthConvArgs &a, int words) {
-    const dim3 grid((unsigned)ceil_div(a.total, 256));
-    if (a.g.sw == 1) {
-        if (words == 1) hipLaunchKernelGGL((conv_depth_kernel<EPI, 1, 1>), grid, 256, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((conv_depth_kernel<EPI, 1, 2>), grid, 256, 0, ctx->stream, a);
-    } else {
-        if (words == 1) hipLaunchKernelGGL((conv_depth_kernel<EPI, 2, 1>), grid, 256, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((conv_depth_kernel<EPI, 2, 2>), grid, 256, 0, ctx->stream, a);
-    }
-    HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, a.g, false);
-    return HIPC_OK;
+    const auto run = [&](auto stride, auto nw) -> int {
+        constexpr int SW = decltype(stride)::value, NW = decltype(nw)::value;
+        hipLaunchKernelGGL((conv_depth_kernel<EPI, SW, NW, false>), dim3((unsigned)ceil_div(a.total, 256)), 256, 0, ctx->stream, a);
+        HIPC_LAUNCHED(ctx);
+        gemm_note_scalars(ctx, a.g, false, reinterpret_cast<const void *>(conv_depth_kernel<EPI, SW, NW, true>));
+        return HIPC_OK;
+    };
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, 2> two{};
+    if (a.g.sw == 1) return words == 1 ? run(one, one) : run(one, two);
+    return words == 1 ? run(two, one) : run(two, two);
 }
 
 int run_conv(hipc_ctx *ctx, const void *X, int x_dtype, const hipc_conv_weight *W, const void *x_zp, const void *w_zp,

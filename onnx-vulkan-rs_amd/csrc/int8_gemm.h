@@ -499,12 +499,13 @@ __global__ void __launch_bounds__(256) int8_gemm_kernel(const GemmArgs p) {
 // After a launch whose argument is a GemmArgs: the scalars of it that a replay of a recorded graph may change
 // (hipc_graph_set_scalar). Zero points only when they were given by value (the QLinear operators).
 // `sums`: the launched instance forms the dynamic operand's sums over k, which a non-zero zero point of the
-// constant operand needs (an instance chosen because that zero point was known to be zero cannot take another).
-inline void gemm_note_scalars(hipc_ctx *ctx, const GemmArgs &g, bool sums) {
+// constant operand needs. An instance chosen because that zero point was known to be zero cannot take another: `with_sums`,
+// where it is given, is the one that can, launched alike.
+inline void gemm_note_scalars(hipc_ctx *ctx, const GemmArgs &g, bool sums, const void *with_sums = nullptr) {
     if (!ctx->capturing) return;
     if (g.host_zp) {
         note_scalar(ctx, HIPC_SCALAR_A_ZERO_POINT, offsetof(GemmArgs, dyn_zp_value));
-        if (sums) note_scalar(ctx, HIPC_SCALAR_B_ZERO_POINT, offsetof(GemmArgs, const_zp_value));
+        if (sums || with_sums) note_scalar(ctx, HIPC_SCALAR_B_ZERO_POINT, offsetof(GemmArgs, const_zp_value), sums ? nullptr : with_sums);
     }
     if (g.ratio) note_scalar(ctx, HIPC_SCALAR_Y_ZERO_POINT, offsetof(GemmArgs, y_zp));
     if (g.scale) note_scalar(ctx, HIPC_SCALAR_RELU, offsetof(GemmArgs, relu));

@@ -98,6 +98,8 @@ struct ScalarPatch {
     int which;              // HIPC_SCALAR_*
     hipGraphNode_t node;
     size_t offset;          // byte offset of the word inside the kernel's argument struct
+    const void *func;       // null, or the kernel (same arguments, grid and LDS) a value other than zero asks for: the recorded one
+                            // was chosen because the scalar is zero and does not read it
 };
 struct RecordedOp {
     std::vector<ScalarPatch> patches;
@@ -207,8 +209,8 @@ inline hipGraphNode_t last_captured_node(hipc_ctx *ctx) {
 }
 // called right after the launch whose argument struct holds the scalar: the word at `offset` of that struct may be
 // changed in the instantiated graph later (hipc_graph_set_scalar)
-inline void note_scalar(hipc_ctx *ctx, int which, size_t offset) {
-    if (hipGraphNode_t node = last_captured_node(ctx)) ctx->cap_patches.push_back(ScalarPatch{which, node, offset});
+inline void note_scalar(hipc_ctx *ctx, int which, size_t offset, const void *func = nullptr) {
+    if (hipGraphNode_t node = last_captured_node(ctx)) ctx->cap_patches.push_back(ScalarPatch{which, node, offset, func});
 }
 
 template <typename F>

@@ -216,7 +216,13 @@ int launch_mm_bdirect_dyn(hipc_ctx *ctx, GemmArgs g) {
     const dim3 grid(gemm_grid(g, T), 1, 1);
     hipLaunchKernelGGL((int8_gemm_bdirect_kernel<EPI, DYN, T, W>), grid, 64 * W, bd_lds(T), ctx->stream, g);
     HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, g, DYN);
+    const void *with_sums = nullptr;
+    if (!DYN && ctx->capturing) {
+        static bool sums_allowed[kMaxDevices] = {};
+        if (int rc = allow_dynamic_lds(ctx, int8_gemm_bdirect_kernel<EPI, true, T, W>, bd_lds(T), sums_allowed)) return rc;
+        with_sums = reinterpret_cast<const void *>(int8_gemm_bdirect_kernel<EPI, true, T, W>);
+    }
+    gemm_note_scalars(ctx, g, DYN, with_sums);
     return HIPC_OK;
 }
 
@@ -257,7 +263,7 @@ int launch_mm_small_dyn(hipc_ctx *ctx, GemmArgs g) {
     const dim3 grid(gemm_grid(g, 64));
     hipLaunchKernelGGL((int8_gemm_small_kernel<EPI, DYN>), grid, 256, kSmallLds, ctx->stream, g);
     HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, g, DYN);
+    gemm_note_scalars(ctx, g, DYN, reinterpret_cast<const void *>(int8_gemm_small_kernel<EPI, true>));
     return HIPC_OK;
 }
 template <int EPI>
@@ -277,6 +283,14 @@ int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {
     static bool lds_allowed[2][kMaxDevices] = {};
     const size_t lds = skinny_lds(waves, RB, cb);
     const dim3 grid((unsigned)ceil_div(cols16, cb));
+    const void *with_sums = nullptr;
+    if (!DYN && ctx->capturing) {
+        static bool sums_allowed[2][kMaxDevices] = {};
+        if (int rc = cb == 2 ? allow_dynamic_lds(ctx, int8_gemm_skinny_kernel<EPI, true, RB, 2>, skinny_lds(16, RB, 2), sums_allowed[1])
+                             : allow_dynamic_lds(ctx, int8_gemm_skinny_kernel<EPI, true, RB, 1>, skinny_lds(16, RB, 1), sums_allowed[0]))
+            return rc;
+        with_sums = cb == 2 ? reinterpret_cast<const void *>(int8_gemm_skinny_kernel<EPI, true, RB, 2>) : reinterpret_cast<const void *>(int8_gemm_skinny_kernel<EPI, true, RB, 1>);
+    }
     if (cb == 2) {
         if (int rc = allow_dynamic_lds(ctx, int8_gemm_skinny_kernel<EPI, DYN, RB, 2>, skinny_lds(16, RB, 2), lds_allowed[1])) return rc;
         hipLaunchKernelGGL((int8_gemm_skinny_kernel<EPI, DYN, RB, 2>), grid, 64 * waves, lds, ctx->stream, g);
@@ -285,7 +299,7 @@ int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {
         hipLaunchKernelGGL((int8_gemm_skinny_kernel<EPI, DYN, RB, 1>), grid, 64 * waves, lds, ctx->stream, g);
     }
     HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, g, DYN);
+    gemm_note_scalars(ctx, g, DYN, with_sums);
     return HIPC_OK;
 }
 // Up to 64 rows. Kernel alone, against the k-split 64x64 tiles (which are ahead of the LDS-staged ones there): 1 x 1024 x

@@ -348,3 +348,33 @@ def test_few_rows(ctx, pkg, oracle, shape, b_dt):
             assert np.array_equal(pkg.ops.qlinear_matmul(ctx, a, 0.02, 131, b, 0.01, 17, 0.5, 3, y_signed=signed, weight=weight),
                                   oracle.qlinear_matmul(a, 0.02, 131, b, 0.01, 17, 0.5, 3, y_signed=signed))
         weight.destroy()
+
+
+@pytest.mark.parametrize("m,k,n", [(5, 256, 96), (40, 250, 200), (64, 128, 4096), (70, 249, 96), (300, 1000, 130), (600, 1001, 900), (2500, 250, 2600)])
+def test_a_recorded_weight_zero_point_of_zero_can_be_patched(ctx, pkg, oracle, m, k, n):
+    """A QLinearMatMul recorded with an int8 weight and zero point 0 -- few rows, rows that are no whole 16 bytes -- and
+    replayed with others."""
+    a = pkg.synth.uniform_ints(m * k, 801, 0, 255).astype(np.uint8).reshape(m, k)
+    b = pkg.synth.int8_weight(k, n, 802)
+    w = pkg.ops.Int8Weight(ctx, b)
+    dA, dY = ctx.upload(a), ctx.alloc(m * n)
+    ys = 0.02 * 0.01 * 74 * 73 * np.sqrt(k) / 40
+    call = lambda: pkg.ops.qlinear_matmul_device(ctx, dA, pkg.U8, 0.02, 128, w, np.float32(0.01), 0, ys, 120, pkg.U8, dY, m)  # noqa: E731
+    call()
+    ctx.flush()
+    ctx.capture_begin()
+    call()
+    graph = ctx.capture_end()
+    rt = pkg.runtime
+    now = {rt.SCALAR_A_ZERO_POINT: 128, rt.SCALAR_B_ZERO_POINT: 0, rt.SCALAR_Y_ZERO_POINT: 120}
+    for which, value in ((None, 0), (rt.SCALAR_A_ZERO_POINT, 90), (rt.SCALAR_B_ZERO_POINT, 3), (rt.SCALAR_Y_ZERO_POINT, 90), (rt.SCALAR_A_ZERO_POINT, 128), (rt.SCALAR_B_ZERO_POINT, 0)):
+        if which:
+            ctx.graph_set_scalar(graph, 0, which, value)
+            now[which] = value
+        ctx.fill(dY, 0, m * n // 4 * 4, 0)
+        ctx.graph_launch(graph)
+        want = oracle.qlinear_matmul(a, 0.02, now[rt.SCALAR_A_ZERO_POINT], b, np.float32(0.01), now[rt.SCALAR_B_ZERO_POINT], ys, now[rt.SCALAR_Y_ZERO_POINT], False)
+        assert np.array_equal(ctx.download(dY, np.uint8, (m, n)), want), (which, value)
+    ctx.graph_destroy(graph)
+    w.destroy()
+    dA.free(), dY.free()

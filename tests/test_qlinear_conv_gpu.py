@@ -350,3 +350,44 @@ def test_scales_with_the_same_quotients_keep_the_resident_ratios(ctx, pkg, oracl
     weight.destroy()
     for b in (dX, dY, dB):
         b.free()
+
+
+PATCHED = [  # convolutions whose recorded weight zero point, 0 of an int8 weight, may be changed: geometry, pads
+    (dict(c_in=24, c_out=24, t=11, kw=3, dil=1, n=2, h=13, kh=3, group=24), (1, 1, 1, 1)),            # depthwise
+    (dict(c_in=10, c_out=20, t=14, kw=7, dil=1, h=9, kh=5, stride=2, group=10), (5, 4, 5, 6)),
+    (dict(c_in=20, c_out=24, t=18, kw=2, dil=3, n=3, h=18, kh=3), (4, 1, 2, 5)),                      # channels off 16
+    (dict(c_in=3, c_out=40, t=57, kw=7, dil=1, n=14, h=61, kh=7, stride=2), (3, 3, 3, 3)),
+    (dict(c_in=16, c_out=130, t=18, kw=1, dil=1, n=130, h=18), (0, 0, 0, 0)),                         # many tiles
+    (dict(c_in=32, c_out=32, t=200, kw=3, dil=1, n=2, h=192, kh=3), (1, 1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("cfg,pads", PATCHED, ids=lambda v: str(v).replace(" ", ""))
+def test_a_recorded_weight_zero_point_of_zero_can_be_patched(ctx, pkg, oracle, cfg, pads):
+    X, W, _, bias, kw = _qconv_case(pkg, seed=180, **cfg)
+    kw["pads"] = pads
+    geom, og = pkg.ConvGeom.make(X.shape, W.shape, **kw), oracle.conv_geom(X.shape, W.shape, **kw)
+    weight = pkg.ops.ConvWeight(ctx, W, geom)
+    shape = pkg.ops.conv_out_shape(ctx, geom)
+    dX, dY, dB = ctx.upload(X), ctx.alloc(int(np.prod(shape))), ctx.upload(bias.astype(np.int32))
+    call = lambda: pkg.ops.qlinear_conv_device(ctx, dX, pkg.U8, 0.03, 100, weight, np.float32(0.004), 0, 0.3, 120, pkg.U8, dB, geom, dY)  # noqa: E731
+    call()
+    ctx.flush()
+    ctx.capture_begin()
+    call()
+    graph = ctx.capture_end()
+    rt = pkg.runtime
+    now = {rt.SCALAR_A_ZERO_POINT: 100, rt.SCALAR_B_ZERO_POINT: 0, rt.SCALAR_Y_ZERO_POINT: 120}
+    for which, value in ((None, 0), (rt.SCALAR_A_ZERO_POINT, 131), (rt.SCALAR_B_ZERO_POINT, -7), (rt.SCALAR_Y_ZERO_POINT, 90), (rt.SCALAR_B_ZERO_POINT, 5),
+                         (rt.SCALAR_A_ZERO_POINT, 128), (rt.SCALAR_B_ZERO_POINT, 0)):
+        if which:
+            ctx.graph_set_scalar(graph, 0, which, value)
+            now[which] = value
+        ctx.fill(dY, 0, int(np.prod(shape)) // 4 * 4, 0)
+        ctx.graph_launch(graph)
+        want = oracle.qlinear_conv(X, 0.03, now[rt.SCALAR_A_ZERO_POINT], W, np.float32(0.004), now[rt.SCALAR_B_ZERO_POINT], 0.3, now[rt.SCALAR_Y_ZERO_POINT], bias, og)
+        assert np.array_equal(ctx.download(dY, np.uint8, shape), want), (which, value)
+    ctx.graph_destroy(graph)
+    weight.destroy()
+    for b in (dX, dY, dB):
+        b.free()
