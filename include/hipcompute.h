@@ -182,7 +182,7 @@ int hipc_matmul_nbits(hipc_ctx *ctx, const void *A, int a_dtype, const void *B, 
  * interp.rs:2712-2768; the reference feeds MatMulNBits the ONNX layout directly).
  * The operands are device pointers in the ONNX layout above and may be released
  * after the next flush. A block_size that is not a power of two or below 16, and one of 16 with
- * K * N < 16384 or K no multiple of 8, has no tiled form:
+ * K * N < 16384, K no multiple of 8 or 4 GiB of nibbles and more, has no tiled form:
  * its handle holds copies of the tensors as they are and hipc_matmul_nbits_packed runs
  * the kernel of hipc_matmul_nbits on them (the same results, bit for bit). */
 int hipc_prepack_matmul_nbits(hipc_ctx *ctx, const void *B, size_t b_len, const void *scales,

@@ -1099,19 +1099,21 @@ int hipc_prepack_matmul_nbits(hipc_ctx *ctx, const void *B, size_t b_len, const 
 namespace {
 
 // Which weights the matrix-core kernels have a form for. Blocks of 16 take it from 16384 values on: one row
-// of a smaller weight is a launch and little else on either kernel, and the handle stays what the caller passed in.
+// of a smaller weight is a launch and little else on either kernel, and the handle stays what the caller passed in; and
+// below 4 GiB, which the kernels' 32-bit offsets reach (larger blocks have no other handle, and are refused there).
+constexpr size_t kTiledLimit = size_t(1) << 32;
+size_t tiled_wq_bytes(int64_t K, int64_t N) { return (size_t)ceil_div(N, 16) * (size_t)ceil_div(K, 128) * 1024; }
 bool has_tiled_form(int64_t K, int64_t N, int64_t block_size) {
-    return is_pow2(block_size) && (block_size >= 32 || (block_size == 16 && K % 8 == 0 && K * N >= 16384));
+    return is_pow2(block_size) && (block_size >= 32 || (block_size == 16 && K % 8 == 0 && K * N >= 16384 && tiled_wq_bytes(K, N) < kTiledLimit));
 }
 // tile counts and scale grouping of the tiled form of a weight (K, N, block_size set), and
 // the bytes of its three arrays
 void tiled_geometry(hipc_nbits_weight *w, size_t *wq_bytes, size_t *sc_bytes, size_t *zb_bytes) {
-    const int n_chunks = (int)ceil_div(w->K, 32);
     w->n_tiles = (int)ceil_div(w->N, 16);
-    w->n_cg = (int)ceil_div(n_chunks, 4);
+    w->n_cg = (int)ceil_div(w->K, 128);
     w->SG = w->block_size >= 128 ? 1 : (int)(128 / w->block_size);
     const size_t tiles = (size_t)w->n_tiles * w->n_cg;
-    *wq_bytes = tiles * 1024, *sc_bytes = tiles * 16 * w->SG * 4, *zb_bytes = tiles * 16 * w->SG;
+    *wq_bytes = tiled_wq_bytes(w->K, w->N), *sc_bytes = tiles * 16 * w->SG * 4, *zb_bytes = tiles * 16 * w->SG;
 }
 // the launch that writes the tiled form from the operator's tensors (device pointers)
 hipError_t tiled_fill(hipc_ctx *ctx, const hipc_nbits_weight *w, const void *B, const void *scales, int scale_dtype, const void *zp) {
@@ -1177,7 +1179,7 @@ int hipc::nbits_prepack(hipc_ctx *ctx, const void *B, size_t b_len, const void *
     w->interleave_half = interleave_half;
     size_t wq_bytes, sc_bytes, zb_bytes;
     tiled_geometry(w, &wq_bytes, &sc_bytes, &zb_bytes);
-    if (wq_bytes >= (size_t(1) << 32)) {
+    if (wq_bytes >= kTiledLimit) {
         delete w;
         return fail(ctx, HIPC_ERR_UNSUPPORTED, "MatMulNBits prepack: a %zu-byte weight exceeds the 4 GiB the kernel addresses", wq_bytes);
     }
@@ -1342,7 +1344,7 @@ int tiled_from_onnx_layout(hipc_ctx *ctx, const void *A, int a_dtype, const void
     w.K = K, w.N = N, w.block_size = block_size;
     size_t wq_bytes, sc_bytes, zb_bytes;
     tiled_geometry(&w, &wq_bytes, &sc_bytes, &zb_bytes);
-    if (wq_bytes >= (size_t(1) << 32)) return HIPC_OK;
+    if (wq_bytes >= kTiledLimit) return HIPC_OK;
     // only where a tiled kernel will take the rows (otherwise sixteen rows at a time on the decode kernel: no gain)
     const bool many = a_dtype == HIPC_F16 ? nbits_prefill_takes(A, &w, M) : nbits_prefill_f32_takes(A, &w, M);
     if (!many) return HIPC_OK;

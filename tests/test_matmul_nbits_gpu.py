@@ -689,3 +689,27 @@ def test_a_first_call_inside_a_capture(pkg, oracle, case, layout):
         c.graph_destroy(graph)
         if layout == "handle":
             w.destroy()
+
+
+def test_a_weight_in_blocks_of_sixteen_beyond_the_tiled_form(ctx, pkg):
+    """4 GiB of nibbles: more than the tiled form's 32-bit offsets reach, so the handle keeps the operator's layout. Codes
+    10 and 5 under zero point 8, scale 1, activations 1: each result is (2 - 3) K / 2."""
+    k, n, bs = 4096, 1 << 21, 16
+    blocks = k // bs
+    b_len = n * blocks * (bs // 2)
+    B, S = ctx.alloc(b_len), ctx.alloc(n * blocks * 4)
+    ctx.fill(B, 0, b_len, 0x5A5A5A5A)
+    ctx.fill(S, 0, n * blocks * 4, 0x3F800000)
+    import ctypes as C
+    h = C.c_void_p()
+    ctx._check(ctx.lib.hipc_prepack_matmul_nbits(ctx.handle, B.ptr, b_len, S.ptr, pkg.F32, n * blocks, None, 0, k, n, bs, C.byref(h)))
+    B.free(), S.free()
+    assert ctx.lib.hipc_nbits_weight_bytes(h) == b_len + n * blocks * 4
+    dA = ctx.upload(np.ones(k, np.float32))
+    dY = ctx.alloc(n * 4)
+    ctx._check(ctx.lib.hipc_matmul_nbits_packed(ctx.handle, dA.ptr, pkg.F32, h, dY.ptr, 1, 0))
+    got = ctx.download(dY, np.float32, (n,))
+    ctx.lib.hipc_nbits_weight_destroy(ctx.handle, h)
+    dA.free(), dY.free()
+    ctx.flush()
+    assert np.all(got == -k / 2)
