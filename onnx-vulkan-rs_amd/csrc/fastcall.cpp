@@ -13,6 +13,7 @@
 #include <cstring>
 #include <new>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 
 #include "../../include/hipcompute.h"
@@ -31,7 +32,7 @@ struct Views {
 };
 
 bool to_integer(PyObject *o, long long *out) {
-    if (!PyLong_CheckExact(o)) {
+    if (!PyLong_Check(o)) {
         if (!PyIndex_Check(o)) return false;   // a NumPy integer
         PyObject *i = PyNumber_Index(o);
         if (!i) {
@@ -87,8 +88,13 @@ struct Arg<T *> {
         const bool holder = Py_TYPE(o) == g_c_void_p;
         if (views.n >= 8 || !(holder || PyObject_TypeCheck(o, g_ndarray) || PyObject_TypeCheck(o, g_structure))) return false;
         Py_buffer *b = &views.held[views.n];
-        if (PyObject_GetBuffer(o, b, PyBUF_SIMPLE) != 0) {
+        constexpr bool floats = std::is_same_v<T, const float>;   // (an array behind a typed pointer has to hold that type)
+        if (PyObject_GetBuffer(o, b, floats ? PyBUF_SIMPLE | PyBUF_FORMAT : PyBUF_SIMPLE) != 0) {
             PyErr_Clear();
+            return false;
+        }
+        if (floats && !holder && !(b->format && strcmp(b->format, "f") == 0)) {
+            PyBuffer_Release(b);
             return false;
         }
         if (holder) {   // the pointer it holds, not where it is held

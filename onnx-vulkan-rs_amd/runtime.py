@@ -9,6 +9,8 @@ import contextlib
 import ctypes as C
 import importlib.util
 import os
+import sysconfig
+import warnings
 
 import numpy as np
 
@@ -64,6 +66,19 @@ class InitializerInfo(C.Structure):
 
 _lib = None
 
+class _FloatArray:
+    """``const float *``: a contiguous float32 NumPy array, as the native entry points take it, or what ctypes takes for one."""
+    _pointer = C.POINTER(C.c_float)
+
+    @classmethod
+    def from_param(cls, value):
+        if isinstance(value, np.ndarray):
+            if value.dtype != np.float32 or not value.flags.c_contiguous:
+                raise TypeError("a contiguous float32 array")
+            return value.ctypes.data_as(cls._pointer)
+        return cls._pointer.from_param(value)
+
+
 # name -> (restype, argtypes); every symbol include/hipcompute.h declares
 _vp, _i64, _sz, _int, _f = C.c_void_p, C.c_int64, C.c_size_t, C.c_int, C.c_float
 SIGNATURES = {
@@ -111,14 +126,14 @@ SIGNATURES = {
     "hipc_matmul_integer_scale_bias": (_int, [_vp, _vp, _int, _vp, _vp, _vp, _vp, _int, _vp, _int, _vp, _int,
                                               _int, _vp, _vp, _i64]),
     "hipc_requantize": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, C.c_int32, _int, _vp]),
-    "hipc_qlinear_matmul": (_int, [_vp, _vp, _int, _f, C.c_int32, _vp, C.POINTER(_f), _i64, C.c_int32, _f,
+    "hipc_qlinear_matmul": (_int, [_vp, _vp, _int, _f, C.c_int32, _vp, _FloatArray, _i64, C.c_int32, _f,
                                    C.c_int32, _int, _vp, _i64]),
     "hipc_conv_out_shape": (_int, [C.POINTER(ConvGeom), C.POINTER(_i64), C.POINTER(_i64)]),
     "hipc_same_pads": (None, [_i64, _i64, _i64, _i64, _int, C.POINTER(_i64), C.POINTER(_i64)]),
     "hipc_prepack_conv_w": (_int, [_vp, _vp, _int, C.POINTER(ConvGeom), C.POINTER(_vp)]),
     "hipc_conv_weight_destroy": (None, [_vp, _vp]),
     "hipc_conv_integer": (_int, [_vp, _vp, _int, _vp, _vp, _vp, C.POINTER(ConvGeom), _vp]),
-    "hipc_qlinear_conv": (_int, [_vp, _vp, _int, _f, C.c_int32, _vp, C.POINTER(_f), _i64, C.c_int32, _f,
+    "hipc_qlinear_conv": (_int, [_vp, _vp, _int, _f, C.c_int32, _vp, _FloatArray, _i64, C.c_int32, _f,
                                  C.c_int32, _int, _vp, C.POINTER(ConvGeom), _vp]),
     "hipc_decoder_create": (_int, [_vp, C.POINTER(DecoderConfig), C.POINTER(_vp)]),
     "hipc_decoder_destroy": (None, [_vp, _vp]),
@@ -175,15 +190,23 @@ def load_library():
     return _lib
 
 
+def fast_path() -> str:
+    """The module with the native entry points for THIS interpreter (its file name carries the ABI)."""
+    return os.path.join(_HERE, "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
 def _bind_fast(lib, build_id: str):
     """Puts the native entry points (csrc/fastcall.cpp) in the place of the ctypes functions that only enqueue. The
-    module belongs to this build of the library, like the library to the sources."""
-    path = os.path.join(_HERE, "_fastcall.so")
-    if not os.path.exists(path):
-        raise HipComputeError(3, f"{path} is missing: build it with __graft_entry__.build() (make -C onnx-vulkan-rs_amd/csrc)")
-    spec = importlib.util.spec_from_file_location("onnx_vulkan_rs_amd._fastcall", path)
-    fast = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(fast)
+    module belongs to this build of the library, like the library to the sources. Without one for this interpreter the
+    ctypes functions stay: the same calls, a microsecond or two slower each."""
+    path = fast_path()
+    try:
+        spec = importlib.util.spec_from_file_location("onnx_vulkan_rs_amd._fastcall", path)
+        fast = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(fast)
+    except (ImportError, OSError) as e:
+        warnings.warn(f"{path} cannot be loaded ({e}): calls go through ctypes (make -C onnx-vulkan-rs_amd/csrc builds it)", RuntimeWarning, stacklevel=3)
+        return
     if fast.build_id != build_id:
         raise HipComputeError(3, f"{path} is stale: built with id {fast.build_id}, the library has {build_id}; rebuild both")
     for name in SIGNATURES:

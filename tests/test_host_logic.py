@@ -217,3 +217,40 @@ def test_kernel_addresses_on_the_cpu_model(tmp_path):
     # f16 and f32 rows, on ragged shapes with operands of exactly the operator's size
     run = subprocess.run([os.path.join(out, "prefill_model")], capture_output=True, text=True, env=env)
     assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout[-2000:] + run.stderr[-2000:]
+
+
+def _ctypes_only(monkeypatch, runtime, tmp_path):
+    """The library as an interpreter without a native module of its own sees it."""
+    monkeypatch.setattr(runtime, "_lib", None)
+    monkeypatch.setattr(runtime, "fast_path", lambda: str(tmp_path / "_fastcall.so"))
+    with pytest.warns(RuntimeWarning, match="calls go through ctypes"):
+        return runtime.load_library()
+
+
+def test_the_library_loads_without_the_native_entry_points(pkg, monkeypatch, tmp_path):
+    """Nothing but speed hangs on the module that spares ctypes: without one every call takes the arguments the wrappers
+    pass, a weight's scales as an array among them, and so does a call the module hands on because it cannot convert one."""
+    runtime = pkg.runtime
+    fast = pkg.load_library()
+    lib = _ctypes_only(monkeypatch, runtime, tmp_path)
+    assert isinstance(lib.hipc_qlinear_matmul, C._CFuncPtr) and not isinstance(fast.hipc_qlinear_matmul, C._CFuncPtr)
+    ws = np.ones(3, np.float32)
+    geom = pkg.ConvGeom.make((1, 16, 1, 8), (3, 16, 1, 1))
+    for library, g in ((lib, geom), (fast, geom), (fast, C.pointer(geom))):     # (a pointer object is ctypes' to convert)
+        # a null context: refused by the library, not by a conversion
+        assert library.hipc_qlinear_matmul(None, None, pkg.U8, 0.1, 0, None, ws, ws.size, 0, 0.1, 0, pkg.U8, None, 1) == 1
+        assert library.hipc_qlinear_conv(None, None, pkg.U8, 0.1, 0, None, ws, ws.size, 0, 0.1, 0, pkg.U8, None, g, None) == 1
+        with pytest.raises(C.ArgumentError):
+            library.hipc_qlinear_matmul(None, None, pkg.U8, 0.1, 0, None, ws.astype(np.float64), ws.size, 0, 0.1, 0, pkg.U8, None, 1)
+
+
+def test_the_native_entry_points_are_built_for_this_interpreter(pkg):
+    """The file name carries the interpreter's ABI, and every target that builds a library builds it."""
+    import subprocess
+    import sysconfig
+    path = pkg.runtime.fast_path()
+    assert path.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and os.path.exists(path)
+    csrc = os.path.join(ROOT, "onnx-vulkan-rs_amd", "csrc")
+    for target in ("all", "stamps"):
+        plan = subprocess.run(["make", "-n", "-B", "-C", csrc, target], capture_output=True, text=True, check=True).stdout
+        assert os.path.basename(path) in plan, target

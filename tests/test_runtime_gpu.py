@@ -217,3 +217,26 @@ def test_scalars_of_a_recorded_graph_can_be_patched(ctx, pkg, oracle):
     w.destroy(), cw.destroy()
     for buf in (dA, dY, dX, dC, dS, dZ, dF):
         buf.free()
+
+
+def test_quantized_operators_without_the_native_entry_points(pkg, oracle, monkeypatch, tmp_path):
+    """An interpreter without a module of its own calls through ctypes: the same operators, the same results."""
+    rt = pkg.runtime
+    monkeypatch.setattr(rt, "_lib", None)
+    monkeypatch.setattr(rt, "fast_path", lambda: str(tmp_path / "_fastcall.so"))
+    with pytest.warns(RuntimeWarning, match="calls go through ctypes"):
+        c = pkg.Context(0)
+    with c:
+        a = pkg.synth.uniform_ints(20 * 64, 1, 0, 255).astype(np.uint8).reshape(20, 64)
+        b = pkg.synth.int8_weight(64, 48, 2)
+        w = pkg.ops.Int8Weight(c, b)
+        dA, dY = c.upload(a), c.alloc(20 * 48)
+        scale = pkg.synth.uniform_f32(48, 3, 0.005, 0.02)
+        pkg.ops.qlinear_matmul_device(c, dA, pkg.U8, 0.02, 128, w, scale, 0, 0.4, 100, pkg.U8, dY, 20)
+        assert np.array_equal(c.download(dY, np.uint8, (20, 48)), oracle.qlinear_matmul(a, 0.02, 128, b, scale, 0, 0.4, 100, False))
+        w.destroy()
+        X = pkg.synth.uniform_ints(16 * 40, 4, 0, 255).astype(np.uint8).reshape(1, 16, 1, 40)
+        W = pkg.synth.uniform_ints(8 * 16 * 3, 5, -127, 127).astype(np.int8).reshape(8, 16, 1, 3)
+        geom, og = pkg.ConvGeom.make(X.shape, W.shape, pads=(0, 1, 0, 1)), oracle.conv_geom(X.shape, W.shape, pads=(0, 1, 0, 1))
+        got = pkg.ops.qlinear_conv(c, X, 0.02, 128, W, scale[:8], 0, 0.3, 120, None, geom)
+        assert np.array_equal(got, oracle.qlinear_conv(X, 0.02, 128, W, scale[:8], 0, 0.3, 120, None, og))
