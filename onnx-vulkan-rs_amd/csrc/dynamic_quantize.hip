@@ -177,15 +177,15 @@ __device__ __forceinline__ void dql_params(const uint32_t *range, float &scale, 
 }
 
 // The codes of four values: sat(rte(v / scale) + zp), packed. `rcp` is 1 / scale where div_by may be used -- a scale within
-// 2^-100 .. 2^100, so that |v| <= 255 scale and the remainders of every quotient that does not round to 0 stay in range --
-// and 0 where it may not.
+// 2^-100 .. 2^100, so that the remainders of every quotient that does not round to 0 stay in range -- and 0 where it may not.
+// Values beyond 1024 scale, which only a caller's own range lets through, saturate like that one (NaN becomes code 0 either way).
 template <bool FAST>
 __device__ __forceinline__ uint32_t dql_four_by(float4 v, float scale, float rcp, float zp) {
     const float in[4] = {v.x, v.y, v.z, v.w};
     uint32_t w = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const float q = FAST ? div_by(in[j], scale, rcp) : __fdiv_rn(in[j], scale);
+        const float q = FAST ? div_by(__builtin_amdgcn_fmed3f(in[j], -1024.f * scale, 1024.f * scale), scale, rcp) : __fdiv_rn(in[j], scale);
         w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(__fadd_rn(rintf(q), zp), 0.f, 255.f), j, w);
     }
     return w;

@@ -160,3 +160,22 @@ def test_scales_at_the_ends_of_the_float_range(ctx, pkg, oracle, scale):
     y, s, z = pkg.ops.dynamic_quantize_linear(ctx, x)
     wy, ws, wz = oracle.dynamic_quantize_linear(x)
     assert np.array_equal(y, wy) and np.float32(s) == np.float32(ws) and z == wz
+
+
+@pytest.mark.parametrize("n", [5000, 262144 * 4 + 5])
+def test_values_outside_a_callers_range_saturate(ctx, pkg, n):
+    """A range slot that does not cover the values: each takes the code its quotient saturates to, also where that
+    quotient is beyond the float range, and NaN the code 0."""
+    x = pkg.synth.normal_f32(n, 93)
+    x[:9] = [np.inf, -np.inf, 3e38, -3e38, 1e37, 2.0, -2.0, 1e-30, np.nan]
+    rng = np.array([np.float32(1.0).view(np.uint32), np.float32(0.5).view(np.uint32)], np.uint32)
+    dX, dR = ctx.upload(x), ctx.upload(rng)
+    dY, dP = ctx.alloc(n), ctx.alloc(8)
+    pkg.ops.dynamic_quantize_linear_device(ctx, dX, n, dY, dP, dP.at(4), range_slot=dR, range_ready=True)
+    scale = np.float32(1.5) / np.float32(255)
+    zp = np.rint(np.float32(1.0) / scale)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = np.where(np.isnan(x), 0, np.clip(np.rint(x / scale) + zp, 0, 255)).astype(np.uint8)
+    assert np.array_equal(ctx.download(dY, np.uint8, (n,)), want)
+    for b in (dX, dR, dY, dP):
+        b.free()
