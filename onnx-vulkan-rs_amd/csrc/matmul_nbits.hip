@@ -1259,8 +1259,8 @@ int launch_plain16(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, voi
 // Blocks of 16: up to 16 rows, and more where it is the better kernel, on the one for a few rows, the others on the tiled
 // kernel. Nothing here accumulates less than the kernel of the operator's layout, which computes in f32: an f32 value keeps all
 // 24 bits (three f16 terms; down to 2^-30 of its row's largest, see split_terms) unless accuracy_level allows less. That kernel, which unpacks the weight and multiplies it
-// with vector instructions once per four rows, took -> this: f32 1 x 6912 x 1152 28.0 -> 8.6 us, 8 rows 145 -> 7.9, 60 x 1152 x
-// 13824 1641 -> 30; f16 20 x 2048 x 11008 384 -> 9.9, 100 rows 1881 -> 22.7; 200 x 256 x 256 27.8 -> 9.5.
+// with vector instructions once per four rows, took -> this: f32 1 x 6912 x 1152 28.0 -> 10.5 us, 8 rows 145 -> 8.6, 60 x 1152 x
+// 13824 1641 -> 30; f16 20 x 2048 x 11008 384 -> 10.9, 100 rows 1881 -> 23.2; f32 200 x 256 x 256 27.8 -> 9.8.
 int packed_run16(hipc_ctx *ctx, const void *A, int a_dtype, const hipc_nbits_weight *w, void *Y, int64_t M, int accuracy_level) {
     const bool f16 = a_dtype == HIPC_F16;
     const size_t esz = f16 ? 2 : 4;

@@ -601,8 +601,8 @@ int nbits_rows_f16(hipc_ctx *ctx, const void *A, int terms, const int *exps, con
 #else
 
 // Which row counts come here (kernel time of the call, before -> after; the streaming kernel 16 rows at a time, the tiled
-// kernel from 17 rows of f16 and 33 of f32 on): 8 x 1152 x 13824 11.5 -> 7.4 us, 16 rows 23 -> 9.8, 32 rows 46 -> 21; 8 x 6912
-// x 1152 10.4 -> 8.6, 16 rows 19 -> 10.2; f16 2048 -> 11008: 1 row 7.3 -> 6.5, 4 rows 11.2 -> 6.5, 16 rows 24 -> 7.8, 17 rows
+// kernel from 17 rows of f16 and 33 of f32 on): 8 x 1152 x 13824 11.5 -> 7.5 us, 16 rows 23 -> 9.4, 32 rows 46 -> 19; 8 x 6912
+// x 1152 10.4 -> 7.1, 16 rows 19 -> 8.2; f16 2048 -> 11008: 1 row 7.3 -> 6.5, 4 rows 11.2 -> 6.5, 16 rows 24 -> 7.8, 17 rows
 // 11.3 -> 8.6; 24 x 512 -> 1152 5.4 -> 4.5, but -> 16384 5.5 -> 5.9. From 33 rows on only where the tiled kernel has few tiles: f16 48 x 6912 x 1152 27.4 -> 11.6, but 48 x 4096 x
 // 4096 18.1 -> 21.4; f32 (which the tiled kernel takes 64 rows at a time) 48 x 6912 x 1152 41 -> 22.7, 48 x 4096 x 4096 39 ->
 // 25, but 64 x 2048 x 8192 32.6 -> 37. A weight of 2048 column tiles or more and up to 16 rows stay on the streaming kernel,
