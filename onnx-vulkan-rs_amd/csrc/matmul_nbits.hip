@@ -1349,7 +1349,9 @@ int tiled_from_onnx_layout(hipc_ctx *ctx, const void *A, int a_dtype, const void
     const bool many = a_dtype == HIPC_F16 ? nbits_prefill_takes(A, &w, M) : nbits_prefill_f32_takes(A, &w, M);
     if (!many) return HIPC_OK;
     const size_t wq_r = (wq_bytes + 255) & ~(size_t)255, sc_r = (sc_bytes + 255) & ~(size_t)255;
-    if (!scratch_fits(ctx, 4, wq_r + sc_r + zb_bytes)) return HIPC_OK;
+    // (a first call inside a capture: blocks of 16 stay on the kernel of the operator's layout, larger ones are refused -- that
+    // kernel reads the whole weight once per four rows, and a graph would keep doing so)
+    if (block_size == 16 && !scratch_fits(ctx, 4, wq_r + sc_r + zb_bytes)) return HIPC_OK;
     *taken = true;
     void *block = nullptr;
     if (int rc = scratch_get(ctx, 4, wq_r + sc_r + zb_bytes, &block)) return rc;
