@@ -382,11 +382,11 @@ def bench_decoder(pkg, ctx, steps, warmup, context=2048):
     tok_s = steps / dt
     out = dict(tok_s=tok_s, ms_per_token=dt / steps * 1e3, context=context, bytes_per_token=byts,
                hbm_bound_tok_s=HBM_PEAK_GBS * 1e9 / byts, frac_of_hbm_bound=tok_s * byts / (HBM_PEAK_GBS * 1e9),
-               # five launches per layer, then the unembedding (whose workgroups leave the argmax candidates) and the
+               # all layers, the unembedding (whose workgroups leave the argmax candidates) and the
                # launch that picks the token and embeds it for the next step
-               launches_per_token=5 * cfg["n_layers"] + 2, final_position=pos)
-    # the same step without the read-ahead helper rows (by default three of a layer's five launches carry extra
-    # workgroups that read what the next launch will read into the L2 of the XCD that will ask for it), and with all five
+               launches_per_token=3, final_position=pos)
+    # the same step as five launches per layer, without read-ahead helper rows and with all five launches carrying them
+    # (extra workgroups that read what the next launch will read into the L2 of the XCD that will ask for it)
     for name, mask in (("no_read_ahead", 0), ("read_ahead_all_five", 31)):
         try:
             with ctx.options(HIPC_DEC_PREFETCH=mask):
@@ -440,12 +440,13 @@ def bench_phases(pkg, ctx, context=2048):
     filler = (rng.standard_normal((cfg["n_kv_heads"], context, cfg["head_dim"])) * 0.5).astype(np.float16)
     for li in range(cfg["n_layers"]):
         dec.fill_cache(li, filler, filler)
-    dec.reset(1234, context - 1)
-    dec.step()
-    ctx.flush()
-    ctx.capture_begin()
-    dec.step()
-    g = ctx.capture_end()
+    with ctx.options(HIPC_DEC_RESIDENT=0):   # a launch per product, which is what is looked into here
+        dec.reset(1234, context - 1)
+        dec.step()
+        ctx.flush()
+        ctx.capture_begin()
+        dec.step()
+        g = ctx.capture_end()
     for _ in range(20):
         ctx.graph_launch(g)
     ctx.flush()

@@ -114,6 +114,7 @@ const OptionName kOptions[] = {
     {"HIPC_DEC_FUSED_ARGMAX", &Tuning::dec_fused_argmax},
     {"HIPC_GEMV_LEAN", &Tuning::gemv_lean},
     {"HIPC_DEC_LEAN", &Tuning::dec_lean},
+    {"HIPC_DEC_RESIDENT", &Tuning::dec_resident},
     {"HIPC_DEC_PREFETCH", &Tuning::dec_prefetch},
 };
 

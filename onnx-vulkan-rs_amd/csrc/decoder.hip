@@ -18,6 +18,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -25,6 +26,7 @@
 #include "internal.h"
 #include "lanes.h"
 #include "prefetch.h"
+#include "resident.h"
 
 namespace hipc {
 
@@ -34,6 +36,7 @@ struct DecState {      // device-resident loop state
     int32_t token;     // the token the next step consumes
     int32_t pos;       // its position = number of tokens already in the cache
     int32_t overflow;  // sticky: a step was asked for with the cache full (pos == max_seq); that step did nothing
+    int32_t broken;    // sticky: a wait inside the resident kernel ran out
 };
 
 __device__ __forceinline__ float block_sum(float v, float *red) {
@@ -741,7 +744,7 @@ dec_argmax_partial_kernel(const float *__restrict__ logits, int n, float *__rest
 // position): a step begins with its q|k|v product, not with a launch of its own for the embedding.
 __global__ void __launch_bounds__(256)
 dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, int nparts, DecState *st,
-                      int32_t *__restrict__ history, int max_hist, int vocab, const EmbedArgs e) {
+                      int32_t *__restrict__ history, int max_hist, int vocab, uint32_t *__restrict__ launch, const EmbedArgs e) {
     __shared__ float red[4];
     __shared__ int next[2];
     // the upper two wavefronts work out the next position's rotary table (it follows from the position alone) while
@@ -776,6 +779,7 @@ dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, 
             } else {
                 if (bi < 0 || bi >= vocab) bi = 0;
                 history[pos] = bi;
+                if (launch) *launch = *launch + 1 == kResLaunches ? 0u : *launch + 1;   // the resident kernel's launch of this step has been
                 st->token = token = bi;
                 st->pos = new_pos = pos + 1;
             }
@@ -786,8 +790,15 @@ dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, 
     dec_embed_token<false>(e, next[0], next[1], red);
 }
 
-__global__ void dec_set_state_kernel(DecState *st, int token, int pos) {
-    if (threadIdx.x == 0) st->token = token, st->pos = pos, st->overflow = 0;
+// (after a resident launch that did not come to its end, its words are made what a new decoder's are)
+__global__ void __launch_bounds__(256) dec_set_state_kernel(DecState *st, int token, int pos, uint32_t *xch, uint32_t *sync) {
+    const bool broken = xch && st->broken;
+    __syncthreads();
+    if (threadIdx.x == 0) st->token = token, st->pos = pos, st->overflow = 0, st->broken = 0;
+    if (broken) {
+        for (uint32_t i = threadIdx.x; i < kResSets * kResWords; i += 256) xch[i] = 0xffffffffu;
+        for (uint32_t i = threadIdx.x; i < kResSyncWords; i += 256) sync[i] = i == 0 ? 1u : 0u;
+    }
 }
 
 }  // namespace hipc
@@ -836,6 +847,12 @@ struct hipc_decoder {
     // x, xn and the rotary table hold the state's token and position (left by the reset or by the step before);
     // anything that changes what they are made of clears it, and a step that finds it cleared embeds first
     bool x_ready = false;
+    // All layers in one launch (decode_resident.hip), where the shape allows it
+    bool resident = false;
+    ResidentLayer *table = nullptr;             // the layers as that kernel reads them
+    std::vector<ResidentLayer> entries;         // what the table holds, or will once `stale` entries are written
+    std::vector<char> stale;
+    uint32_t *xch = nullptr, *sync = nullptr;
     bool one_launch_attn = false;  // head_dim and group size have an instance of dec_attn_chunks_kernel
     std::vector<void *> owned;
 };
@@ -878,6 +895,32 @@ int launch_attn_chunks(hipc_ctx *ctx, hipc_decoder *d, DecLayer &l, float scale,
     }
     HIPC_LAUNCHED(ctx);
     return HIPC_OK;
+}
+
+// Layer li of the resident kernel's table follows what has been set. A recorded step keeps the weights it was recorded
+// with: while graphs exist the change goes into a table of its own.
+int update_entry(hipc_ctx *ctx, hipc_decoder *d, int li) {
+    if (!d->resident) return HIPC_OK;
+    const DecLayer &l = d->layers[li];
+    ResidentLayer e{};
+    const hipc_nbits_weight *w[4] = {l.qkv, l.o, l.gate_up, l.down};
+    for (int i = 0; i < 4; i++)
+        if (w[i]) e.wq[i] = w[i]->Wq, e.sc[i] = w[i]->Sc, e.zb[i] = w[i]->Zb;
+    for (int i = 0; i < 6; i++) e.norm[i] = l.norm[i];
+    e.k_cache = l.k_cache, e.v_cache = l.v_cache, e.window = l.window, e.rope_table = l.rope_table;
+    if (memcmp(&e, &d->entries[li], sizeof e) == 0 && !d->stale[li]) return HIPC_OK;
+    if (ctx->live_graphs > 0 && !ctx->capturing) {
+        ResidentLayer *fresh = nullptr;
+        int rc = dev_alloc(ctx, d, &fresh, d->entries.size());
+        if (rc != HIPC_OK) return rc;
+        HIPC_TRY(ctx, hipMemcpyAsync(fresh, d->table, d->entries.size() * sizeof(ResidentLayer), hipMemcpyDeviceToDevice, ctx->stream));
+        d->table = fresh;
+    }
+    d->entries[li] = e, d->stale[li] = 1;
+    if (ctx->capturing) return HIPC_OK;   // (the next step writes it)
+    int rc = resident_set_layer(ctx, d->table + li, e);
+    if (rc == HIPC_OK) d->stale[li] = 0;
+    return rc;
 }
 
 bool complete(const hipc_decoder *d) {
@@ -970,13 +1013,19 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
                     rc = fail(ctx, HIPC_ERR_BACKEND, "decoder: cannot clear the gated row and the attention partials");
             }
         }
+        d->resident = d->lean && resident_takes(c) && ctx->tune.dec_resident != 0;
+        if (d->resident) {
+            d->entries.resize(c.n_layers), d->stale.assign(c.n_layers, 1);
+            A(&d->table, c.n_layers), A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSyncWords);
+            if (rc == HIPC_OK) rc = resident_clear(ctx, d->xch, d->sync);
+        }
         if (rc == HIPC_OK) {
             for (DecLayer &l : d->layers) {  // an unwritten cache row must not hold NaN bit patterns
                 if (hipMemsetAsync(l.k_cache, 0, k_halfs * 2, ctx->stream) != hipSuccess ||
                     hipMemsetAsync(l.v_cache, 0, v_halfs * 2, ctx->stream) != hipSuccess)
                     rc = fail(ctx, HIPC_ERR_BACKEND, "decoder: cannot clear the KV cache");
             }
-            hipLaunchKernelGGL((dec_set_state_kernel), 1, 64, 0, ctx->stream, d->state, 0, 0);
+            hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, 0, 0, nullptr, nullptr);
         }
         if (rc != HIPC_OK) {
             for (void *p : d->owned) (void)hipFree(p);
@@ -1027,7 +1076,9 @@ int hipc_decoder_set_linear(hipc_ctx *ctx, hipc_decoder *d, int layer, int which
             *slot = nullptr;
         }
         const int half = (d->lean && which == HIPC_DEC_GATE_UP) ? c.ffn : 0;
-        return nbits_prepack(ctx, B, b_len, scales, HIPC_F32, scales_len, zp, zp_len, K, N, c.block_size, slot, half);
+        int rc = nbits_prepack(ctx, B, b_len, scales, HIPC_F32, scales_len, zp, zp_len, K, N, c.block_size, slot, half);
+        if (rc == HIPC_OK && which != HIPC_DEC_LM_HEAD) rc = update_entry(ctx, d, layer);
+        return rc;
     });
 }
 
@@ -1051,7 +1102,7 @@ int hipc_decoder_set_norm(hipc_ctx *ctx, hipc_decoder *d, int layer, int which, 
         }
         HIPC_TRY(ctx, hipMemcpyAsync(*slot, w, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
         d->x_ready = false;
-        return HIPC_OK;
+        return which == HIPC_DEC_NORM_FINAL ? HIPC_OK : update_entry(ctx, d, layer);
     });
 }
 
@@ -1094,7 +1145,7 @@ int hipc_decoder_set_layer_attention(hipc_ctx *ctx, hipc_decoder *d, int layer, 
         l.window = window > 0 ? window : 0;
         l.rope_table = table;
         d->x_ready = false;   // the rotary table may need its second half
-        return HIPC_OK;
+        return update_entry(ctx, d, layer);
     });
 }
 
@@ -1118,7 +1169,7 @@ int hipc_decoder_reset(hipc_ctx *ctx, hipc_decoder *d, int32_t token, int32_t po
     if (!d) return HIPC_ERR_INVALID;
     return entry(ctx, [&]() -> int {
         HIPC_REQUIRE(ctx, token >= 0 && token < d->cfg.vocab && pos >= 0 && pos < d->cfg.max_seq, "decoder: bad token %d or position %d", token, pos);
-        hipLaunchKernelGGL((dec_set_state_kernel), 1, 64, 0, ctx->stream, d->state, token, pos);
+        hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, token, pos, d->xch, d->sync);
         HIPC_LAUNCHED(ctx);
         // the step expects the token embedded (x, xn, the position's rotary table): every step leaves that behind for
         // the next one, the reset does it for the first
@@ -1173,7 +1224,22 @@ int hipc_decoder_step(hipc_ctx *ctx, hipc_decoder *d) {
             const int64_t want = std::min<int64_t>(512, std::max<int64_t>(192, consumers));
             return (int)std::max<int64_t>(1, std::min<int64_t>(32, (want + gx - 1) / gx));
         };
-        for (int li = 0; li < c.n_layers && d->lean; li++) {
+        // All layers in one launch. (Asked for read-ahead by name, the launches that can carry it run instead.)
+        const bool resident = d->resident && ctx->tune.dec_resident != 0 && ctx->tune.dec_prefetch < 0;
+        if (resident) {
+            for (int li = 0; li < c.n_layers; li++) {
+                if (!d->stale[li]) continue;
+                if ((rc = resident_set_layer(ctx, d->table + li, d->entries[li])) != HIPC_OK) return rc;
+                if (!ctx->capturing) d->stale[li] = 0;
+            }
+            ResidentArgs a{};
+            a.table = d->table, a.pos = &d->state->pos, a.broken = &d->state->broken, a.rope = d->rope;
+            a.x_in = xc, a.x_out = xo, a.y_out = d->yd, a.xch = d->xch, a.sync = d->sync;
+            const int groups = ctx->tune.dec_resident > 0 ? std::min<int>(ctx->tune.dec_resident, kResGroups) : std::min<int>(ctx->cu_count, kResGroups);
+            if ((rc = resident_launch(ctx, c, a, groups)) != HIPC_OK) return rc;
+            std::swap(xc, xo);
+        }
+        for (int li = 0; li < c.n_layers && d->lean && !resident; li++) {
             DecLayer &l = d->layers[li];
             LeanPlan pl_qkv, pl_o, pl_gu, pl_down, pl_next;
             HIPC_REQUIRE(ctx, lean_plan(ctx, l.qkv, 1, 1, &pl_qkv, 8), "decoder: no launch plan for the qkv projection");
@@ -1300,7 +1366,7 @@ int hipc_decoder_step(hipc_ctx *ctx, hipc_decoder *d) {
             // the unembedding's prologue adds the last branch to the stream and applies the final norm (every workgroup
             // for itself, while its first weight tiles are on their way)
             GemvPrologue pro;
-            pro.mode = 2, pro.x = xc, pro.y = d->lean ? d->yd : d->y, pro.y_slices = d->lean ? d->down_slices : 1;
+            pro.mode = 2, pro.x = xc, pro.y = d->lean ? d->yd : d->y, pro.y_slices = d->lean && !resident ? d->down_slices : 1;
             pro.w_post = d->layers[c.n_layers - 1].norm[HIPC_DEC_NORM_POST_FFN], pro.w_in = d->final_norm, pro.eps = c.rms_eps;
             if ((rc = nbits_gemv(ctx, xc, HIPC_F32, d->lm_head, d->logits, 1, terms, &pro, &am)) != HIPC_OK) return rc;
         } else {
@@ -1314,7 +1380,7 @@ int hipc_decoder_step(hipc_ctx *ctx, hipc_decoder *d) {
             hipLaunchKernelGGL((dec_argmax_partial_kernel), kArgmaxParts, 256, 0, s, d->logits, c.vocab, d->am_v, d->am_i);
             HIPC_LAUNCHED(ctx);
         }
-        hipLaunchKernelGGL((dec_pick_embed_kernel), 1, 256, 0, s, d->am_v, d->am_i, parts, d->state, d->history, c.max_seq, c.vocab, embed_args(d));
+        hipLaunchKernelGGL((dec_pick_embed_kernel), 1, 256, 0, s, d->am_v, d->am_i, parts, d->state, d->history, c.max_seq, c.vocab, resident ? d->sync : nullptr, embed_args(d));
         HIPC_LAUNCHED(ctx);
         if (!ctx->capturing) d->x_ready = true;
         return HIPC_OK;
@@ -1333,6 +1399,7 @@ int hipc_decoder_read(hipc_ctx *ctx, hipc_decoder *d, int32_t *token, int32_t *p
         if (logits) HIPC_TRY(ctx, hipMemcpy(logits, d->logits, (size_t)d->cfg.vocab * 4, hipMemcpyDeviceToHost));
         if (history && n_history > 0)
             HIPC_TRY(ctx, hipMemcpy(history, d->history, (size_t)std::min<int32_t>(n_history, d->cfg.max_seq) * 4, hipMemcpyDeviceToHost));
+        if (st.broken) return fail(ctx, HIPC_ERR_BACKEND, "decoder: a step did not come to its end (a wait inside it ran out); reset the decoder");
         HIPC_REQUIRE(ctx, !st.overflow, "decoder: a step was enqueued with the cache full (%d positions); it did nothing", d->cfg.max_seq);
         return HIPC_OK;
     });

@@ -24,6 +24,7 @@
 // loads) can compile them: HIPC_HOST_MODEL is defined there and nowhere else.
 #ifndef HIPC_HOST_MODEL
 #define HIPC_PIN_VGPR(v) asm volatile("" : "+v"(v))                                              // the value is needed here, in a vector register
+#define HIPC_PIN_SGPR(v) asm volatile("" : "+s"(v))                                              // ... in a scalar one
 #define HIPC_VGPR_FROM_SGPR(dst, src) asm volatile("v_mov_b32 %0, %1" : "=v"(dst) : "s"(src))   // a uniform value kept in a vector register
 #define HIPC_ARG_NOW(v) asm volatile("" ::"s"(v))                                                // the kernel argument is read here
 // A load whose value may go unused on some paths (it is masked afterwards): on the GPU it is issued whatever the mask
@@ -33,6 +34,7 @@
 #define HIPC_LOAD_ALWAYS(ptr) gpu_model_load_always(ptr)
 #define HIPC_ARG_NOW(v) ((void)0)
 #define HIPC_PIN_VGPR(v) ((void)0)
+#define HIPC_PIN_SGPR(v) ((void)0)
 #define HIPC_VGPR_FROM_SGPR(dst, src) ((dst) = (src))
 #endif
 
@@ -69,6 +71,7 @@ struct Tuning {
     int dec_fused_attn = -1;  // HIPC_DEC_FUSED_ATTN 0 keeps the three-kernel attention (read when a decoder is created)
     int gemv_lean = -1;       // HIPC_GEMV_LEAN      0: one-row products keep the streaming GEMV kernel
     int dec_lean = -1;        // HIPC_DEC_LEAN       0: the decoder keeps the streaming GEMV and its prologues (read when a decoder is created)
+    int dec_resident = -1;    // HIPC_DEC_RESIDENT   0: the decoder keeps a launch per product (read when a decoder is created, too); n: workgroups of the launch that holds all layers
     int dec_prefetch = -1;    // HIPC_DEC_PREFETCH   bits: which launches of a layer carry helper rows that read ahead for the next launch (0 none, 31 all; see hipc_decoder_step)
 };
 

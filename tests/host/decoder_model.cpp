@@ -190,6 +190,20 @@ void full(const Shape &s) {
         for (int pos : g_quick ? few : all)
             if (pos >= 0 && pos <= last) m.step_at(pos, (pos * 7 + 3) % s.vocab);
     }
+    // all layers in one launch, where the shape has that: the whole grid, and a smaller one whose workgroups take several shares
+    if (s.hd != 192) {
+        m.ctx.tune.dec_prefetch = -1;
+        for (int w : windows_of(s)) {
+            m.windows(w);
+            for (int pos : {0, 31, 32, 33, 513, 2048, last})
+                if (pos >= 0 && pos <= last) {
+                    m.ctx.tune.dec_resident = pos == 33 ? 100 : -1;
+                    m.step_at(pos, 1);
+                    if (g_quick && s.layers * s.hidden > 1000) break;
+                }
+        }
+        m.ctx.tune.dec_prefetch = 31, m.ctx.tune.dec_resident = -1;
+    }
     // a step with the cache full changes nothing and reads nothing out of range
     m.step_at(last, s.vocab - 1);
     {

@@ -117,6 +117,16 @@ inline uint8_t gpu_model_load_b8(gpu_model_rsrc r, int v, int s, int aux) { uint
 #define __builtin_amdgcn_raw_buffer_load_b16 gpu_model_load_b16
 #define __builtin_amdgcn_raw_buffer_load_b8 gpu_model_load_b8
 
+// a store under the same rule: dropped past the descriptor's size, else inside one allocation
+inline void gpu_model_store_b32(uint32_t v, gpu_model_rsrc r, int voff_, int soff_, int) {
+    const uint32_t voff = (uint32_t)voff_, soff = (uint32_t)soff_;
+    if ((uint64_t)voff + 4 > r.records) return;
+    const uintptr_t addr = r.base + soff + voff;
+    if (!gpu_model::inside(addr, 4)) gpu_model::fail("buffer store", r.base, r.records, voff, soff, 4);
+    std::memcpy(reinterpret_cast<void *>(addr), &v, 4);
+}
+#define __builtin_amdgcn_raw_buffer_store_b32 gpu_model_store_b32
+
 // ---- stubs: cross-lane operations, matrix cores, barriers, device math -------------------------
 template <typename T>
 inline T gpu_model_same(T v) { return v; }

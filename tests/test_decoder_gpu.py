@@ -338,3 +338,89 @@ def test_gemma3_1b_shape_at_context_2040(ctx, pkg, oracle, route, env):
         token = got_tok
     dec.destroy()
     ctx.flush()
+
+
+RESIDENT = [  # (hidden, ffn, head_dim, query heads, kv heads, block_size): the launch that holds all layers, where its shares run out unevenly
+    (128, 256, 64, 4, 2, 32),     # eight column tiles and two k tiles for 256 workgroups; a head is half a k tile of o
+    (1296, 1552, 256, 2, 1, 32),  # 81 column tiles (three for some ranks), ffn's last k tile one pair wide, more units than are asked for ahead
+    (448, 1088, 128, 8, 2, 64),   # one XCD per head; 3 1/2 k tiles of hidden
+    (2048, 4224, 64, 1, 1, 128),  # the longest row; eight XCDs to a head; uneven slices of ffn
+]
+
+
+@pytest.mark.parametrize("groups", [-1, 255, 100, 3], ids=["all", "255", "100", "3"])
+@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
+def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, nkv, bs, groups):
+    """Three layers by a launch of 256 workgroups, and by launches of fewer, whose workgroups take several shares each
+    (what happens when not all of them find room on the device): logits, cache rows and tokens against the oracle over a
+    filled cache, positions 69 .. 72 (the third pass of 32 begins) with a window of 40 in the second layer. The tolerance is this file's."""
+    from oracle import decoder as od
+    route({"HIPC_DEC_RESIDENT": groups})
+    cfg = dict(SMALL, n_layers=3, hidden=hidden, ffn=ffn, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, block_size=bs, vocab=512, embed_scale=float(np.sqrt(hidden)))
+    p0, max_seq = 69, 80
+    w = pkg.decoder.build_weights(cfg, seed=31)
+    dec = pkg.decoder.Decoder(ctx, cfg, max_seq)
+    dec.load(w)
+    ref = od.Decoder(w, max_seq)
+    dec.set_layer_attention(1, 40, 500.0), ref.set_layer_attention(1, 40, 500.0)
+    rng = np.random.default_rng(hidden)
+    for li in range(cfg["n_layers"]):
+        k_rows, v_rows = ((rng.standard_normal((nkv, max_seq, hd)) * 0.7).astype(np.float16) for _ in range(2))
+        ref.k[li], ref.v[li] = k_rows, v_rows
+        dec.fill_cache(li, k_rows, v_rows)
+    token = 23
+    dec.reset(token, p0)
+    for pos in range(p0, p0 + 4):
+        dec.step()
+        got_tok, got_pos, logits, _ = dec.read(want_logits=True)
+        want_logits, _ = ref.step(token, pos)
+        assert got_pos == pos + 1
+        err = np.abs(logits - want_logits)
+        assert np.all(err <= 2e-3 + 2e-3 * np.abs(want_logits)), (pos, float(err.max()))
+        for li in range(cfg["n_layers"]):
+            k_row = ctx.download(dec.kv_cache(li)[0], np.float16, (hd,), offset=((nkv - 1) * max_seq + pos) * hd * 2)
+            assert np.allclose(k_row.astype(np.float32), ref.k[li, nkv - 1, pos].astype(np.float32), atol=2e-3, rtol=2e-3), (pos, li)
+        token = got_tok
+    dec.destroy()
+
+
+def test_decoders_on_several_streams_at_once(pkg):
+    """Three contexts (a stream each) replay their recorded steps from three threads: launches that do not find room for
+    all their workgroups beside each other go on with those that do, and every decoder picks the tokens it picks alone."""
+    import threading
+    cfg = dict(SMALL, hidden=512, ffn=2048, head_dim=128, n_layers=4, embed_scale=float(np.sqrt(512.0)))
+    w = pkg.decoder.build_weights(cfg, seed=8)
+    steps = 40
+
+    def run(n_threads):
+        ctxs = [pkg.Context(0) for _ in range(n_threads)]
+        decs, graphs, hists = [], [], [None] * n_threads
+        for c in ctxs:
+            d = pkg.decoder.Decoder(c, cfg, steps + 8)
+            d.load(w)
+            d.reset(7, 0)
+            d.step()
+            c.flush()
+            c.capture_begin()
+            d.step()
+            graphs.append(c.capture_end())
+            decs.append(d)
+
+        def go(i):
+            decs[i].reset(7, 0)
+            for _ in range(steps):
+                ctxs[i].graph_launch(graphs[i])
+            hists[i] = decs[i].read(n_history=steps)[3].copy()
+        threads = [threading.Thread(target=go, args=(i,)) for i in range(n_threads)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        for c, d, g in zip(ctxs, decs, graphs):
+            c.graph_destroy(g)
+            d.destroy()
+            c.close()
+        return hists
+    alone = run(1)[0]
+    for h in run(3):
+        assert h is not None and np.array_equal(h, alone)
