@@ -26,10 +26,10 @@
 // L2 only (workgroup scope); whether the members of a group really share one is read from the hardware when the launch
 // starts, and if not all stores are of agent scope.
 //
-// Nothing waits for a workgroup that may never come: a launch begins with the workgroups that have arrived by a deadline
-// (all 256 within microseconds on a free device), workgroup 0 decides who takes part, the 256 shares of the work are dealt
-// to those, and a workgroup that arrives later leaves at once. So two such launches on one device, from other streams or
-// processes, cannot block each other. All waits are bounded beside that: a thread's polls of a whole launch are counted.
+// Nothing waits for a workgroup that may never come: workgroup 0 decides by a deadline whether the launch begins (all 256
+// arrive within microseconds on a free device). If not, everyone leaves, and a launch behind it deals the 256 shares of the
+// work to the workgroups that have arrived there; one that arrives later leaves at once. So such launches on one device, from
+// other streams or processes, cannot block each other. All waits are bounded beside that: a thread's polls of a whole launch are counted.
 #include <hip/hip_fp16.h>
 
 #include "internal.h"
@@ -97,14 +97,16 @@ inline void res_stored() {}
 // A wavefront's share of a phase's product: up to U (column tile, k tile) units, one after the other 128 k of 16 columns.
 // Which units they are does not change between layers: their byte offsets are worked out once and kept in LDS (kept in
 // registers, they and the weights of three phases do not fit).
+// The sums of a unit are the same in all four groups of 16 lanes, so one group's are enough: group g takes those of units
+// g, 4 + g, ... and holds the scales and zero points of these only, asked for together with three other units'.
 template <int U, int SG>
 struct Units {
     uint4 wq[U];
-    ScaleVecLean<SG> sv[U];
+    ScaleVecLean<SG> sv[(U + 3) / 4];
     uint32_t live;   // bit i: unit i exists
 };
 
-// A product unit against the row's terms in LDS (see mmnb_lean_kernel). Every lane returns its column's sum.
+// A product unit against the row's terms in LDS (see mmnb_lean_kernel). The lanes that hold the unit's scales return their column's sum.
 template <int SG>
 __device__ __forceinline__ float res_unit(const uint4 &wq, const ScaleVecLean<SG> &sv, const char *as, uint32_t o_as, uint32_t nib_mask, uint32_t magic) {
     constexpr int CPG = 4 / SG;
@@ -272,28 +274,36 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
     };
     // the lane's offsets of a unit: in the weight (what its scales' and zero points' follow from); in LDS, the row's operand
     // and in the upper half where the sum goes
-    auto offsets_of = [&](const Unit &x, int phase) {
+    auto offsets_of = [&](const Unit &x, int i, int phase) {
         // (a unit that does not exist loads from past the end of everything: zeros, and no traffic. A load that is skipped
         // would keep the registers of the layer before alive.)
-        const uint32_t red = g4 == 0 ? (uint32_t)(phase * 64 * kRedPitch + (x.t * 16 + i16) * kRedPitch + x.kt) : (uint32_t)(4 * 64 * kRedPitch + lane);
+        const uint32_t red = g4 == (i & 3) ? (uint32_t)(phase * 64 * kRedPitch + (x.t * 16 + i16) * kRedPitch + x.kt) : (uint32_t)(4 * 64 * kRedPitch + lane);
         return make_uint2(x.live ? (uint32_t)x.tl * 1024u + (uint32_t)lane * 16u : 0xffff0000u,
                           (uint32_t)x.kt * 512u + (uint32_t)(min(i16 & 3, 1) * 4 + g4) * 16u + (red << 18));
     };
-    auto load_one = [&](const Weight &b, auto &w, int i, uint32_t o_wq) {
+    auto load_scales = [&](const Weight &b, ScaleVecLean<SG> &sv, uint32_t o_wq) {   // of the unit at the lane's o_wq
         const uint32_t o_zb = (o_wq >> 10) * (16u * SG) + (uint32_t)i16 * SG;
-        w.wq[i] = lean_ld16(b.q, o_wq, 0);
-        w.sv[i].load(b.s, b.z, o_zb * 4u, o_zb, 0);
+        sv.load(b.s, b.z, o_zb * 4u, o_zb, 0);
     };
-    auto load_units = [&](auto &w, int at, const Weight &b) {
+    // units from .. to - 1 (from: a multiple of four, or 2 with its neighbours' scales already asked for)
+    auto load_units = [&](auto &w, int at, const Weight &b, int from = 0, int to = 8) {
         constexpr int U = (int)(sizeof w.wq / sizeof w.wq[0]);
-        uint32_t o[U];
+        uint32_t o[U], os[(U + 3) / 4];
 #pragma unroll
-        for (int i = 0; i < U; i++) o[i] = S.off[at + i][tid].x;
+        for (int i = 0; i < U; i++)
+            if (i >= from && i < to) o[i] = S.off[at + i][tid].x;
 #pragma unroll
-        for (int i = 0; i < U; i++) load_one(b, w, i, o[i]);
+        for (int i = 0; i < U; i += 4)
+            if (i >= from && i < to) os[i / 4] = S.off[at + min(i + g4, U - 1)][tid].x;
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            if (i < from || i >= to) continue;
+            if (i % 4 == 0) load_scales(b, w.sv[i / 4], os[i / 4]);
+            w.wq[i] = lean_ld16(b.q, o[i], 0);
+        }
     };
     auto multiply_one = [&](auto &w, int i, uint32_t o_lds) {
-        const float acc = res_unit<SG>(w.wq[i], w.sv[i], as, o_lds & 0xffffu, nib_mask, magic);
+        const float acc = res_unit<SG>(w.wq[i], w.sv[i / 4], as, o_lds & 0xffffu, nib_mask, magic);
         *reinterpret_cast<float *>(reinterpret_cast<char *>(S.red) + (o_lds >> 16)) = acc;
     };
     // a phase's product: what was asked for ahead, then whatever else the share has
@@ -311,8 +321,10 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             const Unit x = unit(v, u);
             if (!x.live) continue;
             Units<1, SG> one;
-            const uint2 o = offsets_of(x, phase);
-            load_one(weight(e, which, tiles), one, 0, o.x);
+            const uint2 o = offsets_of(x, 0, phase);
+            const Weight b = weight(e, which, tiles);
+            load_scales(b, one.sv[0], o.x);
+            one.wq[0] = lean_ld16(b.q, o.x, 0);
             multiply_one(one, 0, o.y);
         }
     };
@@ -327,7 +339,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             w.live = 0;
             for (int i = 0; i < (int)(sizeof w.wq / sizeof w.wq[0]); i++) {
                 const Unit x = unit(first, wave + 8 * i);
-                S.off[at + i][tid] = offsets_of(x, phase);
+                S.off[at + i][tid] = offsets_of(x, i, phase);
                 w.live |= x.live ? 1u << i : 0u;
             }
         };
@@ -380,8 +392,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
     // what a layer's first phases need, asked for while the layer before is in its last one
     auto load_ahead = [&](uint32_t e) {
         load_head_w(e);
-        RES_STAMP(27);
-        if (ALL) load_units(w1, kAt1, weight(e, 0, n1)), load_units(w3, kAt3, weight(e, 1, n3));
+        if (ALL) load_units(w1, kAt1, weight(e, 0, n1));
     };
 
     // ---- hand-overs
@@ -546,6 +557,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
         // ---- q|k|v of the row
         RES_STAMP(0);
         norm_row(wp, wi);
+        if (ALL) load_units(w4, kAt4, weight(ent, 2, n4), 0, 2);
         RES_STAMP(2);
         for (int v = first; v < end; v += step) {
             zero_red(0);
@@ -559,6 +571,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             clear(v);
             if (!ALL) __syncthreads();
         }
+        if (ALL) load_units(w3, kAt3, weight(ent, 1, n3));
         RES_STAMP(4);
         // ---- attention: the share's positions for the XCD's head
         for (int v = first; v < end; v += step) {
@@ -608,7 +621,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             RES_STAMP(5);
             res_stored();   // this workgroup's words of the next layer are empty before it hands anything over (and o's weights and the cache rows are here)
             RES_STAMP(28);
-            if (ALL) load_units(w4, kAt4, weight(ent, 2, n4));
+            if (ALL) load_units(w4, kAt4, weight(ent, 2, n4), 2);
             else load_kv(ent, v);
             RES_STAMP(29);
             __syncthreads();
@@ -721,8 +734,6 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                 for (int i = 0; i < HD / 64; i++) again = again || any_empty(ov[i]);
             } while (again && --tries > 0);
             RES_STAMP(9);
-            if (ALL) load_units(w5, kAt5, weight(ent, 3, n5));
-            RES_STAMP(30);
             // lane i16 holds ranks 2 i16 and 2 i16 + 1
             const float m0 = __uint_as_float(ml.x), m1 = __uint_as_float(ml.z);
             const float M = lean_row_max(fmaxf(m0, m1));
@@ -776,6 +787,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             if (!ALL) __syncthreads();
         }
         RES_STAMP(12);
+        if (ALL) load_units(w5, kAt5, weight(ent, 3, n5));
         if (wave == 6)
             for (int v = first; v < end; v += step)
                 if (tiles3(v) > 0) combine(v, kResG1, kResY, true);
@@ -816,13 +828,13 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                           make_uint2(__builtin_amdgcn_perm(w.y, w.x, 0x07060302u), __builtin_amdgcn_perm(w.w, w.z, 0x07060302u)));
             }
             RES_STAMP(18);
-            if (ALL || v == first) load_ahead(ent_next);   // (behind the last layer: its own again)
             RES_STAMP(24);
             zero_red(3);
             __syncthreads();
             RES_STAMP(19);
             const int tiles = tiles3(v);
             multiply(w5, kAt5, ent, 3, n5, v, tiles * nk, 3, unit5);
+            if (ALL || v == first) load_ahead(ent_next);   // (behind the last layer: its own again)
             RES_STAMP(20);
             __syncthreads();
             if (wave == 7) {
@@ -852,7 +864,10 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
     }
 }
 
-template <int HD, int SG>
+// ALL: begins when all 256 workgroups have arrived, or not at all. Else: does the work of a launch of the other form that
+// did not begin (`behind` is set), or that was never made, with the workgroups that have arrived by the deadline.
+// (Two kernels: in one the second form costs the first 25 us a token, in registers. A launch that finds its work done is 2 us.)
+template <int HD, int SG, bool ALL>
 __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kernel(const ResidentArgs p) {
     __shared__ __attribute__((aligned(16))) ResShared<HD> S;
     const int pos = *p.pos;
@@ -865,12 +880,14 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t epoch = p.sync[0];
+    if (!ALL && p.behind && p.sync[kResAll + kResDecision] == ((epoch << 10) | (kResGroups << 1) | (p.sync[kResAll + kResDecision] & 1u))) return;   // done
+    uint32_t *sync = p.sync + (ALL ? kResAll : kResSome);
     if (tid == 0) {
         const uint32_t xcc = __builtin_amdgcn_s_getreg((31 << 11) | 20) & 15u;   // XCC_ID
-        __hip_atomic_store(p.sync + kResFlags + blockIdx.x, (epoch << 4) | xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(sync + kResFlags + blockIdx.x, (epoch << 4) | xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (blockIdx.x == 0 && wave == 0) {
-        const __amdgpu_buffer_rsrc_t r_s = lean_rsrc(p.sync, kResSyncWords * 4u);
+        const __amdgpu_buffer_rsrc_t r_s = lean_rsrc(sync, kResSyncWords * 4u);
         const unsigned long long t0 = wall_clock64();
         uint4 f;
         uint32_t here;   // bit q: workgroup 4 lane + q has arrived
@@ -889,44 +906,43 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
             const int o = __shfl_up(before, off, 64);
             if (lane >= off) before += o;
         }
-        const int count = __shfl(before, 63, 64);
+        int count = __shfl(before, 63, 64);
         before -= __popc(here);
         // one L2 per group: workgroups 8 j + x are group x, this lane holds groups 4 (lane & 1) ..
         const uint32_t gx = __shfl(f.x, lane & 1, 64), gy = __shfl(f.y, lane & 1, 64), gz = __shfl(f.z, lane & 1, 64), gw = __shfl(f.w, lane & 1, 64);
         const bool one_l2 = count == (int)kResGroups && __all(f.x == gx && f.y == gy && f.z == gz && f.w == gw);
-        if (count < (int)gridDim.x) {
+        if (ALL) {
+            count = count == (int)kResGroups ? count : 0;
+        } else if (count < (int)gridDim.x) {
             for (int q = 0; q < 4; q++) {
                 const bool in = (here >> q) & 1u;
-                __hip_atomic_store(p.sync + kResRankOf + 4 * lane + q, in ? (uint32_t)before : 0xffffu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(sync + kResRankOf + 4 * lane + q, in ? (uint32_t)before : 0xffffu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 before += in;
             }
             res_stored();
         }
-        if (lane == 0) __hip_atomic_store(p.sync + 1, (epoch << 10) | ((uint32_t)count << 1) | (one_l2 ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(sync + kResDecision, (epoch << 10) | ((uint32_t)count << 1) | (one_l2 ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (tid == 0) {
         uint32_t d = 0, rank = 0xffffu;
         do {
-            d = __hip_atomic_load(p.sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            d = __hip_atomic_load(sync + kResDecision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } while ((d >> 10) != (epoch & 0x3fffffu) && --tries > 0);
-        if (tries > 0) {
-            const uint32_t count = (d >> 1) & 0x1ffu;
-            rank = count == gridDim.x ? blockIdx.x : __hip_atomic_load(p.sync + kResRankOf + blockIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            *p.broken = 1;
-        }
+        const uint32_t count = (d >> 1) & 0x1ffu;
+        if (tries <= 0) *p.broken = 1;
+        else if (count == gridDim.x) rank = blockIdx.x;
+        else if (!ALL) rank = __hip_atomic_load(sync + kResRankOf + blockIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         S.decision[0] = d, S.decision[1] = rank;
     }
     __syncthreads();
     {
         const uint32_t d = __builtin_amdgcn_readfirstlane(S.decision[0]), rank = __builtin_amdgcn_readfirstlane(S.decision[1]);
-        if (rank == 0xffffu) return;   // the launch has begun without this workgroup
+        if (rank == 0xffffu) return;   // the launch does not begin, or has begun without this workgroup
         first = (int)rank, n = (int)((d >> 1) & 0x1ffu), wide = !(d & 1u);
     }
     set = (epoch % kResSets) * ((uint32_t)p.n_layers % kResSets) % kResSets;
 #endif
-    if (n == (int)kResGroups) res_layers<HD, SG, true>(p, S, first, n, wide, set, pos, tries);
-    else res_layers<HD, SG, false>(p, S, first, n, wide, set, pos, tries);
+    res_layers<HD, SG, ALL>(p, S, first, n, wide, set, pos, tries);
     if (tries <= 0) *p.broken = 1;
 }
 
@@ -936,7 +952,7 @@ __global__ void resident_set_layer_kernel(ResidentLayer *entry, const ResidentLa
 __global__ void __launch_bounds__(256) resident_clear_kernel(uint32_t *xch, uint32_t *sync) {
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < kResSets * kResWords; i += gridDim.x * 256) xch[i] = kEmpty;
     if (blockIdx.x == 0)
-        for (uint32_t i = threadIdx.x; i < kResSyncWords; i += 256) sync[i] = i == 0 ? 1u : 0u;
+        for (uint32_t i = threadIdx.x; i < kResSync; i += 256) sync[i] = i == 0 ? 1u : 0u;
 }
 
 }  // namespace hipc
@@ -959,13 +975,23 @@ bool hipc::resident_takes(const hipc_decoder_config &c) {
 
 namespace {
 
-template <int HD>
+template <int HD, bool ALL>
 void launch_sg(hipc_ctx *ctx, int sg, const ResidentArgs &a, int workgroups) {
     switch (sg) {
-        case 4: hipLaunchKernelGGL((dec_resident_kernel<HD, 4>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
-        case 2: hipLaunchKernelGGL((dec_resident_kernel<HD, 2>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL((dec_resident_kernel<HD, 1>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
+        case 4: hipLaunchKernelGGL((dec_resident_kernel<HD, 4, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
+        case 2: hipLaunchKernelGGL((dec_resident_kernel<HD, 2, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
+        default: hipLaunchKernelGGL((dec_resident_kernel<HD, 1, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
     }
+}
+template <bool ALL>
+int launch_hd(hipc_ctx *ctx, int hd, int sg, const ResidentArgs &a, int workgroups) {
+    switch (hd) {
+        case 64: launch_sg<64, ALL>(ctx, sg, a, workgroups); break;
+        case 128: launch_sg<128, ALL>(ctx, sg, a, workgroups); break;
+        default: launch_sg<256, ALL>(ctx, sg, a, workgroups); break;
+    }
+    HIPC_LAUNCHED(ctx);
+    return HIPC_OK;
 }
 
 }  // namespace
@@ -983,13 +1009,12 @@ int hipc::resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const Res
     a.nib_mask = 0x000f000fu, a.magic = 0x43004300u;
     a.eps = c.rms_eps, a.scale = c.attn_scale > 0.f ? c.attn_scale : 1.f / sqrtf((float)c.head_dim);
     const int sg = c.block_size == 32 ? 4 : c.block_size == 64 ? 2 : 1;
-    switch (c.head_dim) {
-        case 64: launch_sg<64>(ctx, sg, a, workgroups); break;
-        case 128: launch_sg<128>(ctx, sg, a, workgroups); break;
-        default: launch_sg<256>(ctx, sg, a, workgroups); break;
+    if (workgroups >= (int)kResGroups) {
+        int rc = launch_hd<true>(ctx, c.head_dim, sg, a, kResGroups);
+        if (rc != HIPC_OK) return rc;
+        a.behind = 1, workgroups = 64;   // fewer than there might be: it is there for the device that is shared
     }
-    HIPC_LAUNCHED(ctx);
-    return HIPC_OK;
+    return launch_hd<false>(ctx, c.head_dim, sg, a, workgroups);
 }
 
 int hipc::resident_set_layer(hipc_ctx *ctx, ResidentLayer *entry, const ResidentLayer &value) {

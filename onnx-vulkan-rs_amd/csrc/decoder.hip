@@ -797,7 +797,7 @@ __global__ void __launch_bounds__(256) dec_set_state_kernel(DecState *st, int to
     if (threadIdx.x == 0) st->token = token, st->pos = pos, st->overflow = 0, st->broken = 0;
     if (broken) {
         for (uint32_t i = threadIdx.x; i < kResSets * kResWords; i += 256) xch[i] = 0xffffffffu;
-        for (uint32_t i = threadIdx.x; i < kResSyncWords; i += 256) sync[i] = i == 0 ? 1u : 0u;
+        for (uint32_t i = threadIdx.x; i < kResSync; i += 256) sync[i] = i == 0 ? 1u : 0u;
     }
 }
 
@@ -1016,7 +1016,7 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
         d->resident = d->lean && resident_takes(c) && ctx->tune.dec_resident != 0;
         if (d->resident) {
             d->entries.resize(c.n_layers), d->stale.assign(c.n_layers, 1);
-            A(&d->table, c.n_layers), A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSyncWords);
+            A(&d->table, c.n_layers), A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSync);
             if (rc == HIPC_OK) rc = resident_clear(ctx, d->xch, d->sync);
         }
         if (rc == HIPC_OK) {

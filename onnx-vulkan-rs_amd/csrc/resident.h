@@ -35,9 +35,10 @@ constexpr uint32_t kResWords = kResQ + kResMaxQkv;                         // wo
 constexpr uint32_t kResSets = 3;
 static_assert(kResA % 32 == 0 && kResML % 32 == 0 && kResY % 32 == 0 && kResH % 32 == 0 && kResY2 % 32 == 0 && kResLocal % 32 == 0,
               "no region shares a 128-byte line with another");
-// The words the workgroups of a launch agree through: [0] the launch's number (the token pick counts it up), [1] the
-// decision, then one flag and one rank per workgroup.
-constexpr uint32_t kResFlags = 32, kResRankOf = kResFlags + kResGroups, kResSyncWords = kResRankOf + kResGroups;
+// The words the workgroups of a launch agree through: [0] the step's number (the token pick counts it up, modulo
+// kResLaunches); then, for the launch of all workgroups and for the one that stands in for it, the decision, one flag and one rank per workgroup.
+constexpr uint32_t kResDecision = 0, kResFlags = 32, kResRankOf = kResFlags + kResGroups, kResSyncWords = kResRankOf + kResGroups;
+constexpr uint32_t kResAll = 32, kResSome = kResAll + kResSyncWords, kResSync = kResSome + kResSyncWords;
 constexpr uint32_t kResLaunches = kResSets << 26;   // a multiple of the sets, so that they go on in turn, and 28 bits
 
 struct ResidentArgs {
@@ -49,7 +50,7 @@ struct ResidentArgs {
     uint32_t *xch, *sync;
     int n_layers, hidden, cg_h, cg_o, tiles_h, tiles_qkv, cg_f, pairs;   // cg_*: 128-k tiles of hidden, the heads' channels, ffn; tiles_*: 16-column tiles; pairs: (gate, up) tile pairs
     int n_q, n_kv, lg_group, lg_parts;   // XCDs per head = 1 << lg_parts
-    int max_seq, v_stride;
+    int max_seq, v_stride, behind;
     uint32_t inv_cg_h;                   // 65536 / cg_h, rounded up
     uint32_t nib_mask, magic;
     float eps, scale, inv_hidden;
