@@ -51,14 +51,14 @@ struct PrefillArgs {
     int ksplit, split_stages;
     float *Ypart;
     float *Yf32;   // when set, the result is written here as f32 and Y is not used (rows of f32 activations, see nbits_prefill_f32)
-    // Paired rows (set together; only the kernel that keeps the weight out of LDS): A holds the two
-    // f16 terms of `pair_rows` f32 rows, 32 rows of high terms followed by the 32 rows of their low terms, so that a
-    // wavefront's two row blocks (64-row tiles: two wavefronts') are the two terms of the same 32 rows; it adds them and stores row r of the result
-    // times 2^exps[r] -- into Yf32, or unscaled into the k split's partials [split][pair_rows][N].
+    // Rows in terms (set together; only the kernel that keeps the weight out of LDS): A holds the `terms` (2 or 3) f16 terms of
+    // `pair_rows` f32 rows, the high terms of 32 rows followed by these rows' lower terms, and a wavefront owns all terms of its
+    // rows: they add up in its accumulator. Row r of the result is stored times 2^exps[r] -- into Yf32, or unscaled into the k
+    // split's partials [split][pair_rows][N].
     // exps without pair_rows: A holds one f16 term per f32 row and row r of the f32 result is stored times 2^exps[r]
     // (any of the kernels; the k split's partials stay unscaled).
     const int *exps;
-    int pair_rows;
+    int pair_rows, terms;
 };
 
 // eight nibbles (order k0 k2 k4 k6 k1 k3 k5 k7) -> eight f16 values q - zp in k order, as four words of pairs
@@ -348,17 +348,26 @@ __global__ void __launch_bounds__(256) mmnb_prefill_kernel(const PrefillArgs p) 
 // group hands over the 32-row blocks the other one stores; 64-row tiles: the second hands everything to the first).
 // For launches that leave wavefront slots of the SIMDs empty: a second wavefront issues while the first waits for
 // LDS, a barrier or the matrix core.
-template <int SG, int MI, int NJ, int KG, bool FULL>
-__global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI * NJ <= 4 ? 2 : 1) mmnb_prefill_direct_kernel(const PrefillArgs p) {
-    static_assert(KG == 1 || KG == 2, "one or two groups");
-    constexpr int T = 64 * MI, TN = 64 * NJ, kChunks = T / 32, kF = MI, kWT = 32 * MI, kWN = 32 * NJ;
+// WM, WN: the wavefronts of a group, WM along the rows, WN along the columns.
+// TERMS: 2 or 3, the row blocks of a wavefront are the terms of the same 32 f32 rows (see nbits_prefill_f32; 0: rows as they
+// are). Two terms' products of a quantisation block go into one set of registers, the low ones first, three terms' into three
+// that are joined, and scale x (block sum) is added to a running total. With two terms that is one multiply-add per result
+// and block, where accumulators of their own cost each term one (blocks of 32: 8 of 14 vector instructions a product), and
+// the total is rounded once per block instead of three times: 2.6e-7 -> 1.3e-7 against 64 bits at 333 x 1152 x 13824, 48.2 -> 38.0 us.
+template <int SG, int MI, int NJ, int WM, int WN, int KG, int TERMS, bool FULL>
+__global__ void __launch_bounds__(64 * WM * WN * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI * NJ <= 4 ? 2 : 1) mmnb_prefill_direct_kernel(const PrefillArgs p) {
+    static_assert(KG == 1 || KG == 2 || (TERMS && KG == 4), "one or two groups; four of paired rows");
+    constexpr int GT = 64 * WM * WN;   // threads of a group
+    static_assert(TERMS == 0 || MI % TERMS == 0, "all terms in one wavefront");
+    constexpr int PB = TERMS ? MI / TERMS : 1, TS = TERMS == 3 ? 3 : 1;   // blocks of 32 f32 rows, sets of sums of each
+    constexpr int T = 32 * MI * WM, TN = 32 * NJ * WN, kChunks = T * 8 / GT, kF = MI, kWT = 32 * MI, kWN = 32 * NJ;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-    const int grp = KG > 1 ? (int)(threadIdx.x >> 8) : 0;
+    const int grp = KG > 1 ? (int)threadIdx.x / GT : 0;
     uint8_t *lds_a = lds_raw + grp * 2 * T * kPPitch;  // [KG][2][T * kPPitch]
 
-    const int tid = threadIdx.x & 255;
+    const int tid = threadIdx.x % GT;
     const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WN, wn = wave % WN;
     const int r32 = lane & 31, kg = lane >> 5;
 
     const int tiles_x = (p.N + TN - 1) / TN, tiles_y = (p.M + T - 1) / T;
@@ -368,12 +377,12 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
     if (idx >= rows_per * cols_per || ty >= tiles_y || tx >= tiles_x) return;
     const int i0 = ty * T, j0 = tx * TN;
 
-    // A: chunk c = tid + 256 u -> slab row c / 8, 16-byte column c % 8 (8 halves)
+    // A: chunk c = tid + GT u -> slab row c / 8, 16-byte column c % 8 (8 halves)
     uint32_t a_off[kChunks], a_lds[kChunks];
     int a_k[kChunks];
 #pragma unroll
     for (int u = 0; u < kChunks; u++) {
-        const int c = tid + 256 * u, row = c >> 3, kc = c & 7;
+        const int c = tid + GT * u, row = c >> 3, kc = c & 7;
         a_off[u] = ((uint32_t)min(i0 + row, p.M - 1) * (uint32_t)p.K + kc * 8) * 2;  // rows past M: clamped, never stored
         a_lds[u] = row * kPPitch + kc * 16;
         a_k[u] = kc * 8;
@@ -454,9 +463,9 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
     // below 2^-64 (a block of zeros carries 0) counts as 2^-64: the quotient stays finite, and what such a block
     // adds, at most 2^-64 x 15 x sum |a|, is far below one unit of the last place of any result that has a block
     // with a real scale; a column without one is stored as 0.
-    f32x16 acc[kF][NJ];
+    f32x16 acc[TERMS ? PB * (1 + TS) : kF][NJ];   // TERMS: [0 .. PB - 1] the running totals, behind them the open block's sums
 #pragma unroll
-    for (int i = 0; i < kF; i++)
+    for (int i = 0; i < (TERMS ? PB : kF); i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -468,6 +477,7 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
     // the scales of a weight tile's groups -> the factors that take the accumulators from each group to the next
     // (worked out when the trip begins, next to the loads, not in front of the products that wait for them)
     auto scales_to_ratios = [&](BRegs &b) {
+        if (TERMS) return;
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -518,20 +528,47 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
         for (int step = 0; step < 4; step++) {
             const int word = half * 2 + (step >> 1), h = step & 1;
             const bool opens = SG == 8 ? true : SG == 4 ? h == 0 : SG == 2 ? step == 0 : step == 0 && half == 0;
+            const int g = (SG == 8 ? 2 * word + h : SG == 4 ? word : SG == 2 ? half : 0) % SG;
             f16x8 af[kF], wf[NJ];
-            if (opens) {
-                const int g = SG == 8 ? 2 * word + h : SG == 4 ? word : SG == 2 ? half : 0;
+            if (opens && !TERMS) {
 #pragma unroll
-                for (int j = 0; j < NJ; j++) reopen(j, b.s[j][g % SG]);
+                for (int j = 0; j < NJ; j++) reopen(j, b.s[j][g]);
             }
 #pragma unroll
             for (int i = 0; i < kF; i++) af[i] = *reinterpret_cast<const f16x8 *>(ba + i * 32 * kPPitch + (step >> 1) * 64 + h * (SG == 8 ? 32 : 16));
 #pragma unroll
             for (int j = 0; j < NJ; j++) wf[j] = dequant_operand(word_of(b.w[j][h], word), zp.at[j][SG == 8 ? step : SG == 4 ? step >> 1 : 0], ones);
+            if constexpr (TERMS > 0) {
+                const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                const bool closes = SG == 8 ? true : SG == 4 ? h == 1 : SG == 2 ? step == 3 : step == 3 && half == 1;
 #pragma unroll
-            for (int i = 0; i < kF; i++)
+                for (int t = TERMS - 1; t >= 0; t--)
 #pragma unroll
-                for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], wf[j], acc[i][j], 0, 0, 0);
+                    for (int i = 0; i < PB; i++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) {
+                            f32x16 &sum = acc[PB + i * TS + (TERMS == 3 ? t : 0)][j];
+                            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i * TERMS + t], wf[j], opens && (TERMS == 3 || t == TERMS - 1) ? zero : sum, 0, 0, 0);
+                        }
+                if (closes) {
+#pragma unroll
+                    for (int i = 0; i < PB; i++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++)
+#pragma unroll
+                            for (int r = 0; r < 16; r++) {
+                                float sum = acc[PB + i * TS][j][r];
+                                if constexpr (TERMS == 3) sum = join_terms(sum, acc[PB + i * TS + 1][j][r], acc[PB + i * TS + 2][j][r]);
+                                acc[i][j][r] = fmaf(sum, b.s[j][g], acc[i][j][r]);
+                            }
+                }
+                if (SG >= 4) __builtin_amdgcn_sched_barrier(0);   // (left alone, the blocks of a stage are all opened before one is closed)
+            } else {
+#pragma unroll
+                for (int i = 0; i < kF; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], wf[j], acc[i][j], 0, 0, 0);
+            }
         }
     };
 
@@ -576,45 +613,48 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
         trip(bc, bn, ks0 + 2 * t);
         if (t + 1 < my_trips) trip(bn, bc, ks0 + 2 * t + 2);
     }
+    if constexpr (TERMS > 0) {
+        // the later groups hand their sums to the first ([group - 1][16-byte piece][thread] in LDS), which adds them and stores
+        if constexpr (KG > 1) {
+            float4 *slot = reinterpret_cast<float4 *>(lds_raw);
+            constexpr int kPieces = PB * NJ * 4;
+            if (grp > 0) {
+#pragma unroll
+                for (int i = 0; i < PB; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            slot[((grp - 1) * kPieces + (i * NJ + j) * 4 + q) * GT + tid] = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+            }
+            __syncthreads();
+            if (grp > 0) return;
+#pragma unroll
+            for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+                for (int i = 0; i < PB; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const float4 o = slot[(g * kPieces + (i * NJ + j) * 4 + q) * GT + tid];
+                            acc[i][j][4 * q] += o.x, acc[i][j][4 * q + 1] += o.y, acc[i][j][4 * q + 2] += o.z, acc[i][j][4 * q + 3] += o.w;
+                        }
+        }
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            f32x16 pair[1][NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; j++) pair[0][j] = acc[i][j];
+            prefill_store_pairs<NJ>(p, pair, (i0 + wm * kWT) / TERMS + 32 * i, j0 + wn * kWN, r32, kg);
+        }
+    } else {
 #pragma unroll
     for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int i = 0; i < kF; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] *= scaled[j] ? unit[j] : 0.f;
-    if constexpr (MI == 2) {
-        if (p.pair_rows > 0) {
-            // paired rows: the wavefront's two row blocks are the two terms of the same 32 rows. Every group adds its
-            // own two, the second hands its sums to the first ([16-byte piece][thread] in LDS, as below), which adds
-            // them and stores.
-            f32x16 pair[1][NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) pair[0][j][r] = acc[0][j][r] + acc[1][j][r];
-            if constexpr (KG == 2) {
-                float4 *slot = reinterpret_cast<float4 *>(lds_raw);
-                if (grp > 0) {
-#pragma unroll
-                    for (int j = 0; j < NJ; j++)
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            slot[(j * 4 + q) * 256 + tid] = make_float4(pair[0][j][4 * q], pair[0][j][4 * q + 1], pair[0][j][4 * q + 2], pair[0][j][4 * q + 3]);
-                }
-                __syncthreads();
-                if (grp > 0) return;
-#pragma unroll
-                for (int j = 0; j < NJ; j++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const float4 o = slot[(j * 4 + q) * 256 + tid];
-                        pair[0][j][4 * q] += o.x, pair[0][j][4 * q + 1] += o.y, pair[0][j][4 * q + 2] += o.z, pair[0][j][4 * q + 3] += o.w;
-                    }
-            }
-            prefill_store_pairs<NJ>(p, pair, (i0 + wm * kWT) >> 1, j0 + wn * kWN, r32, kg);
-            return;
-        }
-    }
     if constexpr (KG > 1 && MI == 1) {
         // the later groups hand their accumulators to the first: [group - 1][16-byte piece][thread] in LDS (the A
         // buffers are done with: the last barrier of the loop is behind every read of them), added in group order
@@ -639,31 +679,6 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
                 }
     }
     if constexpr (MI == 1) {
-        if (p.pair_rows > 0) {
-            // paired rows: the tile's two row blocks, of two wavefronts. The one with the low terms hands its sums over
-            // (behind what the groups exchanged; 8 KB, once per tile), the other adds them and stores. Few rows are
-            // bound by the serial chain of each tile: 128-row tiles left most CUs idle (130 x 2048 x 2560: 60 tiles,
-            // 30.8 us; 200 of these, 17.6 us).
-            float4 *slot = reinterpret_cast<float4 *>(lds_raw) + (KG - 1) * NJ * 4 * 256;
-            if (wm == 1) {
-#pragma unroll
-                for (int j = 0; j < NJ; j++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        slot[(j * 4 + q) * 128 + wn * 64 + lane] = make_float4(acc[0][j][4 * q], acc[0][j][4 * q + 1], acc[0][j][4 * q + 2], acc[0][j][4 * q + 3]);
-            }
-            __syncthreads();   // (the second group of wavefronts has left)
-            if (wm == 1) return;
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 o = slot[(j * 4 + q) * 128 + wn * 64 + lane];
-                    acc[0][j][4 * q] += o.x, acc[0][j][4 * q + 1] += o.y, acc[0][j][4 * q + 2] += o.z, acc[0][j][4 * q + 3] += o.w;
-                }
-            prefill_store_pairs<NJ>(p, acc, i0 >> 1, j0 + wn * kWN, r32, kg);
-            return;
-        }
         prefill_store<kF, NJ>(p, acc, i0 + wm * kWT, j0 + wn * kWN, r32, kg);
     } else if constexpr (KG == 2) {
         // group g keeps row block g and hands the other one over: [group][16-byte piece][thread] in LDS (the A
@@ -694,11 +709,12 @@ __global__ void __launch_bounds__(256 * KG, KG > 1 ? 1 : MI * NJ == 1 ? 4 : MI *
     } else {
         prefill_store<kF, NJ>(p, acc, i0 + wm * kWT, j0 + wn * kWN, r32, kg);
     }
+    }
 }
 
 // Y = f16(sum over splits of the f32 partials), in split order; or the f32 sum itself into Yf32. Four results per
 // thread; VEC: the element count is a multiple of four and the rows are aligned for 16-byte loads and one 8- or
-// 16-byte store. (static: this file is compiled twice)
+// 16-byte store. (static: this file is compiled three times)
 template <bool VEC>
 static __global__ void __launch_bounds__(256)
 mmnb_prefill_reduce_kernel(const float *__restrict__ part, __half *__restrict__ Y, float *__restrict__ Yf32, long total, int ksplit,
@@ -802,85 +818,80 @@ int prefill_launch_tile(hipc_ctx *ctx, PrefillArgs a) {
 }
 
 // the weight from memory into the operand registers; A alone in LDS
-template <int SG, int MI, int NJ, int KG>
+template <int SG, int MI, int NJ, int WM, int WN, int KG, int TERMS>
 int prefill_launch_direct_groups(hipc_ctx *ctx, const PrefillArgs &a, dim3 grid) {
     const bool full = a.K % (2 * kPK) == 0;
-    // one group: at most 36 KB, inside the limit that needs no permission; two: their A buffers, then the hand-over
-    constexpr size_t lds = KG == 1 ? prefill_lds(64 * MI) / 2 : std::max(KG * prefill_lds(64 * MI) / 2, (size_t)(MI == 2 ? 4 : 2 * (KG - 1) + 1) * NJ * 4 * 128 * 16);
+    constexpr int T = 32 * MI * WM, kThreads = 64 * WM * WN * KG;
+    // one group: at most 36 KB, inside the limit that needs no permission; more: their A buffers, then the hand-over
+    constexpr size_t hand_over = TERMS ? (size_t)(KG - 1) * (MI / std::max(1, TERMS)) * NJ * 4 * (64 * WM * WN) * 16 : (size_t)(MI == 2 ? 4 : 2 * (KG - 1)) * NJ * 4 * 128 * 16;
+    constexpr size_t lds = KG == 1 ? prefill_lds(T) / 2 : std::max(KG * prefill_lds(T) / 2, hand_over);
     if (KG > 1 && lds > 64 * 1024) {
         static bool lds_allowed[2][kMaxDevices] = {};
-        if (int rc = full ? allow_dynamic_lds(ctx, mmnb_prefill_direct_kernel<SG, MI, NJ, KG, true>, lds, lds_allowed[1])
-                          : allow_dynamic_lds(ctx, mmnb_prefill_direct_kernel<SG, MI, NJ, KG, false>, lds, lds_allowed[0]))
+        if (int rc = full ? allow_dynamic_lds(ctx, mmnb_prefill_direct_kernel<SG, MI, NJ, WM, WN, KG, TERMS, true>, lds, lds_allowed[1])
+                          : allow_dynamic_lds(ctx, mmnb_prefill_direct_kernel<SG, MI, NJ, WM, WN, KG, TERMS, false>, lds, lds_allowed[0]))
             return rc;
     }
     if (full)
-        hipLaunchKernelGGL((mmnb_prefill_direct_kernel<SG, MI, NJ, KG, true>), grid, dim3(256 * KG), lds, ctx->stream, a);
+        hipLaunchKernelGGL((mmnb_prefill_direct_kernel<SG, MI, NJ, WM, WN, KG, TERMS, true>), grid, dim3(kThreads), lds, ctx->stream, a);
     else
-        hipLaunchKernelGGL((mmnb_prefill_direct_kernel<SG, MI, NJ, KG, false>), grid, dim3(256 * KG), lds, ctx->stream, a);
+        hipLaunchKernelGGL((mmnb_prefill_direct_kernel<SG, MI, NJ, WM, WN, KG, TERMS, false>), grid, dim3(kThreads), lds, ctx->stream, a);
     HIPC_LAUNCHED(ctx);
     return HIPC_OK;
 }
-template <int SG, int MI, int NJ>
+template <int SG, int MI, int NJ, int WM, int WN, int TERMS>
 int prefill_launch_direct(hipc_ctx *ctx, PrefillArgs a) {
+    constexpr int T = 32 * MI * WM, TN = 32 * NJ * WN;
     dim3 grid;
     // (64-row tiles split a long k as the larger ones do when even they are too few: f16 100 x 8192 x 1024, 32 tiles,
     // 32.0 us as they are, 13.7 us four ways)
-    if (int rc = prefill_plan(ctx, a, 64 * MI, 64 * NJ, true, &grid)) return rc;
-    if constexpr (MI == 2) {
-        // Two k groups per workgroup when the launch leaves the second wavefront slot of the SIMDs empty (no more
-        // workgroups than CUs) and every group gets two trips or more; prefill_groups 1 / 2 forces the choice.
-        const int trips = (a.split_stages + 1) / 2, forced = ctx->tune.prefill_groups;
-        const long wgs = (long)ceil_div(a.M, 64 * MI) * ceil_div(a.N, 64 * NJ) * a.ksplit;
-        // (three column blocks and two groups leave no register for more than one scale per weight tile)
-        const bool two = (NJ == 2 || SG == 1) && (forced == 1 ? false : forced == 2 ? true : wgs <= ctx->cu_count && trips >= 4);
-        if constexpr (NJ == 2 || SG == 1) if (two) {
-            if (int rc = prefill_launch_direct_groups<SG, MI, NJ, 2>(ctx, a, grid)) return rc;
+    if (int rc = prefill_plan(ctx, a, T, TN, true, &grid)) return rc;
+    const int trips = (a.split_stages + 1) / 2, forced = ctx->tune.prefill_groups;
+    const long wgs = (long)ceil_div(a.M, T) * ceil_div(a.N, TN) * a.ksplit;
+    // Two k groups per workgroup (four of paired rows where a group is two wavefronts) when the launch leaves the second
+    // wavefront slot of the SIMDs empty (128-row tiles: no more workgroups than CUs; 64-row tiles: no more than two per CU,
+    // 512 x 2048 x 2560: 15.9 against 16.9 us, four groups, 18.3 us, cost more in prologues than they hide) and every group
+    // gets two trips or more; prefill_groups 1 / 2 forces the choice. (three column blocks and two groups leave no register
+    // for more than one scale per weight tile)
+    constexpr int kGroups = WM * WN == 2 ? 4 : 2;
+    if constexpr (NJ < 3 || SG == 1) {
+        if (forced == 1 ? false : forced == 2 ? true : wgs <= (T < 128 ? 2 : 1) * ctx->cu_count && trips >= 2 * kGroups) {
+            if (int rc = prefill_launch_direct_groups<SG, MI, NJ, WM, WN, kGroups, TERMS>(ctx, a, grid)) return rc;
             return prefill_join_splits(ctx, a);
         }
     }
-    if constexpr (MI == 1) {
-        // 64-row tiles: two groups when the launch has too few wavefronts to hide one another's waits (no more than
-        // two workgroups per CU) and each group keeps two trips (512 x 2048 x 2560: 15.9 against 16.9 us; four
-        // groups, 18.3 us, cost more in prologues than they hide)
-        const int trips = (a.split_stages + 1) / 2, forced = ctx->tune.prefill_groups;
-        const long wgs = (long)ceil_div(a.M, 64) * ceil_div(a.N, 64 * NJ) * a.ksplit;
-        if (forced == 1 ? false : forced == 2 ? true : wgs <= 2 * ctx->cu_count && trips >= 4) {
-            if (int rc = prefill_launch_direct_groups<SG, MI, NJ, 2>(ctx, a, grid)) return rc;
-            return prefill_join_splits(ctx, a);
-        }
-    }
-    if (int rc = prefill_launch_direct_groups<SG, MI, NJ, 1>(ctx, a, grid)) return rc;
+    if (int rc = prefill_launch_direct_groups<SG, MI, NJ, WM, WN, 1, TERMS>(ctx, a, grid)) return rc;
     return prefill_join_splits(ctx, a);
 }
 
 }  // namespace
 
-// This file is compiled twice. The 128x128 instances live in an object of their own, built with
+// This file is compiled three times. The 128x128 instances live in an object of their own, built with
 // HIPC_PREFILL_WIDE and with the matrix-core accumulators in ordinary vector registers (the block
 // scales then multiply them without copies out of the accumulation file: 48.5 -> 44.7 us for
 // 512 x 2048 x 11008); the 64x64 instances are faster with the accumulation file (80.6 against
 // 87.9 us for 512 x 11008 x 2048), and that is a switch of the whole compilation.
 int prefill_launch_wide(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile);
+int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile);   // rows in terms: an object of its own, too (see the Makefile)
 
 #ifdef HIPC_PREFILL_WIDE
 
 int prefill_launch_wide(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) {
     if (tile == 192) switch (SG) {
-            case 4: return prefill_launch_direct<4, 2, 3>(ctx, a);
-            case 2: return prefill_launch_direct<2, 2, 3>(ctx, a);
-            default: return prefill_launch_direct<1, 2, 3>(ctx, a);
+            case 4: return prefill_launch_direct<4, 2, 3, 2, 2, 0>(ctx, a);
+            case 2: return prefill_launch_direct<2, 2, 3, 2, 2, 0>(ctx, a);
+            default: return prefill_launch_direct<1, 2, 3, 2, 2, 0>(ctx, a);
         }
     if (tile == 64) switch (SG) {
-            case 8: return prefill_launch_direct<8, 1, 1>(ctx, a);
-            case 4: return prefill_launch_direct<4, 1, 1>(ctx, a);
-            case 2: return prefill_launch_direct<2, 1, 1>(ctx, a);
-            default: return prefill_launch_direct<1, 1, 1>(ctx, a);
+            case 8: return prefill_launch_direct<8, 1, 1, 2, 2, 0>(ctx, a);
+            case 4: return prefill_launch_direct<4, 1, 1, 2, 2, 0>(ctx, a);
+            case 2: return prefill_launch_direct<2, 1, 1, 2, 2, 0>(ctx, a);
+            default: return prefill_launch_direct<1, 1, 1, 2, 2, 0>(ctx, a);
         }
     if (ctx->tune.prefill_direct != 0 || SG == 8) switch (SG) {
-            case 8: return prefill_launch_direct<8, 2, 2>(ctx, a);
-            case 4: return prefill_launch_direct<4, 2, 2>(ctx, a);
-            case 2: return prefill_launch_direct<2, 2, 2>(ctx, a);
-            default: return prefill_launch_direct<1, 2, 2>(ctx, a);
+            case 8: return prefill_launch_direct<8, 2, 2, 2, 2, 0>(ctx, a);
+            case 4: return prefill_launch_direct<4, 2, 2, 2, 2, 0>(ctx, a);
+            case 2: return prefill_launch_direct<2, 2, 2, 2, 2, 0>(ctx, a);
+            default: return prefill_launch_direct<1, 2, 2, 2, 2, 0>(ctx, a);
         }
     switch (SG) {
         case 4: return prefill_launch_tile<4, 128>(ctx, a);
@@ -889,13 +900,65 @@ int prefill_launch_wide(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) {
     }
 }
 
+#elif defined(HIPC_PREFILL_TERMS)
+
+int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) {
+    if (a.terms == 3) {   // (tile: 64 -> 96x64, else 96x128)
+        if (tile == 64) switch (SG) {
+                case 4: return prefill_launch_direct<4, 3, 1, 1, 2, 3>(ctx, a);
+                case 2: return prefill_launch_direct<2, 3, 1, 1, 2, 3>(ctx, a);
+                default: return prefill_launch_direct<1, 3, 1, 1, 2, 3>(ctx, a);
+            }
+        switch (SG) {
+            case 4: return prefill_launch_direct<4, 3, 1, 1, 4, 3>(ctx, a);
+            case 2: return prefill_launch_direct<2, 3, 1, 1, 4, 3>(ctx, a);
+            default: return prefill_launch_direct<1, 3, 1, 1, 4, 3>(ctx, a);
+        }
+    }
+    // (tile: 64 -> 64x64, 128 -> 64x128, 192 -> the larger ones of prefill_pair_tile)
+    if (tile == 192) switch (SG) {
+            case 4: return prefill_launch_direct<4, 4, 1, 1, 4, 2>(ctx, a);
+            case 2: return prefill_launch_direct<2, 2, 2, 1, 4, 2>(ctx, a);
+            case 1: return prefill_launch_direct<1, 2, 2, 1, 4, 2>(ctx, a);
+        }
+    if (tile == 64) switch (SG) {
+            case 4: return prefill_launch_direct<4, 2, 1, 1, 2, 2>(ctx, a);
+            case 2: return prefill_launch_direct<2, 2, 1, 1, 2, 2>(ctx, a);
+            default: return prefill_launch_direct<1, 2, 1, 1, 2, 2>(ctx, a);
+        }
+    switch (SG) {
+        case 4: return prefill_launch_direct<4, 2, 1, 1, 4, 2>(ctx, a);
+        case 2: return prefill_launch_direct<2, 2, 1, 1, 4, 2>(ctx, a);
+        default: return prefill_launch_direct<1, 2, 1, 1, 4, 2>(ctx, a);
+    }
+}
+
 #else
 
 namespace {
 
+// Tiles of paired rows: 64x64 where there are few tiles and k is not long enough to split three ways over workgroups; else
+// 64x128, or the larger ones where these take fewer rounds of workgroups times stages: 128x128 (64 f32 rows to a wavefront)
+// with four scales per weight tile, 64x256 with one or two. They do two 64x128 tiles' work in 15/16 of the time. Measured,
+// 64x64 / 64x128 / larger, us: 333 x 1152 x 13824 in blocks of 32 44.0 / 37.1 / 42.1, 1000 x 2048 x 4096 62.1 / 53.1 / 50.4,
+// 100 x 2048 x 2560 14.8 / 18.6 / 28.5, 100 x 6912 x 1152 33.3 / 25.2 / 35.7, 300 x 11008 x 2048 90.2 / 72.1 / 54.9; in blocks
+// of 128 600 x 8192 x 1024 60.9 / 48.3 / 38.4.
+template <int SG>
+int prefill_pair_tile(hipc_ctx *ctx, const PrefillArgs &a) {
+    const int64_t cus = std::max(1, ctx->cu_count), rows64 = ceil_div(a.M, 32 * a.terms), stages = ceil_div(a.K, kPK);
+    const int64_t most = ctx->tune.prefill_split == 0 ? 1 : std::max<int64_t>(1, std::min<int64_t>(4, stages / 32));   // (see prefill_plan)
+    const int64_t mid = rows64 * ceil_div(a.N, 128), large = SG <= 2 ? rows64 * ceil_div(a.N, 256) : ceil_div(a.M, 128) * ceil_div(a.N, 128);
+    if (mid <= cus / 2 && most < 3) return 64;
+    auto cost = [&](int64_t tiles) {
+        const int64_t ways = std::max<int64_t>(1, std::min(most, cus / tiles));
+        return ceil_div(tiles * ways, cus) * ceil_div(stages, ways);
+    };
+    return a.terms == 2 && 2 * 15 * cost(large) < 16 * cost(mid) ? 192 : 128;
+}
 template <int SG>
 int prefill_launch(hipc_ctx *ctx, const PrefillArgs &a) {
     const int forced = ctx->tune.prefill_tile, g_prefill_split = ctx->tune.prefill_split;
+    if (a.pair_rows > 0) return prefill_launch_terms(ctx, a, SG, forced == 64 || forced == 128 || forced == 192 ? forced : prefill_pair_tile<SG>(ctx, a));
     // 128-row tiles when they give every CU a workgroup, directly or (long k) with k split over up
     // to four workgroups per tile; else 64x64
     const int64_t rows128 = ceil_div(a.M, 128), tiles128 = rows128 * ceil_div(a.N, 128), tiles192 = rows128 * ceil_div(a.N, 192);
@@ -934,17 +997,21 @@ int nbits_prefill(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, void
 // lo = f16(a 2^-e - hi) (22 significant bits), with 2^e the row's own power of two that brings its
 // largest magnitude into [2^14, 2^15) -- exact, and no value of the row leaves the f16 range. The rows
 // are stored as A2[m] = hi, A2[M + m] = lo; one workgroup per row. PAIRED: 32 rows of high terms are followed by the
-// 32 rows of their low terms (row m: hi at 64 (m / 32) + m % 32, lo 32 rows on), the grid covers a multiple of 32
+// 32 rows of each further term (row m of two: hi at 64 (m / 32) + m % 32, lo 32 rows on), the grid covers a multiple of 32
 // rows and the rows past M are zeros.
-template <bool PAIRED, int TERMS = 2>   // TERMS 1: the high terms alone, M rows; 3: a third, rows 2 M + m (see split_terms)
+template <bool PAIRED, int TERMS = 2>   // TERMS 1: the high terms alone, M rows; 3: a third, unpaired in rows 2 M + m (see split_terms)
 static __global__ void __launch_bounds__(256)
 mmnb_prefill_split_rows_kernel(const float *__restrict__ A, int M, int K, __half *__restrict__ A2, int *__restrict__ exps) {
     __shared__ float red[4];
     const int m = blockIdx.x, tid = threadIdx.x;
-    const size_t hi_at = PAIRED ? (size_t)(64 * (m >> 5) + (m & 31)) : (size_t)m, lo_at = PAIRED ? hi_at + 32 : (size_t)M + m;
+    const size_t step = PAIRED ? 32 : (size_t)M;   // rows from a term to the next
+    const size_t hi_at = PAIRED ? (size_t)(32 * TERMS * (m >> 5) + (m & 31)) : (size_t)m, lo_at = hi_at + step;
     if (PAIRED && m >= M) {
-        uint4 *hi_row = reinterpret_cast<uint4 *>(A2 + hi_at * K), *lo_row = reinterpret_cast<uint4 *>(A2 + lo_at * K);
-        for (int c = tid; c < K / 8; c += 256) hi_row[c] = make_uint4(0u, 0u, 0u, 0u), lo_row[c] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int t = 0; t < TERMS; t++) {
+            uint4 *to = reinterpret_cast<uint4 *>(A2 + (hi_at + t * step) * K);
+            for (int c = tid; c < K / 8; c += 256) to[c] = make_uint4(0u, 0u, 0u, 0u);
+        }
         return;
     }
     const float4 *row = reinterpret_cast<const float4 *>(A + (size_t)m * K);   // (K is a multiple of 8 and A is aligned: see nbits_prefill_f32_takes)
@@ -982,7 +1049,7 @@ mmnb_prefill_split_rows_kernel(const float *__restrict__ A, int M, int K, __half
         };
         hi_row[c] = piece(0);
         if constexpr (TERMS >= 2) lo_row[c] = piece(1);
-        if constexpr (TERMS == 3) lo_row[c + (size_t)M * (K / 4)] = piece(2);
+        if constexpr (TERMS == 3) lo_row[c + step * (K / 4)] = piece(2);
     };
 #pragma unroll
     for (int u = 0; u < kHeld; u++)
@@ -1009,27 +1076,27 @@ mmnb_prefill_join_rows_kernel(const float *__restrict__ P, const int *__restrict
     }
 }
 
-// Many rows of f32 activations: each row as two f16 rows (22 bits) through the same tiled kernel. Twice the products
-// of the f16 case, against one pass over the whole weight per 16 rows on the decode kernel. With the kernel that
-// keeps the weight out of LDS the two terms of a row are the two row blocks of one wavefront, which adds them and
-// puts the rows' powers of two back itself; the kernel that stages both operands through LDS writes 2 M rows of f32
-// results and a last launch adds the pairs.
+// Many rows of f32 activations: each row as one to three f16 rows (11, 22 or all 24 bits) through the same tiled kernel, against
+// one pass over the whole weight per 16 rows on the decode kernel. With the kernel that keeps the weight out of LDS the terms
+// of a row are row blocks of one wavefront, which adds them and puts the rows' powers of two back itself; else the kernel
+// writes a row of f32 results per term and a last launch adds them.
 bool nbits_prefill_f32_takes(const void *A, const hipc_nbits_weight *w, int64_t M) {
-    return M > 32 && w->K % 8 == 0 && aligned(A, 16) && (3 * M + 64) * w->K < (int64_t(1) << 31) && 3 * M * w->N < (int64_t(1) << 31);
+    return M > 32 && w->K % 8 == 0 && aligned(A, 16) && (3 * M + 96) * w->K < (int64_t(1) << 31) && 3 * M * w->N < (int64_t(1) << 31);
 }
 
 namespace {
 // the exponents of M rows, padded, in front of the f16 rows
 size_t split_exps_bytes(int64_t M) { return ((size_t)M * sizeof(int) + 255) & ~(size_t)255; }
-// two terms: the pairs of the kernel that keeps the weight out of LDS; three (f32 pinned: all 24 bits), or the
-// kernel with both operands in LDS: `terms` M rows, and a launch that adds them
-bool split_paired(hipc_ctx *ctx, const hipc_nbits_weight *w, int terms) { return terms == 2 && (ctx->tune.prefill_direct != 0 || w->SG == 8); }
+// the kernel that keeps the weight out of LDS takes all terms of a row in one wavefront; for the kernel with both operands in
+// LDS, and for blocks of 16 (whose sums and scales would not fit the registers: 130 x 2048 x 2560 58.6 against 30.1 us): `terms`
+// M rows, and a launch that adds them
+bool split_paired(hipc_ctx *ctx, const hipc_nbits_weight *w, int terms) { return terms >= 2 && w->SG != 8 && ctx->tune.prefill_direct != 0; }
 }  // namespace
 size_t nbits_split_bytes(int64_t rows, int64_t M, int64_t K) { return (size_t)rows * K * sizeof(__half) + split_exps_bytes(M); }
 
 bool nbits_prefill_f32_fits(hipc_ctx *ctx, const hipc_nbits_weight *w, int64_t M, int terms) {
     const bool paired = split_paired(ctx, w, terms);
-    if (!scratch_fits(ctx, 2, nbits_split_bytes(paired ? 64 * ceil_div(M, 32) : terms * M, M, w->K))) return false;
+    if (!scratch_fits(ctx, 2, nbits_split_bytes(paired ? 32 * terms * ceil_div(M, 32) : terms * M, M, w->K))) return false;
     return terms == 1 || paired || scratch_fits(ctx, 3, (size_t)terms * M * w->N * sizeof(float));
 }
 
@@ -1055,14 +1122,16 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
         }
     }
     const bool paired = split_paired(ctx, w, terms);
-    const int64_t rows2 = paired ? 64 * ceil_div(M, 32) : terms * M;
+    const int64_t rows2 = paired ? 32 * terms * ceil_div(M, 32) : terms * M;
     void *split = nullptr, *sums = nullptr;
     if (int rc = scratch_get(ctx, 2, nbits_split_bytes(rows2, M, w->K), &split)) return rc;
     if (!paired)
         if (int rc = scratch_get(ctx, 3, (size_t)terms * M * w->N * sizeof(float), &sums)) return rc;
     __half *A2 = reinterpret_cast<__half *>(static_cast<char *>(split) + split_exps_bytes(M));
     int *exps = static_cast<int *>(split);
-    if (paired)
+    if (paired && terms == 3)
+        hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<true, 3>), dim3((unsigned)(rows2 / 3)), dim3(256), 0, ctx->stream, static_cast<const float *>(A), (int)M, (int)w->K, A2, exps);
+    else if (paired)
         hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<true, 2>), dim3((unsigned)(rows2 / 2)), dim3(256), 0, ctx->stream, static_cast<const float *>(A), (int)M, (int)w->K, A2, exps);
     else if (terms == 3)
         hipLaunchKernelGGL((mmnb_prefill_split_rows_kernel<false, 3>), dim3((unsigned)M), dim3(256), 0, ctx->stream, static_cast<const float *>(A), (int)M, (int)w->K, A2, exps);
@@ -1072,7 +1141,7 @@ int nbits_prefill_f32(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *w, 
     PrefillArgs a{};
     a.A = A2, a.Wq = w->Wq, a.Sc = w->Sc, a.Zb = w->Zb, a.Y = nullptr, a.Yf32 = static_cast<float *>(paired ? Y : sums);
     a.M = (int)rows2, a.K = (int)w->K, a.N = (int)w->N, a.n_tiles = w->n_tiles, a.n_cg = w->n_cg;
-    if (paired) a.exps = exps, a.pair_rows = (int)M;
+    if (paired) a.exps = exps, a.pair_rows = (int)M, a.terms = terms;
     int rc;
     switch (w->SG) {
         case 8: rc = prefill_launch<8>(ctx, a); break;

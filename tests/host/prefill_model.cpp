@@ -1,5 +1,5 @@
 // Address model of the tiled MatMulNBits kernels (many rows of f16 or f32 activations): matmul_nbits_prefill.hip,
-// compiled twice as the library does, with matmul_nbits.hip for the prepack and the operator's entry point, as host
+// compiled three times as the library does, with matmul_nbits.hip for the prepack and the operator's entry point, as host
 // code behind gpu_model.h. Every launch runs thread by thread on the CPU; the operands are allocations of exactly the
 // operator's sizes (no slack), and AddressSanitizer checks every load and store of every thread: the clamped rows
 // and tiles past the edges of ragged shapes, the stage past the end of an odd stage count, the k split's partials.

@@ -233,8 +233,8 @@ F32_PREFILL = [  # (M, K, N, block_size, zero points)
 ]
 
 
-F32_ROUTES = [  # the default; the two terms of a row as the two row blocks of a wavefront (128 x 128 and 128 x 192 tiles, two k
-    # groups per workgroup, k split over workgroups, a forced 64-row tile that such rows cannot take); the kernel
+F32_ROUTES = [  # the default; the two terms of a row in one accumulator (64 x 128 tiles and the larger ones, two k
+    # groups per workgroup, k split over workgroups, 64 x 64 tiles); the kernel
     # with both operands in LDS, whose 2 M result rows a last launch adds up
     {}, {"HIPC_PREFILL_TILE": 128}, {"HIPC_PREFILL_TILE": 192}, {"HIPC_PREFILL_TILE": 128, "HIPC_PREFILL_GROUPS": 2},
     {"HIPC_PREFILL_TILE": 128, "HIPC_PREFILL_SPLIT": 2}, {"HIPC_PREFILL_TILE": 192, "HIPC_PREFILL_GROUPS": 2, "HIPC_PREFILL_SPLIT": 2},
@@ -333,6 +333,32 @@ def test_f32_rows_with_f32_pinned(ctx, pkg, oracle, shape, options):
     assert e3.max() <= 2e-5, float(e3.max())
     assert e3.max() <= e2.max() * 1.05 + 1e-7, (float(e3.max()), float(e2.max()))
     assert np.all(got[2] == 0)
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("tile", [64, 128, 192])
+@pytest.mark.parametrize("level", [0, 1])
+@pytest.mark.parametrize("shape", [(33, 70, 70, 32, True), (64, 128, 128, 32, False), (65, 448, 129, 64, True), (97, 1100, 257, 128, False), (129, 576, 300, 256, True)],
+                         ids=lambda s: "M%d_K%d_N%d_bs%d_zp%d" % s)
+def test_terms_of_f32_rows_added_in_one_accumulator(ctx, pkg, shape, level, tile, groups):
+    """Every tile that holds the two (level 1: three) f16 terms of its f32 rows in one wavefront, with one k group per workgroup
+    and with several: rows and columns one past a tile, fewer stages than groups, a partial last stage. Against float64:
+    what the terms leave of a row's largest value times the column's absolute sum, and f32 accumulation over k."""
+    m, k, n, bs, with_zp = shape
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=47, with_zp=with_zp)
+    a = pkg.synth.normal_f32(m * k, 48).reshape(m, k)
+    a[m - 1] *= np.float32(1.0e7)
+    nib, z = _unpack(B, zp if zp is not None else np.full((n, (-(-k // bs) + 1) // 2), 0x88, np.uint8), k, n, bs)
+    f64 = rc.matmul_nbits_f64(a, nib, z, scales.reshape(n, -1), bs)
+    absw = rc.matmul_nbits_f64(np.ones((1, k)), np.abs(nib.astype(np.int64) - z.repeat(bs, axis=1)[:, :k]), np.zeros_like(z), scales.reshape(n, -1), bs)
+    absy = rc.matmul_nbits_f64(np.abs(a), np.abs(nib.astype(np.int64) - z.repeat(bs, axis=1)[:, :k]), np.zeros_like(z), scales.reshape(n, -1), bs)
+    bound = np.abs(a).max(axis=1, keepdims=True).astype(np.float64) * 2.0 ** (-24 if level else -21) * absw + (k + 8) * 2.0 ** -24 * absy
+    w = pkg.ops.NBitsWeight(ctx, B, scales, zp, k, n, bs)
+    with ctx.options(HIPC_PREFILL_TILE=tile, HIPC_PREFILL_GROUPS=groups):
+        got = pkg.ops.matmul_nbits(ctx, a, None, None, None, k, n, bs, accuracy_level=level, weight=w)
+    w.destroy()
+    assert got.dtype == np.float32 and got.shape == (m, n)
+    assert np.all(np.abs(got - f64) <= bound), float(np.max(np.abs(got - f64) / bound))
 
 
 @pytest.mark.parametrize("kn", [(2048, 11008), (11008, 2048), (2048, 2560)], ids=lambda s: "K%d_N%d" % s)
