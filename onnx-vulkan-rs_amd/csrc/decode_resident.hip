@@ -973,6 +973,15 @@ bool hipc::resident_takes(const hipc_decoder_config &c) {
            (c.n_q_heads + 2 * c.n_kv_heads) * c.head_dim <= (int)kResMaxQkv && c.hidden % 16 == 0 && c.hidden <= (int)kResMaxHidden && c.ffn % 16 == 0 && cg_f <= 64;
 }
 
+// One launch against five per layer (8 layers, a token, us): the 256 workgroups read each query head's positions themselves
+// (no more than 8 / heads parts of them), where the attention launch spreads them over as many workgroups as it likes. Heads
+// times positions decide, whatever the other sizes are: hidden 256 to 2048 and 4 heads win at every position that was measured
+// (1152 / 6912 / 4 heads of 256: 130.8 against 179.8 at 100, 143.2 / 191.0 at 2048, 306.6 / 335.3 at 32000; 256 / 1024 / 4 heads of 64:
+// 109.1 / 136.6, 117.5 / 144.1, 198.1 / 206.6), 8 heads up to about 12000 (2048 / 8192 / 8 of 256: 175.9 / 232.1 at 100, 263.0 /
+// 280.8 at 8192, 342.9 / 325.2 at 16384, 517.5 / 390.0 at 32000). The position is the device's and a recorded step covers all of
+// them, so the rule is on the longest one: at 8 heads x 16384 the last quarter loses 5 %, the rest gains 7 to 32 %.
+bool hipc::resident_pays(const hipc_decoder_config &c) { return (int64_t)c.n_q_heads * c.max_seq <= 8 * 16384; }
+
 namespace {
 
 template <int HD, bool ALL>

@@ -126,6 +126,29 @@ def test_attention_over_a_long_filled_cache(ctx, pkg, oracle, route, hd, nq, nkv
     dec.destroy()
 
 
+@pytest.mark.parametrize("nq,max_seq", [(8, 16384), (8, 16385), (4, 32768), (4, 32769)])
+def test_the_longest_context_that_keeps_all_layers_in_one_launch(ctx, pkg, route, nq, max_seq):
+    """Heads times positions choose between one launch and the launches per product: the last length of each side at its
+    last positions, against the launches per product over the same cache."""
+    cfg = dict(SMALL, n_q_heads=nq, n_kv_heads=1, head_dim=64)
+    w = pkg.decoder.build_weights(cfg, seed=14)
+    rng = np.random.default_rng(nq)
+    rows = [tuple((rng.standard_normal((1, max_seq, 64)) * 0.7).astype(np.float16) for _ in range(2)) for _ in range(cfg["n_layers"])]
+    got = []
+    for resident in (-1, 0):
+        route({"HIPC_DEC_RESIDENT": resident})
+        dec = pkg.decoder.Decoder(ctx, cfg, max_seq)
+        dec.load(w)
+        for li, (k_rows, v_rows) in enumerate(rows):
+            dec.fill_cache(li, k_rows, v_rows)
+        dec.reset(29, max_seq - 1)
+        dec.step()
+        got.append(dec.read(want_logits=True))
+        dec.destroy()
+    assert got[0][1] == got[1][1] == max_seq
+    assert np.all(np.abs(got[0][2] - got[1][2]) <= 2e-3 + 2e-3 * np.abs(got[1][2])), float(np.abs(got[0][2] - got[1][2]).max())
+
+
 WINDOWS = [  # (head_dim, query heads, kv heads, first position, window of layer 0, window of layer 1)
     (256, 4, 1, 2300, 512, 0),     # gemma3's local window beside a global layer
     (128, 4, 2, 509, 512, 100),    # the window starts to mask at 512 positions, i.e. during these steps
