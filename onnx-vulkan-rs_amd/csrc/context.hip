@@ -115,6 +115,7 @@ const OptionName kOptions[] = {
     {"HIPC_GEMV_LEAN", &Tuning::gemv_lean},
     {"HIPC_DEC_LEAN", &Tuning::dec_lean},
     {"HIPC_DEC_RESIDENT", &Tuning::dec_resident},
+    {"HIPC_DQL_WAIT", &Tuning::dql_wait},
     {"HIPC_DEC_PREFETCH", &Tuning::dec_prefetch},
 };
 

@@ -15,13 +15,15 @@
 #include <type_traits>
 
 #include "internal.h"
+#include "lanes.h"
 
 namespace hipc {
 
-// up to how many values dql_small_kernel takes: where its repeated reads (of a GELU: evaluations) cost what a second launch
-// does (feed-forward block of 32 tokens of 1024: 26.0 -> 23.4 us, of 60: 28.7 -> 29.5; of 4 tokens through a GELU of 4 x
-// 4096: 25.0 -> 19.1, of 8: 25.0 -> 24.4)
-constexpr int64_t kSmallPlain = 40960, kSmallGelu = 16384;
+// Up to how many values dql_small_kernel, whose every workgroup reads (of a GELU: evaluates) all of them, beats the launch whose
+// workgroups tell each other their ranges. Us, both: 32768 values 4.04 / 4.62, 40960 4.36 / 4.62, 65536 5.7 / 4.65; of a GELU
+// 4097 4.31 / 4.9, 6000 4.59 / 4.9, 8192 5.1 / 5.0, 16384 6.7 / 5.0.
+constexpr int64_t kSmallPlain = 40960, kSmallGelu = 6144;
+constexpr long kMeetTicks = 5000;   // 50 us: several times what the workgroups of a launch are apart on a chip of their own
 
 
 // Range partials of hipc_dynamic_quantize_linear_static: {bits(-min), bits(max)} per workgroup of
@@ -260,9 +262,8 @@ dql_quantize_kernel(const float *__restrict__ x, long n, const uint32_t *__restr
     }
 }
 
-// Few values: one launch instead of two. Every workgroup takes the range of all of them and quantizes its own 4096; what
-// that reads again comes from the caches and costs less than the second launch, whose 1.6 us (2.2 us of the host's time)
-// nothing hides.
+// Few values: every workgroup takes the range of all of them and quantizes its own 4096; what that reads again comes from the
+// caches and costs less than a second launch (1.6 us, 2.2 us of the host's time) or telling each other (1.3 us).
 template <int GELU>
 __global__ void __launch_bounds__(1024)
 dql_small_kernel(const float *__restrict__ x, long n, uint8_t *__restrict__ y, float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, GeluParams g) {
@@ -305,6 +306,146 @@ dql_small_kernel(const float *__restrict__ x, long n, uint8_t *__restrict__ y, f
     }
 }
 
+// All of it in one launch, for as many values as the chip's registers hold: 1024 threads keep V runs of four values each, through
+// the GELU where there is one, publish the workgroup's range, wait for the ranges of all workgroups and quantize what they hold.
+// Every value is read once and every GELU taken once; two launches do both twice. As few runs per thread as 256 workgroups
+// allow, since waiting for 256 costs little more than for 64: 1 M values 5.2 us with one run, 5.3, 5.9 and 7.8 with two, four
+// and eight. What bounds it: 1 M values the launch, the trip for the values and the two of the hand-over (5.2 us of which 1 us
+// is the copy's time), 4 M through a GELU its instructions (4.8 of 9.1 us), 8 M the memory (9.4 us, 4.5 TB/s). Against two
+// launches, us: 64 K values 4.65 / 4.8, 1 M 5.2 / 6.0, 4 M 6.6 / 8.7, 8 M 9.4 / 18.0, 16 M 18.9 / 30.4; through a GELU 16 K 5.0 / 5.6,
+// 1 M 5.6 / 7.3, 4 M 9.1 / 13.8, 8 M 14.5 / 26.2, 16 M 28.2 / 41.3.
+//
+// The ranges are published eight times over and each workgroup reads one copy with one wavefront: all 256 workgroups polling
+// one copy with four wavefronts each took 8 us for what takes one.
+//
+// No workgroup depends on the others being on the chip with it. One that has waited `ticks` says so and leaves; the workgroup
+// that publishes last finds all ranges there, and then quantizes for those that left. (A workgroup that leaves looks once more
+// after it has said so: either it finds all ranges, or the last one publishes, and looks for leavers, after that. Both may
+// write the same values; no other order is possible.)
+//
+// A call uses one of two sets of words, empties the other, which nobody reads any more, and then makes that the next call's.
+#ifndef HIPC_HOST_MODEL
+__device__ __forceinline__ void dql_stored() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }   // this wavefront's stores are where everyone sees them
+__device__ __forceinline__ long dql_now() { return (long)wall_clock64(); }
+#else   // (threads of the address model run one after the other: nobody waits)
+inline void dql_stored() {}
+inline long dql_now() { return 0; }
+#endif
+constexpr uint64_t kThere = 0x8000000080000000ull;
+__device__ __forceinline__ void dql_put(uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <int GELU, int V>
+__global__ void __launch_bounds__(1024)
+dql_once_kernel(const float *__restrict__ x, long n, uint32_t *meet, uint8_t *__restrict__ y, float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, long ticks, GeluParams g) {
+    HIPC_PIN_SGPR(ticks);   // (read with the first arguments, not when the waiting begins)
+    __shared__ float slow[16], shigh[16];
+    __shared__ uint32_t joined[2];
+    __shared__ int seen[2];   // all ranges; at the first look
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, groups = gridDim.x;
+    // the 4096 values of run `r` of a workgroup, four to a thread
+    auto load = [&](long r) {
+        const float *xr = x + r * 4096;
+        const int count = (int)max(min(n - r * 4096, 4096l), 0l), base = 4 * tid;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (__builtin_expect(base + 4 <= count, 1)) {
+            v = reinterpret_cast<const float4 *>(xr)[tid];
+        } else {
+            if (base < count) v.x = xr[base];
+            if (base + 1 < count) v.y = xr[base + 1];
+            if (base + 2 < count) v.z = xr[base + 2];
+        }
+        return v;
+    };
+    auto store = [&](long r, uint32_t w) {
+        uint8_t *yr = y + r * 4096;
+        const int count = (int)max(min(n - r * 4096, 4096l), 0l), base = 4 * tid;
+        if (__builtin_expect(base + 4 <= count, 1)) {
+            reinterpret_cast<uint32_t *>(yr)[tid] = w;
+        } else {
+            for (int j = 0; j < 3; j++)
+                if (base + j < count) yr[base + j] = (uint8_t)(w >> (8 * j));
+        }
+    };
+    const long first = (long)blockIdx.x * V;
+    float4 v[V];
+#pragma unroll
+    for (int u = 0; u < V; u++) v[u] = load(first + u);
+    const uint32_t set = __builtin_amdgcn_readfirstlane(meet[0]) & 1u;   // (asked for behind the values)
+    uint32_t *here = meet + 64 + set * (kMeetSet / 4), *other = meet + 64 + (set ^ 1u) * (kMeetSet / 4);
+    float mn = 0.f, mx = 0.f;
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+        v[u] = gelu_load4<GELU>(v[u], g);
+        mn = fminf(mn, fminf(fminf(v[u].x, v[u].y), fminf(v[u].z, v[u].w)));
+        mx = fmaxf(mx, fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w)));
+    }
+    float low = lean_wave_max(-mn), high = lean_wave_max(mx);
+    if (lane == 0) slow[wave] = low, shigh[wave] = high;
+    __syncthreads();
+    uint64_t *copies = reinterpret_cast<uint64_t *>(here);
+    uint32_t *gone = here + 2 * kMeetMax * kMeetCopies;
+    if (tid < kMeetCopies) {
+#pragma unroll
+        for (int w = 0; w < 16; w++) low = fmaxf(low, slow[w]), high = fmaxf(high, shigh[w]);
+        // (the sign bits, which a range does not need, say that it is there; -0.0 counts as 0)
+        const uint64_t pair = ((uint64_t)(__float_as_uint(low) | 0x80000000u) << 32) | (__float_as_uint(high) | 0x80000000u);
+        __hip_atomic_store(copies + tid * kMeetMax + blockIdx.x, pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (wave == 0) dql_stored();
+    const uint64_t *mine = copies + (blockIdx.x % kMeetCopies) * kMeetMax;
+    int first_look = 0;
+    auto look = [&](long wait) -> bool {   // are all ranges there, within `wait`?
+        if (wave == 0) {
+            uint64_t pair[kMeetMax / 64];
+            bool all;
+            const long t0 = dql_now();
+            for (first_look = 1;; first_look = 0) {
+                bool there = true;
+#pragma unroll
+                for (int q = 0; q < kMeetMax / 64; q++) {
+                    pair[q] = kThere;
+                    if (lane + 64 * q < groups) pair[q] = __hip_atomic_load(mine + lane + 64 * q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int q = 0; q < kMeetMax / 64; q++) there &= (pair[q] & kThere) == kThere;
+                all = __all(there);
+                if (all || dql_now() - t0 >= wait) break;
+            }
+            low = high = 0.f;
+#pragma unroll
+            for (int q = 0; q < kMeetMax / 64; q++)
+                low = fmaxf(low, __uint_as_float((uint32_t)(pair[q] >> 32) & 0x7fffffffu)), high = fmaxf(high, __uint_as_float((uint32_t)pair[q] & 0x7fffffffu));
+            low = lean_wave_max(low), high = lean_wave_max(high);
+            if (lane == 0) joined[0] = __float_as_uint(low), joined[1] = __float_as_uint(high), seen[0] = all, seen[1] = first_look;
+        }
+        __syncthreads();
+        return seen[0];
+    };
+    if (__builtin_expect(!look(ticks), 0)) {
+        if (tid == 0) dql_put(gone + blockIdx.x, 1u), dql_stored();
+        __syncthreads();
+        if (!look(0)) return;
+    }
+    float scale, zp;
+    dql_params(joined, scale, zp);
+    const float rcp = dql_rcp(scale);
+    // workgroup 0, or who does its part, tells the scale and makes the other set the next call's
+    auto once = [&] {
+        for (int i = tid; i < (int)(kMeetSet / 16); i += 1024) reinterpret_cast<uint4 *>(other)[i] = make_uint4(0, 0, 0, 0);
+        if (tid == 0) *meet = set ^ 1u, *scale_out = scale, *zp_out = (uint8_t)zp;
+    };
+    if (blockIdx.x == 0) once();
+    const int left = (int)__hip_atomic_load(gone + min(tid, kMeetMax - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (0 behind the last workgroup's)
+#pragma unroll
+    for (int u = 0; u < V; u++) store(first + u, dql_four(v[u], scale, rcp, zp));
+    if (__builtin_expect(!seen[1] || !__syncthreads_or(left), 1)) return;
+    for (int i = 0; i < groups; i++) {
+        if (i == (int)blockIdx.x || !__syncthreads_or(tid == i ? left : 0)) continue;
+        if (i == 0) once();
+#pragma unroll 1
+        for (int u = 0; u < V; u++) store((long)i * V + u, dql_four(gelu_load4<GELU>(load((long)i * V + u), g), scale, rcp, zp));
+    }
+}
+
 __global__ void dql_empty_kernel(float *scale_out, uint8_t *zp_out) {
     if (threadIdx.x == 0) {
         *scale_out = 1.f;
@@ -342,6 +483,25 @@ int dql_launch(hipc_ctx *ctx, const void *X, int64_t n, void *Y, void *scale_out
         if (!range_ready && !range && vec_ok && n <= (GELU ? kSmallGelu : kSmallPlain)) {
             hipLaunchKernelGGL((dql_small_kernel<GELU>), (unsigned)ceil_div(n, 4096), 1024, 0, ctx->stream, x, (long)n, static_cast<uint8_t *>(Y),
                                static_cast<float *>(scale_out), static_cast<uint8_t *>(zp_out), gelu);
+            HIPC_LAUNCHED(ctx);
+            return HIPC_OK;
+        }
+        // one launch while a workgroup per CU holds all values (16 runs of four per thread at most: 107 registers of the 128
+        // that 1024 threads may have); the forms that must not use the context's memory, and unaligned tensors, keep two
+        const int64_t groups = std::min<int64_t>(ctx->cu_count, kMeetMax);
+        if (!range_ready && !range && !parts && vec_ok && n <= groups * 16 * 4096 && ctx->tune.dql_wait != 0) {
+            const long ticks = ctx->tune.dql_wait > 0 ? ctx->tune.dql_wait : kMeetTicks;
+            auto once = [&](auto runs) {
+                constexpr int V = decltype(runs)::value;
+                hipLaunchKernelGGL((dql_once_kernel<GELU, V>), (unsigned)ceil_div(n, 4096 * V), 1024, 0, ctx->stream, x, (long)n,
+                                   reinterpret_cast<uint32_t *>(static_cast<char *>(ctx->params) + kParamMeet), static_cast<uint8_t *>(Y), static_cast<float *>(scale_out),
+                                   static_cast<uint8_t *>(zp_out), ticks, gelu);
+            };
+            if (n <= groups * 4096) once(std::integral_constant<int, 1>{});
+            else if (n <= groups * 2 * 4096) once(std::integral_constant<int, 2>{});
+            else if (n <= groups * 4 * 4096) once(std::integral_constant<int, 4>{});
+            else if (n <= groups * 8 * 4096) once(std::integral_constant<int, 8>{});
+            else once(std::integral_constant<int, 16>{});
             HIPC_LAUNCHED(ctx);
             return HIPC_OK;
         }

@@ -72,6 +72,7 @@ struct Tuning {
     int gemv_lean = -1;       // HIPC_GEMV_LEAN      0: one-row products keep the streaming GEMV kernel
     int dec_lean = -1;        // HIPC_DEC_LEAN       0: the decoder keeps the streaming GEMV and its prologues (read when a decoder is created)
     int dec_resident = -1;    // HIPC_DEC_RESIDENT   0: the decoder keeps a launch per product (read when a decoder is created, too); n: workgroups of the launch that holds all layers
+    int dql_wait = -1;        // HIPC_DQL_WAIT       0: DynamicQuantizeLinear never in one launch of several workgroups; n: how long these wait for each other, in 10 ns
     int dec_prefetch = -1;    // HIPC_DEC_PREFETCH   bits: which launches of a layer carry helper rows that read ahead for the next launch (0 none, 31 all; see hipc_decoder_step)
 };
 
@@ -499,6 +500,12 @@ int nbits_rows_f32_split(hipc_ctx *ctx, const void *A, const hipc_nbits_weight *
 constexpr size_t kParamRange = 0;   // 8 B  {bits(-min), bits(max)}
 constexpr size_t kParamParts = 256; // 16 KiB: per-workgroup {bits(-min), bits(max)} pairs of DynamicQuantizeLinear
 constexpr int kParamPartsMax = 2048;
-constexpr size_t kParamBytes = 256 + 8 * kParamPartsMax;
+// DynamicQuantizeLinear in one launch: the word that says which of two sets a call uses, and the sets: {max, -min} bits of each
+// workgroup (8 B), a copy for every eighth of the workgroups to read, and behind them a word per workgroup that gave up waiting.
+// All zero when no call runs but for one set.
+constexpr int kMeetMax = 256, kMeetCopies = 8;
+constexpr size_t kParamMeet = kParamParts + 8 * kParamPartsMax;
+constexpr size_t kMeetSet = (8 * kMeetCopies + 4) * kMeetMax;
+constexpr size_t kParamBytes = kParamMeet + 256 + 2 * kMeetSet;
 
 }  // namespace hipc

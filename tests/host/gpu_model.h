@@ -186,6 +186,17 @@ inline uint32_t __float_as_uint(float f) { uint32_t u; std::memcpy(&u, &f, 4); r
 inline float __expf(float v) { return std::exp(v); }
 inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xffffffu) * (b & 0xffffffu); }
 inline int __any(int v) { return v; }
+inline int __all(int) { return 1; }   // (what a wavefront would wait for counts as there: threads run one after the other)
+inline int __syncthreads_or(int v) { return v; }
+#ifndef __HIP_MEMORY_SCOPE_AGENT
+#define __HIP_MEMORY_SCOPE_AGENT 4
+#endif
+template <typename T>
+inline void gpu_model_atomic_store(T *p, T v) { *p = v; }
+template <typename T>
+inline T gpu_model_atomic_load(const T *p) { return *p; }
+#define __hip_atomic_store(p, v, order, scope) gpu_model_atomic_store(p, v)
+#define __hip_atomic_load(p, order, scope) gpu_model_atomic_load(p)
 inline float rsqrtf(float v) { return 1.f / std::sqrt(v); }
 inline float __fmul_rn(float a, float b) { return a * b; }
 inline float __fdiv_rn(float a, float b) { return a / b; }

@@ -168,7 +168,7 @@ int main(int argc, char **argv) {
     ctx.params = gpu_model::alloc(hipc::kParamBytes);
     ctx.cu_count = 256;
     MUST(hipc::dql_static_init(&ctx));
-    for (int64_t n : {0, 1, 3, 4, 5, 255, 256, 257, 1000, 4096, 4099, 65536 + 7, 1000 * 1024})
+    for (int64_t n : {0, 1, 3, 4, 5, 255, 256, 257, 1000, 4096, 4099, 65536 + 7, 1000 * 1024, 8 * 256 * 4096 + 5})
         for (int misalign : {0, 4}) quantize(n, misalign);
     report("DynamicQuantizeLinear and the decomposed GELU");
     // matrix products: tiny, ragged in every direction, aligned, one tile more than a multiple, both signs

@@ -139,9 +139,9 @@ def test_fused_gelu_quantization_of_nothing_and_bad_constants(ctx, pkg):
         pkg.ops.decomposed_gelu(ctx, np.ones(4, np.float32), divisor=0.0)
 
 
-@pytest.mark.parametrize("n", [1, 3, 4095, 4097, 16383, 16384, 16386, 40959, 40960, 40961, 262144 * 4 + 5])
+@pytest.mark.parametrize("n", [1, 3, 4095, 4097, 6144, 6145, 16383, 16384, 16386, 40959, 40960, 40961, 262144 * 4 + 5])
 def test_sizes_around_the_launch_forms(ctx, pkg, oracle, n):
-    """One launch up to 40960 values (16384 through a GELU), two behind it, sixteen values per thread from a million on:
+    """One launch that reads everything up to 40960 values (6144 through a GELU), one of many workgroups behind it:
     the last size of each form and the first of the next; divisors the quotient of which is formed either way."""
     x = pkg.synth.normal_f32(n, 91)
     y, s, z = pkg.ops.dynamic_quantize_linear(ctx, x)
@@ -151,6 +151,49 @@ def test_sizes_around_the_launch_forms(ctx, pkg, oracle, n):
         y, s, z = pkg.ops.dynamic_quantize_linear_gelu(ctx, x, divisor)
         wy, ws, wz = pkg.ops.dynamic_quantize_linear(ctx, pkg.ops.decomposed_gelu(ctx, x, divisor))
         assert np.array_equal(y, wy) and s == ws and z == wz
+
+
+@pytest.mark.parametrize("wait", [-1, 1], ids=["default", "nobody-waits"])
+@pytest.mark.parametrize("n", [40963, 4096 * 255 + 1, 4096 * 256, 4096 * 256 + 1, 2 * 4096 * 256 + 2, 4 * 4096 * 256 + 3, 8 * 4096 * 256 + 4, 16 * 4096 * 256])
+def test_one_launch_of_many_workgroups_equals_two_launches(pkg, n, wait):
+    """Each number of values a thread holds, at its largest size and one past the one before, byte for byte the two launches'
+    result; with workgroups that wait for the others and with ones that leave their part to the last; the range set by the
+    last, by the first and by a value in the middle, infinities and NaN; again from replays with other sizes between them."""
+    ctx = pkg.Context(0)
+    x = pkg.synth.normal_f32(n, 93)
+    x[n - 1], x[0] = 9.0, -7.0
+    special = x.copy()
+    special[n // 2], special[n // 3] = np.inf, np.nan
+    for values in (x, special):
+        d_x, d_y, d_q = ctx.upload(values), ctx.alloc(n + 8), ctx.alloc(16)
+        results = []
+        for w in (0, wait):
+            ctx.set_option("HIPC_DQL_WAIT", w)
+            for gelu in (False, True):
+                def call(count=n):
+                    if gelu:
+                        ctx._check(ctx.lib.hipc_dynamic_quantize_linear_gelu(ctx.handle, d_x.ptr, count, pkg.ops.SQRT2_F32, 1.0, 0.5, 0, d_y.ptr, d_q.ptr, d_q.ptr + 4, None))
+                    else:
+                        pkg.ops.dynamic_quantize_linear_device(ctx, d_x, count, d_y, d_q, d_q.at(4))
+                read = lambda: (ctx.download(d_y, np.uint8, (n,)), ctx.download(d_q, np.uint8, (5,)))
+                ctx.fill(d_y, 0, n // 4 * 4, 0xAAAAAAAA)
+                call()
+                results.append(read())
+                if w:
+                    ctx.capture_begin()
+                    call(n - 5000), call()
+                    graph = ctx.capture_end()
+                    for _ in range(3):
+                        ctx.fill(d_y, 0, n // 4 * 4, 0xAAAAAAAA)
+                        call(30000)
+                        ctx.graph_launch(graph)
+                        again = read()
+                        assert np.array_equal(again[0], results[-1][0]) and np.array_equal(again[1], results[-1][1])
+                    ctx.graph_destroy(graph)
+        for plain in (0, 1):
+            assert np.array_equal(results[plain][1], results[plain + 2][1])
+            assert np.array_equal(results[plain][0], results[plain + 2][0])
+    ctx.close()
 
 
 @pytest.mark.parametrize("scale", [1e-38, 2.0 ** -101, 2.0 ** -99, 1.0, 2.0 ** 99, 2.0 ** 101, 1e38])
