@@ -462,7 +462,10 @@ struct RowsPlan {
 // How many columns a workgroup takes and how many ways k is split over workgroups. A CU takes in about 32 bytes per clock
 // (17.7 TB/s of L2 over 256 CUs), of rows and of weight alike: few columns per workgroup read the rows often, many leave
 // CUs without work, the code of a tile's products is fetched by an empty instruction cache (600 clocks per row block and
-// column tile: 24 x 2048 x 8320 9.2 us without that term, 7.6 with it), and a split costs a second launch, some 6000 clocks with its own trip through memory.
+// column tile: 24 x 2048 x 8320 9.2 us without that term, 7.6 with it), and a split costs a second launch: 3000 clocks with
+// its own trip through memory, most of the launch's 2.4 us hiding behind the first one's last workgroups. (Counted as 6000, the
+// rule kept 2 x 11008 x 1024 and x 2048 whole: 8.8 and 9.7 us, 6.6 and 7.8 split; counted as 2000, it splits 2 x 8192 x 512 and 20 x 2048 x 1024
+// for 8 % more, called one by one. Joining in the workgroup that comes last instead of a launch: 7.6 us for the 6.8 of 8 x 6912 x 1152.)
 bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT, int RB, int NR, bool may_split, RowsPlan *best) {
     const int cus = std::max(1, ctx->cu_count), max_waves = kRowsWaves;
     const int most_splits = may_split ? std::min(w->n_cg, std::max(16, (int)ceil_div(w->n_cg, 8))) : 1;   // (up to eight tiles of k fit any launch)
@@ -506,7 +509,7 @@ bool rows_plan(hipc_ctx *ctx, const hipc_nbits_weight *w, int M, int src, int NT
             const double row_bytes = (double)M * st * 128 * (src == SRC_F32 ? 4 : 2 * NT), weight_bytes = (double)cw * st * (1024 + 80 * w->SG);
             const double rounds = (double)ceil_div(wgs, cus * resident), per_cu = (double)std::min<int64_t>(resident, ceil_div(wgs, cus));
             double cost = 600.0 * RB * pl.T + (pl.loops ? per_cu * row_bytes / 32 + 2500 + rounds * (per_cu * weight_bytes / 32 + 800) : rounds * (per_cu * (row_bytes + weight_bytes) / 32 + 2500));
-            if (splits > 1) cost += 6000 + (double)splits * M * w->N * 8 / (32.0 * cus);
+            if (splits > 1) cost += 3000 + (double)splits * M * w->N * 8 / (32.0 * cus);
             if (!found || cost < best_cost) found = true, best_cost = cost, *best = pl;
         }
     }
