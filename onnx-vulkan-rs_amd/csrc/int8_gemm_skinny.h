@@ -6,8 +6,8 @@
 // workgroup owns 16 or 32 columns -- 64 to 256 workgroups for the usual widths -- and its 4 to 16 wavefronts share out k:
 // each asks for everything it will multiply at once (up to four 64-k steps in flight), both operands straight into the
 // operand registers of v_mfma_i32_16x16x64_i8 -- the fragment-major weight in 256-byte runs, A's rows in 64-byte pieces
-// -- and the partial sums meet in LDS. No stages, one barrier. Rows are taken 16 at a time (RB blocks), so one row costs
-// a quarter of what the 64x64 tile's A costs in load instructions.
+// -- and the partial sums meet in LDS. No stages, one barrier. Rows are taken 16 at a time (RB blocks to a workgroup, and
+// as many workgroups along the rows as it takes), so one row costs a quarter of what the 64x64 tile's A costs in load instructions.
 //
 // Measured (whole call, before -> after): see launch_mm_skinny.
 #pragma once
@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(1024) int8_gemm_skinny_kernel(const GemmArgs p
     const int i16 = lane & 15, kg = lane >> 4;
     i32x4 *red = reinterpret_cast<i32x4 *>(lds_raw);   // [wavefronts][RB][CB][64]: a lane's four rows of its column
     int *lds_sum = reinterpret_cast<int *>(red + waves * (RB * CB * 64));   // [wavefronts][16 RB]
-    const int j0 = blockIdx.x * 16 * CB;
+    const int j0 = blockIdx.x * 16 * CB, i0 = blockIdx.y * 16 * RB;
     const int steps = p.K_pad / 64;
 
     const __amdgpu_buffer_rsrc_t rsrc_p = __builtin_amdgcn_make_buffer_rsrc(
@@ -37,7 +37,7 @@ __global__ void __launch_bounds__(1024) int8_gemm_skinny_kernel(const GemmArgs p
         const_cast<uint8_t *>(p.Q), 0, (int)((uint32_t)((p.J + kBN - 1) / kBN * kBN) * (uint32_t)p.K_pad), 0x00020000);
     uint32_t a_row[RB], q_off[CB];
 #pragma unroll
-    for (int i = 0; i < RB; i++) a_row[i] = (uint32_t)min(i * 16 + i16, p.I - 1) * (uint32_t)p.lda;   // rows past I: clamped, never stored
+    for (int i = 0; i < RB; i++) a_row[i] = (uint32_t)min(i0 + i * 16 + i16, p.I - 1) * (uint32_t)p.lda;   // rows past I: clamped, never stored
 #pragma unroll
     for (int j = 0; j < CB; j++) q_off[j] = qfrag_offset(j0 + j * 16 + i16, kg * 16, p.K_pad);         // B is packed in whole 128-column tiles
 
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(1024) int8_gemm_skinny_kernel(const GemmArgs p
     const bool words = EPI == EPI_REQUANT && ((p.J | (int)(reinterpret_cast<uintptr_t>(p.Y) & 3)) & 3) == 0;   // bytes leave four columns at a time
     const RequantBytes bytes{ecol.s, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
     for (int f = wave; f < RB * CB; f += waves) {   // (waves is a multiple of CB: the column block stays)
-        const int row = (f / CB) * 16 + kg * 4;
+        const int own = (f / CB) * 16 + kg * 4, row = i0 + own;   // (own: of this workgroup's rows)
         if (row - kg * 4 >= p.I) break;
         i32x4 v = {fixed, fixed, fixed, fixed}, sum = {0, 0, 0, 0};
         for (int w = 0; w < waves; w += 4) {        // (and of 4)
@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(1024) int8_gemm_skinny_kernel(const GemmArgs p
             v += (part[0] + part[1]) + (part[2] + part[3]);
             if (DYN) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) sum += *reinterpret_cast<const i32x4 *>(lds_sum + (w + e) * (RB * 16) + row);
+                for (int e = 0; e < 4; e++) sum += *reinterpret_cast<const i32x4 *>(lds_sum + (w + e) * (RB * 16) + own);
             }
         }
         if (DYN) v -= zc * sum;

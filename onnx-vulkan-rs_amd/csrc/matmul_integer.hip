@@ -282,7 +282,7 @@ int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {
     while (waves < 16 && waves * kSkinnyAhead < steps) waves *= 2;
     static bool lds_allowed[2][kMaxDevices] = {};
     const size_t lds = skinny_lds(waves, RB, cb);
-    const dim3 grid((unsigned)ceil_div(cols16, cb));
+    const dim3 grid((unsigned)ceil_div(cols16, cb), (unsigned)ceil_div(g.I, 16 * RB));
     const void *with_sums = nullptr;
     if (!DYN && ctx->capturing) {
         static bool sums_allowed[2][kMaxDevices] = {};
@@ -303,13 +303,20 @@ int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {
     return HIPC_OK;
 }
 // Up to 64 rows. Kernel alone, against the k-split 64x64 tiles (which are ahead of the LDS-staged ones there): 1 x 1024 x
-// 1024 6.4 -> 2.9 us, 1 x 4096 x 4096 11.4 -> 5.1, 23 x 1024 x 4096 6.6 -> 3.7, 23 x 4096 x 1024 11.1 -> 6.1, 60 x 1024 x
-// 4096 6.8 -> 4.9, 60 x 4096 x 1024 11.3 -> 10.2; against the LDS-staged tiles 64 x 256 x 4096 8.2 -> 4.9.
+// 1024 6.4 -> 2.9 us, 1 x 4096 x 4096 11.4 -> 5.1, 23 x 1024 x 4096 6.6 -> 3.7, 23 x 4096 x 1024 11.1 -> 4.9, 60 x 1024 x
+// 4096 6.8 -> 4.9, 60 x 4096 x 1024 11.3 -> 5.1; against the LDS-staged tiles 64 x 256 x 4096 8.2 -> 4.9.
 template <int EPI>
 int launch_mm_skinny(hipc_ctx *ctx, const GemmArgs &g) {
     const bool zero_known = g.const_shift == 0 && (g.host_zp ? g.const_zp_value == 0 : g.const_zp == nullptr);
-    if (g.I <= 16) return zero_known ? launch_mm_skinny_rb<EPI, false, 1>(ctx, g) : launch_mm_skinny_rb<EPI, true, 1>(ctx, g);
-    if (g.I <= 32) return zero_known ? launch_mm_skinny_rb<EPI, false, 2>(ctx, g) : launch_mm_skinny_rb<EPI, true, 2>(ctx, g);
+    // 16-row blocks to a workgroup: as few as leave no more workgroups than CUs. Another workgroup reads the weight again, from
+    // the L2, but a CU without one idles, and a block fewer is a quarter of A's loads and of the sums that meet less. Us, all
+    // blocks in one / two / one block each: 60 x 4096 x 1024 (64 workgroups a block) 10.2 / 6.8 / 5.1, 32 x 4096 x 1024 6.8 / - / 5.0,
+    // 24 x 8192 x 2048 9.5 / - / 7.1, 48 x 2048 x 2048 (128) 6.1 / 4.8 / 4.9; 60 x 1024 x 4096 (256) 4.9 / 4.7 / 5.0, 64 x 4096 x
+    // 4096 10.9 / 12.4 / 13.1, 64 x 2048 x 8192 (512) 10.7 / 11.1 / 12.3.
+    const int64_t cols16 = ceil_div(g.J, 16), cols = cols16 > 2 * (int64_t)ctx->cu_count ? ceil_div(cols16, 2) : cols16, blocks = ceil_div(g.I, 16);
+    const auto fits = [&](int rb) { return blocks <= rb || cols * ceil_div(blocks, rb) <= ctx->cu_count; };
+    if (fits(1)) return zero_known ? launch_mm_skinny_rb<EPI, false, 1>(ctx, g) : launch_mm_skinny_rb<EPI, true, 1>(ctx, g);
+    if (fits(2)) return zero_known ? launch_mm_skinny_rb<EPI, false, 2>(ctx, g) : launch_mm_skinny_rb<EPI, true, 2>(ctx, g);
     return zero_known ? launch_mm_skinny_rb<EPI, false, 4>(ctx, g) : launch_mm_skinny_rb<EPI, true, 4>(ctx, g);
 }
 bool wants_skinny(hipc_ctx *ctx, const GemmArgs &g) {

@@ -350,6 +350,25 @@ def test_few_rows(ctx, pkg, oracle, shape, b_dt):
         weight.destroy()
 
 
+@pytest.mark.parametrize("shape", [(17, 512, 1024), (33, 1100, 2048), (48, 64, 1366), (49, 4160, 500), (64, 1024, 2050), (64, 128, 4100)], ids=lambda s: "M%d_K%d_N%d" % s)
+def test_few_rows_over_several_workgroups(ctx, pkg, oracle, shape):
+    """One, two and all blocks of 16 rows to a workgroup, the last block of one row or of all, columns one past a block: int32
+    and the folded range."""
+    m, k, n = shape
+    a = rc.pseudo_plus1(m * k, 84).reshape(m, k)
+    b = rc.pseudo_plus1(k * n, 85).view(np.int8).reshape(k, n)
+    want = oracle.matmul_integer(a, b, 131, 0)
+    weight = pkg.ops.Int8Weight(ctx, b)
+    with ctx.options(HIPC_GEMM_SKINNY=1):
+        assert np.array_equal(pkg.ops.matmul_integer(ctx, a, b, 131, 0, weight=weight), want)
+        bias = pkg.synth.uniform_f32(n, 86, -0.5, 0.5)
+        got, folded = pkg.ops.matmul_integer_scale_bias(ctx, a, b, 131, 0, np.float32(0.002), bias, fold_range=True, weight=weight)
+    weight.destroy()
+    ref = oracle.rescale(want, np.float32(0.002), bias)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    assert folded[0] == np.float32(-min(ref.min(), 0)).view(np.uint32) & 0x7FFFFFFF and folded[1] == np.float32(max(ref.max(), 0)).view(np.uint32)
+
+
 @pytest.mark.parametrize("m,k,n", [(5, 256, 96), (40, 250, 200), (64, 128, 4096), (70, 249, 96), (300, 1000, 130), (600, 1001, 900), (2500, 250, 2600)])
 def test_a_recorded_weight_zero_point_of_zero_can_be_patched(ctx, pkg, oracle, m, k, n):
     """A QLinearMatMul recorded with an int8 weight and zero point 0 -- few rows, rows that are no whole 16 bytes -- and
