@@ -6,8 +6,8 @@
 // measured (MI355X, per hand-over, all members storing and waiting for all): 0.52 us between the 32 workgroups of an XCD,
 // through its L2; 0.87 us between two workgroups of different XCDs, 1.7 us between all 256. So the work is laid out for
 // the XCDs:
-//   * XCD x serves query head x / P (P = 8 / heads XCDs a head), the (x mod P)th part of the context: its 32 workgroups
-//     multiply the q, k and v columns of that head (k and v by every XCD: cheaper than a hand-over across), attend to
+//   * The q, k and v columns are dealt to all 256 workgroups and handed to the XCDs that want them; XCD x then serves query head
+//     x / P (P = 8 / heads XCDs a head), the (x mod P)th part of the context: its 32 workgroups attend to
 //     their positions, and multiply their joined, unnormalised outputs by o's rows of the head. What leaves the XCD is one
 //     partial row of the o product and the softmax maximum and sum that weigh it.
 //   * Workgroup r of every XCD holds the same columns of the hidden row, so a row is summed over the XCDs by eight

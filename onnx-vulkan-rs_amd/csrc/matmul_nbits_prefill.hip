@@ -953,6 +953,9 @@ int prefill_pair_tile(hipc_ctx *ctx, const PrefillArgs &a) {
         const int64_t ways = std::max<int64_t>(1, std::min(most, cus / tiles));
         return ceil_div(tiles * ways, cus) * ceil_div(stages, ways);
     };
+    // three terms: half as wide where that leaves fewer CUs idle in the last round, at 0.55 of a 96x128 tile's work (512 x 2048 x
+    // 2560 in blocks of 128 39.4 us in two rounds, 35.3 in three of half the work; 2000 x 2048 x 2048 63.6 and 77.5, 512 x 4096 x 4096 70.0 and 74.1)
+    if (a.terms == 3 && mid > cus && 11 * ceil_div(rows64 * ceil_div(a.N, 64), cus) < 20 * ceil_div(mid, cus)) return 64;
     return a.terms == 2 && 2 * 15 * cost(large) < 16 * cost(mid) ? 192 : 128;
 }
 template <int SG>
