@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t epoch = p.sync[0];
-    if (!ALL && p.behind && p.sync[kResAll + kResDecision] == ((epoch << 10) | (kResGroups << 1) | (p.sync[kResAll + kResDecision] & 1u))) return;   // done
+    if (!ALL && p.behind && res_decided_for(p.sync[kResAll + kResDecision]) == kResGroups) return;   // done
     uint32_t *sync = p.sync + (ALL ? kResAll : kResSome);
     if (tid == 0) {
         const uint32_t xcc = __builtin_amdgcn_s_getreg((31 << 11) | 20) & 15u;   // XCC_ID
@@ -921,14 +921,14 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
             }
             res_stored();
         }
-        if (lane == 0) __hip_atomic_store(sync + kResDecision, (epoch << 10) | ((uint32_t)count << 1) | (one_l2 ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(sync + kResDecision, res_decision((uint32_t)count, one_l2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (tid == 0) {
         uint32_t d = 0, rank = 0xffffu;
         do {
             d = __hip_atomic_load(sync + kResDecision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } while ((d >> 10) != (epoch & 0x3fffffu) && --tries > 0);
-        const uint32_t count = (d >> 1) & 0x1ffu;
+        } while (!(d & kResDecided) && --tries > 0);
+        const uint32_t count = res_decided_for(d);
         if (tries <= 0) *p.broken = 1;
         else if (count == gridDim.x) rank = blockIdx.x;
         else if (!ALL) rank = __hip_atomic_load(sync + kResRankOf + blockIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -938,7 +938,7 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     {
         const uint32_t d = __builtin_amdgcn_readfirstlane(S.decision[0]), rank = __builtin_amdgcn_readfirstlane(S.decision[1]);
         if (rank == 0xffffu) return;   // the launch does not begin, or has begun without this workgroup
-        first = (int)rank, n = (int)((d >> 1) & 0x1ffu), wide = !(d & 1u);
+        first = (int)rank, n = (int)res_decided_for(d), wide = !(d & 1u);
     }
     set = (epoch % kResSets) * ((uint32_t)p.n_layers % kResSets) % kResSets;
 #endif

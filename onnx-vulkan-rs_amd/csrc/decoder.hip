@@ -744,7 +744,7 @@ dec_argmax_partial_kernel(const float *__restrict__ logits, int n, float *__rest
 // position): a step begins with its q|k|v product, not with a launch of its own for the embedding.
 __global__ void __launch_bounds__(256)
 dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, int nparts, DecState *st,
-                      int32_t *__restrict__ history, int max_hist, int vocab, uint32_t *__restrict__ launch, const EmbedArgs e) {
+                      int32_t *__restrict__ history, int max_hist, int vocab, uint32_t *__restrict__ sync, const EmbedArgs e) {
     __shared__ float red[4];
     __shared__ int next[2];
     // the upper two wavefronts work out the next position's rotary table (it follows from the position alone) while
@@ -779,7 +779,7 @@ dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, 
             } else {
                 if (bi < 0 || bi >= vocab) bi = 0;
                 history[pos] = bi;
-                if (launch) *launch = *launch + 1 == kResLaunches ? 0u : *launch + 1;   // the resident kernel's launch of this step has been
+                if (sync) res_next_step(sync);   // the resident kernel's launches of this step have been
                 st->token = token = bi;
                 st->pos = new_pos = pos + 1;
             }

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "resident.h"
 
 // ---- what the three sources leave undefined ---------------------------------------------------
 namespace hipc {
@@ -170,6 +171,40 @@ void report(const char *what) {
     g_launches = g_threads = g_loads = g_clipped = 0;
 }
 
+// The words a step's workgroups agree through must be as new for the next step, whatever they held: a decision that is left
+// standing would be taken for the next launch's own.
+void step_words() {
+    const Shape s = kSmall[0];
+    Model m;
+    gpu_model::reg().where = "the words of a step";
+    m.build(s);
+    m.ctx.tune.dec_prefetch = -1;
+    uint32_t *sync = nullptr;
+    for (const auto &[at, bytes] : gpu_model::reg().blocks)
+        if (bytes == hipc::kResSync * sizeof(uint32_t)) sync = reinterpret_cast<uint32_t *>(at);
+    using namespace hipc;
+    const auto expect = [&](bool ok, const char *what, uint32_t step) {
+        if (ok) return;
+        std::printf("FAILED: step %u: %s\n", step, what);
+        std::exit(1);
+    };
+    expect(sync != nullptr, "no words found", 0);
+    expect(sync[0] == 1, "a new decoder's first step is not number 1", 0);
+    hipc_ctx &ctx = m.ctx;
+    MUST(hipc_decoder_reset(&ctx, m.dec, 1, 0));
+    // (2^22: what a decision once held of the number was all zeros there, as the words are when nothing has been decided)
+    for (uint32_t step : {1u, 2u, (1u << 22) - 1, 1u << 22, (1u << 22) + 1, 3u << 22, kResLaunches - 2, kResLaunches - 1}) {
+        sync[0] = step;
+        sync[kResAll + kResDecision] = res_decision(kResGroups, true), sync[kResSome + kResDecision] = res_decision(3, false);
+        MUST(hipc_decoder_step(&ctx, m.dec));
+        expect(sync[kResAll + kResDecision] == 0 && sync[kResSome + kResDecision] == 0, "its decisions stand", step);
+        expect(sync[0] != 0, "followed by number 0, which the flags begin with", step);
+        expect(sync[0] % kResSets == (step + 1) % kResSets, "the sets are not taken in turn", step);
+    }
+    m.destroy();
+    report("the words of a step");
+}
+
 bool g_quick = false;
 std::vector<int> windows_of(const Shape &s) {
     if (g_quick) return {0, 512};
@@ -266,6 +301,7 @@ int main(int argc, char **argv) {
         if (!g_select.on) return true;
         return g_select.rows(g_select.index++, y0, y1);
     };
+    if (mode != "sweep") step_words();
     if (mode == "full") {
         for (const Shape &s : kSmall) full(s);
         full(kGemma);
