@@ -26,10 +26,11 @@
 // L2 only (workgroup scope); whether the members of a group really share one is read from the hardware when the launch
 // starts, and if not all stores are of agent scope.
 //
-// Nothing waits for a workgroup that may never come: workgroup 0 decides by a deadline whether the launch begins (all 256
-// arrive within microseconds on a free device). If not, everyone leaves, and a launch behind it deals the 256 shares of the
-// work to the workgroups that have arrived there; one that arrives later leaves at once. So such launches on one device, from
-// other streams or processes, cannot block each other. All waits are bounded beside that: a thread's polls of a whole launch are counted.
+// Nothing waits for a workgroup that may never come (resident_door.h): the launch begins when all 256 have arrived, which takes
+// microseconds on a free device, or else everyone leaves by a deadline of their own, and a launch behind it deals the 256 shares
+// of the work to the workgroups that have arrived there; one that arrives later leaves at once. So such launches on one device,
+// from other streams or processes, cannot block each other. Waits for workgroups that take part, which are all on the chip,
+// are bounded beside that: a thread's polls of a whole launch are counted.
 #include <hip/hip_fp16.h>
 
 #include "internal.h"
@@ -881,64 +882,54 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t epoch = p.sync[0];
     if (!ALL && p.behind && res_decided_for(p.sync[kResAll + kResDecision]) == kResGroups) return;   // done
-    uint32_t *sync = p.sync + (ALL ? kResAll : kResSome);
-    if (tid == 0) {
+    uint32_t *words = p.sync + (ALL ? kResAll : kResSome);
+    if (ALL && tid == 0) {
         const uint32_t xcc = __builtin_amdgcn_s_getreg((31 << 11) | 20) & 15u;   // XCC_ID
-        __hip_atomic_store(sync + kResFlags + blockIdx.x, (epoch << 4) | xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(words + kResFlags + blockIdx.x, (epoch << 4) | xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (blockIdx.x == 0 && wave == 0) {
-        const __amdgpu_buffer_rsrc_t r_s = lean_rsrc(sync, kResSyncWords * 4u);
+    if (!ALL) {
+        uint32_t here = 0;
+        if (tid == 0) S.decision[1] = res_join(words, gridDim.x, kArriveTicks, &here, tries), S.decision[0] = here;
+    } else if (blockIdx.x != 0) {
+        if (tid == 0) S.decision[0] = res_await(words, 2 * kArriveTicks, tries);
+    } else if (wave == 0) {
+        const __amdgpu_buffer_rsrc_t r_s = lean_rsrc(words, kResSyncWords * 4u);
         const unsigned long long t0 = wall_clock64();
-        uint4 f;
-        uint32_t here;   // bit q: workgroup 4 lane + q has arrived
+        const bool taken = lane == 0 && res_take(words);
+        uint4 f;   // the flags of workgroups 4 lane ..
+        bool all;
         do {
             res_reload();
             f = lean_ld16<kAgent>(r_s, (kResFlags + 4u * lane) * 4u, 0);
             const uint32_t want = epoch << 4;
-            here = ((f.x & ~15u) == want ? 1u : 0u) | ((f.y & ~15u) == want ? 2u : 0u) | ((f.z & ~15u) == want ? 4u : 0u) | ((f.w & ~15u) == want ? 8u : 0u);
-            const int in_grid = min(max((int)gridDim.x - 4 * lane, 0), 4);
-            here &= (1u << in_grid) - 1u;
-            if (__all(here == (1u << in_grid) - 1u)) break;
-        } while (wall_clock64() - t0 < kArriveTicks);
-        int before = __popc(here);   // arrived workgroups up to and with this lane's
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(before, off, 64);
-            if (lane >= off) before += o;
-        }
-        int count = __shfl(before, 63, 64);
-        before -= __popc(here);
+            all = __all((f.x & ~15u) == want && (f.y & ~15u) == want && (f.z & ~15u) == want && (f.w & ~15u) == want);
+        } while (!all && wall_clock64() - t0 < kArriveTicks);
         // one L2 per group: workgroups 8 j + x are group x, this lane holds groups 4 (lane & 1) ..
         const uint32_t gx = __shfl(f.x, lane & 1, 64), gy = __shfl(f.y, lane & 1, 64), gz = __shfl(f.z, lane & 1, 64), gw = __shfl(f.w, lane & 1, 64);
-        const bool one_l2 = count == (int)kResGroups && __all(f.x == gx && f.y == gy && f.z == gz && f.w == gw);
-        if (ALL) {
-            count = count == (int)kResGroups ? count : 0;
-        } else if (count < (int)gridDim.x) {
-            for (int q = 0; q < 4; q++) {
-                const bool in = (here >> q) & 1u;
-                __hip_atomic_store(sync + kResRankOf + 4 * lane + q, in ? (uint32_t)before : 0xffffu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                before += in;
-            }
-            res_stored();
+        const bool one_l2 = __all(f.x == gx && f.y == gy && f.z == gz && f.w == gw);
+        if (lane == 0) {
+            const uint32_t d = all && taken ? res_decision(kResGroups, one_l2) : res_decision(0, false);
+            if (taken) __hip_atomic_store(words + kResDecision, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            S.decision[0] = d;
         }
-        if (lane == 0) __hip_atomic_store(sync + kResDecision, res_decision((uint32_t)count, one_l2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (tid == 0) {
-        uint32_t d = 0, rank = 0xffffu;
-        do {
-            d = __hip_atomic_load(sync + kResDecision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } while (!(d & kResDecided) && --tries > 0);
-        const uint32_t count = res_decided_for(d);
-        if (tries <= 0) *p.broken = 1;
-        else if (count == gridDim.x) rank = blockIdx.x;
-        else if (!ALL) rank = __hip_atomic_load(sync + kResRankOf + blockIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        S.decision[0] = d, S.decision[1] = rank;
     }
     __syncthreads();
     {
-        const uint32_t d = __builtin_amdgcn_readfirstlane(S.decision[0]), rank = __builtin_amdgcn_readfirstlane(S.decision[1]);
-        if (rank == 0xffffu) return;   // the launch does not begin, or has begun without this workgroup
-        first = (int)rank, n = (int)res_decided_for(d), wide = !(d & 1u);
+        const uint32_t d = __builtin_amdgcn_readfirstlane(S.decision[0]);
+        if (ALL) {
+            if (res_decided_for(d) != kResGroups) {   // the launch does not begin
+                if (tries <= 0) *p.broken = 1;
+                return;
+            }
+            wide = !(d & 1u);
+        } else {
+            const uint32_t rank = __builtin_amdgcn_readfirstlane(S.decision[1]);
+            if (rank == kResNoRank) {   // ... has begun without this workgroup
+                if (tries <= 0) *p.broken = 1;
+                return;
+            }
+            first = (int)rank, n = (int)d, wide = true;
+        }
     }
     set = (epoch % kResSets) * ((uint32_t)p.n_layers % kResSets) % kResSets;
 #endif

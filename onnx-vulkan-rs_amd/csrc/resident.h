@@ -4,6 +4,7 @@
 #include <hip/hip_fp16.h>
 
 #include "internal.h"
+#include "resident_door.h"
 
 namespace hipc {
 
@@ -18,7 +19,6 @@ struct ResidentLayer {
 };
 
 // The words workgroups exchange: three sets, taken in turn by the layers. A region that stays inside an XCD is repeated for each.
-constexpr uint32_t kResXcds = 8, kResRanks = 32, kResGroups = kResXcds * kResRanks;
 constexpr uint32_t kResMaxHidden = 2048, kResMaxHead = 256, kResMaxSlice = 1024;
 constexpr uint32_t kResA = 0;                                          // [rank][head]: unnormalised attention outputs
 constexpr uint32_t kResML = kResA + kResRanks * kResMaxHead;           // [rank](max, sum)
@@ -32,25 +32,8 @@ constexpr uint32_t kResG2 = kResM1 + kResRanks * 32;                   // [rank]
 constexpr uint32_t kResQ = kResG2 + kResRanks * kResXcds * 64;         // the q|k|v row
 constexpr uint32_t kResMaxQkv = 2 * kResGroups * 16;
 constexpr uint32_t kResWords = kResQ + kResMaxQkv;                         // words of one set
-constexpr uint32_t kResSets = 3;
 static_assert(kResA % 32 == 0 && kResML % 32 == 0 && kResY % 32 == 0 && kResH % 32 == 0 && kResY2 % 32 == 0 && kResLocal % 32 == 0,
               "no region shares a 128-byte line with another");
-// The words the workgroups of a launch agree through: [0] the step's number, then, for the launch of all workgroups and for
-// the one that stands in for it, the decision (0: none yet), one flag and one rank per workgroup. The token pick closes the
-// step: it counts the number up and takes both decisions back, so no launch finds one that is not its own, however long ago
-// that form last ran. (A flag carries the step's number and needs no clearing; no step has the number 0 that flags begin with.)
-constexpr uint32_t kResDecision = 0, kResFlags = 32, kResRankOf = kResFlags + kResGroups, kResSyncWords = kResRankOf + kResGroups;
-constexpr uint32_t kResAll = 32, kResSome = kResAll + kResSyncWords, kResSync = kResSome + kResSyncWords;
-constexpr uint32_t kResLaunches = kResSets << 26;   // behind the largest number: a multiple of the sets, so that they go on in turn, and 28 bits
-constexpr uint32_t kResDecided = 0x80000000u;       // a decision: this, the workgroups that take part, and (bit 0) whether each group of them shares an L2
-
-__host__ __device__ inline uint32_t res_decision(uint32_t workgroups, bool one_l2) { return kResDecided | (workgroups << 1) | (one_l2 ? 1u : 0u); }
-__host__ __device__ inline uint32_t res_decided_for(uint32_t decision) { return (decision & ~kResDecided) >> 1; }
-// behind a step: the next one's words
-__host__ __device__ inline void res_next_step(uint32_t *sync) {
-    sync[0] = sync[0] + 1 == kResLaunches ? kResSets : sync[0] + 1;
-    sync[kResAll + kResDecision] = sync[kResSome + kResDecision] = 0;
-}
 
 struct ResidentArgs {
     const ResidentLayer *table;

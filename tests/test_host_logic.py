@@ -217,6 +217,10 @@ def test_kernel_addresses_on_the_cpu_model(tmp_path):
     # f16 and f32 rows, on ragged shapes with operands of exactly the operator's size
     run = subprocess.run([os.path.join(out, "prefill_model")], capture_output=True, text=True, env=env)
     assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout[-2000:] + run.stderr[-2000:]
+    # and how the workgroups of the decode step's one launch agree whether it begins, and on who stands in for it
+    # (tests/host/resident_door.cpp): workgroups that come late, workgroup 0 among them, keep nobody waiting
+    run = subprocess.run([os.path.join(out, "resident_door")], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout[-2000:] + run.stderr[-2000:]
 
 
 def _ctypes_only(monkeypatch, runtime, tmp_path):
