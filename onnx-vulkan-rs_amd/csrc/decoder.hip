@@ -849,7 +849,8 @@ struct hipc_decoder {
     bool x_ready = false;
     // All layers in one launch (decode_resident.hip), where the shape allows it
     bool resident = false;
-    ResidentLayer *table = nullptr;             // the layers as that kernel reads them
+    ResidentLayer *table = nullptr;             // the layers as that kernel reads them (not among `owned`: it is replaced)
+    bool table_recorded = false;                // a recorded step reads it
     std::vector<ResidentLayer> entries;         // what the table holds, or will once `stale` entries are written
     std::vector<char> stale;
     uint32_t *xch = nullptr, *sync = nullptr;
@@ -897,8 +898,13 @@ int launch_attn_chunks(hipc_ctx *ctx, hipc_decoder *d, DecLayer &l, float scale,
     return HIPC_OK;
 }
 
+int table_alloc(hipc_ctx *ctx, hipc_decoder *d, ResidentLayer **out) {
+    HIPC_TRY(ctx, hipMalloc(reinterpret_cast<void **>(out), d->entries.size() * sizeof(ResidentLayer)));
+    return HIPC_OK;
+}
+
 // Layer li of the resident kernel's table follows what has been set. A recorded step keeps the weights it was recorded
-// with: while graphs exist the change goes into a table of its own.
+// with: where one reads the table, the change goes into a new one, and the old one lives as long as the graphs do.
 int update_entry(hipc_ctx *ctx, hipc_decoder *d, int li) {
     if (!d->resident) return HIPC_OK;
     const DecLayer &l = d->layers[li];
@@ -909,12 +915,20 @@ int update_entry(hipc_ctx *ctx, hipc_decoder *d, int li) {
     for (int i = 0; i < 6; i++) e.norm[i] = l.norm[i];
     e.k_cache = l.k_cache, e.v_cache = l.v_cache, e.window = l.window, e.rope_table = l.rope_table;
     if (memcmp(&e, &d->entries[li], sizeof e) == 0 && !d->stale[li]) return HIPC_OK;
-    if (ctx->live_graphs > 0 && !ctx->capturing) {
-        ResidentLayer *fresh = nullptr;
-        int rc = dev_alloc(ctx, d, &fresh, d->entries.size());
-        if (rc != HIPC_OK) return rc;
-        HIPC_TRY(ctx, hipMemcpyAsync(fresh, d->table, d->entries.size() * sizeof(ResidentLayer), hipMemcpyDeviceToDevice, ctx->stream));
-        d->table = fresh;
+    if (d->table_recorded && !ctx->capturing) {
+        if (ctx->live_graphs > 0) {
+            ResidentLayer *fresh = nullptr;
+            int rc = table_alloc(ctx, d, &fresh);
+            if (rc != HIPC_OK) return rc;
+            hipError_t e = hipMemcpyAsync(fresh, d->table, d->entries.size() * sizeof(ResidentLayer), hipMemcpyDeviceToDevice, ctx->stream);
+            if (e != hipSuccess) {
+                (void)hipFree(fresh);
+                return fail(ctx, HIPC_ERR_BACKEND, "decoder: cannot copy the layer table: %s", hipGetErrorString(e));
+            }
+            retire(ctx, d->table);
+            d->table = fresh;
+        }
+        d->table_recorded = false;
     }
     d->entries[li] = e, d->stale[li] = 1;
     if (ctx->capturing) return HIPC_OK;   // (the next step writes it)
@@ -1016,7 +1030,8 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
         d->resident = d->lean && resident_takes(c) && (ctx->tune.dec_resident < 0 ? resident_pays(c) : ctx->tune.dec_resident > 0);
         if (d->resident) {
             d->entries.resize(c.n_layers), d->stale.assign(c.n_layers, 1);
-            A(&d->table, c.n_layers), A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSync);
+            A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSync);
+            if (rc == HIPC_OK) rc = table_alloc(ctx, d, &d->table);
             if (rc == HIPC_OK) rc = resident_clear(ctx, d->xch, d->sync);
         }
         if (rc == HIPC_OK) {
@@ -1029,6 +1044,7 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
         }
         if (rc != HIPC_OK) {
             for (void *p : d->owned) (void)hipFree(p);
+            if (d->table) (void)hipFree(d->table);
             delete d;
             return rc;
         }
@@ -1045,6 +1061,7 @@ void hipc_decoder_destroy(hipc_ctx *ctx, hipc_decoder *d) {
         }
         nbits_release(ctx, d->lm_head);
         for (void *p : d->owned) ctx->deferred.push_back(p);
+        if (d->table) ctx->deferred.push_back(d->table);
         delete d;
     });
 }
@@ -1232,6 +1249,7 @@ int hipc_decoder_step(hipc_ctx *ctx, hipc_decoder *d) {
                 if ((rc = resident_set_layer(ctx, d->table + li, d->entries[li])) != HIPC_OK) return rc;
                 if (!ctx->capturing) d->stale[li] = 0;
             }
+            if (ctx->capturing) d->table_recorded = true;
             ResidentArgs a{};
             a.table = d->table, a.pos = &d->state->pos, a.broken = &d->state->broken, a.rope = d->rope;
             a.x_in = xc, a.x_out = xo, a.y_out = d->yd, a.xch = d->xch, a.sync = d->sync;

@@ -205,6 +205,49 @@ void step_words() {
     report("the words of a step");
 }
 
+// Replacing what a layer is made of while graphs live: a new layer table only where a recorded step reads the old one, and
+// that one goes when the graphs do.
+void table_changes() {
+    const Shape s = kSmall[0];
+    Model m;
+    gpu_model::reg().where = "changes beside graphs";
+    m.build(s);
+    hipc_ctx &ctx = m.ctx;
+    ctx.tune.dec_prefetch = -1;
+    const auto change = [&](int times) {
+        for (int i = 0; i < times; i++) MUST(hipc_decoder_set_layer_attention(&ctx, m.dec, i % s.layers, 10 + i % 7, 0.f));
+    };
+    const auto expect = [&](size_t blocks, size_t retained, const char *what) {
+        if (gpu_model::reg().blocks.size() == blocks && ctx.retained.size() == retained) return;
+        std::printf("FAILED: %s: %zu allocations for %zu, %zu retired for %zu\n", what, gpu_model::reg().blocks.size(), blocks, ctx.retained.size(), retained);
+        std::exit(1);
+    };
+    const auto record = [&] {
+        ctx.capturing = true;
+        MUST(hipc_decoder_step(&ctx, m.dec));
+        ctx.capturing = false, ctx.live_graphs++;
+    };
+    MUST(hipc_decoder_reset(&ctx, m.dec, 1, 0));
+    const size_t before = gpu_model::reg().blocks.size();
+    ctx.live_graphs = 1;   // somebody else's
+    change(50);
+    expect(before, 0, "no recorded step of this decoder");
+    record();
+    change(50);
+    expect(before + 1, 1, "one recorded step");
+    record(), record();
+    change(50);
+    expect(before + 2, 2, "recorded again");
+    record();
+    ctx.live_graphs = 0;   // all of them destroyed
+    for (void *p : ctx.retained) gpu_model::release(p);
+    ctx.retained.clear();
+    change(50);
+    expect(before, 0, "no graph left");
+    m.destroy();
+    report("changes beside graphs");
+}
+
 bool g_quick = false;
 std::vector<int> windows_of(const Shape &s) {
     if (g_quick) return {0, 512};
@@ -301,7 +344,7 @@ int main(int argc, char **argv) {
         if (!g_select.on) return true;
         return g_select.rows(g_select.index++, y0, y1);
     };
-    if (mode != "sweep") step_words();
+    if (mode != "sweep") step_words(), table_changes();
     if (mode == "full") {
         for (const Shape &s : kSmall) full(s);
         full(kGemma);
