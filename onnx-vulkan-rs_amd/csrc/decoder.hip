@@ -851,8 +851,8 @@ struct hipc_decoder {
     bool resident = false;
     ResidentLayer *table = nullptr;             // the layers as that kernel reads them (not among `owned`: it is replaced)
     bool table_recorded = false;                // a recorded step reads it
-    std::vector<ResidentLayer> entries;         // what the table holds, or will once `stale` entries are written
-    std::vector<char> stale;
+    bool table_behind = false;                  // a change did not reach it (no memory for a new one): the next step makes up for that
+    std::vector<ResidentLayer> entries;         // what the table holds
     uint32_t *xch = nullptr, *sync = nullptr;
     bool one_launch_attn = false;  // head_dim and group size have an instance of dec_attn_chunks_kernel
     std::vector<void *> owned;
@@ -914,8 +914,11 @@ int update_entry(hipc_ctx *ctx, hipc_decoder *d, int li) {
         if (w[i]) e.wq[i] = w[i]->Wq, e.sc[i] = w[i]->Sc, e.zb[i] = w[i]->Zb;
     for (int i = 0; i < 6; i++) e.norm[i] = l.norm[i];
     e.k_cache = l.k_cache, e.v_cache = l.v_cache, e.window = l.window, e.rope_table = l.rope_table;
-    if (memcmp(&e, &d->entries[li], sizeof e) == 0 && !d->stale[li]) return HIPC_OK;
-    if (d->table_recorded && !ctx->capturing) {
+    if (memcmp(&e, &d->entries[li], sizeof e) == 0) return HIPC_OK;
+    HIPC_REFUSE(ctx, ctx->capturing, "decoder: a layer changed while a capture is open");   // (what would change one allocates, which a capture refuses first)
+    const bool behind = d->table_behind;
+    d->table_behind = true;
+    if (d->table_recorded) {
         if (ctx->live_graphs > 0) {
             ResidentLayer *fresh = nullptr;
             int rc = table_alloc(ctx, d, &fresh);
@@ -930,10 +933,8 @@ int update_entry(hipc_ctx *ctx, hipc_decoder *d, int li) {
         }
         d->table_recorded = false;
     }
-    d->entries[li] = e, d->stale[li] = 1;
-    if (ctx->capturing) return HIPC_OK;   // (the next step writes it)
     int rc = resident_set_layer(ctx, d->table + li, e);
-    if (rc == HIPC_OK) d->stale[li] = 0;
+    if (rc == HIPC_OK) d->entries[li] = e, d->table_behind = behind;
     return rc;
 }
 
@@ -1029,7 +1030,7 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
         }
         d->resident = d->lean && resident_takes(c) && (ctx->tune.dec_resident < 0 ? resident_pays(c) : ctx->tune.dec_resident > 0);
         if (d->resident) {
-            d->entries.resize(c.n_layers), d->stale.assign(c.n_layers, 1);
+            d->entries.resize(c.n_layers);
             A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSync);
             if (rc == HIPC_OK) rc = table_alloc(ctx, d, &d->table);
             if (rc == HIPC_OK) rc = resident_clear(ctx, d->xch, d->sync);
@@ -1244,11 +1245,9 @@ int hipc_decoder_step(hipc_ctx *ctx, hipc_decoder *d) {
         // All layers in one launch. (Asked for read-ahead by name, the launches that can carry it run instead.)
         const bool resident = d->resident && ctx->tune.dec_resident != 0 && ctx->tune.dec_prefetch < 0;
         if (resident) {
-            for (int li = 0; li < c.n_layers; li++) {
-                if (!d->stale[li]) continue;
-                if ((rc = resident_set_layer(ctx, d->table + li, d->entries[li])) != HIPC_OK) return rc;
-                if (!ctx->capturing) d->stale[li] = 0;
-            }
+            for (int li = 0; li < c.n_layers && d->table_behind; li++)
+                if ((rc = update_entry(ctx, d, li)) != HIPC_OK) return rc;
+            d->table_behind = false;
             if (ctx->capturing) d->table_recorded = true;
             ResidentArgs a{};
             a.table = d->table, a.pos = &d->state->pos, a.broken = &d->state->broken, a.rope = d->rope;

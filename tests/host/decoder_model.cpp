@@ -239,6 +239,19 @@ void table_changes() {
     change(50);
     expect(before + 2, 2, "recorded again");
     record();
+    // a change for which there was no memory is made up for by the next step: it must not run on what was replaced
+    gpu_model::reg().no_memory = true;
+    if (hipc_decoder_set_layer_attention(&ctx, m.dec, 0, 77, 0.f) == HIPC_OK || hipc_decoder_step(&ctx, m.dec) == HIPC_OK) {
+        std::printf("FAILED: a change without memory, or a step behind it, went through\n");
+        std::exit(1);
+    }
+    gpu_model::reg().no_memory = false;
+    MUST(hipc_decoder_step(&ctx, m.dec));
+    expect(before + 3, 3, "made up for");
+    bool found = false;
+    for (const auto &[at, bytes] : gpu_model::reg().blocks)
+        found = found || (bytes == s.layers * sizeof(hipc::ResidentLayer) && reinterpret_cast<const hipc::ResidentLayer *>(at)->window == 77);
+    if (!found) std::printf("FAILED: the change did not reach the table\n"), std::exit(1);
     ctx.live_graphs = 0;   // all of them destroyed
     for (void *p : ctx.retained) gpu_model::release(p);
     ctx.retained.clear();

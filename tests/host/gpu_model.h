@@ -34,6 +34,7 @@ struct Registry {
     std::map<uintptr_t, size_t> blocks;   // start -> bytes
     size_t loads = 0, loads_clipped = 0, launches = 0, threads = 0;
     bool failed = false;
+    bool no_memory = false;   // hipMalloc fails
     std::string where;   // what is being launched (printed with a failure)
 };
 // one registry per host thread: a thread of the driver builds its own model (its own allocations)
@@ -218,7 +219,11 @@ using std::min;
 #define hipGetSymbolAddress(pp, sym) (*(pp) = const_cast<void *>(static_cast<const void *>(sym)), hipSuccess)
 #define hipFuncSetAttribute(...) hipSuccess
 template <typename T>
-inline hipError_t gpu_model_hipMalloc(T **p, size_t bytes) { *p = static_cast<T *>(gpu_model::alloc(bytes)); return hipSuccess; }
+inline hipError_t gpu_model_hipMalloc(T **p, size_t bytes) {
+    if (gpu_model::reg().no_memory) return hipErrorOutOfMemory;
+    *p = static_cast<T *>(gpu_model::alloc(bytes));
+    return hipSuccess;
+}
 inline hipError_t gpu_model_hipFree(void *p) { gpu_model::release(p); return hipSuccess; }
 inline hipError_t gpu_model_hipMemsetAsync(void *p, int v, size_t n, hipStream_t) { std::memset(p, v, n); return hipSuccess; }
 inline hipError_t gpu_model_hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
