@@ -971,7 +971,11 @@ bool hipc::resident_takes(const hipc_decoder_config &c) {
 // 109.1 / 136.6, 117.5 / 144.1, 198.1 / 206.6), 8 heads up to about 12000 (2048 / 8192 / 8 of 256: 175.9 / 232.1 at 100, 263.0 /
 // 280.8 at 8192, 342.9 / 325.2 at 16384, 517.5 / 390.0 at 32000). The position is the device's and a recorded step covers all of
 // them, so the rule is on the longest one: at 8 heads x 16384 the last quarter loses 5 %, the rest gains 7 to 32 %.
-bool hipc::resident_pays(const hipc_decoder_config &c) { return (int64_t)c.n_q_heads * c.max_seq <= 8 * 16384; }
+// Only where every workgroup has a CU: with fewer, all steps would be the stand-in's, whose workgroups take shares in turn (gemma3-1b
+// at 2048: 832 us a token with 255 workgroups, 990 with 128, 1680 with 64; 654 by the launches per product, 452 in one launch).
+bool hipc::resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c) {
+    return ctx->cu_count >= (int)kResGroups && (int64_t)c.n_q_heads * c.max_seq <= 8 * 16384;
+}
 
 namespace {
 

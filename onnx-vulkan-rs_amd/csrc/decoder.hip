@@ -1028,7 +1028,7 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
                     rc = fail(ctx, HIPC_ERR_BACKEND, "decoder: cannot clear the gated row and the attention partials");
             }
         }
-        d->resident = d->lean && resident_takes(c) && (ctx->tune.dec_resident < 0 ? resident_pays(c) : ctx->tune.dec_resident > 0);
+        d->resident = d->lean && resident_takes(c) && (ctx->tune.dec_resident < 0 ? resident_pays(ctx, c) : ctx->tune.dec_resident > 0);
         if (d->resident) {
             d->entries.resize(c.n_layers);
             A(&d->xch, (size_t)kResSets * kResWords), A(&d->sync, kResSync);

@@ -51,7 +51,7 @@ struct ResidentArgs {
 };
 
 bool resident_takes(const hipc_decoder_config &c);
-bool resident_pays(const hipc_decoder_config &c);   // against the launch per product
+bool resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c);   // against the launch per product
 int resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const ResidentArgs &a, int workgroups);
 int resident_set_layer(hipc_ctx *ctx, ResidentLayer *entry, const ResidentLayer &value);   // in stream order
 int resident_clear(hipc_ctx *ctx, uint32_t *xch, uint32_t *sync);                          // exchange words empty, launch number 1

@@ -261,6 +261,35 @@ void table_changes() {
     report("changes beside graphs");
 }
 
+// Where a decoder takes all layers in one launch by itself: a device with a CU for each workgroup, and contexts up to the
+// length where the launches per product, which spread a head over more workgroups, are the faster form.
+void which_form() {
+    struct Case {
+        int cus, nq, nkv, max_seq;
+        bool one_launch;
+    };
+    const Case cases[] = {{256, 4, 2, 80, true}, {255, 4, 2, 80, false}, {64, 4, 2, 80, false}, {304, 4, 2, 80, true},
+                          {256, 4, 1, 32768, true}, {256, 4, 1, 32769, false}, {256, 1, 1, 131072, true}};
+    for (const Case &k : cases) {
+        hipc_ctx ctx;
+        ctx.cu_count = k.cus;
+        hipc_decoder_config cfg{};
+        cfg.n_layers = 1, cfg.hidden = 128, cfg.ffn = 256, cfg.n_q_heads = k.nq, cfg.n_kv_heads = k.nkv, cfg.head_dim = 64;
+        cfg.vocab = 512, cfg.max_seq = k.max_seq, cfg.block_size = 32, cfg.rms_eps = 1e-6f, cfg.rope_theta = 10000.f, cfg.embed_scale = 1.f;
+        hipc_decoder *dec = nullptr;
+        MUST(hipc_decoder_create(&ctx, &cfg, &dec));
+        bool found = false;
+        for (const auto &[at, bytes] : gpu_model::reg().blocks) found = found || bytes == hipc::kResSync * sizeof(uint32_t);
+        if (found != k.one_launch) {
+            std::printf("FAILED: %d CUs, %d / %d heads, %d positions: %s\n", k.cus, k.nq, k.nkv, k.max_seq, found ? "one launch" : "a launch per product");
+            std::exit(1);
+        }
+        hipc_decoder_destroy(&ctx, dec);
+        for (void *p : ctx.deferred) gpu_model::release(p);
+    }
+    report("which form a decoder takes");
+}
+
 bool g_quick = false;
 std::vector<int> windows_of(const Shape &s) {
     if (g_quick) return {0, 512};
@@ -357,7 +386,7 @@ int main(int argc, char **argv) {
         if (!g_select.on) return true;
         return g_select.rows(g_select.index++, y0, y1);
     };
-    if (mode != "sweep") step_words(), table_changes();
+    if (mode != "sweep") step_words(), table_changes(), which_form();
     if (mode == "full") {
         for (const Shape &s : kSmall) full(s);
         full(kGemma);
