@@ -964,17 +964,23 @@ bool hipc::resident_takes(const hipc_decoder_config &c) {
            (c.n_q_heads + 2 * c.n_kv_heads) * c.head_dim <= (int)kResMaxQkv && c.hidden % 16 == 0 && c.hidden <= (int)kResMaxHidden && c.ffn % 16 == 0 && cg_f <= 64;
 }
 
-// One launch against five per layer (8 layers, a token, us): the 256 workgroups read each query head's positions themselves
-// (no more than 8 / heads parts of them), where the attention launch spreads them over as many workgroups as it likes. Heads
-// times positions decide, whatever the other sizes are: hidden 256 to 2048 and 4 heads win at every position that was measured
-// (1152 / 6912 / 4 heads of 256: 130.8 against 179.8 at 100, 143.2 / 191.0 at 2048, 306.6 / 335.3 at 32000; 256 / 1024 / 4 heads of 64:
-// 109.1 / 136.6, 117.5 / 144.1, 198.1 / 206.6), 8 heads up to about 12000 (2048 / 8192 / 8 of 256: 175.9 / 232.1 at 100, 263.0 /
-// 280.8 at 8192, 342.9 / 325.2 at 16384, 517.5 / 390.0 at 32000). The position is the device's and a recorded step covers all of
-// them, so the rule is on the longest one: at 8 heads x 16384 the last quarter loses 5 %, the rest gains 7 to 32 %.
+// One launch against five per layer: the 256 workgroups read each query head's positions themselves (no more than 8 / heads
+// parts of them), where the attention launch spreads them over as many workgroups as it likes, and heads that share a kv head
+// there share its reading. So heads and positions decide, whatever the other sizes are. Per product / one launch, us a token of 8 layers (query
+// / kv heads of channels, hidden / ffn, at position):
+//   8/1 of 256, 2048 / 8192     272 / 259 at 8192, 292 / 308 at 12288, 314 / 350 at 16384
+//   8/2 of 64, 512 / 2048       162 / 156 at 8192, 169 / 179 at 12288, 178 / 201 at 16384
+//   8/4 of 256, 1152 / 6912     284 / 269 at 12288, 311 / 318 at 16384
+//   8/8 of 128, 1024 / 4096     204 / 184 at 8192, 240 / 222 at 12288, 258 / 258 at 16384
+//   4/1 of 256, 1152 / 6912     246 / 212 at 16384, 330 / 308 at 32768;  4/4 of 128, 512 / 2048  276 / 251 at 32768
+//   2/1 of 128, 512 / 2048      353 / 224 at 65536;  1/1 of 256, 1152 / 6912  804 / 339 at 131072
+// and at position 100 one launch takes about three quarters. The position is the device's and a recorded step covers all of
+// them, so the rule is on the longest one: no position of a decoder that takes one launch is slower for it.
 // Only where every workgroup has a CU: with fewer, all steps would be the stand-in's, whose workgroups take shares in turn (gemma3-1b
 // at 2048: 832 us a token with 255 workgroups, 990 with 128, 1680 with 64; 654 by the launches per product, 452 in one launch).
 bool hipc::resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c) {
-    return ctx->cu_count >= (int)kResGroups && (int64_t)c.n_q_heads * c.max_seq <= 8 * 16384;
+    const int64_t most = c.n_q_heads <= 4 ? 131072 / c.n_q_heads : c.n_kv_heads >= 4 ? 12288 : 8192;
+    return ctx->cu_count >= (int)kResGroups && c.max_seq <= most;
 }
 
 namespace {

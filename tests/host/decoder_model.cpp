@@ -269,7 +269,8 @@ void which_form() {
         bool one_launch;
     };
     const Case cases[] = {{256, 4, 2, 80, true}, {255, 4, 2, 80, false}, {64, 4, 2, 80, false}, {304, 4, 2, 80, true},
-                          {256, 4, 1, 32768, true}, {256, 4, 1, 32769, false}, {256, 1, 1, 131072, true}};
+                          {256, 4, 1, 32768, true}, {256, 4, 1, 32769, false}, {256, 1, 1, 131072, true},
+                          {256, 8, 1, 8192, true}, {256, 8, 1, 8193, false}, {256, 8, 2, 8193, false}, {256, 8, 4, 12288, true}, {256, 8, 8, 12289, false}};
     for (const Case &k : cases) {
         hipc_ctx ctx;
         ctx.cu_count = k.cus;
