@@ -115,6 +115,9 @@ const OptionName kOptions[] = {
     {"HIPC_GEMV_LEAN", &Tuning::gemv_lean},
     {"HIPC_DEC_LEAN", &Tuning::dec_lean},
     {"HIPC_DEC_RESIDENT", &Tuning::dec_resident},
+    {"HIPC_DEC_WAIT", &Tuning::dec_wait},
+    {"HIPC_DEC_WIDE", &Tuning::dec_wide},
+    {"HIPC_DEC_POLLS", &Tuning::dec_polls},
     {"HIPC_DQL_WAIT", &Tuning::dql_wait},
     {"HIPC_DEC_PREFETCH", &Tuning::dec_prefetch},
 };

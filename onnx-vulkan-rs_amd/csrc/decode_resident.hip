@@ -73,7 +73,7 @@ constexpr int kPollBudget = 1 << 23;                   // polls of one thread in
 #else
 constexpr int kPollBudget = 1;                         // (one thread after the other: there is nobody to wait for)
 #endif
-constexpr unsigned long long kArriveTicks = 20000;     // 200 us of the 100 MHz clock: how long the launch waits for workgroups that have not started
+constexpr int kArriveTicks = 20000;                    // 200 us of the 100 MHz clock: how long the launch waits for workgroups that have not started
 constexpr int kResThreads = 512, kResWaves = 8;
 constexpr int kRedPitch = 20;                          // words per column of the reduction area: 16 k tiles, 16-byte rows
 constexpr int kSumsAt = 64 * 2 * 4 * 16;               // bytes from the row's terms to their chunks' sums (ResShared)
@@ -873,7 +873,7 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     __shared__ __attribute__((aligned(16))) ResShared<HD> S;
     const int pos = *p.pos;
     if (pos >= p.max_seq) return;   // the cache is full: the step is a no-op (the token pick reports it)
-    int tries = kPollBudget;
+    int tries = p.polls;
     int first = blockIdx.x, n = gridDim.x;
     bool wide = false;
     uint32_t set = 0;
@@ -889,9 +889,9 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     }
     if (!ALL) {
         uint32_t here = 0;
-        if (tid == 0) S.decision[1] = res_join(words, gridDim.x, kArriveTicks, &here, tries), S.decision[0] = here;
+        if (tid == 0) S.decision[1] = res_join(words, gridDim.x, (unsigned long long)p.arrive, &here, tries), S.decision[0] = here;
     } else if (blockIdx.x != 0) {
-        if (tid == 0) S.decision[0] = res_await(words, 2 * kArriveTicks, tries);
+        if (tid == 0) S.decision[0] = res_await(words, 2ull * (unsigned)p.arrive, tries);
     } else if (wave == 0) {
         const __amdgpu_buffer_rsrc_t r_s = lean_rsrc(words, kResSyncWords * 4u);
         const unsigned long long t0 = wall_clock64();
@@ -903,12 +903,12 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
             f = lean_ld16<kAgent>(r_s, (kResFlags + 4u * lane) * 4u, 0);
             const uint32_t want = epoch << 4;
             all = __all((f.x & ~15u) == want && (f.y & ~15u) == want && (f.z & ~15u) == want && (f.w & ~15u) == want);
-        } while (!all && wall_clock64() - t0 < kArriveTicks);
+        } while (!all && wall_clock64() - t0 < (unsigned long long)p.arrive);
         // one L2 per group: workgroups 8 j + x are group x, this lane holds groups 4 (lane & 1) ..
         const uint32_t gx = __shfl(f.x, lane & 1, 64), gy = __shfl(f.y, lane & 1, 64), gz = __shfl(f.z, lane & 1, 64), gw = __shfl(f.w, lane & 1, 64);
         const bool one_l2 = __all(f.x == gx && f.y == gy && f.z == gz && f.w == gw);
         if (lane == 0) {
-            const uint32_t d = all && taken ? res_decision(kResGroups, one_l2) : res_decision(0, false);
+            const uint32_t d = all && taken && p.arrive != 0 ? res_decision(kResGroups, one_l2) : res_decision(0, false);
             if (taken) __hip_atomic_store(words + kResDecision, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             S.decision[0] = d;
         }
@@ -921,7 +921,7 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
                 if (tries <= 0) *p.broken = 1;
                 return;
             }
-            wide = !(d & 1u);
+            wide = p.wide || !(d & 1u);
         } else {
             const uint32_t rank = __builtin_amdgcn_readfirstlane(S.decision[1]);
             if (rank == kResNoRank) {   // ... has begun without this workgroup
@@ -1018,6 +1018,9 @@ int hipc::resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const Res
     a.inv_hidden = 1.f / (float)c.hidden;
     a.nib_mask = 0x000f000fu, a.magic = 0x43004300u;
     a.eps = c.rms_eps, a.scale = c.attn_scale > 0.f ? c.attn_scale : 1.f / sqrtf((float)c.head_dim);
+    a.arrive = ctx->tune.dec_wait >= 0 ? ctx->tune.dec_wait : kArriveTicks;
+    a.polls = ctx->tune.dec_polls > 0 ? ctx->tune.dec_polls : kPollBudget;
+    a.wide = ctx->tune.dec_wide > 0;
     const int sg = c.block_size == 32 ? 4 : c.block_size == 64 ? 2 : 1;
     if (workgroups >= (int)kResGroups) {
         int rc = launch_hd<true>(ctx, c.head_dim, sg, a, kResGroups);

@@ -72,6 +72,10 @@ struct Tuning {
     int gemv_lean = -1;       // HIPC_GEMV_LEAN      0: one-row products keep the streaming GEMV kernel
     int dec_lean = -1;        // HIPC_DEC_LEAN       0: the decoder keeps the streaming GEMV and its prologues (read when a decoder is created)
     int dec_resident = -1;    // HIPC_DEC_RESIDENT   0: the decoder keeps a launch per product (read when a decoder is created, too); n: workgroups of the launch that holds all layers
+    // The ways out of the launch that holds all layers, for tests:
+    int dec_wait = -1;        // HIPC_DEC_WAIT       how long its workgroups wait for ones that have not started, in 10 ns; 0: it does not begin
+    int dec_wide = -1;        // HIPC_DEC_WIDE       1: as where the workgroups of a group do not share an L2
+    int dec_polls = -1;       // HIPC_DEC_POLLS      polls a thread may make before the step is given up
     int dql_wait = -1;        // HIPC_DQL_WAIT       0: DynamicQuantizeLinear never in one launch of several workgroups; n: how long these wait for each other, in 10 ns
     int dec_prefetch = -1;    // HIPC_DEC_PREFETCH   bits: which launches of a layer carry helper rows that read ahead for the next launch (0 none, 31 all; see hipc_decoder_step)
 };

@@ -45,6 +45,7 @@ struct ResidentArgs {
     int n_layers, hidden, cg_h, cg_o, tiles_h, tiles_qkv, cg_f, pairs;   // cg_*: 128-k tiles of hidden, the heads' channels, ffn; tiles_*: 16-column tiles; pairs: (gate, up) tile pairs
     int n_q, n_kv, lg_group, lg_parts;   // XCDs per head = 1 << lg_parts
     int max_seq, v_stride, behind;
+    int arrive, polls, wide;             // how long workgroups are waited for, in 10 ns; polls of a thread; stores at agent scope whatever the launch finds
     uint32_t inv_cg_h;                   // 65536 / cg_h, rounded up
     uint32_t nib_mask, magic;
     float eps, scale, inv_hidden;

@@ -72,7 +72,8 @@ DEEP = [  # (head_dim, query heads, kv heads, first position): every head_dim / 
 # launch of a layer. By default three of the five producers carry helpers; the other cases run all five and none.
 READ_AHEAD = {"HIPC_DEC_PREFETCH": 31}
 NO_READ_AHEAD = {"HIPC_DEC_PREFETCH": 0}
-PATHS = [{}, READ_AHEAD, {"HIPC_DEC_LEAN": 0}, {"HIPC_DEC_FUSED_GLUE": 0}, {"HIPC_DEC_FUSED_ATTN": 0}]
+PER_PRODUCT = {"HIPC_DEC_RESIDENT": 0}   # the launches per product with their default read-ahead, which longer contexts and other shapes take
+PATHS = [{}, PER_PRODUCT, READ_AHEAD, {"HIPC_DEC_LEAN": 0}, {"HIPC_DEC_FUSED_GLUE": 0}, {"HIPC_DEC_FUSED_ATTN": 0}]
 
 
 @pytest.fixture
@@ -89,7 +90,7 @@ def route(ctx):
         ctx.set_option(k, -1)
 
 
-@pytest.mark.parametrize("env", PATHS, ids=["default", "read-ahead", "streaming-gemv", "separate-glue", "three-kernel-attention"])
+@pytest.mark.parametrize("env", PATHS, ids=["default", "per-product", "read-ahead", "streaming-gemv", "separate-glue", "three-kernel-attention"])
 @pytest.mark.parametrize("hd,nq,nkv,p0", DEEP)
 def test_attention_over_a_long_filled_cache(ctx, pkg, oracle, route, hd, nq, nkv, p0, env):
     """Steps taken deep into a context whose cache rows hold random f16 values on both sides: the
@@ -157,7 +158,7 @@ WINDOWS = [  # (head_dim, query heads, kv heads, first position, window of layer
 ]
 
 
-@pytest.mark.parametrize("env", PATHS, ids=["default", "read-ahead", "streaming-gemv", "separate-glue", "three-kernel-attention"])
+@pytest.mark.parametrize("env", PATHS, ids=["default", "per-product", "read-ahead", "streaming-gemv", "separate-glue", "three-kernel-attention"])
 @pytest.mark.parametrize("hd,nq,nkv,p0,w0,w1", WINDOWS)
 def test_sliding_windows_and_a_second_rotary_base(ctx, pkg, oracle, route, hd, nq, nkv, p0, w0, w1, env):
     """Local layers: the last `window` positions only, the step's own included (the reference's
@@ -371,16 +372,11 @@ RESIDENT = [  # (hidden, ffn, head_dim, query heads, kv heads, block_size): the 
 ]
 
 
-@pytest.mark.parametrize("groups", [-1, 255, 100, 3], ids=["all", "255", "100", "3"])
-@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
-def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, nkv, bs, groups):
-    """Three layers by a launch of 256 workgroups, and by launches of fewer, whose workgroups take several shares each
-    (what happens when not all of them find room on the device): logits, cache rows and tokens against the oracle over a
-    filled cache, positions 69 .. 72 (the third pass of 32 begins) with a window of 40 in the second layer. The tolerance is this file's."""
+def three_layers(pkg, ctx, hidden, ffn, hd, nq, nkv, bs):
+    """A decoder and the oracle's over the same filled cache of 80 positions, a window of 40 in the second layer."""
     from oracle import decoder as od
-    route({"HIPC_DEC_RESIDENT": groups})
     cfg = dict(SMALL, n_layers=3, hidden=hidden, ffn=ffn, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, block_size=bs, vocab=512, embed_scale=float(np.sqrt(hidden)))
-    p0, max_seq = 69, 80
+    max_seq = 80
     w = pkg.decoder.build_weights(cfg, seed=31)
     dec = pkg.decoder.Decoder(ctx, cfg, max_seq)
     dec.load(w)
@@ -391,7 +387,12 @@ def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, 
         k_rows, v_rows = ((rng.standard_normal((nkv, max_seq, hd)) * 0.7).astype(np.float16) for _ in range(2))
         ref.k[li], ref.v[li] = k_rows, v_rows
         dec.fill_cache(li, k_rows, v_rows)
-    token = 23
+    return dec, ref
+
+
+def steps_match(ctx, dec, ref, p0=69):
+    """Four steps from position 69 (the third pass of 32 begins): logits, cache rows and tokens. The tolerance is this file's."""
+    token, nkv, hd = 23, dec.cfg["n_kv_heads"], dec.cfg["head_dim"]
     dec.reset(token, p0)
     for pos in range(p0, p0 + 4):
         dec.step()
@@ -400,10 +401,31 @@ def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, 
         assert got_pos == pos + 1
         err = np.abs(logits - want_logits)
         assert np.all(err <= 2e-3 + 2e-3 * np.abs(want_logits)), (pos, float(err.max()))
-        for li in range(cfg["n_layers"]):
-            k_row = ctx.download(dec.kv_cache(li)[0], np.float16, (hd,), offset=((nkv - 1) * max_seq + pos) * hd * 2)
+        for li in range(dec.cfg["n_layers"]):
+            k_row = ctx.download(dec.kv_cache(li)[0], np.float16, (hd,), offset=((nkv - 1) * dec.max_seq + pos) * hd * 2)
             assert np.allclose(k_row.astype(np.float32), ref.k[li, nkv - 1, pos].astype(np.float32), atol=2e-3, rtol=2e-3), (pos, li)
         token = got_tok
+
+
+@pytest.mark.parametrize("groups", [-1, 255, 100, 3], ids=["all", "255", "100", "3"])
+@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
+def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, nkv, bs, groups):
+    """Three layers by a launch of 256 workgroups, and by launches of fewer, whose workgroups take several shares each."""
+    route({"HIPC_DEC_RESIDENT": groups})
+    dec, ref = three_layers(pkg, ctx, hidden, ffn, hd, nq, nkv, bs)
+    steps_match(ctx, dec, ref)
+    dec.destroy()
+
+
+@pytest.mark.parametrize("env", [{"HIPC_DEC_WAIT": 0}, {"HIPC_DEC_WAIT": 100}, {"HIPC_DEC_WIDE": 1}, {"HIPC_DEC_RESIDENT": 40, "HIPC_DEC_WAIT": 0}],
+                         ids=["does-not-begin", "waits-a-microsecond", "no-shared-l2", "those-there-at-once"])
+@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
+def test_the_ways_out_of_the_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, nkv, bs, env):
+    """The launch of 256 workgroups does not begin and the one behind it goes on with the workgroups it has by then, however
+    few; the same where some may come in time; and hand-overs that leave the L2 everywhere."""
+    route(env)
+    dec, ref = three_layers(pkg, ctx, hidden, ffn, hd, nq, nkv, bs)
+    steps_match(ctx, dec, ref)
     dec.destroy()
 
 
