@@ -416,7 +416,9 @@ const char *hipc_host_error(void);
  * Limits kept on the device: the cache holds `max_seq` positions, so at most `max_seq` steps can
  * follow a reset to position 0. A step enqueued (or replayed) with the cache full writes nothing,
  * leaves token and position as they are and raises a sticky flag that `hipc_decoder_read` reports
- * as HIPC_ERR_INVALID until the next `hipc_decoder_reset`. The chosen token is always inside
+ * as HIPC_ERR_INVALID until the next `hipc_decoder_reset`. A step that had to be given up (a wait inside it
+ * ran out) is reported as HIPC_ERR_BACKEND in the same way; the cache holds nothing useful from its position
+ * on, so the reset goes there or further back. The chosen token is always inside
  * [0, vocab): if no logit compares (all NaN) it is 0, ArgMax's answer for such a row.
  */
 typedef struct hipc_decoder hipc_decoder;

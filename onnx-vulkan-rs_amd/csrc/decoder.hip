@@ -790,14 +790,22 @@ dec_pick_embed_kernel(const float *__restrict__ pv, const int *__restrict__ pi, 
     dec_embed_token<false>(e, next[0], next[1], red);
 }
 
-// (after a resident launch that did not come to its end, its words are made what a new decoder's are)
-__global__ void __launch_bounds__(256) dec_set_state_kernel(DecState *st, int token, int pos, uint32_t *xch, uint32_t *sync) {
-    const bool broken = xch && st->broken;
+// Behind a resident launch that did not come to its end, its words are made what a new decoder's are, and so are the value rows
+// that launch and later ones wrote from `pos` on: rows past the position have no weight in the attention, but NaN times nothing
+// is NaN. (Without a resident launch `r.xch` is null.)
+__global__ void __launch_bounds__(256) dec_set_state_kernel(DecState *st, int token, int pos, const ResidentReset r) {
+    const bool broken = r.xch && st->broken;
+    const int end = st->pos;
     __syncthreads();
     if (threadIdx.x == 0) st->token = token, st->pos = pos, st->overflow = 0, st->broken = 0;
     if (broken) {
-        for (uint32_t i = threadIdx.x; i < kResSets * kResWords; i += 256) xch[i] = 0xffffffffu;
-        for (uint32_t i = threadIdx.x; i < kResSync; i += 256) sync[i] = i == 0 ? 1u : 0u;
+        for (uint32_t i = threadIdx.x; i < kResSets * kResWords; i += 256) r.xch[i] = 0xffffffffu;
+        for (uint32_t i = threadIdx.x; i < kResSync; i += 256) r.sync[i] = i == 0 ? 1u : 0u;
+        for (int l = 0; l < r.n_layers; l++) {
+            __half *v = r.table[l].v_cache;
+            for (int row = threadIdx.x; row < r.v_rows; row += 256)
+                for (int t = pos; t < end; t++) v[(size_t)row * r.v_stride + t] = __float2half(0.f);
+        }
     }
 }
 
@@ -850,7 +858,7 @@ struct hipc_decoder {
     // All layers in one launch (decode_resident.hip), where the shape allows it
     bool resident = false;
     ResidentLayer *table = nullptr;             // the layers as that kernel reads them (not among `owned`: it is replaced)
-    bool table_recorded = false;                // a recorded step reads it
+    bool table_recorded = false;                // a recorded step or reset reads it
     bool table_behind = false;                  // a change did not reach it (no memory for a new one): the next step makes up for that
     std::vector<ResidentLayer> entries;         // what the table holds
     uint32_t *xch = nullptr, *sync = nullptr;
@@ -1041,7 +1049,7 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
                     hipMemsetAsync(l.v_cache, 0, v_halfs * 2, ctx->stream) != hipSuccess)
                     rc = fail(ctx, HIPC_ERR_BACKEND, "decoder: cannot clear the KV cache");
             }
-            hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, 0, 0, nullptr, nullptr);
+            hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, 0, 0, ResidentReset{});
         }
         if (rc != HIPC_OK) {
             for (void *p : d->owned) (void)hipFree(p);
@@ -1187,7 +1195,12 @@ int hipc_decoder_reset(hipc_ctx *ctx, hipc_decoder *d, int32_t token, int32_t po
     if (!d) return HIPC_ERR_INVALID;
     return entry(ctx, [&]() -> int {
         HIPC_REQUIRE(ctx, token >= 0 && token < d->cfg.vocab && pos >= 0 && pos < d->cfg.max_seq, "decoder: bad token %d or position %d", token, pos);
-        hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, token, pos, d->xch, d->sync);
+        ResidentReset words{};
+        if (d->resident) {
+            words = ResidentReset{d->xch, d->sync, d->table, d->cfg.n_layers, d->cfg.n_kv_heads * d->cfg.head_dim, attn_v_stride(d->cfg.max_seq)};
+            if (ctx->capturing) d->table_recorded = true;
+        }
+        hipLaunchKernelGGL((dec_set_state_kernel), 1, 256, 0, ctx->stream, d->state, token, pos, words);
         HIPC_LAUNCHED(ctx);
         // the step expects the token embedded (x, xn, the position's rotary table): every step leaves that behind for
         // the next one, the reset does it for the first

@@ -51,6 +51,13 @@ struct ResidentArgs {
     float eps, scale, inv_hidden;
 };
 
+// What a reset puts in order behind a step that did not come to its end.
+struct ResidentReset {
+    uint32_t *xch, *sync;
+    const ResidentLayer *table;
+    int n_layers, v_rows, v_stride;   // v_rows: channels of all kv heads
+};
+
 bool resident_takes(const hipc_decoder_config &c);
 bool resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c);   // against the launch per product
 int resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const ResidentArgs &a, int workgroups);

@@ -429,6 +429,24 @@ def test_the_ways_out_of_the_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd
     dec.destroy()
 
 
+@pytest.mark.parametrize("polls", [1, 4, 10])
+@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
+def test_a_step_that_was_given_up(ctx, pkg, oracle, route, hidden, ffn, hd, nq, nkv, bs, polls):
+    """Steps whose threads run out of polls, with the launch just begun or within it, end, and the read reports them. A reset
+    to where they began makes the decoder as good as new, whatever they left in the cache and in the words workgroups exchange."""
+    dec, ref = three_layers(pkg, ctx, hidden, ffn, hd, nq, nkv, bs)
+    steps_match(ctx, dec, ref)
+    for _ in range(2):
+        route({"HIPC_DEC_POLLS": polls})
+        dec.reset(23, 69)
+        dec.step(), dec.step(), dec.step()
+        with pytest.raises(pkg.HipComputeError, match="did not come to its end"):
+            dec.read()
+        route({"HIPC_DEC_POLLS": -1})
+        steps_match(ctx, dec, ref)
+    dec.destroy()
+
+
 def test_decoders_on_several_streams_at_once(pkg):
     """Three contexts (a stream each) replay their recorded steps from three threads: launches that do not find room for
     all their workgroups beside each other go on with those that do, and every decoder picks the tokens it picks alone."""
