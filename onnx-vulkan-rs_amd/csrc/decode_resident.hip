@@ -73,7 +73,16 @@ constexpr int kPollBudget = 1 << 23;                   // polls of one thread in
 #else
 constexpr int kPollBudget = 1;                         // (one thread after the other: there is nobody to wait for)
 #endif
-constexpr int kArriveTicks = 20000;                    // 200 us of the 100 MHz clock: how long the launch waits for workgroups that have not started
+// How long workgroups that have not started are waited for, in ticks of the 100 MHz clock. All of them, 50 us: they arrive within
+// microseconds on a free device, and within the 50 us another decoder's unembedding and token pick keep some CUs. In the
+// stand-in until nobody has come for 5 us.
+// Beside other work, us a token of gemma3-1b at 2048 (454 alone; launches per product 654 alone), the launches per product / 50 us and
+// 256 workgroups standing in / 200 us and 256 / 200 us and 64: beside a softmax of eight workgroups of a millisecond 763 / 773 / 923 / 1602;
+// launches that hold 64 CUs for 220 us 730 / 908 / 835 / 1191, 128 CUs for 140 us 788 / 777 / 570 / 569; products that fill the chip for 125 us
+// at a time - / 860 / 860 / 872. Two decoders side by side, a token of each: 780 / 878 / 877 / 877; three 918 / 1900 / 2490 / 2060,
+// four 1061 / 2190 / 2880 / 2180: launches that each want the whole chip take turns at best, where short ones fill each other's
+// gaps (these figures scatter by a fifth), so contexts that decode at the same time are better off with HIPC_DEC_RESIDENT=0.
+constexpr int kArriveTicks = 5000, kJoinTicks = 500;
 constexpr int kResThreads = 512, kResWaves = 8;
 constexpr int kRedPitch = 20;                          // words per column of the reduction area: 16 k tiles, 16-byte rows
 constexpr int kSumsAt = 64 * 2 * 4 * 16;               // bytes from the row's terms to their chunks' sums (ResShared)
@@ -889,7 +898,7 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     }
     if (!ALL) {
         uint32_t here = 0;
-        if (tid == 0) S.decision[1] = res_join(words, gridDim.x, (unsigned long long)p.arrive, &here, tries), S.decision[0] = here;
+        if (tid == 0) S.decision[1] = res_join(words, gridDim.x, (unsigned long long)min(p.arrive, kJoinTicks), &here, tries), S.decision[0] = here;
     } else if (blockIdx.x != 0) {
         if (tid == 0) S.decision[0] = res_await(words, 2ull * (unsigned)p.arrive, tries);
     } else if (wave == 0) {
@@ -1025,7 +1034,7 @@ int hipc::resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const Res
     if (workgroups >= (int)kResGroups) {
         int rc = launch_hd<true>(ctx, c.head_dim, sg, a, kResGroups);
         if (rc != HIPC_OK) return rc;
-        a.behind = 1, workgroups = 64;   // fewer than there might be: it is there for the device that is shared
+        a.behind = 1, workgroups = kResGroups;   // (where it finds its work done, 256 workgroups that leave at once take no longer than 64)
     }
     return launch_hd<false>(ctx, c.head_dim, sg, a, workgroups);
 }

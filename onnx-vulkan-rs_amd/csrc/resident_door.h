@@ -57,14 +57,19 @@ __device__ __forceinline__ uint32_t res_await(uint32_t *words, unsigned long lon
     return d;
 }
 // Workgroups of the stand-in: the rank among the *n that take part, kResNoRank for one that comes too late. The first waits
-// `ticks` for `groups`; the others wait for the first, `tries` times at most.
+// for `groups`, until nobody has come for `ticks`; the others wait for the first, `tries` times at most.
 __device__ __forceinline__ uint32_t res_join(uint32_t *words, uint32_t groups, unsigned long long ticks, uint32_t *n, int &tries) {
     const uint32_t ticket = __hip_atomic_fetch_add(words + kResTickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (ticket & kResClosed) return kResNoRank;
     uint32_t d;
     if (ticket == 0) {
-        const unsigned long long t0 = wall_clock64();
-        while (res_look(words + kResTickets) < groups && wall_clock64() - t0 < ticks) {}
+        unsigned long long last = wall_clock64();   // when the last one came
+        uint32_t here, before = 1;
+        while ((here = res_look(words + kResTickets)) < groups) {
+            const unsigned long long now = wall_clock64();
+            if (here != before) before = here, last = now;
+            else if (now - last >= ticks) break;
+        }
         d = res_decision(__hip_atomic_fetch_or(words + kResTickets, kResClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), false);
         __hip_atomic_store(words + kResDecision, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
