@@ -23,7 +23,7 @@ namespace hipc {
 // workgroups tell each other their ranges. Us, both: 32768 values 4.04 / 4.62, 40960 4.36 / 4.62, 65536 5.7 / 4.65; of a GELU
 // 4097 4.31 / 4.9, 6000 4.59 / 4.9, 8192 5.1 / 5.0, 16384 6.7 / 5.0.
 constexpr int64_t kSmallPlain = 40960, kSmallGelu = 6144;
-constexpr long kMeetTicks = 5000;   // 50 us: several times what the workgroups of a launch are apart on a chip of their own
+constexpr long kMeetTicks = 1000;   // 10 us: twice what the workgroups of a launch are apart on a chip of their own (16 M values: 20.3 us with 5 us and more, 28 with 2 us)
 
 
 // Range partials of hipc_dynamic_quantize_linear_static: {bits(-min), bits(max)} per workgroup of
@@ -310,18 +310,23 @@ dql_small_kernel(const float *__restrict__ x, long n, uint8_t *__restrict__ y, f
 // the GELU where there is one, publish the workgroup's range, wait for the ranges of all workgroups and quantize what they hold.
 // Every value is read once and every GELU taken once; two launches do both twice. As few runs per thread as 256 workgroups
 // allow, since waiting for 256 costs little more than for 64: 1 M values 5.2 us with one run, 5.3, 5.9 and 7.8 with two, four
-// and eight. What bounds it: 1 M values the launch, the trip for the values and the two of the hand-over (5.2 us of which 1 us
-// is the copy's time), 4 M through a GELU its instructions (4.8 of 9.1 us), 8 M the memory (9.4 us, 4.5 TB/s). Against two
-// launches, us: 64 K values 4.65 / 4.8, 1 M 5.2 / 6.0, 4 M 6.6 / 8.7, 8 M 9.4 / 18.0, 16 M 18.9 / 30.4; through a GELU 16 K 5.0 / 5.6,
-// 1 M 5.6 / 7.3, 4 M 9.1 / 13.8, 8 M 14.5 / 26.2, 16 M 28.2 / 41.3.
+// and eight. What bounds it: 1 M values the launch, the trip for the values and the two of the hand-over (4.9 us of which 1 us
+// is the copy's time), 4 M through a GELU its instructions (4.8 of 9.0 us), 8 M the memory (9.4 us, 4.5 TB/s). Against two
+// launches, us: 64 K values 4.6 / 5.2, 1 M 4.9 / 6.1, 4 M 6.3 / 9.2, 8 M 9.4 / 18.2, 16 M 20.3 / 31.3; through a GELU 64 K 5.2 / 6.2,
+// 1 M 5.5 / 7.7, 4 M 9.0 / 14.3, 8 M 14.1 / 26.3, 16 M 29.4 / 42.2.
 //
 // The ranges are published eight times over and each workgroup reads one copy with one wavefront: all 256 workgroups polling
 // one copy with four wavefronts each took 8 us for what takes one.
 //
-// No workgroup depends on the others being on the chip with it. One that has waited `ticks` says so and leaves; the workgroup
-// that publishes last finds all ranges there, and then quantizes for those that left. (A workgroup that leaves looks once more
-// after it has said so: either it finds all ranges, or the last one publishes, and looks for leavers, after that. Both may
-// write the same values; no other order is possible.)
+// No workgroup depends on the others being on the chip with it. One that has waited long enough says so beside its range and
+// leaves, which makes room for one that has not started: of each XCD (to which a launch's workgroups are dealt in turn) the first
+// after `ticks`, then two, four, ... more at a time, the last after twice `ticks`, so that about as many leave as are missing.
+// Whoever finds all ranges there takes parts of those that left, one at a time. (A workgroup that leaves looks once more after it
+// has said so: either it finds all ranges, or the one that publishes last looks for leavers after that, and takes what
+// nobody else takes. Both may write the same values; no other order is possible.)
+// Calls waited for one by one, beside launches that hold CUs whole, us, two launches / one: 128 CUs for 140 us at a time, 4 M values
+// 24 / 21, 8 M 32 / 50, 16 M 45 / 62; 200 CUs, 1 M 19 / 33, 16 M 50 / 140; beside products that fill the chip for 125 us 220 / 110 to
+// 124 at any size. (When all left after 50 us and the last workgroup did their parts alone: 16 M beside 64 CUs held 1610.)
 //
 // A call uses one of two sets of words, empties the other, which nobody reads any more, and then makes that the next call's.
 #ifndef HIPC_HOST_MODEL
@@ -331,15 +336,16 @@ __device__ __forceinline__ long dql_now() { return (long)wall_clock64(); }
 inline void dql_stored() {}
 inline long dql_now() { return 0; }
 #endif
-constexpr uint64_t kThere = 0x8000000080000000ull;
-__device__ __forceinline__ void dql_put(uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+constexpr uint64_t kThere = 0x80000000ull, kLeft = 0x8000000000000000ull;   // (the sign bits, which a range does not need)
 template <int GELU, int V>
 __global__ void __launch_bounds__(1024)
 dql_once_kernel(const float *__restrict__ x, long n, uint32_t *meet, uint8_t *__restrict__ y, float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, long ticks, GeluParams g) {
     HIPC_PIN_SGPR(ticks);   // (read with the first arguments, not when the waiting begins)
     __shared__ float slow[16], shigh[16];
     __shared__ uint32_t joined[2];
-    __shared__ int seen[2];   // all ranges; at the first look
+    __shared__ int seen[2];   // all ranges; that some left
+    __shared__ uint64_t free_parts[kMeetMax / 64];
+    __shared__ int mine_now;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, groups = gridDim.x;
     // the 4096 values of run `r` of a workgroup, four to a thread
     auto load = [&](long r) {
@@ -382,31 +388,34 @@ dql_once_kernel(const float *__restrict__ x, long n, uint32_t *meet, uint8_t *__
     if (lane == 0) slow[wave] = low, shigh[wave] = high;
     __syncthreads();
     uint64_t *copies = reinterpret_cast<uint64_t *>(here);
-    uint32_t *gone = here + 2 * kMeetMax * kMeetCopies;
+    uint32_t *taken = here + 2 * kMeetMax * kMeetCopies;
+    uint64_t own = kThere;
+    auto publish = [&](uint64_t left) {
+        if (tid < kMeetCopies) __hip_atomic_store(copies + tid * kMeetMax + blockIdx.x, own | left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (wave == 0) dql_stored();
+    };
     if (tid < kMeetCopies) {
 #pragma unroll
         for (int w = 0; w < 16; w++) low = fmaxf(low, slow[w]), high = fmaxf(high, shigh[w]);
-        // (the sign bits, which a range does not need, say that it is there; -0.0 counts as 0)
-        const uint64_t pair = ((uint64_t)(__float_as_uint(low) | 0x80000000u) << 32) | (__float_as_uint(high) | 0x80000000u);
-        __hip_atomic_store(copies + tid * kMeetMax + blockIdx.x, pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        own |= ((uint64_t)(__float_as_uint(low) & 0x7fffffffu) << 32) | (__float_as_uint(high) & 0x7fffffffu);   // (-0.0 counts as 0)
     }
-    if (wave == 0) dql_stored();
+    publish(0);
     const uint64_t *mine = copies + (blockIdx.x % kMeetCopies) * kMeetMax;
-    int first_look = 0;
     auto look = [&](long wait) -> bool {   // are all ranges there, within `wait`?
         if (wave == 0) {
             uint64_t pair[kMeetMax / 64];
-            bool all;
+            bool all, left;
             const long t0 = dql_now();
-            for (first_look = 1;; first_look = 0) {
+            for (;;) {
                 bool there = true;
+                left = false;
 #pragma unroll
                 for (int q = 0; q < kMeetMax / 64; q++) {
                     pair[q] = kThere;
                     if (lane + 64 * q < groups) pair[q] = __hip_atomic_load(mine + lane + 64 * q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
 #pragma unroll
-                for (int q = 0; q < kMeetMax / 64; q++) there &= (pair[q] & kThere) == kThere;
+                for (int q = 0; q < kMeetMax / 64; q++) there &= (pair[q] & kThere) != 0, left |= (pair[q] & kLeft) != 0;
                 all = __all(there);
                 if (all || dql_now() - t0 >= wait) break;
             }
@@ -415,14 +424,15 @@ dql_once_kernel(const float *__restrict__ x, long n, uint32_t *meet, uint8_t *__
             for (int q = 0; q < kMeetMax / 64; q++)
                 low = fmaxf(low, __uint_as_float((uint32_t)(pair[q] >> 32) & 0x7fffffffu)), high = fmaxf(high, __uint_as_float((uint32_t)pair[q] & 0x7fffffffu));
             low = lean_wave_max(low), high = lean_wave_max(high);
-            if (lane == 0) joined[0] = __float_as_uint(low), joined[1] = __float_as_uint(high), seen[0] = all, seen[1] = first_look;
+            left = __any(left);
+            if (lane == 0) joined[0] = __float_as_uint(low), joined[1] = __float_as_uint(high), seen[0] = all, seen[1] = left;
         }
         __syncthreads();
         return seen[0];
     };
-    if (__builtin_expect(!look(ticks), 0)) {
-        if (tid == 0) dql_put(gone + blockIdx.x, 1u), dql_stored();
+    if (__builtin_expect(!look(ticks + ticks / 5 * (31 - __builtin_clz((blockIdx.x >> 3) + 1))), 0)) {
         __syncthreads();
+        publish(kLeft);
         if (!look(0)) return;
     }
     float scale, zp;
@@ -434,12 +444,31 @@ dql_once_kernel(const float *__restrict__ x, long n, uint32_t *meet, uint8_t *__
         if (tid == 0) *meet = set ^ 1u, *scale_out = scale, *zp_out = (uint8_t)zp;
     };
     if (blockIdx.x == 0) once();
-    const int left = (int)__hip_atomic_load(gone + min(tid, kMeetMax - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (0 behind the last workgroup's)
 #pragma unroll
     for (int u = 0; u < V; u++) store(first + u, dql_four(v[u], scale, rcp, zp));
-    if (__builtin_expect(!seen[1] || !__syncthreads_or(left), 1)) return;
-    for (int i = 0; i < groups; i++) {
-        if (i == (int)blockIdx.x || !__syncthreads_or(tid == i ? left : 0)) continue;
+    if (__builtin_expect(!seen[1], 1)) return;
+    for (;;) {   // (every round somebody takes a part: there are no more rounds than parts)
+        if (wave < kMeetMax / 64) {
+            bool free = false;
+            if (tid < groups && tid != (int)blockIdx.x)
+                free = (__hip_atomic_load(mine + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLeft) && !__hip_atomic_load(taken + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t parts = __ballot(free);
+            if (lane == 0) free_parts[wave] = parts;
+        }
+        __syncthreads();
+        int count = 0;
+#pragma unroll
+        for (int q = 0; q < kMeetMax / 64; q++) count += __popcll(free_parts[q]);
+        if (count == 0) return;
+        // not everyone the same: the workgroup's number modulo how many there are
+        int nth = (int)blockIdx.x % count, q = 0;
+        while (nth >= __popcll(free_parts[q])) nth -= __popcll(free_parts[q++]);
+        uint64_t parts = free_parts[q];
+        while (nth-- > 0) parts &= parts - 1;
+        const int i = 64 * q + __builtin_ctzll(parts);
+        if (tid == 0) mine_now = __hip_atomic_exchange(taken + i, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+        __syncthreads();
+        if (!mine_now) continue;
         if (i == 0) once();
 #pragma unroll 1
         for (int u = 0; u < V; u++) store((long)i * V + u, dql_four(gelu_load4<GELU>(load((long)i * V + u), g), scale, rcp, zp));

@@ -505,7 +505,7 @@ constexpr size_t kParamRange = 0;   // 8 B  {bits(-min), bits(max)}
 constexpr size_t kParamParts = 256; // 16 KiB: per-workgroup {bits(-min), bits(max)} pairs of DynamicQuantizeLinear
 constexpr int kParamPartsMax = 2048;
 // DynamicQuantizeLinear in one launch: the word that says which of two sets a call uses, and the sets: {max, -min} bits of each
-// workgroup (8 B), a copy for every eighth of the workgroups to read, and behind them a word per workgroup that gave up waiting.
+// workgroup (8 B), a copy for every eighth of the workgroups to read, and behind them a word per workgroup whose part another one took.
 // All zero when no call runs but for one set.
 constexpr int kMeetMax = 256, kMeetCopies = 8;
 constexpr size_t kParamMeet = kParamParts + 8 * kParamPartsMax;

@@ -188,7 +188,8 @@ inline float __expf(float v) { return std::exp(v); }
 inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xffffffu) * (b & 0xffffffu); }
 inline int __any(int v) { return v; }
 inline int __all(int) { return 1; }   // (what a wavefront would wait for counts as there: threads run one after the other)
-inline int __syncthreads_or(int v) { return v; }
+inline unsigned long long __ballot(int v) { return v ? 1 : 0; }
+inline int __popcll(unsigned long long v) { return __builtin_popcountll(v); }
 #ifndef __HIP_MEMORY_SCOPE_AGENT
 #define __HIP_MEMORY_SCOPE_AGENT 4
 #endif
@@ -196,6 +197,9 @@ template <typename T>
 inline void gpu_model_atomic_store(T *p, T v) { *p = v; }
 template <typename T>
 inline T gpu_model_atomic_load(const T *p) { return *p; }
+template <typename T>
+inline T gpu_model_atomic_exchange(T *p, T v) { const T was = *p; *p = v; return was; }
+#define __hip_atomic_exchange(p, v, order, scope) gpu_model_atomic_exchange(p, v)
 #define __hip_atomic_store(p, v, order, scope) gpu_model_atomic_store(p, v)
 #define __hip_atomic_load(p, order, scope) gpu_model_atomic_load(p)
 inline float rsqrtf(float v) { return 1.f / std::sqrt(v); }

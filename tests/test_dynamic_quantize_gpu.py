@@ -153,11 +153,11 @@ def test_sizes_around_the_launch_forms(ctx, pkg, oracle, n):
         assert np.array_equal(y, wy) and s == ws and z == wz
 
 
-@pytest.mark.parametrize("wait", [-1, 1], ids=["default", "nobody-waits"])
+@pytest.mark.parametrize("wait", [-1, 1, 100], ids=["default", "nobody-waits", "some-wait"])
 @pytest.mark.parametrize("n", [40963, 4096 * 255 + 1, 4096 * 256, 4096 * 256 + 1, 2 * 4096 * 256 + 2, 4 * 4096 * 256 + 3, 8 * 4096 * 256 + 4, 16 * 4096 * 256])
 def test_one_launch_of_many_workgroups_equals_two_launches(pkg, n, wait):
     """Each number of values a thread holds, at its largest size and one past the one before, byte for byte the two launches'
-    result; with workgroups that wait for the others and with ones that leave their part to the last; the range set by the
+    result; with workgroups that wait for the others, with ones that leave their parts to whoever comes last, and with some of each; the range set by the
     last, by the first and by a value in the middle, infinities and NaN; again from replays with other sizes between them."""
     ctx = pkg.Context(0)
     x = pkg.synth.normal_f32(n, 93)
