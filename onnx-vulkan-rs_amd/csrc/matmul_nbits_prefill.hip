@@ -749,16 +749,21 @@ mmnb_prefill_reduce_kernel(const float *__restrict__ part, __half *__restrict__ 
 
 namespace {
 
-// The tile grid cut into one rectangle per XCD, the k split (prefill_split option: 0 never splits k, n > 0 forces n
-// ways; unset: chosen by shape) with its partials in scratch memory; returns the launch grid in *grid.
-int prefill_plan(hipc_ctx *ctx, PrefillArgs &a, int TM, int TN, bool may_split, dim3 *grid) {
-    const int tiles_x = (int)ceil_div(a.N, TN), tiles_y = (int)ceil_div(a.M, TM);
-    int best = 8, best_cost = 1 << 30;
+// the rectangles the tile grid is cut into, one per XCD: how many along the rows (of eight)
+[[maybe_unused]] int prefill_xcd_rows(int64_t tiles_x, int64_t tiles_y) {
+    int best = 8;
+    int64_t best_cost = int64_t(1) << 40;
     for (int r = 1; r <= 8; r *= 2) {
-        const int cost = (int)(ceil_div(tiles_y, r) + ceil_div(tiles_x, 8 / r));
+        const int64_t cost = ceil_div(tiles_y, r) + ceil_div(tiles_x, 8 / r);
         if (cost < best_cost) best_cost = cost, best = r;
     }
-    a.xcd_rows = best, a.xcd_cols = 8 / best;
+    return best;
+}
+// The tile grid cut into one rectangle per XCD, the k split (prefill_split option: 0 never splits k, n > 0 forces n
+// ways; unset: as a.ksplit says, or, where that is 0, chosen by shape) with its partials in scratch memory; returns the launch grid in *grid.
+int prefill_plan(hipc_ctx *ctx, PrefillArgs &a, int TM, int TN, bool may_split, dim3 *grid) {
+    const int tiles_x = (int)ceil_div(a.N, TN), tiles_y = (int)ceil_div(a.M, TM);
+    a.xcd_rows = prefill_xcd_rows(tiles_x, tiles_y), a.xcd_cols = 8 / a.xcd_rows;
     const unsigned gx = 8u * (unsigned)(ceil_div(tiles_y, a.xcd_rows) * ceil_div(tiles_x, a.xcd_cols));
     // Too few tiles for the chip: split k over workgroups, as many ways as gives every CU a
     // workgroup, at least 32 stages each (with fewer, the second launch and the partials cost more
@@ -769,13 +774,14 @@ int prefill_plan(hipc_ctx *ctx, PrefillArgs &a, int TM, int TN, bool may_split, 
     const int g_prefill_split = ctx->tune.prefill_split;
     if (may_split && g_prefill_split != 0) {
         const int tiles = tiles_x * tiles_y;
-        ksplit = g_prefill_split > 0 ? g_prefill_split : std::min(4, ctx->cu_count / std::max(1, tiles));
-        ksplit = std::max(1, std::min(ksplit, g_prefill_split > 0 ? nk / 2 : nk / 32));
+        const int asked = g_prefill_split > 0 ? g_prefill_split : a.ksplit;
+        ksplit = asked > 0 ? asked : std::min(4, ctx->cu_count / std::max(1, tiles));
+        ksplit = std::max(1, std::min(ksplit, asked > 0 ? nk / 2 : nk / 32));
     }
     a.split_stages = (int)(ceil_div(ceil_div(nk, ksplit), 2) * 2);
     a.ksplit = (int)ceil_div(nk, a.split_stages);
     a.Ypart = nullptr;
-    const size_t part_bytes = (size_t)a.ksplit * a.M * a.N * sizeof(float);
+    const size_t part_bytes = (size_t)a.ksplit * (a.pair_rows > 0 ? a.pair_rows : a.M) * a.N * sizeof(float);
     if (a.ksplit > 1 && !scratch_fits(ctx, 0, part_bytes)) a.split_stages = (int)(ceil_div(nk, 2) * 2), a.ksplit = 1;
     if (a.ksplit > 1) {
         void *part = nullptr;
@@ -848,13 +854,14 @@ int prefill_launch_direct(hipc_ctx *ctx, PrefillArgs a) {
     const int trips = (a.split_stages + 1) / 2, forced = ctx->tune.prefill_groups;
     const long wgs = (long)ceil_div(a.M, T) * ceil_div(a.N, TN) * a.ksplit;
     // Two k groups per workgroup (four of paired rows where a group is two wavefronts) when the launch leaves the second
-    // wavefront slot of the SIMDs empty (128-row tiles: no more workgroups than CUs; 64-row tiles: no more than two per CU,
+    // wavefront slot of the SIMDs empty (128-row tiles and 96x128 ones of three terms: no more workgroups than CUs, 400 x 1152 x 4096
+    // in three terms 26.5 us with one group, 33.4 with two; 64-row tiles: no more than two per CU,
     // 512 x 2048 x 2560: 15.9 against 16.9 us, four groups, 18.3 us, cost more in prologues than they hide) and every group
     // gets two trips or more; prefill_groups 1 / 2 forces the choice. (three column blocks and two groups leave no register
     // for more than one scale per weight tile)
     constexpr int kGroups = WM * WN == 2 ? 4 : 2;
     if constexpr (NJ < 3 || SG == 1) {
-        if (forced == 1 ? false : forced == 2 ? true : wgs <= (T < 128 ? 2 : 1) * ctx->cu_count && trips >= 2 * kGroups) {
+        if (forced == 1 ? false : forced == 2 ? true : wgs <= (T < 128 && !(TERMS == 3 && WM * WN == 4) ? 2 : 1) * ctx->cu_count && trips >= 2 * kGroups) {
             if (int rc = prefill_launch_direct_groups<SG, MI, NJ, WM, WN, kGroups, TERMS>(ctx, a, grid)) return rc;
             return prefill_join_splits(ctx, a);
         }
@@ -937,7 +944,7 @@ int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) 
 
 namespace {
 
-// Tiles of paired rows: 64x64 where there are few tiles and k is not long enough to split three ways over workgroups; else
+// Tiles of rows in two terms: 64x64 where there are few tiles and k is not long enough to split three ways over workgroups; else
 // 64x128, or the larger ones where these take fewer rounds of workgroups times stages: 128x128 (64 f32 rows to a wavefront)
 // with four scales per weight tile, 64x256 with one or two. They do two 64x128 tiles' work in 15/16 of the time. Measured,
 // 64x64 / 64x128 / larger, us: 333 x 1152 x 13824 in blocks of 32 44.0 / 37.1 / 42.1, 1000 x 2048 x 4096 62.1 / 53.1 / 50.4,
@@ -953,15 +960,48 @@ int prefill_pair_tile(hipc_ctx *ctx, const PrefillArgs &a) {
         const int64_t ways = std::max<int64_t>(1, std::min(most, cus / tiles));
         return ceil_div(tiles * ways, cus) * ceil_div(stages, ways);
     };
-    // three terms: half as wide where that leaves fewer CUs idle in the last round, at 0.55 of a 96x128 tile's work (512 x 2048 x
-    // 2560 in blocks of 128 39.4 us in two rounds, 35.3 in three of half the work; 2000 x 2048 x 2048 63.6 and 77.5, 512 x 4096 x 4096 70.0 and 74.1)
-    if (a.terms == 3 && mid > cus && 11 * ceil_div(rows64 * ceil_div(a.N, 64), cus) < 20 * ceil_div(mid, cus)) return 64;
-    return a.terms == 2 && 2 * 15 * cost(large) < 16 * cost(mid) ? 192 : 128;
+    return 2 * 15 * cost(large) < 16 * cost(mid) ? 192 : 128;
+}
+// Rows in three terms: tiles of 96x64 or 96x128, and how many ways k is split over workgroups, by an estimate of the call in us:
+// a workgroup's stages times the rounds of workgroups on the XCD that has most of them (less than proportionally, since rounds overlap;
+// 96x64 tiles of one group go two to a CU), and the join of a split's partials. Its constants are a fit to calls of 40 to 1000
+// rows, k 1152 to 11008, n 1024 to 6912; over 133 of them what it picks is 1 % behind the best of the eight on average. Measured, us, each
+// term's rows by themselves through the kernel for f16 rows / the fewest rounds, split only where that leaves CUs idle / this:
+// 64 x 1152 x 1152 in blocks of 32 14.7 / 16.1 / 13.1, 200 x 6912 x 1152 in blocks of 64 43.3 / 47.4 / 39.1, 400 x 4096 x 1152 in blocks
+// of 64 41.3 / 54.4 / 35.1, 1000 x 11008 x 1152 in blocks of 32 154 / 187 / 135, 400 x 6912 x 4096 in blocks of 32 166 / 123 / 107; 64 x 11008 x 1024
+// in blocks of 128 stays at 28.6 / 33.6 / 30.9.
+template <int SG>
+int prefill_pinned_tile(hipc_ctx *ctx, const PrefillArgs &a, int *ways_out) {
+    const int64_t cus = std::max(1, ctx->cu_count), xcd_cus = std::max<int64_t>(1, cus / 8), stages = ceil_div(a.K, kPK), rows = ceil_div(a.M, 96);
+    const double scales = SG == 4 ? 1.07 : SG == 2 ? 1. : 0.85, values = (double)a.pair_rows * a.N;
+    const int most = ctx->tune.prefill_split == 0 ? 1 : 4;
+    int tile = 128;
+    double best = 1e30;
+    *ways_out = 1;
+    for (int T : {64, 128}) {
+        const int64_t cols = ceil_div(a.N, T);
+        const int r = prefill_xcd_rows(cols, rows);
+        for (int asked = 1; asked <= most; asked++) {   // (as prefill_plan and prefill_launch_direct will have it)
+            const int64_t split = std::max<int64_t>(1, std::min<int64_t>(asked, stages / 2)), own = ceil_div(ceil_div(stages, split), 2) * 2, ways = ceil_div(stages, own);
+            const bool groups = rows * cols * ways <= (T == 64 ? 2 : 1) * cus && (own + 1) / 2 >= (T == 64 ? 8 : 4);
+            const double load = (double)(ceil_div(rows, r) * ceil_div(cols, 8 / r) * ways) / xcd_cus;
+            const double rounds = std::max(1., T == 64 && !groups ? std::ceil(2 * load) / 2 : std::ceil(load));
+            const double first = T == 64 ? (groups ? 0.33 : 0.39) : 0.48, more = T == 64 ? (groups ? 0.39 : 0.33) : groups ? 0.48 : 0.4;
+            double us = (T == 64 ? (groups ? 10.23 : 9.46) : groups ? 8.36 : 7.23) + scales * own * (first + more * (rounds - 1));
+            if (ways > 1) us += 2.34 + 1.35e-6 * ways * values;
+            if (us < best) best = us, tile = T, *ways_out = asked;
+        }
+    }
+    return tile;
 }
 template <int SG>
 int prefill_launch(hipc_ctx *ctx, const PrefillArgs &a) {
     const int forced = ctx->tune.prefill_tile, g_prefill_split = ctx->tune.prefill_split;
-    if (a.pair_rows > 0) return prefill_launch_terms(ctx, a, SG, forced == 64 || forced == 128 || forced == 192 ? forced : prefill_pair_tile<SG>(ctx, a));
+    if (a.pair_rows > 0) {
+        PrefillArgs b = a;
+        const int tile = forced == 64 || forced == 128 || forced == 192 ? forced : a.terms == 3 ? prefill_pinned_tile<SG>(ctx, a, &b.ksplit) : prefill_pair_tile<SG>(ctx, a);
+        return prefill_launch_terms(ctx, b, SG, tile);
+    }
     // 128-row tiles when they give every CU a workgroup, directly or (long k) with k split over up
     // to four workgroups per tile; else 64x64
     const int64_t rows128 = ceil_div(a.M, 128), tiles128 = rows128 * ceil_div(a.N, 128), tiles192 = rows128 * ceil_div(a.N, 192);
