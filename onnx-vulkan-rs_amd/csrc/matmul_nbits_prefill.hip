@@ -944,7 +944,8 @@ int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile) 
 
 namespace {
 
-// Tiles of rows in two terms: 64x64 where there are few tiles and k is not long enough to split three ways over workgroups; else
+// Tiles of rows in two terms: 64x64 where there are few tiles, k is not long enough to split three ways over workgroups and no
+// XCD gets more workgroups than it has CUs (400 x 1152 x 1152, 234 tiles of which one XCD gets 35: 21.0 us, 15.5 on 64x128); else
 // 64x128, or the larger ones where these take fewer rounds of workgroups times stages: 128x128 (64 f32 rows to a wavefront)
 // with four scales per weight tile, 64x256 with one or two. They do two 64x128 tiles' work in 15/16 of the time. Measured,
 // 64x64 / 64x128 / larger, us: 333 x 1152 x 13824 in blocks of 32 44.0 / 37.1 / 42.1, 1000 x 2048 x 4096 62.1 / 53.1 / 50.4,
@@ -952,10 +953,12 @@ namespace {
 // of 128 600 x 8192 x 1024 60.9 / 48.3 / 38.4.
 template <int SG>
 int prefill_pair_tile(hipc_ctx *ctx, const PrefillArgs &a) {
-    const int64_t cus = std::max(1, ctx->cu_count), rows64 = ceil_div(a.M, 32 * a.terms), stages = ceil_div(a.K, kPK);
+    const int64_t cus = std::max(1, ctx->cu_count), rows64 = ceil_div(a.M, 64), stages = ceil_div(a.K, kPK);
     const int64_t most = ctx->tune.prefill_split == 0 ? 1 : std::max<int64_t>(1, std::min<int64_t>(4, stages / 32));   // (see prefill_plan)
     const int64_t mid = rows64 * ceil_div(a.N, 128), large = SG <= 2 ? rows64 * ceil_div(a.N, 256) : ceil_div(a.M, 128) * ceil_div(a.N, 128);
-    if (mid <= cus / 2 && most < 3) return 64;
+    const int64_t cols64 = ceil_div(a.N, 64), xcd_rows = prefill_xcd_rows(cols64, rows64);
+    const int64_t per_xcd = ceil_div(rows64, xcd_rows) * ceil_div(cols64, 8 / xcd_rows) * std::max<int64_t>(1, std::min(most, cus / (rows64 * cols64)));
+    if (mid <= cus / 2 && most < 3 && 8 * per_xcd <= cus) return 64;
     auto cost = [&](int64_t tiles) {
         const int64_t ways = std::max<int64_t>(1, std::min(most, cus / tiles));
         return ceil_div(tiles * ways, cus) * ceil_div(stages, ways);
