@@ -129,14 +129,14 @@ def test_attention_over_a_long_filled_cache(ctx, pkg, oracle, route, hd, nq, nkv
 
 @pytest.mark.parametrize("nq,max_seq", [(8, 16384), (8, 16385), (4, 32768), (4, 32769)])
 def test_the_longest_context_that_keeps_all_layers_in_one_launch(ctx, pkg, route, nq, max_seq):
-    """Heads times positions choose between one launch and the launches per product: the last length of each side at its
-    last positions, against the launches per product over the same cache."""
+    """All layers in one launch over the longest contexts, at the last position, against the launches per product over the
+    same cache. (Which of the two forms a decoder takes by itself: tests/host/decoder_model.cpp.)"""
     cfg = dict(SMALL, n_q_heads=nq, n_kv_heads=1, head_dim=64)
     w = pkg.decoder.build_weights(cfg, seed=14)
     rng = np.random.default_rng(nq)
     rows = [tuple((rng.standard_normal((1, max_seq, 64)) * 0.7).astype(np.float16) for _ in range(2)) for _ in range(cfg["n_layers"])]
     got = []
-    for resident in (-1, 0):
+    for resident in (256, 0):
         route({"HIPC_DEC_RESIDENT": resident})
         dec = pkg.decoder.Decoder(ctx, cfg, max_seq)
         dec.load(w)
