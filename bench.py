@@ -382,9 +382,10 @@ def bench_decoder(pkg, ctx, steps, warmup, context=2048):
     tok_s = steps / dt
     out = dict(tok_s=tok_s, ms_per_token=dt / steps * 1e3, context=context, bytes_per_token=byts,
                hbm_bound_tok_s=HBM_PEAK_GBS * 1e9 / byts, frac_of_hbm_bound=tok_s * byts / (HBM_PEAK_GBS * 1e9),
-               # all layers, the unembedding (whose workgroups leave the argmax candidates) and the
-               # launch that picks the token and embeds it for the next step
-               launches_per_token=3, final_position=pos)
+               # all layers, the launch that stands in for that one where it finds no room, the unembedding (whose workgroups
+               # leave the argmax candidates) and the one that picks the token and embeds it for the next step (unknown
+               # where a switch may have chosen other launches)
+               launches_per_token=None if any(k.startswith(("HIPC_DEC_", "HIPC_GEMV_")) for k in os.environ) else 4, final_position=pos)
     # the same step as five launches per layer, without read-ahead helper rows and with all five launches carrying them
     # (extra workgroups that read what the next launch will read into the L2 of the XCD that will ask for it)
     for name, mask in (("no_read_ahead", 0), ("read_ahead_all_five", 31)):
@@ -421,12 +422,52 @@ ATTN_PHASES = {0: "first instruction (arguments read)", 1: "position arrived", 2
                8: "first pass: value product", 9: "all passes done", 10: "partials stored"}
 
 
+# in the order a workgroup passes them
+RESIDENT_PHASES = {0: "layer begins", 2: "norm of the row, terms in LDS", 3: "q|k|v products", 4: "q|k|v handed over", 1: "query, key, value arrived",
+                   5: "heads normed and rotated", 28: "own stores and loads done", 6: "workgroup barrier", 7: "cache passes", 8: "attention handed over",
+                   9: "the XCD's chunks arrived", 26: "chunks joined", 10: "terms in LDS", 11: "o products", 12: "o's partial row handed over",
+                   13: "partial rows summed", 14: "the row arrived", 15: "norm of the row", 16: "gate|up products", 17: "gated row handed over",
+                   18: "gated row arrived", 19: "workgroup barrier (2)", 20: "down products", 21: "down's partial row handed over",
+                   22: "partial rows summed (2)", 23: "the next row arrived"}
+
+
+def resident_phases(lib, ctx, dec, context):
+    """The same of one layer inside the launch that holds all of them: shader clocks since the workgroup began the layer, of its
+    last wavefront to pass each point (the clocks of two workgroups cannot be compared)."""
+    import ctypes
+    dec.reset(1234, context - 1)
+    dec.step()
+    ctx.flush()
+    ctx.capture_begin()
+    dec.step()
+    g = ctx.capture_end()
+    for _ in range(20):
+        ctx.graph_launch(g)
+    ctx.flush()
+    ctx.graph_destroy(g)
+    st = np.zeros(256 * 8 * 32, dtype=np.uint64)
+    fn = lib.hipc_debug_resident_stamps
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_size_t]
+    if fn(st.ctypes.data_as(ctypes.c_void_p), st.nbytes) != 0:
+        raise RuntimeError("reading the stamps failed")
+    st = st.reshape(256, 8, 32).astype(np.int64)
+    begin = st[:, :, 0].min(axis=1)
+    since = st - begin[:, None, None]
+    out = {}
+    for ph, label in RESIDENT_PHASES.items():
+        v = np.where((since[:, :, ph] >= 0) & (since[:, :, ph] < 1 << 20), since[:, :, ph], -1).max(axis=1)   # (a place no wavefront passed holds an older stamp)
+        v = v[v >= 0]
+        if v.size:
+            out[label] = dict(workgroups=int(v.size), median=int(np.median(v)), p90=int(np.percentile(v, 90)), max=int(v.max()))
+    return dict(clocks_since_the_layer_began=out)
+
+
 def bench_phases(pkg, ctx, context=2048):
     """Where the time of a decode step's launches goes: the library built by `make stamps` (load it with
     HIPC_LIBRARY=libhipcompute_stamps.so) records the device clock (10 ns ticks) at fixed points of the one-row kernels
     and of the attention kernel; this reads the stamps the LAST layer's launches left after a replayed step and
     reports, per launch, the median / 90th percentile / maximum over its wavefronts of the time since the launch's
-    first wavefront started, and the gaps between the launches."""
+    first wavefront started, and the gaps between the launches; then the points of one layer of the launch that holds all."""
     import ctypes
     lib = pkg.runtime.load_library()
     if not hasattr(lib, "hipc_debug_lean_stamps"):
@@ -489,9 +530,10 @@ def bench_phases(pkg, ctx, context=2048):
         prev_end = end
         out[name] = rec
     ctx.graph_destroy(g)
+    one = resident_phases(lib, ctx, dec, context)
     dec.destroy()
     ctx.flush()
-    return out
+    return out, one
 
 
 F16_PEAK_TFLOPS = 2500.0    # MI355X dense f16 MFMA, published
@@ -645,13 +687,17 @@ def main():
         extras["gemma3_1b_int4_decode"] = bench_decoder(pkg, ctx, max(args.steps, 20), args.warmup)
         log("[bench] decoder:", json.dumps(extras["gemma3_1b_int4_decode"]))
     if "phases" in only:
-        extras["decode_step_phases_last_layer"] = bench_phases(pkg, ctx)
+        extras["decode_step_phases_last_layer"], one = bench_phases(pkg, ctx)
+        extras["decode_step_phases_one_launch"] = one
         for name, rec in extras["decode_step_phases_last_layer"].items():
             log(f"[bench] {name}: {rec['wavefronts']} wavefronts, {rec['duration_ns']} ns" +
                 (f", {rec['gap_from_previous_launch_ns']} ns after the launch before it ended" if "gap_from_previous_launch_ns" in rec else "") +
                 (f"; helper rows {json.dumps(rec['helper_rows_ns'])}" if "helper_rows_ns" in rec else ""))
             for label, v in rec["phases_ns"].items():
                 log(f"[bench]     {label:52s} median {v['median']:6d}  p90 {v['p90']:6d}  max {v['max']:6d} ns")
+        log("[bench] one layer of the launch that holds all: clocks since the workgroup began it")
+        for label, v in one["clocks_since_the_layer_began"].items():
+            log(f"[bench]     {label:52s} median {v['median']:6d}  p90 {v['p90']:6d}  max {v['max']:6d}  ({v['workgroups']} workgroups)")
     if "copy" in only:
         extras["copy_256MiB"] = bench_copy(ctx)
         log("[bench] copy:", json.dumps(extras["copy_256MiB"]))
