@@ -872,13 +872,14 @@ int prefill_launch_direct(hipc_ctx *ctx, PrefillArgs a) {
 
 }  // namespace
 
-// This file is compiled three times. The 128x128 instances live in an object of their own, built with
-// HIPC_PREFILL_WIDE and with the matrix-core accumulators in ordinary vector registers (the block
-// scales then multiply them without copies out of the accumulation file: 48.5 -> 44.7 us for
-// 512 x 2048 x 11008); the 64x64 instances are faster with the accumulation file (80.6 against
-// 87.9 us for 512 x 11008 x 2048), and that is a switch of the whole compilation.
+// This file is compiled three times, since where the compiler keeps matrix-core accumulators is a switch of the whole
+// compilation. HIPC_PREFILL_WIDE: the kernel that keeps the weight out of LDS, and the 128x128 tiles of the other one, with
+// accumulators in ordinary vector registers (the block scales then multiply them without copies out of the accumulation file:
+// 48.5 -> 44.7 us for 512 x 2048 x 11008). HIPC_PREFILL_TERMS: the instances for rows in terms, in ordinary registers, too, and without
+// sinking (see the Makefile). Without either: the 64x64 tiles with both operands in LDS, which are faster with the accumulation
+// file (80.6 against 87.9 us for 512 x 11008 x 2048), the rules and the entry points.
 int prefill_launch_wide(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile);
-int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile);   // rows in terms: an object of its own, too (see the Makefile)
+int prefill_launch_terms(hipc_ctx *ctx, const PrefillArgs &a, int SG, int tile);
 
 #ifdef HIPC_PREFILL_WIDE
 
