@@ -361,6 +361,22 @@ def test_terms_of_f32_rows_added_in_one_accumulator(ctx, pkg, shape, level, tile
     assert np.all(np.abs(got - f64) <= bound), float(np.max(np.abs(got - f64) / bound))
 
 
+@pytest.mark.parametrize("shape", [(400, 192, 1152, 32, True), (400, 136, 1090, 64, False), (384, 192, 1024, 128, True)], ids=lambda s: "M%d_K%d_N%d_bs%d_zp%d" % s)
+def test_f32_rows_by_the_tiles_an_xcd_gets(ctx, pkg, shape):
+    """Two terms on either side of the rule that leaves 64x64 tiles where one XCD would get more of them than it has CUs (35, 35
+    and 32 of 32): against float64, within the bound of the test above."""
+    m, k, n, bs, with_zp = shape
+    B, scales, zp = pkg.synth.nbits_weight(n, k, bs, seed=67, with_zp=with_zp)
+    a = pkg.synth.normal_f32(m * k, 68).reshape(m, k)
+    nib, z = _unpack(B, zp if zp is not None else np.full((n, (-(-k // bs) + 1) // 2), 0x88, np.uint8), k, n, bs)
+    w64 = (nib.astype(np.float64) - z.repeat(bs, axis=1)[:, :k]) * scales.reshape(n, -1).astype(np.float64).repeat(bs, axis=1)[:, :k]
+    absw = np.abs(w64)
+    bound = np.abs(a).max(axis=1, keepdims=True).astype(np.float64) * 2.0 ** -21 * absw.sum(axis=1) + (k + 8) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ absw.T)
+    got = pkg.ops.matmul_nbits(ctx, a, B, scales, zp, k, n, bs)
+    err = np.abs(got - a.astype(np.float64) @ w64.T)
+    assert np.all(err <= bound), float(np.max(err / bound))
+
+
 @pytest.mark.parametrize("shape", [(33, 1152, 64, 32, True), (64, 1096, 1154, 64, False), (100, 2056, 257, 128, True), (200, 4096, 130, 32, False),
                                    (400, 1152, 1152, 128, True), (1000, 776, 1030, 256, False)], ids=lambda s: "M%d_K%d_N%d_bs%d_zp%d" % s)
 def test_f32_pinned_rows_with_k_split_by_shape(ctx, pkg, shape):
