@@ -15,7 +15,7 @@
 //   * XCD x holds the ffn columns of the 128-k tiles x, x + 8, ... of the down projection: gate|up columns and down rows
 //     of its own, so the gated row never leaves it; the down product's partial rows are summed like o's.
 // Per layer four hand-overs stay inside the XCDs and three cross them. Weights and cache rows do not depend on the row, so
-// every phase's are asked for two phases ahead, straight into registers (17 MB a layer are 68 KB a workgroup).
+// they are asked for ahead: weights (17 MB a layer are 68 KB a workgroup) into LDS, by wavefronts of their own; cache rows into registers.
 //
 // Hand-overs carry their own "ready": an empty word is all ones (no result has that pattern, see put()), readers poll the
 // words themselves (agent scope loads), so a hand-over is one store and one load, without flags or fences. There are three
@@ -33,6 +33,8 @@
 // are bounded beside that: a thread's polls of a whole launch are counted.
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "internal.h"
 #include "lanes.h"
 #include "lean_ops.h"
@@ -41,9 +43,9 @@
 namespace hipc {
 
 #ifndef HIPC_HOST_MODEL
-#define RES_ONE_PER_CU __attribute__((amdgpu_waves_per_eu(2, 2)))   // two wavefronts a SIMD: 256 registers each
+#define RES_ONE_PER_CU(all) __attribute__((amdgpu_waves_per_eu((all) ? 3 : 2, (all) ? 3 : 2)))   // three (two) wavefronts a SIMD: 168 (256) registers each
 #else
-#define RES_ONE_PER_CU
+#define RES_ONE_PER_CU(all)
 #endif
 
 // phase time stamps (library built with `make stamps` only; see gemv_lean.hip): res_stamps[workgroup][wavefront][phase] of one
@@ -54,7 +56,7 @@ __device__ unsigned long long res_stamps[256 * 8 * 32];
 #define RES_STAMP(ph)                                                                      \
     do {                                                                                   \
         const unsigned long long t_ = (unsigned long long)clock64();                       \
-        if ((threadIdx.x & 63) == 0) S.stamp[threadIdx.x >> 6][ph] = t_;                   \
+        if ((threadIdx.x & 63) == 0) S.stamp[threadIdx.x >> 6][ph] = (uint32_t)t_;                   \
     } while (0)
 #define RES_STAMPS_OUT()                                                                   \
     do {                                                                                   \
@@ -83,10 +85,10 @@ constexpr int kPollBudget = 1;                         // (one thread after the 
 // four 1061 / 2190 / 2880 / 2180: launches that each want the whole chip take turns at best, where short ones fill each other's
 // gaps (these figures scatter by a fifth), so contexts that decode at the same time are better off with HIPC_DEC_RESIDENT=0.
 constexpr int kArriveTicks = 5000, kJoinTicks = 500;
-constexpr int kResThreads = 512, kResWaves = 8;
-constexpr int kRedPitch = 20;                          // words per column of the reduction area: 16 k tiles, 16-byte rows
-constexpr int kSumsAt = 64 * 2 * 4 * 16;               // bytes from the row's terms to their chunks' sums (ResShared)
-constexpr int kResUnits = 12;                          // units a thread's wavefront asks for ahead, all phases
+constexpr int kResThreads = 512, kResWaves = 8;        // those that compute
+constexpr int kFeedWaves = 4;                          // and, in the launch of all, those that bring the weights: one per product
+constexpr int kResSlots = 104;                         // units of weights in LDS (see resident_launch)
+constexpr int kRowPitch = 384;                         // bytes of a k tile of the row: three digits of 128 values
 constexpr int kEntryWords = (int)(sizeof(ResidentLayer) / 4);
 
 typedef _Float16 rh16x8 __attribute__((ext_vector_type(8)));
@@ -100,67 +102,90 @@ __device__ __forceinline__ void res_stored() {
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), in a form the compiler takes into account
     res_reload();
 }   // every store of this wavefront is where its scope says
+#define RES_TOGETHER() __builtin_amdgcn_sched_barrier(0)   // no instruction is moved across
+#define RES_BARRIER()                  \
+    do {                               \
+        res_reload();                  \
+        __builtin_amdgcn_s_barrier();  \
+        res_reload();                  \
+    } while (0)   // without a wait for anything
 #else
 inline void res_stored() {}
+#define RES_TOGETHER() ((void)0)
+#define RES_BARRIER() __syncthreads()
 #endif
 
-// A wavefront's share of a phase's product: up to U (column tile, k tile) units, one after the other 128 k of 16 columns.
-// Which units they are does not change between layers: their byte offsets are worked out once and kept in LDS (kept in
-// registers, they and the weights of three phases do not fit).
-// The sums of a unit are the same in all four groups of 16 lanes, so one group's are enough: group g takes those of units
-// g, 4 + g, ... and holds the scales and zero points of these only, asked for together with three other units'.
-template <int U, int SG>
-struct Units {
-    uint4 wq[U];
-    ScaleVecLean<SG> sv[(U + 3) / 4];
-    uint32_t live;   // bit i: unit i exists
+// A product is done in units: 128 k (a k tile) of 16 columns (a tile), 1 KB of weight. In the launch of all, four wavefronts of
+// their own bring a workgroup's units into LDS (res_feed), one product's each, a whole layer ahead: what a phase has consumed is
+// asked for again, for the next layer or for this one, as the product leaves its places. When matters: a CU's loads return in the order
+// they were asked for, whichever wavefront asked, so a poll behind weights waits for HBM (measured: a poll of 0.09 us takes up to 1 us
+// behind 4 KB of them, 1.5 us behind 36 KB). So they are asked for behind the barrier that follows a poll, with work in front
+// of the next one: gate|up's where a layer begins (kFeedFirst units), behind the heads' barrier (up to kFeedHeads) and where
+// the chunks have arrived; o's where a layer begins, down's where the hidden row has arrived, the next layer's q|k|v where
+// the gated row has. Us for eight tokens of gemma3-1b at 2048: all of a product's at once as soon as its places are free 3955; so spread
+// 3560; in the registers of the polling wavefronts, two phases ahead, 3725. (Eight layers of 2048 / 8192 with 8/1 heads of 256 at 2040,
+// where those registers held half of the units: 201 -> 185; of 512 / 2048 with 8/2 heads of 64: 123 -> 119.)
+//
+// The row takes part as whole numbers: 23 bits below the largest of every 32 values, as three signed bytes (digits), so a
+// product of a unit is two int8 matrix instructions with exact sums, and a weight's nibbles need no conversion beyond being
+// spread to bytes. The 16 rows of the matrix operand are the four 32-k chunks times the digits (the fourth of each is
+// empty): lane group g ends with the sums of chunk g. Two bf16 terms per value (17 bits) took twice the instructions a unit.
+typedef int ri32x4 __attribute__((ext_vector_type(4)));
+
+struct UnitWeight {
+    uint4 w;
+    float s;      // of the lane's column and chunk
+    uint32_t z;   // 128 + zero point
 };
 
-// A product unit against the row's terms in LDS (see mmnb_lean_kernel). The lanes that hold the unit's scales return their column's sum.
-template <int SG>
-__device__ __forceinline__ float res_unit(const uint4 &wq, const ScaleVecLean<SG> &sv, const char *as, uint32_t o_as, uint32_t nib_mask, uint32_t magic) {
-    constexpr int CPG = 4 / SG;
-    uint4 a[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) a[j] = *reinterpret_cast<const uint4 *>(as + o_as + j * 128);
-    const float4 bs = *reinterpret_cast<const float4 *>(as + kSumsAt + ((o_as >> 9) << 4));
-    lf32x4 d[SG];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t word = j == 0 ? wq.x : j == 1 ? wq.y : j == 2 ? wq.z : wq.w;
-        const uint4 bw = make_uint4((word & nib_mask) | magic, ((word >> 4) & nib_mask) | magic, ((word >> 8) & nib_mask) | magic, ((word >> 12) & nib_mask) | magic);
-        const int g = j / CPG;
-        d[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lbf16x8, a[j]), __builtin_bit_cast(lbf16x8, bw), (j % CPG) == 0 ? lf32x4{0.f, 0.f, 0.f, 0.f} : d[g], 0, 0, 0);
-    }
-    float acc = 0.f;
-#pragma unroll
-    for (int g = 0; g < SG; g++) {
-        const float dsum = d[g][0] + d[g][1];
-        float asg;
-        if (SG == 4) asg = g == 0 ? bs.x : g == 1 ? bs.y : g == 2 ? bs.z : bs.w;
-        else if (SG == 2) asg = g == 0 ? bs.x + bs.y : bs.z + bs.w;
-        else asg = (bs.x + bs.y) + (bs.z + bs.w);
-        const float zb = (float)((sv.z >> (8 * g)) & 0xffu);
-        acc = fmaf(sv.s[g], fmaf(-zb, asg, dsum), acc);
-    }
-    return acc;
+// the place of column c in a row of words that others turn into digits: a thread takes four words, and the bytes of a digit
+// lie as the nibbles of a weight do (0 4 1 5, 2 6 3 7), so bits 1 and 2 change places
+__device__ __forceinline__ uint32_t res_place(uint32_t c) { return (c & ~6u) | ((c & 2u) << 1) | ((c & 4u) >> 1); }
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t res_dpp(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
+
+// the sum over two neighbouring groups of 16 lanes, in both
+__device__ __forceinline__ float res_rows_sum(float v) {
+#ifndef HIPC_HOST_MODEL
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+#endif
+    return v;
 }
+
+// the sum over the four groups of 16 lanes, in all lanes
+__device__ __forceinline__ float res_groups_sum(float v) {
+#ifndef HIPC_HOST_MODEL
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+#endif
+    return res_rows_sum(v);
+}
+
+// 16 (4) bytes a lane from memory to LDS, without a register: lane l's to `to` + 16 (4) l
+#ifndef HIPC_HOST_MODEL
+#define RES_TO_LDS(BYTES, r, to, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)(to), BYTES, (int)(voff), 0, 0, 0)
+#else
+#define RES_TO_LDS(BYTES, r, to, voff) gpu_model_load<BYTES>(r, (int)(voff), 0, 0, reinterpret_cast<char *>(to) + (threadIdx.x & 63) * BYTES)
+#endif
 
 // gelu_tanh: 0.5 v (1 + tanh u) = v / (1 + exp(-2 u)), without the difference that loses digits where tanh is near -1
 __device__ __forceinline__ float res_gelu(float v) {
     return v / (1.f + __expf(-1.5957691216057308f * fmaf(0.044715f, v * v * v, v)));
 }
 
-// the LDS of a workgroup
-template <int HD>
+// the LDS of a workgroup (the stand-in's, which loads weights where it uses them, fits beside other work's)
+template <int HD, int SG, bool ALL>
 struct ResShared {
-    uint4 As[64 * 2 * 4];                                // the row as two bf16 terms: [32-k chunk][term][8-k group]
-    float bsum[64];                                      // the sum of the terms per chunk
-    float red[4][64 * kRedPitch];                        // per phase: [column][k tile]; places that no k tile has stay zero
-    float trash[64];                                     // where lanes without a result store
-    uint2 off[kResUnits][kResThreads];                   // the offsets of every thread's units
+    static constexpr int SLOTS = ALL ? kResSlots : 1;
+    uint32_t row[16 * kRowPitch / 4];                    // the row's digits: [k tile][digit][128 bytes]
+    float2 chunk[64];                                    // per 32 values: what a 1 stands for, their sum in such units
     float4 red4[4 * kResWaves];
-    float join[kResThreads * 4];
+    union {
+        float red[4 * kResWaves * 64];                   // a product: [tile][part of its k tiles][lane]
+        float join[kResThreads * 4];                     // (between two products)
+    };
     float rope[2 * HD];
     __half qa[2 * (HD + 8)];
     __half pa[kResWaves][2 * (kAttnPass + 8)];
@@ -169,32 +194,177 @@ struct ResShared {
     float sown;
     uint32_t decision[2];
 #ifdef HIPC_PHASE_STAMPS
-    unsigned long long stamp[kResWaves][32];
+    uint32_t stamp[kResWaves][32];
 #endif
+    // (last: the others' offsets fit the instructions')
+    float sc[SLOTS][16 * SG];
+    uint8_t zb[SLOTS][16 * SG];
+    uint4 wq[SLOTS][64];                                 // units: as in memory, lane by lane
+};
+static_assert(sizeof(ResShared<256, 4, true>) <= 160 * 1024, "a workgroup's LDS");
+
+// ---- what a share v (of XCD v & 7, rank v >> 3) has of each product
+__device__ __forceinline__ int res_tiles_qkv(const ResidentArgs &p, int v) { return (v < p.tiles_qkv) + (v + (int)kResGroups < p.tiles_qkv); }   // v, v + 256
+__device__ __forceinline__ int res_tiles_h(const ResidentArgs &p, int v) { return (p.tiles_h - (v >> 3) + 31) >> 5; }                             // of the hidden row: r, r + 32, ..
+__device__ __forceinline__ int res_slice_tiles(const ResidentArgs &p, int v) { return (p.cg_f - (v & 7) + 7) >> 3; }                              // down's k tiles of the XCD
+__device__ __forceinline__ int res_pairs(const ResidentArgs &p, int v) {   // (gate, up) pairs: eight per k tile of the slice; r, r + 32
+    const int m = res_slice_tiles(p, v) * 8;
+    return ((v >> 3) < m) + ((v >> 3) + 32 < m);
+}
+__device__ __forceinline__ int res_pair(const ResidentArgs &p, int v, int q) {   // global pair, or p.pairs: nothing there
+    const int lp = (v >> 3) + 32 * q;
+    return min(((v & 7) + 8 * (lp >> 3)) * 8 + (lp & 7), p.pairs);
+}
+// A share of product `ph`: `tiles` tiles of `kts` k tiles each; unit (t, kt) is number t * kts + kt.
+template <int HD>
+struct ResShare {
+    int v, ph, tiles, kts;
+    __device__ __forceinline__ ResShare(const ResidentArgs &p, int v_, int ph_) : v(v_), ph(ph_) {
+        tiles = ph == 0 ? res_tiles_qkv(p, v) : ph == 2 ? 2 * res_pairs(p, v) : res_tiles_h(p, v);
+        kts = ph == 1 ? (HD >= 128 ? HD / 128 : 1) : ph == 3 ? res_slice_tiles(p, v) : p.cg_h;
+    }
+    __device__ __forceinline__ bool has(const ResidentArgs &p, int t) const { return ph != 2 || res_pair(p, v, t >> 1) < p.pairs; }
+    __device__ __forceinline__ uint32_t at(const ResidentArgs &p, int t, int kt) const {   // which 128 k x 16 columns of the weight
+        const int r = v >> 3, x = v & 7;
+        if (ph == 0) return (uint32_t)((v + (int)kResGroups * t) * p.cg_h + kt);
+        if (ph == 1) return (uint32_t)((r + 32 * t) * p.cg_o + ((x >> p.lg_parts) * HD) / 128 + kt);
+        if (ph == 2) return (uint32_t)((2 * res_pair(p, v, t >> 1) + (t & 1)) * p.cg_h + kt);
+        return (uint32_t)((r + 32 * t) * p.cg_f + x + 8 * kt);
+    }
+};
+__device__ __forceinline__ uint32_t res_units(const ResidentArgs &p, int ph) {   // of the whole weight
+    return (uint32_t)(ph == 0 ? p.tiles_qkv * p.cg_h : ph == 1 ? p.tiles_h * p.cg_o : ph == 2 ? 2 * p.pairs * p.cg_h : p.tiles_h * p.cg_f);
+}
+
+// the cache positions of share v: its part of its head's context, 32 at a time
+struct ResSpan {
+    int begin, end, first;
+    bool dead;
+    __device__ __forceinline__ ResSpan(const ResidentArgs &p, int v, int total, int window) {
+        const int base = attn_base(total, window), lg = p.lg_parts + 10;   // kAttnPass * kResRanks positions a part
+        static_assert(kAttnPass * kResRanks == 1 << 10, "positions of a part per pass");
+        const int chunk = kAttnPass * max(1, (total - base + (1 << lg) - 1) >> lg);
+        begin = base + (((v & 7) & ((1 << p.lg_parts) - 1)) * (int)kResRanks + (v >> 3)) * chunk;
+        dead = begin >= total;
+        end = min(total, begin + chunk);
+        first = attn_first(total, window);
+    }
+    __device__ __forceinline__ int barriers() const {   // that the passes take: one, and two for each further pass
+        const int passes = dead ? 0 : (end - begin + kAttnPass - 1) / kAttnPass;
+        return max(0, 2 * passes - 1);
+    }
 };
 
-// The work of a launch. ALL: the 256 workgroups are there and workgroup v does share v of every phase; what follows needs no
-// division and no loop over shares, and weights are asked for phases ahead. Else `n` workgroups take the shares in turn.
+// The wavefronts that bring the weights of the launch of all: wavefront `ph` those of product `ph`. It passes the barriers the
+// computing wavefronts do, asks for weights behind some of them, and waits for them before the one that opens the product.
+// Which units these are does not change: their offsets stay in registers, and each of the four wavefronts has code of its own for
+// the fixed places where it asks, so that four units take twelve instructions and the next barrier, which may be 0.3 us away, does
+// not wait for this wavefront (one code for all, which skipped what it did not ask for: 3860 us instead of 3560).
+constexpr int kFeedFirst = 16, kFeedHeads = 24;
+template <int HD, int SG, int ph>
+__device__ __forceinline__ void res_feed(const ResidentArgs &p, ResShared<HD, SG, true> &S, const int v, const int total) {
+    constexpr int MOST = ph == 0 ? 32 : ph == 1 ? 8 : ph == 2 ? 64 : 32;   // units of a share
+    const int lane = threadIdx.x & 63;
+    const ResShare<HD> share(p, v, ph);
+    const int base = p.slot[ph], units = share.tiles * share.kts;
+    const uint32_t tiles = res_units(p, ph);
+    constexpr uint32_t none = 0xffff0000u;   // past the end of everything: zeros, and no traffic
+    uint32_t o_q[MOST], o_s[MOST / 4];   // (a zero point's is a quarter of its scale's)
+    {
+        const uint32_t part = (uint32_t)lane / (4 * SG), in = (uint32_t)lane % (4 * SG);   // of four units' scales: whose, and which 16 (4) bytes
+        // (tile by tile: worked out unit by unit these would take microseconds of every launch)
+        const uint32_t row0 = share.has(p, 0) ? share.at(p, 0, 0) : none, row1 = share.has(p, 1) ? share.at(p, 1, 0) : none;
+        const uint32_t row2 = share.has(p, 2) ? share.at(p, 2, 0) : none, row3 = share.has(p, 3) ? share.at(p, 3, 0) : none;
+        auto row_of = [&](int t) { return t == 0 ? row0 : t == 1 ? row1 : t == 2 ? row2 : row3; };
+        const int kstep = ph == 3 ? 8 : 1;
+        int t = 0, kt = 0;
+        uint32_t row = row0;
+#pragma unroll
+        for (int u = 0; u < MOST; u++) {
+            if (u % 4 == 0 && u >= units) break;
+            const bool live = u < units && row != none;
+            const uint32_t tl = row + (uint32_t)(kt * kstep);
+            o_q[u] = live ? tl * 1024u + (uint32_t)lane * 16u : none;
+            if (u % 4 == 0) o_s[u / 4] = none;
+            if (live && part == (uint32_t)(u % 4)) o_s[u / 4] = tl * 64u * SG + in * 16u;
+            if (++kt == share.kts) kt = 0, t++, row = row_of(t);
+        }
+    }
+    struct Entry {
+        const void *q, *s, *z;
+        int window;
+    };
+    auto entry = [&](int l) {
+#ifndef HIPC_HOST_MODEL
+        const auto *e = (const __attribute__((address_space(4))) ResidentLayer *)(uintptr_t)(p.table + min(l, p.n_layers - 1));   // (scalar loads: they wait for no weights)
+#else
+        const ResidentLayer *e = p.table + min(l, p.n_layers - 1);
+#endif
+        return Entry{e->wq[ph], e->sc[ph], e->zb[ph], e->window};
+    };
+    auto ask = [&](const Entry &e, auto from, auto to) {   // units from .. to - 1, in whole fours
+        const __amdgpu_buffer_rsrc_t q = lean_rsrc(e.q, tiles * 1024u), s = lean_rsrc(e.s, tiles * 64u * SG), z = lean_rsrc(e.z, tiles * 16u * SG);
+#pragma unroll
+        for (int u = decltype(from)::value; u < decltype(to)::value; u += 4) {
+            if (u >= units) break;
+#pragma unroll
+            for (int i = 0; i < 4; i++) RES_TO_LDS(16, q, S.wq[base + u + i], o_q[u + i]);
+            if (lane < 16 * SG) {
+                RES_TO_LDS(16, s, S.sc[base + u], o_s[u / 4]);
+                RES_TO_LDS(4, z, S.zb[base + u], o_s[u / 4] >> 2);
+            }
+        }
+    };
+    Entry e = entry(0), e_next = entry(1);
+    constexpr std::integral_constant<int, 0> none_yet{};
+    constexpr std::integral_constant<int, kFeedFirst> first{};
+    constexpr std::integral_constant<int, kFeedHeads> second{};
+    constexpr std::integral_constant<int, MOST> all{};
+    if (ph == 0) ask(e, none_yet, all);
+    RES_BARRIER();   // (the one in front of the layers)
+    for (int l = 0; l < p.n_layers; l++) {
+        const int inner = ResSpan(p, v, total, e.window).barriers();
+        const int opens = ph == 0 ? 1 : ph == 1 ? 5 + inner : ph == 2 ? 8 + inner : 10 + inner;   // the barrier in front of the product
+        for (int b = 0; b < 12 + inner; b++) {
+            if (b == opens) res_stored();   // (here: what was asked for has arrived)
+            RES_BARRIER();
+            if constexpr (ph == 0) {
+                if (b == 10 + inner && l + 1 < p.n_layers) ask(e_next, none_yet, all);
+            } else if constexpr (ph == 1) {
+                if (b == 0) ask(e, none_yet, all);
+            } else if constexpr (ph == 2) {
+                if (b == 0) ask(e, none_yet, first);
+                if (b == 3) ask(e, first, second);
+                if (b == 4 + inner) ask(e, second, all);
+            } else {
+                if (b == 7 + inner) ask(e, none_yet, all);
+            }
+        }
+        e = e_next;
+        e_next = entry(l + 2);
+    }
+}
+
+// The work of a launch. ALL: the 256 workgroups are there and workgroup v does share v of every phase, with the weights in LDS.
+// Else `n` workgroups take the shares in turn and load weights where they use them.
+// (In the launch of all the loops over shares run once. They stay loops to the compiler, which otherwise moves instructions from phase
+// to phase: 3570 against 3650 to 3800 us for eight tokens of gemma3-1b.)
+#define RES_SHARES(v) for (int v = first, step_ = ALL ? (int)kResGroups : n, end_ = ALL ? mine + 1 : (int)kResGroups; v < end_; v += step_)
 template <int HD, int SG, bool ALL>
-__device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> &S, int first, const int n, const bool wide, uint32_t set, const int pos, int &tries) {
+__device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, SG, ALL> &S, int first, const int n, const bool wide, uint32_t set, const int pos, int &tries) {
     constexpr int KT3 = HD >= 128 ? HD / 128 : 1;  // k tiles of a head in o's weight (half of one at 64 channels)
     constexpr int KS = HD >= 128 ? HD / 128 : 1;   // 32-channel steps of a wavefront's share of the scores
     constexpr int DQ = HD / (32 * KS);             // wavefronts that share the channels of the scores
     constexpr int NB = HD >= 128 ? HD / 128 : 1;   // 16-channel blocks of a wavefront's outputs
     constexpr int QS = HD + 8, PS = kAttnPass + 8; // halfs per operand row (16 bytes of padding)
     constexpr int NJ = kResThreads * 4 / HD;       // rows of chunks that are joined side by side
-    constexpr int U1 = 2, U3 = 1, U4 = 5, U5 = 3;   // units asked for ahead; a wavefront's further ones when it comes to them
     constexpr float NEG = -3.0e38f;
 
     int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int i16 = lane & 15, g4 = lane >> 4;
-    uint32_t magic;
-    HIPC_VGPR_FROM_SGPR(magic, p.magic);
-    const uint32_t nib_mask = p.nib_mask;
-    const int total = pos + 1;
+    const int total = pos + 1, mine = first;
     const __amdgpu_buffer_rsrc_t r_x = lean_rsrc(p.xch, kResSets * kResWords * 4u);
-    const char *as = reinterpret_cast<const char *>(S.As);
 
     // ---- the layer's entry: lane i holds word i of it, a pointer is read from two lanes. (Scalar loads would miss the
     // scalar cache once per phase.) The next layer's is asked for a layer ahead.
@@ -205,7 +375,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
         return (uint32_t)l;
 #endif
     };
-    uint32_t ent = entry_of(0), ent_next = entry_of(1);
+    uint32_t ent = entry_of(0), ent_next = entry_of(1), ent_after = ent_next;
     auto word_of = [&](uint32_t e, int i) {
 #ifndef HIPC_HOST_MODEL
         return (uint32_t)__builtin_amdgcn_readlane((int)e, i);
@@ -217,194 +387,128 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
     constexpr int kNorm = 12, kCache = 18, kWindow = 40, kRope = 41;
     static_assert(offsetof(ResidentLayer, norm) == kNorm * 8 && offsetof(ResidentLayer, k_cache) == kCache * 8 && offsetof(ResidentLayer, window) == kWindow * 4, "entries are read as words");
 
-    struct Weight {
-        __amdgpu_buffer_rsrc_t q, s, z;
-    };
-    auto weight = [&](uint32_t e, int which, uint32_t tiles) {
-        return Weight{lean_rsrc(ptr_of(e, which), tiles * 1024u), lean_rsrc(ptr_of(e, 4 + which), tiles * 64u * SG), lean_rsrc(ptr_of(e, 8 + which), tiles * 16u * SG)};
-    };
-    const uint32_t n1 = (uint32_t)(p.tiles_qkv * p.cg_h), n3 = (uint32_t)(p.tiles_h * p.cg_o), n4 = (uint32_t)(2 * p.pairs * p.cg_h), n5 = (uint32_t)(p.tiles_h * p.cg_f);
+    auto tiles1 = [&](int v) { return res_tiles_qkv(p, v); };
+    auto tiles3 = [&](int v) { return res_tiles_h(p, v); };
+    auto slice_tiles = [&](int v) { return res_slice_tiles(p, v); };
+    auto pairs4 = [&](int v) { return res_pairs(p, v); };
 
-    // ---- which units share v of a phase has
-    struct Unit {
-        int tl, kt, t;   // tile of the weight, k tile of the row in LDS, column tile of the workgroup
-        bool live;
-    };
-    auto split_unit = [&](int u, int *kt) {   // unit u = (column tile u / cg_h, k tile u % cg_h)
-        const int t = (int)(((uint32_t)u * p.inv_cg_h) >> 16);
-        *kt = u - t * p.cg_h;
-        return t;
-    };
-    // q|k|v: column tiles v and v + 256, all of hidden's k tiles
-    auto tiles1 = [&](int v) { return (v < p.tiles_qkv) + (v + (int)kResGroups < p.tiles_qkv); };
-    auto unit1 = [&](int v, int u) {
-        Unit x;
-        x.t = split_unit(u, &x.kt);
-        x.tl = (v + (int)kResGroups * x.t) * p.cg_h + x.kt;
-        x.live = u < tiles1(v) * p.cg_h;
-        return x;
-    };
-    // o: the columns of the hidden row that rank r holds, tiles r, r + 32, ...; the k tiles of the XCD's head
-    auto tiles3 = [&](int v) { return (p.tiles_h - (v >> 3) + 31) >> 5; };
-    auto unit3 = [&](int v, int u) {
-        const int h = (v & 7) >> p.lg_parts;
-        Unit x;
-        x.t = u / KT3, x.kt = u % KT3;
-        x.tl = ((v >> 3) + 32 * x.t) * p.cg_o + (h * HD) / 128 + x.kt;
-        x.live = x.t < tiles3(v);
-        return x;
-    };
-    // gate|up: the XCD holds the pairs of the down projection's k tiles x, x + 8, ..., 8 pairs each; rank r its pairs r, r + 32
-    auto slice_tiles = [&](int v) { return (p.cg_f - (v & 7) + 7) >> 3; };
-    auto pair_of = [&](int v, int q) {   // global pair, or one past the last: nothing there
-        const int lp = (v >> 3) + 32 * q;
-        return min(((v & 7) + 8 * (lp >> 3)) * 8 + (lp & 7), p.pairs);
-    };
-    auto pairs4 = [&](int v) {
-        const int m = slice_tiles(v) * 8;
-        return ((v >> 3) < m) + ((v >> 3) + 32 < m);
-    };
-    auto unit4 = [&](int v, int u) {
-        Unit x;
-        x.t = split_unit(u, &x.kt);
-        const int pair = pair_of(v, x.t >> 1);
-        x.tl = (2 * pair + (x.t & 1)) * p.cg_h + x.kt;
-        x.live = u < 2 * pairs4(v) * p.cg_h && pair < p.pairs;
-        return x;
-    };
-    // down: rank r's columns, the XCD's k tiles; unit u = (tile u % tiles, k tile u / tiles), at most four tiles
-    auto unit5 = [&](int v, int u) {
-        const int tiles = tiles3(v);
-        Unit x;
-        x.kt = tiles <= 1 ? u : tiles == 2 ? u >> 1 : tiles == 4 ? u >> 2 : (int)(((uint32_t)u * 21846u) >> 16);
-        x.t = u - x.kt * tiles;
-        x.tl = ((v >> 3) + 32 * x.t) * p.cg_f + (v & 7) + 8 * x.kt;
-        x.live = u < tiles * slice_tiles(v);
-        return x;
-    };
-    // the lane's offsets of a unit: in the weight (what its scales' and zero points' follow from); in LDS, the row's operand
-    // and in the upper half where the sum goes
-    auto offsets_of = [&](const Unit &x, int i, int phase) {
-        // (a unit that does not exist loads from past the end of everything: zeros, and no traffic. A load that is skipped
-        // would keep the registers of the layer before alive.)
-        const uint32_t red = g4 == (i & 3) ? (uint32_t)(phase * 64 * kRedPitch + (x.t * 16 + i16) * kRedPitch + x.kt) : (uint32_t)(4 * 64 * kRedPitch + lane);
-        return make_uint2(x.live ? (uint32_t)x.tl * 1024u + (uint32_t)lane * 16u : 0xffff0000u,
-                          (uint32_t)x.kt * 512u + (uint32_t)(min(i16 & 3, 1) * 4 + g4) * 16u + (red << 18));
-    };
-    auto load_scales = [&](const Weight &b, ScaleVecLean<SG> &sv, uint32_t o_wq) {   // of the unit at the lane's o_wq
-        const uint32_t o_zb = (o_wq >> 10) * (16u * SG) + (uint32_t)i16 * SG;
-        sv.load(b.s, b.z, o_zb * 4u, o_zb, 0);
-    };
-    // units from .. to - 1 (from: a multiple of four, or 2 with its neighbours' scales already asked for)
-    auto load_units = [&](auto &w, int at, const Weight &b, int from = 0, int to = 8) {
-        constexpr int U = (int)(sizeof w.wq / sizeof w.wq[0]);
-        uint32_t o[U], os[(U + 3) / 4];
+    // ---- products
+    // NT tiles of a product, t0 .. t0 + NT - 1, over its k tiles kt0, kt0 + step, .. (once: there is no second): this lane's sums
+    // for its chunk go to `part`
+    auto multiply = [&](auto nt, auto once, int ph, uint32_t e, const ResShare<HD> &share, int t0, int kt0, int step, int part) {
+        constexpr int NT = decltype(nt)::value;
+        float acc[NT];
 #pragma unroll
-        for (int i = 0; i < U; i++)
-            if (i >= from && i < to) o[i] = S.off[at + i][tid].x;
-#pragma unroll
-        for (int i = 0; i < U; i += 4)
-            if (i >= from && i < to) os[i / 4] = S.off[at + min(i + g4, U - 1)][tid].x;
-#pragma unroll
-        for (int i = 0; i < U; i++) {
-            if (i < from || i >= to) continue;
-            if (i % 4 == 0) load_scales(b, w.sv[i / 4], os[i / 4]);
-            w.wq[i] = lean_ld16(b.q, o[i], 0);
-        }
-    };
-    auto multiply_one = [&](auto &w, int i, uint32_t o_lds) {
-        const float acc = res_unit<SG>(w.wq[i], w.sv[i / 4], as, o_lds & 0xffffu, nib_mask, magic);
-        *reinterpret_cast<float *>(reinterpret_cast<char *>(S.red) + (o_lds >> 16)) = acc;
-    };
-    // a phase's product: what was asked for ahead, then whatever else the share has
-    auto multiply = [&](auto &w, int at, uint32_t e, int which, uint32_t tiles, int v, int units, int phase, auto &&unit) {
-        constexpr int U = (int)(sizeof w.wq / sizeof w.wq[0]);
-        if (ALL) {
-            uint32_t o[U];
-#pragma unroll
-            for (int i = 0; i < U; i++) o[i] = S.off[at + i][tid].y;
-#pragma unroll
-            for (int i = 0; i < U; i++)
-                if ((w.live >> i) & 1u) multiply_one(w, i, o[i]);
-        }
-        for (int u = wave + (ALL ? 8 * U : 0); u < units; u += 8) {
-            const Unit x = unit(v, u);
-            if (!x.live) continue;
-            Units<1, SG> one;
-            const uint2 o = offsets_of(x, 0, phase);
-            const Weight b = weight(e, which, tiles);
-            load_scales(b, one.sv[0], o.x);
-            one.wq[0] = lean_ld16(b.q, o.x, 0);
-            multiply_one(one, 0, o.y);
-        }
-    };
-    Units<U1, SG> w1;
-    Units<U3, SG> w3;
-    Units<U4, SG> w4;
-    Units<U5, SG> w5;
-    constexpr int kAt1 = 0, kAt3 = U1, kAt4 = U1 + U3, kAt5 = U1 + U3 + U4;
-    static_assert(kAt5 + U5 <= kResUnits, "places for the units' offsets");
-    if (ALL) {
-        auto set_units = [&](auto &w, int at, int phase, auto &&unit) {
-            w.live = 0;
-            for (int i = 0; i < (int)(sizeof w.wq / sizeof w.wq[0]); i++) {
-                const Unit x = unit(first, wave + 8 * i);
-                S.off[at + i][tid] = offsets_of(x, i, phase);
-                w.live |= x.live ? 1u << i : 0u;
-            }
+        for (int j = 0; j < NT; j++) acc[j] = 0.f;
+        const int t3 = min(i16 & 3, 2), mine = i16 >> 2;
+        const char *row = reinterpret_cast<const char *>(S.row) + t3 * 128 + mine * 32 + g4 * 8;
+        const float2 *chunk = S.chunk + g4;
+        const bool digit = (i16 & 3) < 3;
+        const uint32_t m0 = digit && mine == 0 ? ~0u : 0u, m1 = digit && mine == 1 ? ~0u : 0u, m2 = digit && mine == 2 ? ~0u : 0u, m3 = digit && mine == 3 ? ~0u : 0u;
+        const int sg = SG == 4 ? g4 : SG == 2 ? g4 >> 1 : 0;
+        struct Operands {
+            uint2 a;     // the lane's digits of the row
+            float2 c;
+            UnitWeight w[NT];
         };
-        set_units(w1, kAt1, 0, unit1), set_units(w3, kAt3, 1, unit3), set_units(w4, kAt4, 2, unit4), set_units(w5, kAt5, 3, unit5);
-    }
+        auto row_here = [&](Operands &o, int kt) { o.a = *reinterpret_cast<const uint2 *>(row + kt * kRowPitch), o.c = chunk[kt * 4]; };
+        auto product = [&](const Operands &o, const UnitWeight &w, float sum) {
+            constexpr uint32_t F = 0x0f0f0f0fu;
+            const ri32x4 a0 = {(int)(o.a.x & m0), (int)(o.a.y & m0), (int)(o.a.x & m1), (int)(o.a.y & m1)}, a1 = {(int)(o.a.x & m2), (int)(o.a.y & m2), (int)(o.a.x & m3), (int)(o.a.y & m3)};
+            const uint4 q = w.w;
+            const ri32x4 b0 = {(int)(q.x & F), (int)((q.x >> 4) & F), (int)(q.y & F), (int)((q.y >> 4) & F)}, b1 = {(int)(q.z & F), (int)((q.z >> 4) & F), (int)(q.w & F), (int)((q.w >> 4) & F)};
+            ri32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, ri32x4{0, 0, 0, 0}, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
+            const float f = fmaf((float)d[0], 65536.f, (float)(d[1] * 256 + d[2]));   // (each sum is below 2^16: the second is exact)
+            return fmaf(w.s * o.c.x, fmaf(-(float)(w.z & 127u), o.c.y, f), sum);
+        };
+        if (ALL) {
+            if (kt0 < share.kts) {
+                Operands o;
+                auto load = [&](int kt) {
+                    row_here(o, kt);
+#pragma unroll
+                    for (int j = 0; j < NT; j++) {
+                        const int at = p.slot[ph] + (t0 + j) * share.kts + kt;
+                        o.w[j] = UnitWeight{S.wq[at][lane], S.sc[at][i16 * SG + sg], S.zb[at][i16 * SG + sg]};
+                    }
+                };
+                load(kt0);
+#pragma unroll 1
+                for (int kt = kt0 + step; !decltype(once)::value && kt < share.kts; kt += step) {
+                    const Operands now = o;
+                    load(kt);
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[j] = product(now, now.w[j], acc[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[j] = product(o, o.w[j], acc[j]);
+            }
+        } else {
+#pragma unroll 1
+            for (int j = 0, kt = kt0; j < NT && kt0 < share.kts; kt = kt + step < share.kts ? kt + step : (j++, kt0)) {
+                if (t0 + j >= share.tiles) break;
+                Operands o;
+                row_here(o, kt);
+                const uint32_t tl = share.at(p, t0 + j, kt), all = res_units(p, ph);
+                UnitWeight w;
+                w.w = lean_ld16(lean_rsrc(ptr_of(e, ph), all * 1024u), (uint32_t)lane * 16u, tl * 1024u);
+                w.s = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(lean_rsrc(ptr_of(e, 4 + ph), all * 64u * SG), (int)((i16 * SG + sg) * 4), (int)(tl * 64u * SG), 0));
+                w.z = __builtin_amdgcn_raw_buffer_load_b8(lean_rsrc(ptr_of(e, 8 + ph), all * 16u * SG), i16 * SG + sg, (int)(tl * 16u * SG), 0);
+                const float r = product(o, w, 0.f);
+#pragma unroll
+                for (int i = 0; i < NT; i++)
+                    if (i == j) acc[i] += r;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NT; j++) S.red[((t0 + j) * kResWaves + part) * 64 + lane] = acc[j];
+    };
+    // the sum of tile t's columns over `parts` parts: column i16's, in all lanes
+    auto tile_sum = [&](int t, int parts) {
+        const float *r = S.red + t * kResWaves * 64 + lane;
+        float s = r[0];
+        if (parts >= 2) s += r[64];
+        if (parts >= 4) s += r[128] + r[192];
+        if (parts >= 8) s += (r[256] + r[320]) + (r[384] + r[448]);
+        return res_groups_sum(s);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using Three = std::integral_constant<int, 3>;
+    using Four = std::integral_constant<int, 4>;
 
     // ---- the cache rows of a share's positions: 32 at a time
-    uint4 kreg[KS], vreg[NB];
-    struct Span {
-        int begin, end, first;
-        bool dead;
+    struct CacheRows {
+        uint4 k[KS], v[NB];
     };
-    auto span_of = [&](int v, int window) {
-        const int base = attn_base(total, window), parts = 1 << p.lg_parts;
-        const int per_pass = kAttnPass * (int)kResRanks * parts, len = total - base;
-        const int chunk = len <= per_pass ? kAttnPass : kAttnPass * ((len + per_pass - 1) / per_pass);
-        Span s;
-        s.begin = base + (((v & 7) & (parts - 1)) * (int)kResRanks + (v >> 3)) * chunk;
-        s.dead = s.begin >= total;
-        s.end = min(total, s.begin + chunk);
-        s.first = attn_first(total, window);
-        return s;
-    };
+    CacheRows kv;
     const int pb = wave & 1, dq = min(wave >> 1, DQ - 1);
     const uint32_t v_k = (uint32_t)((pb * 16 + i16) * HD + dq * 32 * KS + g4 * 8) * 2u;
     const uint32_t v_v = ((uint32_t)(min(wave * 16 * NB, HD - 16 * NB) + i16) * (uint32_t)p.v_stride + (uint32_t)(g4 * 8)) * 2u;
     auto load_k = [&](__amdgpu_buffer_rsrc_t r, int kvh, int t0) {
         const uint32_t s_k = ((uint32_t)kvh * (uint32_t)p.max_seq + (uint32_t)t0) * HD * 2u;
 #pragma unroll
-        for (int u = 0; u < KS; u++) kreg[u] = lean_ld16(r, v_k + u * 64u, s_k);
+        for (int u = 0; u < KS; u++) kv.k[u] = lean_ld16(r, v_k + u * 64u, s_k);
     };
     auto load_v = [&](__amdgpu_buffer_rsrc_t r, int kvh, int t0) {
 #pragma unroll
-        for (int b = 0; b < NB; b++) vreg[b] = lean_ld16(r, v_v, (((uint32_t)kvh * HD + b * 16u) * (uint32_t)p.v_stride + (uint32_t)t0) * 2u);
+        for (int b = 0; b < NB; b++) kv.v[b] = lean_ld16(r, v_v, (((uint32_t)kvh * HD + b * 16u) * (uint32_t)p.v_stride + (uint32_t)t0) * 2u);
     };
     auto rsrc_k = [&](uint32_t e, bool dead) { return lean_rsrc(ptr_of(e, kCache), dead ? 0u : ((uint32_t)p.n_kv * (uint32_t)p.max_seq + 64u) * HD * 2u); };
     auto rsrc_v = [&](uint32_t e, bool dead) { return lean_rsrc(ptr_of(e, kCache + 1), dead ? 0u : (uint32_t)p.n_kv * HD * (uint32_t)p.v_stride * 2u); };
     auto load_kv = [&](uint32_t e, int v) {
-        const Span s = span_of(v, (int)word_of(e, kWindow));
+        const ResSpan s(p, v, total, (int)word_of(e, kWindow));
         const int kvh = ((v & 7) >> p.lg_parts) >> p.lg_group, t0 = s.dead ? 0 : s.begin;   // (the scalar offset stays inside whatever the descriptor says)
         load_k(rsrc_k(e, s.dead), kvh, t0), load_v(rsrc_v(e, s.dead), kvh, t0);
     };
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    // norm weights of the heads: the query's for wavefront 0, the key's for wavefront 1. (A load under a condition would be
-    // waited for where the condition ends: none of the loads ahead has one.)
+    // norm weights of the heads: the query's for wavefront 0, the key's for wavefront 1; asked for a layer ahead. (A load under a
+    // condition would be waited for where the condition ends: none of the loads ahead has one.)
     float4 head_w = zero4;
     auto load_head_w = [&](uint32_t e) {
         head_w = __builtin_bit_cast(float4, lean_ld16(lean_rsrc(ptr_of(e, kNorm + 4 + (wave & 1)), HD * 4u), (uint32_t)lane * 16u, 0));
     };
-    // what a layer's first phases need, asked for while the layer before is in its last one
-    auto load_ahead = [&](uint32_t e) {
-        load_head_w(e);
-        if (ALL) load_units(w1, kAt1, weight(e, 0, n1));
-    };
-
     // ---- hand-overs
     uint32_t cur = set * kResWords * 4u, next = (set == kResSets - 1 ? 0u : set + 1u) * kResWords * 4u;   // byte offsets of this layer's and the next layer's words
     auto store = [&](uint32_t word, uint32_t bits, uint32_t in, bool agent) {
@@ -438,35 +542,38 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
         } while (any_empty(v) && --tries > 0);
         return v;
     };
-    // four values of the row as two bf16 terms into LDS, and their chunk's sum; eight neighbouring threads make a chunk
-    auto put_terms = [&](int i4, uint2 hi, uint2 lo) {
-        uint2 *dst = reinterpret_cast<uint2 *>(S.As) + (i4 >> 3) * 16 + (i4 & 7);
-        dst[0] = hi, dst[8] = lo;
-        const lbf16pair ones = __builtin_bit_cast(lbf16pair, 0x3f803f80u);
-        float s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(lbf16pair, hi.x), ones, 0.f, false);
-        float t = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(lbf16pair, hi.y), ones, 0.f, false);
-        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(lbf16pair, lo.x), ones, s, false);
-        t = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(lbf16pair, lo.y), ones, t, false);
-        s += t;
+    // four values of the row (words 4 i4 .. of it, see res_place) as digits into LDS; eight neighbouring threads make a chunk. (Its
+    // sum is one of the values themselves: an infinity or a NaN among them, which has no digits, makes the products NaN.)
+    auto put_digits = [&](int i4, float a, float b, float c, float d) {
+        uint32_t mx = __float_as_uint(fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d))));
+        mx = max(mx, res_dpp<0xB1>(mx));
+        mx = max(mx, res_dpp<0x4E>(mx));
+        mx = max(mx, res_dpp<0x141>(mx));   // row_half_mirror: the other quad of the eight
+        const uint32_t ex = max(mx >> 23, 22u);
+        const float to = __uint_as_float((275u - ex) << 23);   // the largest comes to 2^21 .. 2^22
+        float s = fmaf(a, to, b * to) + fmaf(c, to, d * to);
         s += lean_dpp<0xB1>(s);
         s += lean_dpp<0x4E>(s);
-        s += lean_dpp<0x141>(s);   // row_half_mirror: the other quad of the eight
-        if ((i4 & 7) == 0) S.bsum[i4 >> 3] = s;
-    };
-    auto split_terms4 = [&](int i4, float a, float b, float c, float d) {
-        uint2 hi, lo;
-        hi.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(lf32x2{a, b}, lbf16x2));
-        hi.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(lf32x2{c, d}, lbf16x2));
-        a -= __uint_as_float(hi.x << 16), b -= __uint_as_float(hi.x & 0xffff0000u);
-        c -= __uint_as_float(hi.y << 16), d -= __uint_as_float(hi.y & 0xffff0000u);
-        lo.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(lf32x2{a, b}, lbf16x2));
-        lo.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(lf32x2{c, d}, lbf16x2));
-        put_terms(i4, hi, lo);
+        s += lean_dpp<0x141>(s);
+        // the nearest whole number in the low bits, 0x80 added to each of its bytes and taken away without borrowing
+        auto digits = [&](float x) { return (__float_as_uint(fmaf(x, to, 12582912.f)) + (0x00808080u - 0x4b400000u)) ^ 0x00808080u; };
+        const uint32_t q0 = digits(a), q1 = digits(c), q2 = digits(b), q3 = digits(d);   // (in the order of the bytes)
+        const uint32_t lo01 = __builtin_amdgcn_perm(q1, q0, 0x05010400u), lo23 = __builtin_amdgcn_perm(q3, q2, 0x05010400u);
+        const uint32_t hi01 = __builtin_amdgcn_perm(q1, q0, 0x0c0c0602u), hi23 = __builtin_amdgcn_perm(q3, q2, 0x0c0c0602u);
+        uint32_t *dst = S.row + (i4 >> 5) * (kRowPitch / 4) + (i4 & 31);   // (= i4 + 64 (i4 >> 5))
+        dst[0] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+        dst[32] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+        dst[64] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+        if ((i4 & 7) == 0) S.chunk[i4 >> 3] = make_float2(__uint_as_float((ex - 21u) << 23), s);
     };
     // stream += rmsnorm(branch, w_post); the row rmsnorm(stream, w_in) goes to LDS. One reduction for both norms (see mmnb_lean_kernel).
     float4 x4 = zero4, y4 = zero4;   // this thread's four values of the stream, and of the branch to be added
     const bool holds = tid * 4 < p.hidden;
-    if (holds) x4 = *reinterpret_cast<const float4 *>(p.x_in + tid * 4);
+    auto place = [&] { return (tid >> 1) * 8 + (tid & 1) * 2; };   // its first value's column; the others: + 1, + 4, + 5
+    if (holds) {
+        const float2 lo = *reinterpret_cast<const float2 *>(p.x_in + place()), hi = *reinterpret_cast<const float2 *>(p.x_in + place() + 4);
+        x4 = make_float4(lo.x, lo.y, hi.x, hi.y);
+    }
     const int pw = (p.cg_h * 32 + 63) >> 6;   // wavefronts that hold parts of the row
     auto norm_row = [&](const float4 &wp, const float4 &wi) {
         const float4 yw = make_float4(y4.x * wp.x, y4.y * wp.y, y4.z * wp.z, y4.w * wp.w);
@@ -480,33 +587,22 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
         }
         __syncthreads();
         if (wave < pw) {
-            const float4 r = lane < pw * 4 ? S.red4[lane & 31] : zero4;
+            const float4 r = S.red4[lane & 31];   // (zeros behind the wavefronts that hold parts)
             const float r_yy = lean_row_sum(r.x), r_xx = lean_row_sum(r.y), r_xy = lean_row_sum(r.z), r_ww = lean_row_sum(r.w);
-            const float t_yy = lean_lane(r_yy, 0) + lean_lane(r_yy, 16), t_xx = lean_lane(r_xx, 0) + lean_lane(r_xx, 16);
-            const float t_xy = lean_lane(r_xy, 0) + lean_lane(r_xy, 16), t_ww = lean_lane(r_ww, 0) + lean_lane(r_ww, 16);
+            const float t_yy = res_rows_sum(r_yy), t_xx = res_rows_sum(r_xx), t_xy = res_rows_sum(r_xy), t_ww = res_rows_sum(r_ww);
             const float f1 = rsqrtf(t_yy * p.inv_hidden + p.eps);
             const float sq2 = fmaf(f1 * f1, t_ww, fmaf(2.f * f1, t_xy, t_xx));
             const float f2 = rsqrtf(fmaxf(sq2, 0.f) * p.inv_hidden + p.eps);
             x4.x = fmaf(yw.x, f1, x4.x), x4.y = fmaf(yw.y, f1, x4.y), x4.z = fmaf(yw.z, f1, x4.z), x4.w = fmaf(yw.w, f1, x4.w);
-            if (tid < p.cg_h * 32) split_terms4(tid, x4.x * f2 * wi.x, x4.y * f2 * wi.y, x4.z * f2 * wi.z, x4.w * f2 * wi.w);
+            if (tid < p.cg_h * 32) put_digits(tid, x4.x * f2 * wi.x, x4.y * f2 * wi.y, x4.z * f2 * wi.z, x4.w * f2 * wi.w);
         }
         __syncthreads();
     };
-    // the sum of a column's k tiles, in order (places past the last k tile hold zeros)
-    auto column = [&](int phase, int col) {
-        const float4 *c = reinterpret_cast<const float4 *>(S.red[phase] + col * kRedPitch);
-        float4 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = c[q];
-        return (((v[0].x + v[0].y) + (v[0].z + v[0].w)) + ((v[1].x + v[1].y) + (v[1].z + v[1].w))) +
-               (((v[2].x + v[2].y) + (v[2].z + v[2].w)) + ((v[3].x + v[3].y) + (v[3].z + v[3].w)));
+    auto row4 = [&](uint32_t e, int which) {   // (past the row: zeros)
+        const __amdgpu_buffer_rsrc_t r = lean_rsrc(ptr_of(e, kNorm + which), (uint32_t)p.hidden * 4u);
+        const float2 lo = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, place() * 4, 0, 0)), hi = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, place() * 4 + 16, 0, 0));
+        return make_float4(lo.x, lo.y, hi.x, hi.y);
     };
-    auto zero_red = [&](int phase) {   // (before another share's product, which may have fewer k tiles)
-        if (ALL) return;
-        for (int i = tid; i < 64 * kRedPitch; i += kResThreads) S.red[phase][i] = 0.f;
-        __syncthreads();
-    };
-    auto row4 = [&](uint32_t e, int which) { return __builtin_bit_cast(float4, lean_ld16(lean_rsrc(ptr_of(e, kNorm + which), (uint32_t)p.hidden * 4u), (uint32_t)tid * 16u, 0)); };   // (past the row: zeros)
     // rank r's columns of a row, summed over the XCDs' partial rows (weighed: with their softmax sums) and given to the XCD
     auto combine = [&](int v, uint32_t g, uint32_t to, bool weighed) {
         const int r = v >> 3, x = v & 7, cols = tiles3(v) * 16;
@@ -545,17 +641,15 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             for (int s = 0; s < 8; s++) f[s] = __uint_as_float(part[s]);
             y = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
         }
-        if (lane < cols) put((uint32_t)x * kResLocal + to + (uint32_t)((r + 32 * g4) * 16 + i16), __float_as_uint(y), wide);
+        if (lane < cols) put((uint32_t)x * kResLocal + to + res_place((uint32_t)((r + 32 * g4) * 16 + i16)), __float_as_uint(y), wide);
     };
     const uint32_t home = (uint32_t)(first & 7) * kResLocal;   // where this workgroup reads rows all XCDs hold
-    const int step = ALL ? (int)kResGroups : n;                // (ALL: every loop over shares runs once)
-    const int end = ALL ? first + 1 : (int)kResGroups;
 
-    for (int i = tid; i < 4 * 64 * kRedPitch; i += kResThreads) S.red[0][i] = 0.f;
     for (int i = tid; i < 2 * HD; i += kResThreads) S.rope[i] = p.rope[i];
+    if (tid < 4 * kResWaves) S.red4[tid] = zero4;
     if (ALL) load_kv(ent, first);
-    load_ahead(ent);
-    float4 wp = zero4, wi = row4(ent, 0);
+    load_head_w(ent);
+    float4 wp = zero4, wi = zero4, wp1 = zero4, wi1 = row4(ent, 0);   // of the norm in the middle of a layer, and where one begins
     __syncthreads();
     for (int l = 0; l < p.n_layers; l++) {
         // What follows from these is worked out where it is used: kept for all layers it would not fit the registers.
@@ -566,28 +660,27 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
         HIPC_PIN_VGPR(tid);
         // ---- q|k|v of the row
         RES_STAMP(0);
-        norm_row(wp, wi);
-        if (ALL) load_units(w4, kAt4, weight(ent, 2, n4), 0, 2);
+        norm_row(wp1, wi1);
         RES_STAMP(2);
-        for (int v = first; v < end; v += step) {
-            zero_red(0);
-            multiply(w1, kAt1, ent, 0, n1, v, tiles1(v) * p.cg_h, 0, unit1);
+        RES_SHARES(v) {
+            const ResShare<HD> share(p, v, 0);
+            const int parts = share.tiles == 2 ? 4 : 8;
+            if (share.tiles > 0) multiply(One{}, std::false_type{}, 0, ent, share, share.tiles == 2 ? wave >> 2 : 0, wave & (parts - 1), parts, wave & (parts - 1));
             RES_STAMP(3);
             __syncthreads();
-            if (wave == 7) {
-                const float s = column(0, lane & 31);
-                if (lane < tiles1(v) * 16) put(kResQ + (uint32_t)((v + (int)kResGroups * g4) * 16 + i16), __float_as_uint(s), true);
+            if (wave >= 4 && wave - 4 < share.tiles) {
+                const float s = tile_sum(wave - 4, parts);
+                if (lane < 16) put(kResQ + (uint32_t)((v + (int)kResGroups * (wave - 4)) * 16 + lane), __float_as_uint(s), true);
             }
             clear(v);
             if (!ALL) __syncthreads();
         }
-        if (ALL) load_units(w3, kAt3, weight(ent, 1, n3));
         RES_STAMP(4);
         // ---- attention: the share's positions for the XCD's head
-        for (int v = first; v < end; v += step) {
+        RES_SHARES(v) {
             const uint32_t mine = (uint32_t)(v & 7) * kResLocal;
             const int h = (v & 7) >> p.lg_parts, kvh = h >> p.lg_group;
-            const Span s = span_of(v, (int)word_of(ent, kWindow));
+            const ResSpan s(p, v, total, (int)word_of(ent, kWindow));
             const bool is_last = !s.dead && s.end == total;
             const int hist_end = min(s.end, pos);
             float rq[4];
@@ -629,13 +722,13 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                 }
             }
             RES_STAMP(5);
-            res_stored();   // this workgroup's words of the next layer are empty before it hands anything over (and o's weights and the cache rows are here)
+            res_stored();   // this workgroup's words of the next layer are empty before it hands anything over
             RES_STAMP(28);
-            if (ALL) load_units(w4, kAt4, weight(ent, 2, n4), 2);
-            else load_kv(ent, v);
+            if (!ALL) load_kv(ent, v);
             RES_STAMP(29);
             __syncthreads();
             RES_STAMP(6);
+            if (ALL) load_head_w(ent_next);
             if (is_last) {
                 if ((h & ((1 << p.lg_group) - 1)) == 0 && tid < HD) {   // one of the heads that share the kv head appends to its cache
                     static_cast<__half *>(ptr_of(ent, kCache))[((size_t)kvh * p.max_seq + pos) * HD + tid] = __float2half(S.kn[tid]);
@@ -665,7 +758,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                 const bool more = t0 + kAttnPass < s.end;
                 lf32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int u = 0; u < KS; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(aq[u], __builtin_bit_cast(rh16x8, kreg[u]), acc, 0, 0, 0);
+                for (int u = 0; u < KS; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(aq[u], __builtin_bit_cast(rh16x8, kv.k[u]), acc, 0, 0, 0);
                 if (g4 == 0) S.sp[wave][i16] = acc[0] + acc[1];
                 if (more) load_k(rsrc_k(ent, false), kvh, t0 + kAttnPass);
                 __syncthreads();
@@ -698,17 +791,14 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
 #pragma unroll
                 for (int b = 0; b < NB; b++) {
                     o[b][0] *= f, o[b][1] *= f;
-                    o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ap, __builtin_bit_cast(rh16x8, vreg[b]), o[b], 0, 0, 0);
+                    o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ap, __builtin_bit_cast(rh16x8, kv.v[b]), o[b], 0, 0, 0);
                 }
                 if (more) {
                     load_v(rsrc_v(ent, false), kvh, t0 + kAttnPass);
                     __syncthreads();   // the next pass's scores must not overtake this pass's reads
                 }
             };
-            // (the first pass apart: its cache rows are here, and a loop that also waits for rows it asks for itself would
-            // wait for gate|up's weights with them)
-            if (s.begin < s.end) pass(s.begin);
-            for (int t0 = s.begin + kAttnPass; t0 < s.end; t0 += kAttnPass) pass(t0);
+            for (int t0 = s.begin; t0 < s.end; t0 += kAttnPass) pass(t0);
             RES_STAMP(7);
             float f = 1.f, e_own = 0.f;
             if (is_last) {   // the step's own position
@@ -727,9 +817,9 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             if (!ALL) __syncthreads();
         }
         RES_STAMP(8);
+        if (!ALL) load_head_w(ent_next);
         // ---- o: the XCD's chunks joined (unnormalised), times the head's rows of o
-        wp = row4(ent, 1), wi = row4(ent, 2);
-        for (int v = first; v < end; v += step) {
+        RES_SHARES(v) {
             const uint32_t mine = (uint32_t)(v & 7) * kResLocal;
             const int h = (v & 7) >> p.lg_parts;
             uint4 ov[HD / 64], ml;
@@ -744,6 +834,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                 for (int i = 0; i < HD / 64; i++) again = again || any_empty(ov[i]);
             } while (again && --tries > 0);
             RES_STAMP(9);
+            if (ALL || v == first) wp = row4(ent, 1), wi = row4(ent, 2);
             // lane i16 holds ranks 2 i16 and 2 i16 + 1
             const float m0 = __uint_as_float(ml.x), m1 = __uint_as_float(ml.z);
             const float M = lean_row_max(fmaxf(m0, m1));
@@ -766,7 +857,6 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             }
             reinterpret_cast<float4 *>(S.join)[tid] = a4;   // [tid / (HD / 4)][HD]
             RES_STAMP(31);
-            zero_red(1);
             __syncthreads();
             RES_STAMP(26);
             const int skip = (h * HD) % 128 / 4;            // a head of 64 channels is half of a k tile: the other half counts for nothing
@@ -774,32 +864,39 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
                 const int c = tid - skip;
                 float4 sum = zero4;
                 if (c >= 0 && c < HD / 4) {
-                    float4 t[NJ];
+#pragma unroll 1
+                    for (int q0 = 0; q0 < NJ; q0 += 8) {
+                        float2 lo[8], hi[8];
 #pragma unroll
-                    for (int q = 0; q < NJ; q++) t[q] = reinterpret_cast<const float4 *>(S.join)[q * (HD / 4) + c];
+                        for (int q = 0; q < 8; q++) {
+                            const float2 *t = reinterpret_cast<const float2 *>(S.join + (q0 + q) * HD + (c >> 1) * 8 + (c & 1) * 2);
+                            lo[q] = t[0], hi[q] = t[2];
+                        }
 #pragma unroll
-                    for (int q = 0; q < NJ; q++) sum.x += t[q].x, sum.y += t[q].y, sum.z += t[q].z, sum.w += t[q].w;
+                        for (int q = 0; q < 8; q++) sum.x += lo[q].x, sum.y += lo[q].y, sum.z += hi[q].x, sum.w += hi[q].y;
+                    }
                 }
-                split_terms4(tid, sum.x, sum.y, sum.z, sum.w);
+                put_digits(tid, sum.x, sum.y, sum.z, sum.w);
             }
             __syncthreads();
             RES_STAMP(10);
-            const int tiles = tiles3(v);
-            multiply(w3, kAt3, ent, 1, n3, v, tiles * KT3, 1, unit3);
+            const ResShare<HD> share(p, v, 1);
+            if (wave / KT3 < share.tiles) multiply(One{}, std::true_type{}, 1, ent, share, wave / KT3, wave % KT3, KT3, wave % KT3);
             RES_STAMP(11);
             __syncthreads();
-            if (wave == 7) {
-                const float s = column(1, lane);
-                const uint32_t r = (uint32_t)(v >> 3), x = (uint32_t)(v & 7);
-                if (lane < 2) put(kResM1 + 32u * r + 2u * x + (uint32_t)lane, __float_as_uint(lane == 0 ? M : L), true);
-                if (lane < tiles * 16) put(kResG1 + r * 512u + x * 64u + (uint32_t)lane, __float_as_uint(s), true);
+            if (wave >= 4) {
+                const uint32_t r = (uint32_t)(v >> 3), x = (uint32_t)(v & 7), t = (uint32_t)wave - 4;
+                if (wave == 4 && lane < 2) put(kResM1 + 32u * r + 2u * x + (uint32_t)lane, __float_as_uint(lane == 0 ? M : L), true);
+                if ((int)t < share.tiles) {
+                    const float s = tile_sum((int)t, KT3);
+                    if (lane < 16) put(kResG1 + r * 512u + x * 64u + t * 16u + (uint32_t)lane, __float_as_uint(s), true);
+                }
             }
             if (!ALL) __syncthreads();
         }
         RES_STAMP(12);
-        if (ALL) load_units(w5, kAt5, weight(ent, 3, n5));
         if (wave == 6)
-            for (int v = first; v < end; v += step)
+            RES_SHARES(v)
                 if (tiles3(v) > 0) combine(v, kResG1, kResY, true);
         RES_STAMP(13);
         // ---- gate | up of the row, and the gated row
@@ -808,54 +905,61 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             y4 = make_float4(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z), __uint_as_float(raw.w));
         }
         RES_STAMP(14);
+        // What the norm needs is here: said in so many words, and what is asked for next kept together, or the norm's first
+        // instructions would be among these loads and wait for them.
+        res_stored();
+        RES_TOGETHER();
         if (ALL) load_kv(ent_next, first);   // (behind the last layer: its own again)
+        wp1 = row4(ent, 3), wi1 = row4(ent_next, 0);
+        ent_after = entry_of(l + 2);
+        RES_TOGETHER();
         RES_STAMP(25);
         norm_row(wp, wi);
         RES_STAMP(15);
-        wp = row4(ent, 3), wi = row4(ent_next, 0);
-        for (int v = first; v < end; v += step) {
-            zero_red(2);
-            multiply(w4, kAt4, ent, 2, n4, v, 2 * pairs4(v) * p.cg_h, 2, unit4);
+        RES_SHARES(v) {
+            const ResShare<HD> share(p, v, 2);
+            const int parts = share.tiles == 4 ? 4 : 8, q = share.tiles == 4 ? wave >> 2 : 0;
+            // (a pair's k tiles start one wavefront later than the other's: the SIMDs, which have two of the wavefronts each, get as many)
+            if (share.tiles > 0 && share.has(p, 2 * q)) multiply(Two{}, std::false_type{}, 2, ent, share, 2 * q, (wave + q) & (parts - 1), parts, wave & (parts - 1));
             RES_STAMP(16);
             __syncthreads();
-            if (wave == 7) {
-                const int q = (lane >> 4) & 1;
-                const float gate = column(2, 32 * q + i16), up = column(2, 32 * q + 16 + i16);
-                const float g = pair_of(v, q) < p.pairs ? res_gelu(gate) * up : 0.f;   // columns past ffn: zeros
-                uint16_t t[3];
-                lean_split1<2>(g, t);
-                if (lane < 16 * pairs4(v)) put((uint32_t)(v & 7) * kResLocal + kResH + (uint32_t)(((v >> 3) + 32 * q) * 16 + i16), (uint32_t)t[0] | ((uint32_t)t[1] << 16), wide);
+            if (wave >= 4 && 2 * (wave - 4) < share.tiles) {
+                const int t = 2 * (wave - 4);
+                const float gate = tile_sum(t, parts), up = tile_sum(t + 1, parts);
+                const float g = res_pair(p, v, wave - 4) < p.pairs ? res_gelu(gate) * up : 0.f;   // columns past ffn: zeros
+                if (lane < 16) put((uint32_t)(v & 7) * kResLocal + kResH + res_place((uint32_t)(((v >> 3) + 32 * (wave - 4)) * 16 + lane)), __float_as_uint(g), wide);
             }
             if (!ALL) __syncthreads();
         }
         RES_STAMP(17);
         // ---- down: the XCD's slice of the gated row times its rows of the weight
-        for (int v = first; v < end; v += step) {
+        RES_SHARES(v) {
             const int nk = slice_tiles(v);
             if (tid < nk * 32) {
                 const uint4 w = take16((uint32_t)(v & 7) * kResLocal + kResH + (uint32_t)tid * 4u);
-                put_terms(tid, make_uint2(__builtin_amdgcn_perm(w.y, w.x, 0x05040100u), __builtin_amdgcn_perm(w.w, w.z, 0x05040100u)),
-                          make_uint2(__builtin_amdgcn_perm(w.y, w.x, 0x07060302u), __builtin_amdgcn_perm(w.w, w.z, 0x07060302u)));
+                put_digits(tid, __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
             }
             RES_STAMP(18);
             RES_STAMP(24);
-            zero_red(3);
             __syncthreads();
             RES_STAMP(19);
-            const int tiles = tiles3(v);
-            multiply(w5, kAt5, ent, 3, n5, v, tiles * nk, 3, unit5);
-            if (ALL || v == first) load_ahead(ent_next);   // (behind the last layer: its own again)
+            const ResShare<HD> share(p, v, 3);
+            // (a k tile per wavefront, which takes all its tiles; one that has none leaves zeros)
+            if (share.tiles == 1 || share.tiles == 2) multiply(Two{}, std::true_type{}, 3, ent, share, 0, wave, kResWaves, wave);
+            else if (share.tiles == 3) multiply(Three{}, std::true_type{}, 3, ent, share, 0, wave, kResWaves, wave);
+            else if (share.tiles == 4) multiply(Four{}, std::true_type{}, 3, ent, share, 0, wave, kResWaves, wave);
             RES_STAMP(20);
             __syncthreads();
-            if (wave == 7) {
-                const float s = column(3, lane);
-                if (lane < tiles * 16) put(kResG2 + (uint32_t)(v >> 3) * 512u + (uint32_t)(v & 7) * 64u + (uint32_t)lane, __float_as_uint(s), true);
+            if (wave >= 4 && wave - 4 < share.tiles) {
+                const uint32_t t = (uint32_t)wave - 4;
+                const float s = tile_sum((int)t, kResWaves);
+                if (lane < 16) put(kResG2 + (uint32_t)(v >> 3) * 512u + (uint32_t)(v & 7) * 64u + t * 16u + (uint32_t)lane, __float_as_uint(s), true);
             }
             if (!ALL) __syncthreads();
         }
         RES_STAMP(21);
         if (wave == 6)
-            for (int v = first; v < end; v += step)
+            RES_SHARES(v)
                 if (tiles3(v) > 0) combine(v, kResG2, kResY2, false);
         RES_STAMP(22);
         if (holds && (l + 1 < p.n_layers || first == 0)) {
@@ -863,14 +967,16 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
             y4 = make_float4(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z), __uint_as_float(raw.w));
         }
         RES_STAMP(23);
+        res_stored();   // (the next norm's operands are here)
         RES_STAMPS_OUT();
         cur = next;
         next = next == (kResSets - 1) * kResWords * 4u ? 0u : next + kResWords * 4u;
-        ent = ent_next, ent_next = entry_of(l + 2);
+        ent = ent_next, ent_next = ent_after;
     }
     if (first == 0 && holds) {
-        *reinterpret_cast<float4 *>(p.x_out + tid * 4) = x4;
-        *reinterpret_cast<float4 *>(p.y_out + tid * 4) = y4;
+        float *x = p.x_out + place(), *y = p.y_out + place();
+        *reinterpret_cast<float2 *>(x) = make_float2(x4.x, x4.y), *reinterpret_cast<float2 *>(x + 4) = make_float2(x4.z, x4.w);
+        *reinterpret_cast<float2 *>(y) = make_float2(y4.x, y4.y), *reinterpret_cast<float2 *>(y + 4) = make_float2(y4.z, y4.w);
     }
 }
 
@@ -878,8 +984,8 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD> 
 // did not begin (`behind` is set), or that was never made, with the workgroups that have arrived by the deadline.
 // (Two kernels: in one the second form costs the first 25 us a token, in registers. A launch that finds its work done is 2 us.)
 template <int HD, int SG, bool ALL>
-__global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kernel(const ResidentArgs p) {
-    __shared__ __attribute__((aligned(16))) ResShared<HD> S;
+__global__ void __launch_bounds__(kResThreads + (ALL ? 64 * kFeedWaves : 0)) RES_ONE_PER_CU(ALL) dec_resident_kernel(const ResidentArgs p) {
+    __shared__ __attribute__((aligned(16))) ResShared<HD, SG, ALL> S;
     const int pos = *p.pos;
     if (pos >= p.max_seq) return;   // the cache is full: the step is a no-op (the token pick reports it)
     int tries = p.polls;
@@ -942,6 +1048,17 @@ __global__ void __launch_bounds__(kResThreads) RES_ONE_PER_CU dec_resident_kerne
     }
     set = (epoch % kResSets) * ((uint32_t)p.n_layers % kResSets) % kResSets;
 #endif
+    if constexpr (ALL) {
+        if ((int)threadIdx.x >= kResThreads) {
+            switch (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) - kResWaves) {
+                case 0: res_feed<HD, SG, 0>(p, S, first, pos + 1); break;
+                case 1: res_feed<HD, SG, 1>(p, S, first, pos + 1); break;
+                case 2: res_feed<HD, SG, 2>(p, S, first, pos + 1); break;
+                default: res_feed<HD, SG, 3>(p, S, first, pos + 1); break;
+            }
+            return;
+        }
+    }
     res_layers<HD, SG, ALL>(p, S, first, n, wide, set, pos, tries);
     if (tries <= 0) *p.broken = 1;
 }
@@ -994,12 +1111,14 @@ bool hipc::resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c) {
 
 namespace {
 
+constexpr int whole_units(int units) { return (units + 3) / 4 * 4; }   // four units' scales are asked for together
+
 template <int HD, bool ALL>
 void launch_sg(hipc_ctx *ctx, int sg, const ResidentArgs &a, int workgroups) {
     switch (sg) {
-        case 4: hipLaunchKernelGGL((dec_resident_kernel<HD, 4, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
-        case 2: hipLaunchKernelGGL((dec_resident_kernel<HD, 2, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL((dec_resident_kernel<HD, 1, ALL>), dim3(workgroups), dim3(kResThreads), 0, ctx->stream, a); break;
+        case 4: hipLaunchKernelGGL((dec_resident_kernel<HD, 4, ALL>), dim3(workgroups), dim3(kResThreads + (ALL ? 64 * kFeedWaves : 0)), 0, ctx->stream, a); break;
+        case 2: hipLaunchKernelGGL((dec_resident_kernel<HD, 2, ALL>), dim3(workgroups), dim3(kResThreads + (ALL ? 64 * kFeedWaves : 0)), 0, ctx->stream, a); break;
+        default: hipLaunchKernelGGL((dec_resident_kernel<HD, 1, ALL>), dim3(workgroups), dim3(kResThreads + (ALL ? 64 * kFeedWaves : 0)), 0, ctx->stream, a); break;
     }
 }
 template <bool ALL>
@@ -1023,9 +1142,15 @@ int hipc::resident_launch(hipc_ctx *ctx, const hipc_decoder_config &c, const Res
     a.n_layers = c.n_layers, a.n_q = c.n_q_heads, a.n_kv = c.n_kv_heads;
     a.lg_group = __builtin_ctz((unsigned)(c.n_q_heads / c.n_kv_heads)), a.lg_parts = 3 - __builtin_ctz((unsigned)c.n_q_heads);
     a.max_seq = c.max_seq, a.v_stride = attn_v_stride(c.max_seq);
-    a.inv_cg_h = (65536u + (uint32_t)a.cg_h - 1u) / (uint32_t)a.cg_h;
     a.inv_hidden = 1.f / (float)c.hidden;
-    a.nib_mask = 0x000f000fu, a.magic = 0x43004300u;
+    // Places in LDS for the units of the largest share of each product. q|k|v's are among gate|up's, those that are asked for when
+    // the former are done with; the next layer's q|k|v are asked for behind gate|up.
+    const int down_kts = (int)ceil_div(a.cg_f, kResXcds), h_tiles = (int)ceil_div(a.tiles_h, kResRanks);
+    a.slot[1] = 0;
+    a.slot[3] = whole_units(h_tiles * std::max(1, c.head_dim / 128));
+    a.slot[2] = a.slot[3] + whole_units(h_tiles * down_kts);
+    a.slot[0] = a.slot[2] + kFeedFirst;
+    static_assert(whole_units(4 * 2) + whole_units(4 * 8) + std::max(whole_units(4 * 16), kFeedFirst + whole_units(2 * 16)) <= kResSlots, "the largest shapes resident_takes");
     a.eps = c.rms_eps, a.scale = c.attn_scale > 0.f ? c.attn_scale : 1.f / sqrtf((float)c.head_dim);
     a.arrive = ctx->tune.dec_wait >= 0 ? ctx->tune.dec_wait : kArriveTicks;
     a.polls = ctx->tune.dec_polls > 0 ? ctx->tune.dec_polls : kPollBudget;

@@ -23,7 +23,7 @@ constexpr uint32_t kResMaxHidden = 2048, kResMaxHead = 256, kResMaxSlice = 1024;
 constexpr uint32_t kResA = 0;                                          // [rank][head]: unnormalised attention outputs
 constexpr uint32_t kResML = kResA + kResRanks * kResMaxHead;           // [rank](max, sum)
 constexpr uint32_t kResY = kResML + 2 * kResRanks;                     // the attention branch's row
-constexpr uint32_t kResH = kResY + kResMaxHidden;                      // the XCD's slice of the gated row, two bf16 terms a word
+constexpr uint32_t kResH = kResY + kResMaxHidden;                      // the XCD's slice of the gated row
 constexpr uint32_t kResY2 = kResH + kResMaxSlice;                      // the feed-forward branch's row
 constexpr uint32_t kResLocal = kResY2 + kResMaxHidden;                 // words of one XCD
 constexpr uint32_t kResG1 = kResXcds * kResLocal;                      // [rank][XCD][64 columns]: o's partial rows
@@ -46,8 +46,7 @@ struct ResidentArgs {
     int n_q, n_kv, lg_group, lg_parts;   // XCDs per head = 1 << lg_parts
     int max_seq, v_stride, behind;
     int arrive, polls, wide;             // how long workgroups are waited for, in 10 ns; polls of a thread; stores at agent scope whatever the launch finds
-    uint32_t inv_cg_h;                   // 65536 / cg_h, rounded up
-    uint32_t nib_mask, magic;
+    int slot[4];                         // where the units of product i begin in LDS
     float eps, scale, inv_hidden;
 };
 

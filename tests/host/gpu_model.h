@@ -177,7 +177,9 @@ inline T atomicMax(T *p, T v) { const T old = *p; if (v > old) *p = v; return ol
 #define __builtin_nontemporal_load gpu_model_nt_load
 #define __builtin_nontemporal_store gpu_model_nt_store
 #define __launch_bounds__(...)
-inline void __syncthreads() {}
+// barriers a thread has passed: where a kernel's wavefronts take different ways through it, they must pass as many (see gpu_model_launch)
+inline thread_local size_t gpu_model_barriers = 0;
+inline void __syncthreads() { gpu_model_barriers++; }
 template <typename T>
 inline T __shfl_xor(T v, int, int = 64) { return v; }
 template <typename T>
@@ -254,12 +256,19 @@ inline void gpu_model_launch(const char *name, dim3 grid, dim3 block, size_t lds
         for (unsigned by = y0; by < y1; by++)
             for (unsigned bx = 0; bx < grid.x; bx++) {
                 blockIdx = dim3(bx, by, bz);
+                size_t first = 0;
                 for (unsigned tz = 0; tz < block.z; tz++)
                     for (unsigned ty = 0; ty < block.y; ty++)
                         for (unsigned tx = 0; tx < block.x; tx++) {
                             threadIdx = dim3(tx, ty, tz);
                             g.threads++;
+                            gpu_model_barriers = 0;
                             body();
+                            if (tx == 0 && ty == 0 && tz == 0) first = gpu_model_barriers;
+                            if (gpu_model_barriers != first && std::strstr(name, "resident")) {
+                                std::printf("FAILED (%s): workgroup %u: thread %u passes %zu barriers, thread 0 %zu\n", g.where.c_str(), bx, tx, gpu_model_barriers, first);
+                                std::exit(1);
+                            }
                         }
             }
     g.where = outer;

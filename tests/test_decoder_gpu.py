@@ -417,6 +417,35 @@ def test_all_layers_in_one_launch(ctx, pkg, oracle, route, hidden, ffn, hd, nq, 
     dec.destroy()
 
 
+LDS_LIMITS = [  # the weights of a share in LDS: every place taken; two tiles of q|k|v a workgroup among gate|up's places; one place in four
+    (2048, 8192, 256, 8, 1, 32),
+    (512, 1040, 256, 8, 8, 32),
+    (144, 128, 64, 2, 1, 128),
+]
+
+
+@pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", LDS_LIMITS)
+def test_weights_of_the_one_launch_in_lds(ctx, pkg, oracle, hidden, ffn, hd, nq, nkv, bs):
+    dec, ref = three_layers(pkg, ctx, hidden, ffn, hd, nq, nkv, bs)
+    steps_match(ctx, dec, ref)
+    dec.destroy()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_a_row_that_is_not_finite(ctx, pkg, oracle, value):
+    """One channel of a norm's weight: the row it goes into the products with has no digits there, and every result is NaN."""
+    dec, ref = three_layers(pkg, ctx, 448, 1088, 128, 8, 2, 64)
+    w = ref.w.norms[(1, pkg.decoder.NORM_PRE_FFN)].copy()
+    w[77] = value
+    ref.w.norms[(1, pkg.decoder.NORM_PRE_FFN)] = w
+    dec.load(ref.w)
+    dec.reset(23, 69)
+    dec.step()
+    token, _, logits, _ = dec.read(want_logits=True)
+    assert np.all(np.isnan(logits)) and token == 0
+    dec.destroy()
+
+
 @pytest.mark.parametrize("env", [{"HIPC_DEC_WAIT": 0}, {"HIPC_DEC_WAIT": 100}, {"HIPC_DEC_WIDE": 1}, {"HIPC_DEC_RESIDENT": 40, "HIPC_DEC_WAIT": 0}],
                          ids=["does-not-begin", "waits-a-microsecond", "no-shared-l2", "those-there-at-once"])
 @pytest.mark.parametrize("hidden,ffn,hd,nq,nkv,bs", RESIDENT)
