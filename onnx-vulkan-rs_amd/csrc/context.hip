@@ -81,6 +81,8 @@ void release_block(hipc_ctx *ctx, void *p) {
 int release_deferred(hipc_ctx *ctx) {
     for (void *p : ctx->deferred) release_block(ctx, p);
     ctx->deferred.clear();
+    for (void *p : ctx->deferred_host) (void)hipHostFree(p);
+    ctx->deferred_host.clear();
     // the stream is idle: every staging slot is free again
     for (bool &b : ctx->stage.pending) b = false;
     ctx->stage.used = 0;

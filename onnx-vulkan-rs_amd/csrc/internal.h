@@ -123,6 +123,7 @@ struct hipc_ctx {
     std::mutex mu;
     std::string err;
     std::vector<void *> deferred;        // released at the next flush
+    std::vector<void *> deferred_host;   // the same, pinned host memory
     // Blocks the library itself retired (a scratch slot that grew, requantisation ratios that changed, a
     // replaced decoder weight) while recorded graphs exist: a graph may hold their addresses, so they stay
     // allocated until the last graph of the context is destroyed.

@@ -138,6 +138,8 @@ struct Model {
         hipc_decoder_destroy(&ctx, dec);
         for (void *p : ctx.deferred) gpu_model::release(p);
         ctx.deferred.clear();
+        for (void *p : ctx.deferred_host) gpu_model::release(p);
+        ctx.deferred_host.clear();
         for (void *p : inputs) gpu_model::release(p);
         inputs.clear();
         for (hipc::Scratch &s : ctx.scratch)
@@ -287,6 +289,7 @@ void which_form() {
         }
         hipc_decoder_destroy(&ctx, dec);
         for (void *p : ctx.deferred) gpu_model::release(p);
+        for (void *p : ctx.deferred_host) gpu_model::release(p);
     }
     report("which form a decoder takes");
 }

@@ -214,6 +214,8 @@ using std::min;
 // ---- the host API the sources call: allocations are registered host blocks, the stream is immediate ----
 #define hipMalloc gpu_model_hipMalloc
 #define hipFree gpu_model_hipFree
+#define hipHostMalloc(p, bytes, flags) gpu_model_hipMalloc(p, bytes)
+#define hipHostFree gpu_model_hipFree
 #define hipMemsetAsync gpu_model_hipMemsetAsync
 #define hipMemcpyAsync gpu_model_hipMemcpyAsync
 #define hipGetLastError gpu_model_hipGetLastError
