@@ -547,28 +547,37 @@ int gemm_launch(hipc_ctx *ctx, const GemmArgs &g, unsigned batch) {
 //   * only A goes through LDS (8 KB stored, 8 KB read per stage); the fragments of the prepacked,
 //     fragment-major B come straight from memory into the matrix-core layout, one fully coalesced
 //     1 KB load each, four stages ahead;
-//   * the four partial tiles are added through LDS at the end, wavefront w finishing fragment w.
+//   * the four partial tiles are added through LDS at the end, wavefront w finishing fragment w, four words
+//     at a time (LDS serves an instruction in 16 clocks whatever its width: 1000 x 4096 x 1024 11.3 -> 11.0 us).
 // Measured against the LDS-staged 64x64 tiles: 12.8 against 17.3 us for 1000 x 4096 x 1024, 7.8
 // against 8.5 us at k = 1024; from about four tiles per CU on, or with very short k, the reduction
 // at the end costs more than the loop saves. (The same kernel with 128x128 tiles, wavefronts 2x2
 // and no k split was slower than either: 16 products per stage issued back to back keep the
 // wavefront from issuing the stage's memory instructions, as in the 128x128 LDS-staged kernel.)
+// With no more tiles than CUs and a long k a workgroup is two groups of four wavefronts (GROUPS), with LDS buffers of their
+// own, that take the stages in turn: the second wavefront of a SIMD fills the chain barrier - LDS - products - LDS of the
+// first, 0.19 us a stage becomes 0.15, towards the 0.12 that 16 KB take at the CU's 64 bytes a clock. For that the hand-over
+// is 112 KB instead of 48. The epilogue is dealt to eight wavefronts.
 constexpr int kSmallSets = 4;  // register sets of A chunks and of B fragments: stages in flight
-// the hand-over of three fragments per wavefront reuses the two A buffers (18 KB of its 48 KB)
-constexpr size_t kSmallLds = 4 * 3 * 16 * 64 * sizeof(int) + 4 * 64 * sizeof(int);
+// the hand-over, of which an owner gets (4 GROUPS - 1) parts of 16 / GROUPS words a lane, reuses the A buffers (18 KB a group of its 48 or 112 KB)
+constexpr size_t small_lds(int groups) { return (size_t)(4 * (4 * groups - 1) * 16 + 4 * groups) * 64 * sizeof(int); }
+constexpr size_t kSmallLds = small_lds(1);
 
-template <int EPI, bool DYN>
-__global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs p) {  // three workgroups per CU (LDS allows no more): 168 registers
+template <int EPI, bool DYN, int GROUPS>
+__global__ void __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) int8_gemm_small_kernel(const GemmArgs p) {  // (one group: three workgroups per CU, LDS allows no more: 168 registers)
     constexpr int T = 64;                       // edge of the workgroup's tile
+    constexpr int kOwn = 16 / GROUPS;           // accumulator words of a fragment that a wavefront finishes
+    constexpr int kParts = 4 * GROUPS - 1;      // wavefronts that hand theirs over to it
     constexpr int kCh = T / 32;                 // 16-byte chunks of an A slab per thread
     constexpr int kSteps = 1;                   // product steps of a stage per wavefront
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-    uint8_t *lds_a = lds_raw;                                              // [2][T * kPitch]
-    int *lds_acc = reinterpret_cast<int *>(lds_raw);                       // after the loop: [owner][source 0..2][16][64]
-    int *lds_sum = lds_acc + 4 * 3 * 16 * 64;                              // [4 wavefronts][64 rows]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;   // of the group
+    const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8), self = group * 4 + wave;
+    uint8_t *lds_a = lds_raw + group * 2 * T * kPitch;                     // [group][2][T * kPitch]
+    int *lds_acc = reinterpret_cast<int *>(lds_raw);                       // after the loop: [owner][source][kOwn / 4][64] four words at a time
+    int *lds_sum = lds_acc + 4 * kParts * 16 * 64;                         // [wavefront][64 rows]
     const int r32 = lane & 31, kg = lane >> 5;
-    auto handed = [&](int owner, int slot, int r) -> int & { return lds_acc[((owner * 3 + slot) * 16 + r) * 64 + lane]; };
+    auto handed = [&](int owner, int slot, int r) -> i32x4 & { return reinterpret_cast<i32x4 *>(lds_acc)[((owner * kParts + slot) * (kOwn / 4) + r / 4) * 64 + lane]; };   // words r .. r + 3
 
     const int tiles_x = (p.J + T - 1) / T, tiles_y = (p.I + T - 1) / T;
     const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
@@ -606,12 +615,15 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
         const_cast<uint8_t *>(p.Q), 0, (int)((uint32_t)(j_last + 1) * (uint32_t)p.K_pad), 0x00020000);
 
     u32x4 ra[kSmallSets][kCh], rb[kSmallSets][kSteps][2];
-    auto load_a = [&](int set, int stage) {
+    // (stages are the group's own: its s-th is the product's stage GROUPS s + group)
+    auto load_a = [&](int set, int s) {
+        const int stage = GROUPS * s + group;
 #pragma unroll
         for (int u = 0; u < kCh; u++)
             ra[set][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, p_off[u] - (stage >= nk - 1 ? tail_back : 0u), min(stage, nk - 1) * kBK, 0);
     };
-    auto load_b = [&](int set, int stage) {
+    auto load_b = [&](int set, int s) {
+        const int stage = GROUPS * s + group;
 #pragma unroll
         for (int step = 0; step < kSteps; step++)
 #pragma unroll
@@ -620,7 +632,8 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
     };
     // a stage past the end is stored as zeros: its products add nothing whatever B holds (and so is, where the sums over
     // A's rows count, what the last stage read from the row's end: see gemm_tail_back)
-    auto store_a = [&](int set, int buf, int stage) {
+    auto store_a = [&](int set, int buf, int s) {
+        const int stage = GROUPS * s + group;
         const uint32_t keep = stage < nk && !(DYN && stage == nk - 1 && tail_back) ? 0xffffffffu : 0u;
 #pragma unroll
         for (int u = 0; u < kCh; u++)
@@ -672,8 +685,10 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
     // Stage s: multiply it out of LDS buffer s & 1 with B set s % 4, refill that B set with stage
     // s + 4, move stage s + 1 from its A set into the other LDS buffer (last read during stage s - 1,
     // before the previous barrier) and refill that A set with stage s + 5. Nothing in the loop is
-    // conditional, so the memory counters stay exact.
-    for (int s = 0; s < nk; s += kSmallSets) {
+    // conditional but its ends, so the memory counters stay exact. Two groups, which take as many stages each, leave behind
+    // any: whole rounds of four cost them up to six stages' time (1000 x 2560 x 1024 9.2 -> 8.6 us). One group leaves behind
+    // whole rounds, whose four stages the compiler orders as one (1000 x 4096 x 1024 11.0 us, behind any 11.5).
+    for (int s = 0, stages = (nk + GROUPS - 1) / GROUPS;; s += kSmallSets) {
 #pragma unroll
         for (int d = 0; d < kSmallSets; d++) {
             compute(d & 1, d);
@@ -681,8 +696,10 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
             store_a((d + 1) % kSmallSets, (d + 1) & 1, s + d + 1);
             load_a((d + 1) % kSmallSets, s + d + 1 + kSmallSets);
             __syncthreads();
+            if ((GROUPS == 2 || d == kSmallSets - 1) && s + d + 1 >= stages) goto multiplied;
         }
     }
+multiplied:
 
     // row sums of A over this wavefront's product steps: the two k halves of a row live in lanes l and l + 32
     const int ifr = wave >> 1, jf = wave & 1;
@@ -691,62 +708,69 @@ __global__ void __launch_bounds__(256, 3) int8_gemm_small_kernel(const GemmArgs 
         for (int f = 0; f < 2; f++) dsum[f] += __shfl_xor(dsum[f], 32, 64);
         if (kg == 0) {
 #pragma unroll
-            for (int f = 0; f < 2; f++) lds_sum[wave * 64 + (f ^ ifr) * 32 + r32] = dsum[f];
+            for (int f = 0; f < 2; f++) lds_sum[self * 64 + (f ^ ifr) * 32 + r32] = dsum[f];
         }
     }
-    // the other three fragments are handed over (the A buffers are free: the loop ended with a barrier)
+    // everything but its own part is handed over (the A buffers are free: the loop ended with a barrier). Group g finishes words
+    // kOwn g .. of a fragment.
+    int own[kOwn];
+#pragma unroll
+    for (int r = 0; r < kOwn; r++) own[r] = GROUPS == 2 && group ? acc[0][0][16 - kOwn + r] : acc[0][0][r];
 #pragma unroll
     for (int di = 0; di < 2; di++)
 #pragma unroll
-        for (int dj = 0; dj < 2; dj++) {
-            if (di == 0 && dj == 0) continue;
-            const int owner = ((ifr ^ di) << 1) | (jf ^ dj);
-            const int slot = wave < owner ? wave : wave - 1;  // 0..2 among the three sources
+        for (int dj = 0; dj < 2; dj++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) handed(owner, slot, r) = acc[di][dj][r];
-        }
+            for (int g = 0; g < GROUPS; g++) {
+                const int owner = g * 4 + (((ifr ^ di) << 1) | (jf ^ dj));
+                if (GROUPS == 1 ? di == 0 && dj == 0 : owner == self) continue;
+                const int slot = self < owner ? self : self - 1;  // among the sources
+#pragma unroll
+                for (int r = 0; r < kOwn; r += 4)
+                    handed(owner, slot, r) = i32x4{acc[di][dj][g * kOwn + r], acc[di][dj][g * kOwn + r + 1], acc[di][dj][g * kOwn + r + 2], acc[di][dj][g * kOwn + r + 3]};
+            }
     __syncthreads();
 
     // The handed-over parts are read four output rows ahead of their use: the LDS latency is paid
     // once, not per output, and the stores still leave spread out (other workgroups of the CU are
     // in their product loops meanwhile).
     const int fixed = p.K * zd * zc - zd * my_csum;
-    const int gj = j0 + jf * 32 + r32;
+    const int gj = j0 + jf * 32 + r32, row0 = ifr * 32 + group * 2 * kOwn;   // of its first outputs
     float fmn = 0.f, fmx = 0.f;
-    int part[2][4], rs[2][4];
+    i32x4 part[2], rs[2];
     auto read_group = [&](int g, int par) {
+        part[par] = handed(self, 0, 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int r = 4 * g + e;
-            part[par][e] = handed(wave, 0, r) + handed(wave, 1, r) + handed(wave, 2, r);
-            if (DYN) {
-                const int at = ifr * 32 + g * 8 + kg * 4 + e;
-                rs[par][e] = lds_sum[at] + lds_sum[64 + at] + lds_sum[128 + at] + lds_sum[192 + at];
-            }
+        for (int slot = 1; slot < kParts; slot++) part[par] += handed(self, slot, 4 * g);
+        if (DYN) {
+            const i32x4 *sums = reinterpret_cast<const i32x4 *>(lds_sum + row0 + g * 8 + kg * 4);
+            rs[par] = sums[0];
+#pragma unroll
+            for (int w = 1; w < 4 * GROUPS; w++) rs[par] += sums[w * 16];
         }
     };
     const bool words = EPI == EPI_REQUANT && ((p.J | (int)(reinterpret_cast<uintptr_t>(p.Y) & 3)) & 3) == 0;   // bytes leave four columns at a time
     const RequantBytes bytes{my_emit.s, (float)p.y_zp + (p.out_signed ? 128.f : 0.f), p.out_signed ? 0x80808080u : 0u};
     read_group(0, 0);
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        if (g + 1 < 4) read_group(g + 1, (g + 1) & 1);
+    for (int g = 0; g < kOwn / 4; g++) {
+        if (g + 1 < kOwn / 4) read_group(g + 1, (g + 1) & 1);
         int q[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int gi = i0 + ifr * 32 + g * 8 + kg * 4 + e;
-            int v = acc[0][0][4 * g + e] + part[g & 1][e] + fixed;
+            const int gi = i0 + row0 + g * 8 + kg * 4 + e;
+            int v = own[4 * g + e] + part[g & 1][e] + fixed;
             if (DYN) v -= zc * rs[g & 1][e];
             if (EPI == EPI_REQUANT && words) q[e] = v + my_emit.qb;
             else if (gi < p.I && gj < p.J) gemm_emit_mm<EPI>(p, my_emit, gi, gj, v, fmn, fmx);
         }
         if (EPI == EPI_REQUANT && words) {
             const uint32_t w = gemm_quad_row(gemm_requant4(bytes, q));
-            const int gi = i0 + ifr * 32 + g * 8 + kg * 4 + (lane & 3);
+            const int gi = i0 + row0 + g * 8 + kg * 4 + (lane & 3);
             if (gi < p.I && gj < p.J) *reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(p.Y) + (size_t)gi * p.J + (gj & ~3)) = w;
         }
     }
-    if (EPI == EPI_SCALE_BIAS) gemm_emit_range(p, lane, wave, 4, fmn, fmx);
+    if (EPI == EPI_SCALE_BIAS) gemm_emit_range(p, lane, self, 4 * GROUPS, fmn, fmx);
 }
 
 // What the k-split convolution kernels below end with. The four wavefronts hold partial products

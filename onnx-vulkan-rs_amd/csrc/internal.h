@@ -59,7 +59,7 @@ struct Tuning {
     int gemv_per_cu = -1;     // HIPC_GEMV_PER_CU    resident GEMV wavefronts per CU of the persistent grid
     int gemm_tile = -1;       // HIPC_GEMM_TILE      LDS-staged int8 tiles: 64 or 128
     int gemm_big = -1;        // HIPC_GEMM_BIG       the int8 kernels that keep B out of LDS: 0 never, 1 / 2 the 256x256 / 128x128 tile whenever A allows
-    int gemm_small = -1;      // HIPC_GEMM_SMALL     the k-split 64x64 kernels: 0 never, 1 whenever A allows
+    int gemm_small = -1;      // HIPC_GEMM_SMALL     the k-split 64x64 kernels: 0 never, 1 / 2 (groups of four wavefronts; products only) whenever A allows
     int gemm_skinny = -1;     // HIPC_GEMM_SKINNY    the kernel for up to 64 rows: 0 never, 1 whenever A allows
     int conv_row = -1;        // HIPC_CONV_ROW       0: convolutions along one axis take the general route
     int prefill_tile = -1;    // HIPC_PREFILL_TILE   64, 128 or 192 (columns; 192 has 128 rows)

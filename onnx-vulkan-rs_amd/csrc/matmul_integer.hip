@@ -248,7 +248,7 @@ int launch_mm_big(hipc_ctx *ctx, const GemmArgs &g, int choice) {
 }
 
 // Products of a few 64x64 tiles per CU and a long enough k run on the kernel that keeps B out of LDS
-// and splits k over the wavefronts of a workgroup. The gemm_small option (0 / 1) overrides (tuning, tests).
+// and splits k over the wavefronts of a workgroup. The gemm_small option (0 / 1 / 2, see small_groups) overrides (tuning, tests).
 bool wants_small_tiles(hipc_ctx *ctx, const GemmArgs &g) {
     const int forced = ctx->tune.gemm_small;
     if (!g.p_aligned) return false;
@@ -258,18 +258,33 @@ bool wants_small_tiles(hipc_ctx *ctx, const GemmArgs &g) {
     const int64_t tiles64 = ceil_div(g.I, 64) * ceil_div(g.J, 64);
     return (tiles64 <= 2 * (int64_t)ctx->cu_count && g.K >= 4 * kBK) || (tiles64 <= 4 * (int64_t)ctx->cu_count && g.K >= 8 * kBK);
 }
-template <int EPI, bool DYN>
+// How many groups of four wavefronts a workgroup is. Us, one / two: 1000 x 4096 x 1024 (256 tiles) 10.95 / 10.5, with the sums
+// over A's rows 11.1 / 10.6, to bytes 10.4 / 10.2; 128 x 4096 x 512 10.9 / 10.0; 70 x 11008 x 1024 21.8 / 18.9; 1001 x 4000 x 1010
+// 11.5 / 11.4. With fewer stages the larger hand-over costs what they save: 1000 x 3072 x 1024 9.4 / 9.2, to bytes 8.7 / 8.9;
+// 200 x 3000 x 512 12.0 / 12.0, to bytes 11.2 / 11.7; 1000 x 1024 x 1024 6.4 / 6.6. Beyond a tile per CU, where three workgroups
+// of one group share a CU but not two of two groups: 1000 x 4096 x 1200 14.8 / 19.6.
+int small_groups(hipc_ctx *ctx, const GemmArgs &g) {
+    if (ctx->tune.gemm_small == 2) return 2;
+    return ctx->tune.gemm_small != 1 && ceil_div(g.I, 64) * ceil_div(g.J, 64) <= (int64_t)ctx->cu_count && g.K >= 28 * kBK ? 2 : 1;
+}
+template <int EPI, bool DYN, int GROUPS>
 int launch_mm_small_dyn(hipc_ctx *ctx, GemmArgs g) {
     const dim3 grid(gemm_grid(g, 64));
-    hipLaunchKernelGGL((int8_gemm_small_kernel<EPI, DYN>), grid, 256, kSmallLds, ctx->stream, g);
+    static bool lds_allowed[2][kMaxDevices] = {};
+    if (GROUPS == 2)
+        if (int rc = allow_dynamic_lds(ctx, int8_gemm_small_kernel<EPI, DYN, GROUPS>, small_lds(GROUPS), lds_allowed[0])) return rc;
+    if (GROUPS == 2 && !DYN && ctx->capturing)   // the instance that a recorded launch may be given later
+        if (int rc = allow_dynamic_lds(ctx, int8_gemm_small_kernel<EPI, true, GROUPS>, small_lds(GROUPS), lds_allowed[1])) return rc;
+    hipLaunchKernelGGL((int8_gemm_small_kernel<EPI, DYN, GROUPS>), grid, 256 * GROUPS, small_lds(GROUPS), ctx->stream, g);
     HIPC_LAUNCHED(ctx);
-    gemm_note_scalars(ctx, g, DYN, reinterpret_cast<const void *>(int8_gemm_small_kernel<EPI, true>));
+    gemm_note_scalars(ctx, g, DYN, reinterpret_cast<const void *>(int8_gemm_small_kernel<EPI, true, GROUPS>));
     return HIPC_OK;
 }
 template <int EPI>
 int launch_mm_small(hipc_ctx *ctx, const GemmArgs &g) {
     const bool zero_known = g.const_shift == 0 && (g.host_zp ? g.const_zp_value == 0 : g.const_zp == nullptr);
-    return zero_known ? launch_mm_small_dyn<EPI, false>(ctx, g) : launch_mm_small_dyn<EPI, true>(ctx, g);
+    if (small_groups(ctx, g) == 2) return zero_known ? launch_mm_small_dyn<EPI, false, 2>(ctx, g) : launch_mm_small_dyn<EPI, true, 2>(ctx, g);
+    return zero_known ? launch_mm_small_dyn<EPI, false, 1>(ctx, g) : launch_mm_small_dyn<EPI, true, 1>(ctx, g);
 }
 template <int EPI, bool DYN, int RB>
 int launch_mm_skinny_rb(hipc_ctx *ctx, const GemmArgs &g) {

@@ -93,6 +93,7 @@ struct Route {
 const Route kRoutes[] = {
     {"library's choice", -1, -1, -1},       {"LDS-staged 64x64", 64, 0, 0},       {"LDS-staged 128x128", 128, 0, 0},
     {"k-split 64x64 (B not in LDS)", -1, 0, 1}, {"B-direct 256x256", -1, 1, 0},   {"B-direct 128x128", -1, 2, 0},
+    {"k-split 64x64, two groups", -1, 0, 2},
 };
 
 // one matrix product through the three epilogues
@@ -177,7 +178,7 @@ int main(int argc, char **argv) {
         products(s[0], s[1], s[2], HIPC_U8, HIPC_I8, true);
         products(s[0], s[1], s[2], HIPC_I8, HIPC_U8, false);
     }
-    report("matrix products, six routes x four epilogue calls");
+    report("matrix products, seven routes x four epilogue calls");
     if (!quick) {
         products(1000, 1024, 4096, HIPC_U8, HIPC_I8, true);   // the benchmark's pair
         products(1000, 4096, 1024, HIPC_U8, HIPC_I8, true);

@@ -294,6 +294,19 @@ def test_rows_that_are_not_whole_stages(ctx, pkg, oracle, shape, route):
             assert np.array_equal(pkg.ops.matmul_integer(ctx, a, b, za, zb), want)
 
 
+@pytest.mark.parametrize("shape", [(70, 16, 7), (65, 128, 64), (64, 144, 130), (129, 256, 131), (257, 1040, 65), (70, 1136, 190), (133, 1280, 260)],
+                         ids=lambda s: "M%d_K%d_N%d" % s)
+def test_two_groups_share_the_stages(ctx, pkg, oracle, shape):
+    """64x64 tiles whose stages two groups of wavefronts take in turn: fewer stages than groups, an odd count (one group's last is
+    past the end), one more than a group has in flight; ragged tiles; sums over A's rows; every epilogue."""
+    m, k, n = shape
+    with ctx.options(HIPC_GEMM_BIG=0, HIPC_GEMM_SMALL=2):
+        _mm_three_epilogues(ctx, pkg, oracle, m, k, n, np.uint8, np.int8, seed=75)
+        _mm_three_epilogues(ctx, pkg, oracle, m, k, n, np.int8, np.uint8, seed=77)
+        a, b = rc.pseudo_plus1(m * k, 78).reshape(m, k), rc.pseudo_plus1(k * n, 79).view(np.int8).reshape(k, n)
+        assert np.array_equal(pkg.ops.matmul_integer(ctx, a, b, 131, None), oracle.matmul_integer(a, b, 131, 0))
+
+
 @pytest.mark.parametrize("offset,k", [(4, 256), (3, 128), (1, 45), (2, 16)])
 def test_rows_at_any_address(ctx, pkg, oracle, offset, k):
     """A inside a larger buffer, at an address that is not a multiple of 16 (or of 4)."""
