@@ -78,7 +78,7 @@ constexpr int kPollBudget = 1;                         // (one thread after the 
 // How long workgroups that have not started are waited for, in ticks of the 100 MHz clock. All of them, 50 us: they arrive within
 // microseconds on a free device, and within the 50 us another decoder's unembedding and token pick keep some CUs. In the
 // stand-in until nobody has come for 5 us.
-// Beside other work, us a token of gemma3-1b at 2048 (454 alone; launches per product 654 alone), the launches per product / 50 us and
+// Beside other work, us a token of gemma3-1b at 2048 (454 alone then, 435 since; launches per product 654 alone), the launches per product / 50 us and
 // 256 workgroups standing in / 200 us and 256 / 200 us and 64: beside a softmax of eight workgroups of a millisecond 763 / 773 / 923 / 1602;
 // launches that hold 64 CUs for 220 us 730 / 908 / 835 / 1191, 128 CUs for 140 us 788 / 777 / 570 / 569; products that fill the chip for 125 us
 // at a time - / 860 / 860 / 872. Two decoders side by side, a token of each: 780 / 878 / 877 / 877; three 918 / 1900 / 2490 / 2060,
