@@ -39,6 +39,7 @@
 #include "lanes.h"
 #include "lean_ops.h"
 #include "resident.h"
+#include "row_digits.h"
 
 namespace hipc {
 
@@ -88,7 +89,7 @@ constexpr int kArriveTicks = 5000, kJoinTicks = 500;
 constexpr int kResThreads = 512, kResWaves = 8;        // those that compute
 constexpr int kFeedWaves = 4;                          // and, in the launch of all, those that bring the weights: one per product
 constexpr int kResSlots = 104;                         // units of weights in LDS (see resident_launch)
-constexpr int kRowPitch = 384;                         // bytes of a k tile of the row: three digits of 128 values
+constexpr int kRowPitch = 512;                         // bytes of a k tile of the row: four digits of 128 values
 constexpr int kEntryWords = (int)(sizeof(ResidentLayer) / 4);
 
 typedef _Float16 rh16x8 __attribute__((ext_vector_type(8)));
@@ -126,10 +127,11 @@ inline void res_stored() {}
 // 3560; in the registers of the polling wavefronts, two phases ahead, 3725. (Eight layers of 2048 / 8192 with 8/1 heads of 256 at 2040,
 // where those registers held half of the units: 201 -> 185; of 512 / 2048 with 8/2 heads of 64: 123 -> 119.)
 //
-// The row takes part as whole numbers: 23 bits below the largest of every 32 values, as three signed bytes (digits), so a
-// product of a unit is two int8 matrix instructions with exact sums, and a weight's nibbles need no conversion beyond being
-// spread to bytes. The 16 rows of the matrix operand are the four 32-k chunks times the digits (the fourth of each is
-// empty): lane group g ends with the sums of chunk g. Two bf16 terms per value (17 bits) took twice the instructions a unit.
+// The row takes part as whole numbers of four signed bytes (row_digits.h has what that keeps of a value), so a product of a
+// unit is two int8 matrix instructions with exact sums, and a weight's nibbles need no conversion beyond being spread to bytes.
+// The 16 rows of the matrix operand are the four 32-k chunks times the digits: lane group g ends with the sums of chunk g.
+// The digits' own sums, for the zero points, are whole numbers too, so a weight of zero takes nothing from its row's value. Two
+// bf16 terms per value took twice the instructions a unit.
 typedef int ri32x4 __attribute__((ext_vector_type(4)));
 
 struct UnitWeight {
@@ -179,25 +181,29 @@ __device__ __forceinline__ float res_gelu(float v) {
 template <int HD, int SG, bool ALL>
 struct ResShared {
     static constexpr int SLOTS = ALL ? kResSlots : 1;
-    uint32_t row[16 * kRowPitch / 4];                    // the row's digits: [k tile][digit][128 bytes]
-    float2 chunk[64];                                    // per 32 values: what a 1 stands for, their sum in such units
+    union {
+        uint32_t row[16 * kRowPitch / 4];                // the row's digits: [k tile][digit, the highest first][128 bytes]
+        struct {                                         // (between q|k|v and o)
+            __half qa[2 * (HD + 8)];
+            __half pa[kResWaves][2 * (kAttnPass + 8)];
+            float sp[kResWaves][16];
+            float kn[HD], vn[HD];
+            float sown;
+        };
+    };
+    int4 chunk[64];                                      // per 32 values: digits_unit(), their sum (two words)
     float4 red4[4 * kResWaves];
     union {
         float red[4 * kResWaves * 64];                   // a product: [tile][part of its k tiles][lane]
         float join[kResThreads * 4];                     // (between two products)
     };
     float rope[2 * HD];
-    __half qa[2 * (HD + 8)];
-    __half pa[kResWaves][2 * (kAttnPass + 8)];
-    float sp[kResWaves][16];
-    float kn[HD], vn[HD];
-    float sown;
     uint32_t decision[2];
 #ifdef HIPC_PHASE_STAMPS
     uint32_t stamp[kResWaves][32];
 #endif
     // (last: the others' offsets fit the instructions')
-    float sc[SLOTS][16 * SG];
+    alignas(16) float sc[SLOTS][16 * SG];
     uint8_t zb[SLOTS][16 * SG];
     uint4 wq[SLOTS][64];                                 // units: as in memory, lane by lane
 };
@@ -400,15 +406,14 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
         float acc[NT];
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[j] = 0.f;
-        const int t3 = min(i16 & 3, 2), mine = i16 >> 2;
-        const char *row = reinterpret_cast<const char *>(S.row) + t3 * 128 + mine * 32 + g4 * 8;
-        const float2 *chunk = S.chunk + g4;
-        const bool digit = (i16 & 3) < 3;
-        const uint32_t m0 = digit && mine == 0 ? ~0u : 0u, m1 = digit && mine == 1 ? ~0u : 0u, m2 = digit && mine == 2 ? ~0u : 0u, m3 = digit && mine == 3 ? ~0u : 0u;
+        const int mine = i16 >> 2;
+        const char *row = reinterpret_cast<const char *>(S.row) + (i16 & 3) * 128 + mine * 32 + g4 * 8;
+        const int4 *chunk = S.chunk + g4;
+        const uint32_t m0 = mine == 0 ? ~0u : 0u, m1 = mine == 1 ? ~0u : 0u, m2 = mine == 2 ? ~0u : 0u, m3 = mine == 3 ? ~0u : 0u;
         const int sg = SG == 4 ? g4 : SG == 2 ? g4 >> 1 : 0;
         struct Operands {
             uint2 a;     // the lane's digits of the row
-            float2 c;
+            int4 c;
             UnitWeight w[NT];
         };
         auto row_here = [&](Operands &o, int kt) { o.a = *reinterpret_cast<const uint2 *>(row + kt * kRowPitch), o.c = chunk[kt * 4]; };
@@ -419,8 +424,9 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
             const ri32x4 b0 = {(int)(q.x & F), (int)((q.x >> 4) & F), (int)(q.y & F), (int)((q.y >> 4) & F)}, b1 = {(int)(q.z & F), (int)((q.z >> 4) & F), (int)(q.w & F), (int)((q.w >> 4) & F)};
             ri32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, ri32x4{0, 0, 0, 0}, 0, 0, 0);
             d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
-            const float f = fmaf((float)d[0], 65536.f, (float)(d[1] * 256 + d[2]));   // (each sum is below 2^16: the second is exact)
-            return fmaf(w.s * o.c.x, fmaf(-(float)(w.z & 127u), o.c.y, f), sum);
+            const int nz = 128 - (int)(w.z & 255u);
+            const float f = digits_join(d[0] * 256 + d[1] + __mul24(nz, o.c.y), d[2] * 256 + d[3] + __mul24(nz, o.c.z));
+            return fmaf(w.s * __int_as_float(o.c.x), f, sum);
         };
         if (ALL) {
             if (kt0 < share.kts) {
@@ -542,29 +548,29 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
         } while (any_empty(v) && --tries > 0);
         return v;
     };
-    // four values of the row (words 4 i4 .. of it, see res_place) as digits into LDS; eight neighbouring threads make a chunk. (Its
-    // sum is one of the values themselves: an infinity or a NaN among them, which has no digits, makes the products NaN.)
+    // four values of the row (words 4 i4 .. of it, see res_place) as digits into LDS; eight neighbouring threads make a chunk.
+    // (The sums of the digits from two more matrix instructions against ones per k tile, instead of here: 3710 against 3610 us
+    // for eight tokens of gemma3-1b at 2048.)
     auto put_digits = [&](int i4, float a, float b, float c, float d) {
-        uint32_t mx = __float_as_uint(fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d))));
+        uint32_t mx = __float_as_uint(__builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), __builtin_elementwise_maximum(fabsf(c), fabsf(d))));
         mx = max(mx, res_dpp<0xB1>(mx));
         mx = max(mx, res_dpp<0x4E>(mx));
         mx = max(mx, res_dpp<0x141>(mx));   // row_half_mirror: the other quad of the eight
-        const uint32_t ex = max(mx >> 23, 22u);
-        const float to = __uint_as_float((275u - ex) << 23);   // the largest comes to 2^21 .. 2^22
-        float s = fmaf(a, to, b * to) + fmaf(c, to, d * to);
-        s += lean_dpp<0xB1>(s);
-        s += lean_dpp<0x4E>(s);
-        s += lean_dpp<0x141>(s);
-        // the nearest whole number in the low bits, 0x80 added to each of its bytes and taken away without borrowing
-        auto digits = [&](float x) { return (__float_as_uint(fmaf(x, to, 12582912.f)) + (0x00808080u - 0x4b400000u)) ^ 0x00808080u; };
-        const uint32_t q0 = digits(a), q1 = digits(c), q2 = digits(b), q3 = digits(d);   // (in the order of the bytes)
+        const uint32_t ex = digits_exponent(mx);
+        const float to = digits_scale(ex);
+        const uint32_t q0 = digits_of(a * to), q1 = digits_of(c * to), q2 = digits_of(b * to), q3 = digits_of(d * to);   // (in the order of the bytes)
         const uint32_t lo01 = __builtin_amdgcn_perm(q1, q0, 0x05010400u), lo23 = __builtin_amdgcn_perm(q3, q2, 0x05010400u);
-        const uint32_t hi01 = __builtin_amdgcn_perm(q1, q0, 0x0c0c0602u), hi23 = __builtin_amdgcn_perm(q3, q2, 0x0c0c0602u);
-        uint32_t *dst = S.row + (i4 >> 5) * (kRowPitch / 4) + (i4 & 31);   // (= i4 + 64 (i4 >> 5))
-        dst[0] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-        dst[32] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-        dst[64] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-        if ((i4 & 7) == 0) S.chunk[i4 >> 3] = make_float2(__uint_as_float((ex - 21u) << 23), s);
+        const uint32_t hi01 = __builtin_amdgcn_perm(q1, q0, 0x07030602u), hi23 = __builtin_amdgcn_perm(q3, q2, 0x07030602u);
+        uint32_t *dst = S.row + (i4 >> 5) * (kRowPitch / 4) + (i4 & 31);
+        const uint32_t w0 = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u), w1 = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+        const uint32_t w2 = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u), w3 = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+        dst[0] = w0, dst[32] = w1, dst[64] = w2, dst[96] = w3;
+        auto sum4 = [](uint32_t w, int more) { return __builtin_amdgcn_sdot4((int)w, 0x01010101, more, false); };
+        uint32_t hi = (uint32_t)sum4(w1, sum4(w0, 0) * 256), lo = (uint32_t)sum4(w3, sum4(w2, 0) * 256);
+        hi += res_dpp<0xB1>(hi), lo += res_dpp<0xB1>(lo);
+        hi += res_dpp<0x4E>(hi), lo += res_dpp<0x4E>(lo);
+        hi += res_dpp<0x141>(hi), lo += res_dpp<0x141>(lo);
+        if ((i4 & 7) == 0) S.chunk[i4 >> 3] = make_int4(__float_as_int(digits_unit(ex)), (int)hi, (int)lo, 0);
     };
     // stream += rmsnorm(branch, w_post); the row rmsnorm(stream, w_in) goes to LDS. One reduction for both norms (see mmnb_lean_kernel).
     float4 x4 = zero4, y4 = zero4;   // this thread's four values of the stream, and of the branch to be added

@@ -1,12 +1,15 @@
 // Host-side checks of the index arithmetic that host and device code share (compiled for the host
-// only, run without a GPU): the split of a decode step's context into chunks, and which weight tiles
-// the read-ahead helper workgroups of a launch ask for.
+// only, run without a GPU): the split of a decode step's context into chunks, which weight tiles
+// the read-ahead helper workgroups of a launch ask for, and a row's values as digits.
+#include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <set>
 #include <vector>
 
 #include "internal.h"
+#include "row_digits.h"
 
 using namespace hipc;
 
@@ -77,8 +80,55 @@ static void read_ahead(int n_tiles, int n_cg, int WN, int slice_tiles, int gy, i
     if (H % 8 == 0 && H >= 8) CHECK(covered == total_tiles, "%zu of %zu tiles read ahead (H = %d)", covered, total_tiles, H);
 }
 
+// Chunks of any finite bit patterns: the digits are the value's nearest whole number of steps (half a step at most off, which is
+// 2^-30 of the largest), each fits a signed byte, and sums over them with a weight's codes come back as the exact sum, to one
+// rounding of f32 where they have more digits than it.
+static void digits() {
+    uint64_t state = 88172645463325252ull;
+    auto random = [&] { state ^= state << 13, state ^= state >> 7, state ^= state << 17; return (uint32_t)(state >> 16); };
+    auto value = [](uint32_t bits) { return __builtin_bit_cast(float, bits); };
+    for (int round = 0; round < 60000; round++) {
+        // exponents: anything; near one value; the smallest; the largest
+        const uint32_t top = round % 4 == 0 ? 254 : round % 4 == 1 ? 1 + random() % 254 : round % 4 == 2 ? random() % 40 : 127;
+        const uint32_t spread = 1 + random() % (round % 3 == 0 ? 60 : 8);
+        float x[32];
+        uint32_t largest = 0;
+        for (float &v : x) {
+            const uint32_t down = random() % spread, ex = down < top ? top - down : 0, sign = random() & 1, mantissa = random() % 8 ? random() & 0x7fffff : 0x7fffff;
+            const uint32_t bits = ex << 23 | mantissa;
+            largest = std::max(largest, bits);
+            v = value(bits | sign << 31);
+        }
+        const uint32_t ex = digits_exponent(largest);
+        const float to = digits_scale(ex), unit = digits_unit(ex);
+        CHECK(std::isfinite(to) && std::isnormal(unit), "scale %g unit %g of exponent %u", to, unit, ex);
+        CHECK((double)to * unit == 65536.0, "scale %g unit %g", to, unit);
+        const int z = (int)(random() & 15);
+        int64_t sum = 0;
+        int digit_sums[4] = {0, 0, 0, 0}, sums[4] = {0, 0, 0, 0};
+        for (float v : x) {
+            const uint32_t word = digits_of(v * to);
+            const int8_t d[4] = {(int8_t)(word >> 24), (int8_t)(word >> 16), (int8_t)(word >> 8), (int8_t)word};
+            const int64_t n = ((int64_t)d[0] << 24) + d[1] * 65536 + d[2] * 256 + d[3];
+            CHECK(std::fabs((double)v * to - (double)n) <= 0.5, "%a: %lld for %a", (double)v, (long long)n, (double)v * to);
+            CHECK(d[0] >= -64 && d[0] <= 64, "highest digit %d", d[0]);
+            CHECK(0.5 * unit / 65536.0 <= std::ldexp((double)std::max(value(largest), 0x1p-98f), -30), "half a step of %a beside %a", (double)unit, (double)value(largest));
+            const int q = round % 5 == 0 ? z : (int)(random() & 15);
+            sum += (q - z) * n;
+            for (int i = 0; i < 4; i++) sums[i] += q * d[i], digit_sums[i] += d[i];
+        }
+        const int hi = sums[0] * 256 + sums[1] - z * (digit_sums[0] * 256 + digit_sums[1]), lo = sums[2] * 256 + sums[3] - z * (digit_sums[2] * 256 + digit_sums[3]);
+        CHECK(std::abs(hi) < 1 << 24 && std::abs(lo) < 1 << 24 && (int64_t)hi * 65536 + lo == sum, "sums %d %d of %lld", hi, lo, (long long)sum);
+        CHECK(digits_join(hi, lo) == (float)((double)sum / 65536.0), "joined %a of %lld", (double)digits_join(hi, lo), (long long)sum);
+        CHECK(round % 5 != 0 || digits_join(hi, lo) == 0.f, "weights of zero");
+    }
+    for (uint32_t bits : {0x7f800000u, 0x7f800001u, 0x7fffffffu}) CHECK(std::isnan(digits_unit(digits_exponent(bits))), "unit of %x", bits);
+    CHECK(digits_of(0.f) == 0 && std::isfinite(digits_unit(digits_exponent(0))), "a chunk of zeros");
+}
+
 int main() {
     attention_chunks();
+    digits();
     // the decoder's launches at the 1152 / 6912 shape: consumer o (read ahead by the attention launch,
     // 64 x (1 + 3) workgroups), gate | up (by o: 18 x (4 + 8)), down (by gate | up: 432 x (1 + 1)), qkv (by down: 72 x (3 + 3))
     read_ahead(72, 8, 4, 2, 4, 64, 1, 3);

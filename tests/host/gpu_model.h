@@ -187,6 +187,7 @@ inline T __shfl(T v, int, int = 64) { return v; }
 inline float __uint_as_float(uint32_t u) { float f; std::memcpy(&f, &u, 4); return f; }
 inline uint32_t __float_as_uint(float f) { uint32_t u; std::memcpy(&u, &f, 4); return u; }
 inline float __expf(float v) { return std::exp(v); }
+inline int __mul24(int a, int b) { return a * b; }
 inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xffffffu) * (b & 0xffffffu); }
 inline int __any(int v) { return v; }
 inline int __all(int) { return 1; }   // (what a wavefront would wait for counts as there: threads run one after the other)
