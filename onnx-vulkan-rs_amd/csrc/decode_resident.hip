@@ -426,7 +426,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
             d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
             const int nz = 128 - (int)(w.z & 255u);
             const float f = digits_join(d[0] * 256 + d[1] + __mul24(nz, o.c.y), d[2] * 256 + d[3] + __mul24(nz, o.c.z));
-            return fmaf(w.s * __int_as_float(o.c.x), f, sum);
+            return fmaf(w.s * __builtin_bit_cast(float, o.c.x), f, sum);
         };
         if (ALL) {
             if (kt0 < share.kts) {
@@ -570,7 +570,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
         hi += res_dpp<0xB1>(hi), lo += res_dpp<0xB1>(lo);
         hi += res_dpp<0x4E>(hi), lo += res_dpp<0x4E>(lo);
         hi += res_dpp<0x141>(hi), lo += res_dpp<0x141>(lo);
-        if ((i4 & 7) == 0) S.chunk[i4 >> 3] = make_int4(__float_as_int(digits_unit(ex)), (int)hi, (int)lo, 0);
+        if ((i4 & 7) == 0) S.chunk[i4 >> 3] = make_int4(__builtin_bit_cast(int, digits_unit(ex)), (int)hi, (int)lo, 0);
     };
     // stream += rmsnorm(branch, w_post); the row rmsnorm(stream, w_in) goes to LDS. One reduction for both norms (see mmnb_lean_kernel).
     float4 x4 = zero4, y4 = zero4;   // this thread's four values of the stream, and of the branch to be added
