@@ -863,14 +863,24 @@ struct hipc_decoder {
     std::vector<ResidentLayer> entries;         // what the table holds
     uint32_t *xch = nullptr, *sync = nullptr;
     bool one_launch_attn = false;  // head_dim and group size have an instance of dec_attn_chunks_kernel
-    uint8_t *host = nullptr;       // pinned: what hipc_decoder_read brings, the state (in kHostState bytes), the logits, the history
+    uint8_t *host = nullptr;       // pinned, from the first read on: the state (in kHostState bytes) and the history
+    uint8_t *host_logits = nullptr;   // ... and, from the first that wants them on, the logits
     std::vector<void *> owned;
 };
 
 namespace {
 
 constexpr size_t kHostState = 64;
-static_assert(sizeof(DecState) <= kHostState, "the state in front of the logits");
+static_assert(sizeof(DecState) <= kHostState, "the state in front of the history");
+
+// `*p` is `bytes` of pinned host memory, allocated here if it was not yet
+bool host_words(uint8_t **p, size_t bytes) {
+    if (*p) return true;
+    if (hipHostMalloc(reinterpret_cast<void **>(p), bytes, hipHostMallocDefault) == hipSuccess) return true;
+    (void)hipGetLastError();   // not the next launch's
+    *p = nullptr;
+    return false;
+}
 
 template <typename T>
 int dev_alloc(hipc_ctx *ctx, hipc_decoder *d, T **p, size_t count) {
@@ -1046,8 +1056,6 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
             if (rc == HIPC_OK) rc = table_alloc(ctx, d, &d->table);
             if (rc == HIPC_OK) rc = resident_clear(ctx, d->xch, d->sync);
         }
-        if (rc == HIPC_OK && hipHostMalloc(reinterpret_cast<void **>(&d->host), kHostState + ((size_t)c.vocab + c.max_seq) * 4, hipHostMallocDefault) != hipSuccess)
-            rc = fail(ctx, HIPC_ERR_BACKEND, "decoder: no pinned host memory for what is read back");
         if (rc == HIPC_OK) {
             for (DecLayer &l : d->layers) {  // an unwritten cache row must not hold NaN bit patterns
                 if (hipMemsetAsync(l.k_cache, 0, k_halfs * 2, ctx->stream) != hipSuccess ||
@@ -1059,7 +1067,6 @@ int hipc_decoder_create(hipc_ctx *ctx, const hipc_decoder_config *cfg, hipc_deco
         if (rc != HIPC_OK) {
             for (void *p : d->owned) (void)hipFree(p);
             if (d->table) (void)hipFree(d->table);
-            if (d->host) (void)hipHostFree(d->host);
             delete d;
             return rc;
         }
@@ -1077,7 +1084,8 @@ void hipc_decoder_destroy(hipc_ctx *ctx, hipc_decoder *d) {
         nbits_release(ctx, d->lm_head);
         for (void *p : d->owned) ctx->deferred.push_back(p);
         if (d->table) ctx->deferred.push_back(d->table);
-        ctx->deferred_host.push_back(d->host);
+        if (d->host) ctx->deferred_host.push_back(d->host);
+        if (d->host_logits) ctx->deferred_host.push_back(d->host_logits);
         delete d;
     });
 }
@@ -1428,21 +1436,29 @@ int hipc_decoder_read(hipc_ctx *ctx, hipc_decoder *d, int32_t *token, int32_t *p
     if (!d) return HIPC_ERR_INVALID;
     return entry(ctx, [&]() -> int {
         HIPC_REFUSE(ctx, ctx->capturing, "decoder read while a capture is open");
-        // Everything through the decoder's pinned words, behind the steps on their stream, with one wait: a copy of the logits of
-        // 262144 columns straight to pageable memory takes 88 us, and each of three copies with a wait of its own 13.
+        // Everything through pinned words of the decoder's, behind the steps on their stream, with one wait: a copy of the logits of
+        // 262144 columns straight to pageable memory takes 88 us, and each of three copies with a wait of its own 13. A read
+        // that finds no pinned memory takes those.
         const size_t n_logits = logits ? (size_t)d->cfg.vocab * 4 : 0;
         const size_t n_hist = history && n_history > 0 ? (size_t)std::min<int32_t>(n_history, d->cfg.max_seq) * 4 : 0;
-        uint8_t *host = d->host, *host_logits = host + kHostState, *host_hist = host_logits + (size_t)d->cfg.vocab * 4;
-        HIPC_TRY(ctx, hipMemcpyAsync(host, d->state, sizeof(DecState), hipMemcpyDeviceToHost, ctx->stream));
-        if (n_hist) HIPC_TRY(ctx, hipMemcpyAsync(host_hist, d->history, n_hist, hipMemcpyDeviceToHost, ctx->stream));
-        if (n_logits) HIPC_TRY(ctx, hipMemcpyAsync(host_logits, d->logits, n_logits, hipMemcpyDeviceToHost, ctx->stream));
-        HIPC_TRY(ctx, hipStreamSynchronize(ctx->stream));
-        DecState st;
-        std::memcpy(&st, host, sizeof st);
+        const bool pinned = host_words(&d->host, kHostState + (size_t)d->cfg.max_seq * 4) && (!n_logits || host_words(&d->host_logits, n_logits));
+        DecState st{};
+        if (pinned) {
+            HIPC_TRY(ctx, hipMemcpyAsync(d->host, d->state, sizeof st, hipMemcpyDeviceToHost, ctx->stream));
+            if (n_hist) HIPC_TRY(ctx, hipMemcpyAsync(d->host + kHostState, d->history, n_hist, hipMemcpyDeviceToHost, ctx->stream));
+            if (n_logits) HIPC_TRY(ctx, hipMemcpyAsync(d->host_logits, d->logits, n_logits, hipMemcpyDeviceToHost, ctx->stream));
+            HIPC_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            std::memcpy(&st, d->host, sizeof st);
+            if (n_hist) std::memcpy(history, d->host + kHostState, n_hist);
+            if (n_logits) std::memcpy(logits, d->host_logits, n_logits);
+        } else {
+            HIPC_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            HIPC_TRY(ctx, hipMemcpy(&st, d->state, sizeof st, hipMemcpyDeviceToHost));
+            if (n_hist) HIPC_TRY(ctx, hipMemcpy(history, d->history, n_hist, hipMemcpyDeviceToHost));
+            if (n_logits) HIPC_TRY(ctx, hipMemcpy(logits, d->logits, n_logits, hipMemcpyDeviceToHost));
+        }
         if (token) *token = st.token;
         if (pos) *pos = st.pos;
-        if (n_logits) std::memcpy(logits, host_logits, n_logits);
-        if (n_hist) std::memcpy(history, host_hist, n_hist);
         if (st.broken) return fail(ctx, HIPC_ERR_BACKEND, "decoder: a step did not come to its end (a wait inside it ran out); reset the decoder");
         HIPC_REQUIRE(ctx, !st.overflow, "decoder: a step was enqueued with the cache full (%d positions); it did nothing", d->cfg.max_seq);
         return HIPC_OK;

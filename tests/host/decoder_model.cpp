@@ -207,6 +207,41 @@ void step_words() {
     report("the words of a step");
 }
 
+// A read brings state, history and logits with pinned host memory and without; the decoder takes none before it, and for logits
+// only where they are wanted.
+void reads() {
+    const Shape s = kSmall[0];
+    Model m;
+    gpu_model::reg().where = "reads";
+    gpu_model::reg().no_pinned = true;
+    m.ctx.tune.dec_resident = 0;   // (in the one launch threads wait for each other, which here run in turn)
+    m.build(s);
+    hipc_ctx &ctx = m.ctx;
+    ctx.tune.dec_prefetch = -1;
+    const size_t blocks = gpu_model::reg().blocks.size();
+    const auto expect = [&](bool ok, const char *what) {
+        if (!ok) std::printf("FAILED: a read: %s\n", what), std::exit(1);
+    };
+    std::vector<float> logits[2];
+    std::vector<int32_t> history[2];
+    MUST(hipc_decoder_reset(&ctx, m.dec, 1, 5));
+    MUST(hipc_decoder_step(&ctx, m.dec));
+    for (int pinned = 0; pinned < 2; pinned++) {
+        gpu_model::reg().no_pinned = !pinned;
+        int32_t token = -1, pos = -1;
+        logits[pinned].assign(s.vocab, -1.f), history[pinned].assign(s.max_seq + 3, -7);
+        MUST(hipc_decoder_read(&ctx, m.dec, &token, &pos, nullptr, nullptr, 0));
+        expect(pos == 6 && token >= 0 && token < s.vocab, "token and position");
+        expect(gpu_model::reg().blocks.size() == blocks + pinned, "memory for logits nobody wanted");
+        MUST(hipc_decoder_read(&ctx, m.dec, &token, &pos, logits[pinned].data(), history[pinned].data(), s.max_seq + 3));
+        expect(gpu_model::reg().blocks.size() == blocks + 2 * pinned, "memory for logits");
+        expect(history[pinned][s.max_seq] == -7, "a history longer than there is");
+    }
+    expect(std::memcmp(logits[0].data(), logits[1].data(), s.vocab * 4) == 0 && history[0] == history[1], "not the same without pinned memory");
+    m.destroy();
+    report("reads");
+}
+
 // Replacing what a layer is made of while graphs live: a new layer table only where a recorded step reads the old one, and
 // that one goes when the graphs do.
 void table_changes() {
@@ -390,7 +425,7 @@ int main(int argc, char **argv) {
         if (!g_select.on) return true;
         return g_select.rows(g_select.index++, y0, y1);
     };
-    if (mode != "sweep") step_words(), table_changes(), which_form();
+    if (mode != "sweep") step_words(), reads(), table_changes(), which_form();
     if (mode == "full") {
         for (const Shape &s : kSmall) full(s);
         full(kGemma);

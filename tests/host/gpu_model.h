@@ -35,6 +35,7 @@ struct Registry {
     size_t loads = 0, loads_clipped = 0, launches = 0, threads = 0;
     bool failed = false;
     bool no_memory = false;   // hipMalloc fails
+    bool no_pinned = false;   // hipHostMalloc does
     std::string where;   // what is being launched (printed with a failure)
 };
 // one registry per host thread: a thread of the driver builds its own model (its own allocations)
@@ -215,7 +216,7 @@ using std::min;
 // ---- the host API the sources call: allocations are registered host blocks, the stream is immediate ----
 #define hipMalloc gpu_model_hipMalloc
 #define hipFree gpu_model_hipFree
-#define hipHostMalloc(p, bytes, flags) gpu_model_hipMalloc(p, bytes)
+#define hipHostMalloc(p, bytes, flags) (gpu_model::reg().no_pinned ? hipErrorOutOfMemory : gpu_model_hipMalloc(p, bytes))
 #define hipHostFree gpu_model_hipFree
 #define hipMemsetAsync gpu_model_hipMemsetAsync
 #define hipMemcpyAsync gpu_model_hipMemcpyAsync
