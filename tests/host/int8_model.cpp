@@ -121,6 +121,32 @@ void products(int64_t M, int64_t K, int64_t N, int a_dtype, int b_dtype, bool zp
     release_all();
 }
 
+// Which products of 64x64 tiles take two groups of wavefronts a workgroup, on four CUs: tiles of 64 rows, k, the groups of an int32
+// result without and with sums over A's rows.
+void which_groups() {
+    ctx.cu_count = 4;
+    const struct { int64_t tiles, K; size_t plain, sums; } cases[] = {{3, 3584, 2, 2}, {4, 3584, 1, 2}, {4, 6144, 1, 2}, {3, 3568, 1, 1}, {5, 3584, 1, 1}};
+    for (const auto &c : cases)
+        for (const bool sums : {false, true}) {
+            const int64_t M = c.tiles * 64, N = 64;
+            void *A = input((size_t)M * c.K, 3), *B = input((size_t)c.K * N, 5), *azp = input(1, 7), *bzp = input(1, 2), *Y = input((size_t)M * N * 4);
+            hipc_int8_weight *w = nullptr;
+            MUST(hipc_prepack_int8_b(&ctx, B, HIPC_I8, c.K, N, &w));
+            ctx.tune.gemm_skinny = ctx.tune.gemm_big = 0;
+            const size_t before = gpu_model::reg().threads;
+            MUST(hipc_matmul_integer(&ctx, A, HIPC_U8, w, azp, sums ? bzp : nullptr, Y, M));
+            const size_t groups = (gpu_model::reg().threads - before) / 256 / (size_t)((c.tiles + 7) / 8 * 8);
+            if (groups != (sums ? c.sums : c.plain)) {
+                std::printf("FAILED: %lld tiles, k = %lld, %s: %zu groups\n", (long long)c.tiles, (long long)c.K, sums ? "with sums" : "without", groups);
+                std::exit(1);
+            }
+            ctx.tune.gemm_skinny = ctx.tune.gemm_big = -1;
+            hipc_int8_weight_destroy(&ctx, w);
+            release_all();
+        }
+    ctx.cu_count = 256;
+}
+
 void conv(int64_t n, int64_t c_in, int64_t h, int64_t w, int64_t c_out, int64_t kh, int64_t kw, int64_t sh, int64_t sw, int64_t dh, int64_t dw,
           int64_t pt, int64_t pl, int64_t pb, int64_t pr, int64_t group, int x_dtype, const char *what) {
     hipc_conv_geom g{n, c_in, h, w, c_out, kh, kw, sh, sw, dh, dw, pt, pl, pb, pr, group};
@@ -179,6 +205,7 @@ int main(int argc, char **argv) {
         products(s[0], s[1], s[2], HIPC_I8, HIPC_U8, false);
     }
     report("matrix products, seven routes x four epilogue calls");
+    which_groups();
     if (!quick) {
         products(1000, 1024, 4096, HIPC_U8, HIPC_I8, true);   // the benchmark's pair
         products(1000, 4096, 1024, HIPC_U8, HIPC_I8, true);
