@@ -554,9 +554,9 @@ int gemm_launch(hipc_ctx *ctx, const GemmArgs &g, unsigned batch) {
 // at the end costs more than the loop saves. (The same kernel with 128x128 tiles, wavefronts 2x2
 // and no k split was slower than either: 16 products per stage issued back to back keep the
 // wavefront from issuing the stage's memory instructions, as in the 128x128 LDS-staged kernel.)
-// With no more tiles than CUs and a long k a workgroup is two groups of four wavefronts (GROUPS), with LDS buffers of their
+// With few tiles and a long k (see small_groups) a workgroup is two groups of four wavefronts (GROUPS), with LDS buffers of their
 // own, that take the stages in turn: the second wavefront of a SIMD fills the chain barrier - LDS - products - LDS of the
-// first, 0.19 us a stage becomes 0.15, towards the 0.12 that 16 KB take at the CU's 64 bytes a clock. For that the hand-over
+// first, 0.19 us a stage becomes 0.16 (0.17 with the weight from memory), towards the 0.12 that 16 KB take at the CU's 64 bytes a clock. For that the hand-over
 // is 112 KB instead of 48. The epilogue is dealt to eight wavefronts.
 constexpr int kSmallSets = 4;  // register sets of A chunks and of B fragments: stages in flight
 // the hand-over, of which an owner gets (4 GROUPS - 1) parts of 16 / GROUPS words a lane, reuses the A buffers (18 KB a group of its 48 or 112 KB)

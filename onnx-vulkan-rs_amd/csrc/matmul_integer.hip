@@ -258,23 +258,31 @@ bool wants_small_tiles(hipc_ctx *ctx, const GemmArgs &g) {
     const int64_t tiles64 = ceil_div(g.I, 64) * ceil_div(g.J, 64);
     return (tiles64 <= 2 * (int64_t)ctx->cu_count && g.K >= 4 * kBK) || (tiles64 <= 4 * (int64_t)ctx->cu_count && g.K >= 8 * kBK);
 }
-// How many groups of four wavefronts a workgroup is (k in whole stages; back to back in a graph, both in turn, us with one / two):
-//                       float rescaled   int32, sums over A's rows   to bytes       int32
-//   1000 x 4096 x 1024   11.2 / 10.7        11.3 / 10.8           10.6 / 10.35   10.3 / 10.3    256 tiles
-//   1000 x 3584 x 1024   10.4 / 10.1        10.5 / 10.2            9.8 / 9.75     9.5 / 9.65
-//   1000 x 6144 x 1024   15.7 / 15.4        15.7 / 14.9           14.5 / 14.2    14.2 / 14.45
-//    800 x 3584 x 1024   10.4 / 10.0        10.5 / 10.15           9.75 / 9.65    9.45 / 9.45   208
-//    640 x 4096 x 1024   11.1 / 10.5        11.3 / 10.7           10.5 / 10.1    10.2 / 10.0    160
-//    100 x 6912 x 1152   15.8 / 13.8        16.3 / 14.2           15.4 / 13.6    15.0 / 13.3     36
-//     70 x 11008 x 1024  21.9 / 19.0        23.0 / 19.5           21.6 / 18.8    21.4 / 18.4     32
-// So from 28 stages on where no CU gets a second tile; int32 results without sums, whose epilogue has nothing to fill the larger
-// hand-over with, up to three tiles for four CUs. With fewer stages the hand-over costs what they save: 1000 x 3072 x 1024 9.4 / 9.2,
-// to bytes 8.7 / 8.9; 200 x 3000 x 512 12.0 / 12.0, to bytes 11.2 / 11.7; 1000 x 1024 x 1024 6.4 / 6.6. Beyond a tile per CU, where three
-// workgroups of one group share a CU but not two of two groups: 1000 x 4096 x 1200 14.8 / 19.6.
-int small_groups(hipc_ctx *ctx, const GemmArgs &g, bool light) {
-    if (ctx->tune.gemm_small == 2) return 2;
-    const int64_t tiles = ceil_div(g.I, 64) * ceil_div(g.J, 64);
-    return ctx->tune.gemm_small != 1 && (light ? tiles * 4 <= ctx->cu_count * 3 : tiles <= ctx->cu_count) && g.K >= 28 * kBK ? 2 : 1;
+// How many groups of four wavefronts a workgroup is. Two groups save 0.02 to 0.03 us a stage and their larger hand-over costs about a
+// microsecond of what the epilogue overlaps. us with one / two, both in turn, random bytes, eight weights in turn so that none
+// is in an L2 (k in whole stages):
+//                      tiles   float rescaled   int32, sums over A's rows   to bytes         int32
+//    96 x  4096 x  512    16    10.8 / 10.2       11.1 / 10.4            10.4 /  9.9       9.96 /  9.67
+//   500 x  4096 x 1024   128    11.6 / 11.5       11.8 / 11.3            11.0 / 10.9      10.6  / 10.8
+//   768 x  3584 x 1024   192    10.9 / 10.9       11.0 / 10.75           10.25 / 10.25     9.86 / 10.2
+//   768 x  4096 x 1024   192    11.7 / 11.6       11.85 / 11.4           11.1 / 10.95     10.7  / 10.9
+//   768 x  5120 x 1024   192    13.25 / 13.0      13.55 / 12.85          12.7 / 12.4      12.3  / 12.4
+//   768 x  6144 x 1024   192    15.4 / 14.85      15.8 / 14.8            14.4 / 13.8      14.05 / 14.0
+//   900 x  4096 x 1024   240    11.9 / 12.0       12.0 / 11.9            11.25 / 11.4     10.9  / 11.4
+//  1000 x  4096 x 1024   256    12.25 / 12.35     12.3 / 12.3            11.6 / 11.95     11.25 / 11.8
+//  1000 x  6144 x 1024   256    16.9 / 16.5       17.0 / 16.65           15.6 / 15.6      15.45 / 15.7
+//   100 x  6912 x 1152    36    16.1 / 15.1       16.7 / 14.95           15.7 / 14.7      15.45 / 14.4
+//    70 x 11008 x 1024    32    22.2 / 20.6       23.45 / 20.4           22.1 / 20.1      21.6  / 19.8
+// With one weight in the L2s two groups gain more: 1000 x 4096 x 1024 11.2 / 10.7, 11.3 / 10.8, 10.6 / 10.35, 10.3 / 10.3. So from 32 stages
+// on, up to a tile per CU where the epilogue is a long one, which fills the hand-over's waits (floats, sums over A's rows: the second
+// product of a feed-forward block of 1000 rows between its quantizers takes 0.2 us less), three tiles for four CUs where it is not;
+// int32 results without sums, the shortest, from 48 stages on. Beyond a tile per CU, where three workgroups of one group share a
+// CU but not two of two groups: 1000 x 4096 x 1200 14.8 / 19.6.
+int small_groups(hipc_ctx *ctx, const GemmArgs &g, bool floats, bool sums, bool bytes) {
+    if (ctx->tune.gemm_small >= 1) return ctx->tune.gemm_small == 2 ? 2 : 1;
+    const int64_t tiles = ceil_div(g.I, 64) * ceil_div(g.J, 64), cus = ctx->cu_count;
+    const bool room = floats || sums ? tiles <= cus : tiles * 4 <= cus * 3;
+    return room && g.K >= (floats || sums || bytes ? 32 : 48) * kBK ? 2 : 1;
 }
 template <int EPI, bool DYN, int GROUPS>
 int launch_mm_small_dyn(hipc_ctx *ctx, GemmArgs g) {
@@ -292,7 +300,7 @@ int launch_mm_small_dyn(hipc_ctx *ctx, GemmArgs g) {
 template <int EPI>
 int launch_mm_small(hipc_ctx *ctx, const GemmArgs &g) {
     const bool zero_known = g.const_shift == 0 && (g.host_zp ? g.const_zp_value == 0 : g.const_zp == nullptr);
-    if (small_groups(ctx, g, EPI == EPI_I32 && zero_known) == 2) return zero_known ? launch_mm_small_dyn<EPI, false, 2>(ctx, g) : launch_mm_small_dyn<EPI, true, 2>(ctx, g);
+    if (small_groups(ctx, g, EPI == EPI_SCALE_BIAS, !zero_known, EPI == EPI_REQUANT) == 2) return zero_known ? launch_mm_small_dyn<EPI, false, 2>(ctx, g) : launch_mm_small_dyn<EPI, true, 2>(ctx, g);
     return zero_known ? launch_mm_small_dyn<EPI, false, 1>(ctx, g) : launch_mm_small_dyn<EPI, true, 1>(ctx, g);
 }
 template <int EPI, bool DYN, int RB>

@@ -125,7 +125,7 @@ void products(int64_t M, int64_t K, int64_t N, int a_dtype, int b_dtype, bool zp
 // result without and with sums over A's rows.
 void which_groups() {
     ctx.cu_count = 4;
-    const struct { int64_t tiles, K; size_t plain, sums; } cases[] = {{3, 3584, 2, 2}, {4, 3584, 1, 2}, {4, 6144, 1, 2}, {3, 3568, 1, 1}, {5, 3584, 1, 1}};
+    const struct { int64_t tiles, K; size_t plain, sums; } cases[] = {{3, 6144, 2, 2}, {3, 6128, 1, 2}, {3, 4096, 1, 2}, {3, 4080, 1, 1}, {4, 6144, 1, 2}, {5, 6144, 1, 1}};
     for (const auto &c : cases)
         for (const bool sums : {false, true}) {
             const int64_t M = c.tiles * 64, N = 64;
