@@ -455,7 +455,7 @@ def resident_phases(lib, ctx, dec, context):
     since = st - begin[:, None, None]
     out = {}
     for ph, label in RESIDENT_PHASES.items():
-        v = np.where((since[:, :, ph] >= 0) & (since[:, :, ph] < 1 << 20), since[:, :, ph], -1).max(axis=1)   # (a place no wavefront passed holds an older stamp)
+        v = np.where((since[:, :, ph] >= 0) & (since[:, :, ph] < 1 << 17), since[:, :, ph], -1).max(axis=1)   # (a place no wavefront passed holds an older stamp)
         v = v[v >= 0]
         if v.size:
             out[label] = dict(workgroups=int(v.size), median=int(np.median(v)), p90=int(np.percentile(v, 90)), max=int(v.max()))
