@@ -415,8 +415,8 @@ const char *hipc_host_error(void);
  * so a captured graph of one step replays without patching.
  * A step on a device of its own is one launch that takes every CU. Contexts that decode at the same time on one
  * device get more tokens per second from a launch per product (HIPC_DEC_RESIDENT=0, read when a decoder is created
- * and at each step): a token of each of two takes 878 us so and 780 us by products, of each of three 1900 and 918
- * (gemma3-1b at 2048; alone 451 and 653, of which the first is 435 since).
+ * and at each step): a token of each of two takes 860 us in one launch and 790 us by products, of each of three 1660 to
+ * 2510 and 928 (gemma3-1b at 2048; alone 445 and 655).
  * Limits kept on the device: the cache holds `max_seq` positions, so at most `max_seq` steps can
  * follow a reset to position 0. A step enqueued (or replayed) with the cache full writes nothing,
  * leaves token and position as they are and raises a sticky flag that `hipc_decoder_read` reports

@@ -79,12 +79,15 @@ constexpr int kPollBudget = 1;                         // (one thread after the 
 // How long workgroups that have not started are waited for, in ticks of the 100 MHz clock. All of them, 50 us: they arrive within
 // microseconds on a free device, and within the 50 us another decoder's unembedding and token pick keep some CUs. In the
 // stand-in until nobody has come for 5 us.
-// Beside other work, us a token of gemma3-1b at 2048 (454 alone then, 435 since; launches per product 654 alone), the launches per product / 50 us and
-// 256 workgroups standing in / 200 us and 256 / 200 us and 64: beside a softmax of eight workgroups of a millisecond 763 / 773 / 923 / 1602;
-// launches that hold 64 CUs for 220 us 730 / 908 / 835 / 1191, 128 CUs for 140 us 788 / 777 / 570 / 569; products that fill the chip for 125 us
-// at a time - / 860 / 860 / 872. Two decoders side by side, a token of each: 780 / 878 / 877 / 877; three 918 / 1900 / 2490 / 2060,
-// four 1061 / 2190 / 2880 / 2180: launches that each want the whole chip take turns at best, where short ones fill each other's
-// gaps (these figures scatter by a fifth), so contexts that decode at the same time are better off with HIPC_DEC_RESIDENT=0.
+// Beside other work, us a token of gemma3-1b at 2048, the launches per product / one launch (655 / 445 alone), on another stream without a
+// pause: softmaxes of eight workgroups and a millisecond 766 / 511; of 64 workgroups and 220 us 783 / 612; of 128 and 140 us 844 / 585 (the
+// softmaxes get on as well beside one launch as beside the other within a fifth); products of 4096^3 of 105 us, which let few small
+// launches in between, 3400 / 764. Two decoders side by side, a token of each: 790 / 860; three 928 / 1660 to 2510, four 1585 /
+// 2080 to 2720: launches that each want the whole chip take turns at best, where short ones fill each other's gaps, so contexts
+// that decode at the same time are better off with HIPC_DEC_RESIDENT=0.
+// The two waits are from the kernel before the present one, whose workgroups had eight wavefronts and 94 KB of LDS, so more could share a CU
+// with them (launches per product / 50 us and 256 workgroups standing in / 200 us and 256 / 200 us and 64): beside the eight workgroups
+// 763 / 773 / 923 / 1602, the 64 730 / 908 / 835 / 1191, the 128 788 / 777 / 570 / 569; three decoders 918 / 1900 / 2490 / 2060.
 constexpr int kArriveTicks = 5000, kJoinTicks = 500;
 constexpr int kResThreads = 512, kResWaves = 8;        // those that compute
 constexpr int kFeedWaves = 4;                          // and, in the launch of all, those that bring the weights: one per product
@@ -123,9 +126,9 @@ inline void res_stored() {}
 // behind 4 KB of them, 1.5 us behind 36 KB). So they are asked for behind the barrier that follows a poll, with work in front
 // of the next one: gate|up's where a layer begins (kFeedFirst units), behind the heads' barrier (up to kFeedHeads) and where
 // the chunks have arrived; o's where a layer begins, down's where the hidden row has arrived, the next layer's q|k|v where
-// the gated row has. Us for eight tokens of gemma3-1b at 2048: all of a product's at once as soon as its places are free 3955; so spread
-// 3560; in the registers of the polling wavefronts, two phases ahead, 3725. (Eight layers of 2048 / 8192 with 8/1 heads of 256 at 2040,
-// where those registers held half of the units: 201 -> 185; of 512 / 2048 with 8/2 heads of 64: 123 -> 119.)
+// the gated row has. Us for eight tokens of gemma3-1b at 2048 (a row as three bytes a value then): all of a product's at once as soon as its
+// places are free 3955; so spread 3560; in the registers of the polling wavefronts, two phases ahead, 3725. (Eight layers of 2048 / 8192 with
+// 8/1 heads of 256 at 2040, where those registers held half of the units: 201 -> 185; of 512 / 2048 with 8/2 heads of 64: 123 -> 119.)
 //
 // The row takes part as whole numbers of four signed bytes (row_digits.h has what that keeps of a value), so a product of a
 // unit is two int8 matrix instructions with exact sums, and a weight's nibbles need no conversion beyond being spread to bytes.
@@ -266,6 +269,13 @@ struct ResSpan {
 // Which units these are does not change: their offsets stay in registers, and each of the four wavefronts has code of its own for
 // the fixed places where it asks, so that four units take twelve instructions and the next barrier, which may be 0.3 us away, does
 // not wait for this wavefront (one code for all, which skipped what it did not ask for: 3860 us instead of 3560).
+// kFeedFirst: as many of gate|up's places are no place of q|k|v's, whose units lie behind them (up to 32, see resident_launch), so
+// these can be asked for while q|k|v's product is still to come. kFeedHeads: what the short work in front of the cache passes covers.
+// A larger q|k|v share or window moves neither: the places stay free, longer passes leave the later ones more time. Us a token with
+// 16/24, 16/16, 16/32, 8/16, 24/24, 24/32: gemma3-1b at 2048 (a vocabulary of 4096) 412 411 421 415 414 415; at 8000, 22 layers with windows
+// of 512, 398 392 405 400 395 401; eight layers at 2040 of 2048 / 8192 with 8/1 heads of 256 180 180 181 182 178 178, with 8/8 (two
+// tiles of q|k|v a workgroup) 193 195 194 196 192 192; of 1024 / 4096 with 4/4 of 128 121 123 121 121 124 121; of 1152 / 6912 at 16000 220 222
+// 225 222 222 223.
 constexpr int kFeedFirst = 16, kFeedHeads = 24;
 template <int HD, int SG, int ph>
 __device__ __forceinline__ void res_feed(const ResidentArgs &p, ResShared<HD, SG, true> &S, const int v, const int total) {
@@ -988,7 +998,7 @@ __device__ __forceinline__ void res_layers(const ResidentArgs &p, ResShared<HD, 
 
 // ALL: begins when all 256 workgroups have arrived, or not at all. Else: does the work of a launch of the other form that
 // did not begin (`behind` is set), or that was never made, with the workgroups that have arrived by the deadline.
-// (Two kernels: in one the second form costs the first 25 us a token, in registers. A launch that finds its work done is 2 us.)
+// (Two kernels: in one the second form costs the first 25 us a token, in registers. A launch that finds its work done is 4.6 us by kernel trace, the launch itself included.)
 template <int HD, int SG, bool ALL>
 __global__ void __launch_bounds__(kResThreads + (ALL ? 64 * kFeedWaves : 0)) RES_ONE_PER_CU(ALL) dec_resident_kernel(const ResidentArgs p) {
     __shared__ __attribute__((aligned(16))) ResShared<HD, SG, ALL> S;
@@ -1100,16 +1110,16 @@ bool hipc::resident_takes(const hipc_decoder_config &c) {
 // parts of them), where the attention launch spreads them over as many workgroups as it likes, and heads that share a kv head
 // there share its reading. So heads and positions decide, whatever the other sizes are. Per product / one launch, us a token of 8 layers (query
 // / kv heads of channels, hidden / ffn, at position):
-//   8/1 of 256, 2048 / 8192     272 / 259 at 8192, 292 / 308 at 12288, 314 / 350 at 16384
-//   8/2 of 64, 512 / 2048       162 / 156 at 8192, 169 / 179 at 12288, 178 / 201 at 16384
-//   8/4 of 256, 1152 / 6912     284 / 269 at 12288, 311 / 318 at 16384
-//   8/8 of 128, 1024 / 4096     204 / 184 at 8192, 240 / 222 at 12288, 258 / 258 at 16384
-//   4/1 of 256, 1152 / 6912     246 / 212 at 16384, 330 / 308 at 32768;  4/4 of 128, 512 / 2048  276 / 251 at 32768
-//   2/1 of 128, 512 / 2048      353 / 224 at 65536;  1/1 of 256, 1152 / 6912  804 / 339 at 131072
-// and at position 100 one launch takes about three quarters. The position is the device's and a recorded step covers all of
+//   8/1 of 256, 2048 / 8192     273 / 243 at 8192, 299 / 293 at 12288, 316 / 335 at 16384
+//   8/2 of 64, 512 / 2048       162 / 151 at 8192, 171 / 174 at 12288, 179 / 194 at 16384
+//   8/4 of 256, 1152 / 6912     285 / 268 at 12288, 312 / 318 at 16384
+//   8/8 of 128, 1024 / 4096     207 / 181 at 8192, 242 / 220 at 12288, 259 / 257 at 16384
+//   4/1 of 256, 1152 / 6912     247 / 212 at 16384, 327 / 309 at 32768;  4/4 of 128, 512 / 2048  275 / 251 at 32768
+//   2/1 of 128, 512 / 2048      353 / 229 at 65536;  1/1 of 256, 1152 / 6912  805 / 341 at 131072
+// and at positions 100 and 2040 one launch takes two thirds to four fifths. The position is the device's and a recorded step covers all of
 // them, so the rule is on the longest one: no position of a decoder that takes one launch is slower for it.
 // Only where every workgroup has a CU: with fewer, all steps would be the stand-in's, whose workgroups take shares in turn (gemma3-1b
-// at 2048: 832 us a token with 255 workgroups, 990 with 128, 1680 with 64; 654 by the launches per product, 452 in one launch).
+// at 2048: 846 us a token with 255 workgroups, 983 with 128, 1672 with 64; 654 by the launches per product, 444 in one launch).
 bool hipc::resident_pays(hipc_ctx *ctx, const hipc_decoder_config &c) {
     const int64_t most = c.n_q_heads <= 4 ? 131072 / c.n_q_heads : c.n_kv_heads >= 4 ? 12288 : 8192;
     return ctx->cu_count >= (int)kResGroups && c.max_seq <= most;
