@@ -121,23 +121,32 @@ void products(int64_t M, int64_t K, int64_t N, int a_dtype, int b_dtype, bool zp
     release_all();
 }
 
-// Which products of 64x64 tiles take two groups of wavefronts a workgroup, on four CUs: tiles of 64 rows, k, the groups of an int32
-// result without and with sums over A's rows.
+// Which products of 64x64 tiles take two groups of wavefronts a workgroup, on four CUs: tiles of 64 rows, k, the groups of each result.
 void which_groups() {
     ctx.cu_count = 4;
-    const struct { int64_t tiles, K; size_t plain, sums; } cases[] = {{3, 6144, 2, 2}, {3, 6128, 1, 2}, {3, 4096, 1, 2}, {3, 4080, 1, 1}, {4, 6144, 1, 2}, {5, 6144, 1, 1}};
+    enum { kPlain, kSums, kFloats, kBytes, kBytesSums, kForms };
+    const char *const names[kForms] = {"int32", "int32 with sums", "floats", "bytes", "bytes with sums"};
+    const struct { int64_t tiles, K; size_t groups[kForms]; } cases[] = {
+        {3, 6144, {2, 2, 2, 2, 2}}, {3, 6128, {1, 2, 2, 2, 2}}, {3, 4096, {1, 2, 2, 2, 2}}, {3, 4080, {1, 1, 1, 1, 1}}, {4, 6144, {1, 2, 2, 1, 2}}, {5, 6144, {1, 1, 1, 1, 1}}};
     for (const auto &c : cases)
-        for (const bool sums : {false, true}) {
+        for (int form = 0; form < kForms; form++) {
             const int64_t M = c.tiles * 64, N = 64;
-            void *A = input((size_t)M * c.K, 3), *B = input((size_t)c.K * N, 5), *azp = input(1, 7), *bzp = input(1, 2), *Y = input((size_t)M * N * 4);
+            void *A = input((size_t)M * c.K, 3), *B = input((size_t)c.K * N, 5), *azp = input(1, 7), *bzp = input(1, 2), *scale = input(4), *Y = input((size_t)M * N * 4);
+            const float b_scale = 0.01f;
             hipc_int8_weight *w = nullptr;
             MUST(hipc_prepack_int8_b(&ctx, B, HIPC_I8, c.K, N, &w));
             ctx.tune.gemm_skinny = ctx.tune.gemm_big = 0;
+            const auto call = [&] {
+                if (form == kPlain || form == kSums) MUST(hipc_matmul_integer(&ctx, A, HIPC_U8, w, azp, form == kSums ? bzp : nullptr, Y, M));
+                else if (form == kFloats) MUST(hipc_matmul_integer_scale_bias(&ctx, A, HIPC_U8, w, azp, nullptr, scale, 0, nullptr, 0, nullptr, 0, 0, nullptr, Y, M));
+                else MUST(hipc_qlinear_matmul(&ctx, A, HIPC_U8, 0.02f, 128, w, &b_scale, 1, form == kBytes ? 0 : 3, 0.05f, 128, HIPC_U8, Y, M));
+            };
+            call();   // (the first also prepares what the handle keeps)
             const size_t before = gpu_model::reg().threads;
-            MUST(hipc_matmul_integer(&ctx, A, HIPC_U8, w, azp, sums ? bzp : nullptr, Y, M));
+            call();
             const size_t groups = (gpu_model::reg().threads - before) / 256 / (size_t)((c.tiles + 7) / 8 * 8);
-            if (groups != (sums ? c.sums : c.plain)) {
-                std::printf("FAILED: %lld tiles, k = %lld, %s: %zu groups\n", (long long)c.tiles, (long long)c.K, sums ? "with sums" : "without", groups);
+            if (groups != c.groups[form]) {
+                std::printf("FAILED: %lld tiles, k = %lld, %s: %zu groups\n", (long long)c.tiles, (long long)c.K, names[form], groups);
                 std::exit(1);
             }
             ctx.tune.gemm_skinny = ctx.tune.gemm_big = -1;
